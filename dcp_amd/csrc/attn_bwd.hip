@@ -94,6 +94,27 @@ __global__ __launch_bounds__(64) void bwd_tile_hull_kernel(const AttnBwdParams p
 // dK/dV kernel
 // ---------------------------------------------------------------------------
 constexpr int kDkvBN = 128;  // keys per workgroup: four waves of 32 keys each
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// The workgroup that holds a tile's keys visits the rows that attend to them one after the other: a
+// single row (dcp_attn_bwd), or up to kDkvMaxVisits rows of a launch that list the same kv block
+// (dcp_attn_bwd_grouped), whose dK/dV then never leave the registers between rows.  The step loop
+// runs through the visits without a break -- the first tiles of the next row are requested during
+// the last step of the one before -- so that everything it needs of a row is put into LDS once, at
+// the start: a record per visit, the tiles its keys see and the ones they see whole.  With one
+// visit per workgroup and one-head blocks of 512 tokens (8 steps a visit) the kernel takes 1044 us on
+// 32768 causal tokens of 8 heads and the sums of the replicas 150; with groups of up to 12 rows 850
+// and 23; at 64 steps a visit (four-head blocks of 1024 tokens, 65536 tokens, 32 heads) the kernel
+// takes the same time either way (8.3 ms: two workgroups per CU hide each other's prologues) and
+// the sums' 0.24 ms are saved.
+// What the kernel needs to know of one row (a "visit" of it) while it holds a kv block's keys.
+struct DkvVisit {
+  int q_begin, seqlen_q, seqlen_kv, q_entry, out_entry;
+  int ds_tile0;  // the row's first 64-key tile in the dS workspace
+  int k_row;     // the row's key position of the workgroup's first key
+  int row;
+  static constexpr int kQBegin = 0, kSeqlenQ = 1, kSeqlenKv = 2, kQEntry = 3, kOutEntry = 4, kDsTile0 = 5, kKRow = 6, kRow = 7;
+};
 
 // WRITE_DS: the kernel also leaves dS (the storage type, zero where masked) in the workspace, for
 // the dQ kernel that contracts it with K instead of recomputing S and dP (attn_bwd_ds.hip).  A
@@ -111,7 +132,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
   __shared__ __attribute__((aligned(16))) int rng_lds[2][4][BM];  // planes: start0, end0, start1, end1
   __shared__ __attribute__((aligned(16))) float lse_lds[2][BM];
   __shared__ __attribute__((aligned(16))) float delta_lds[2][BM];
-  __shared__ unsigned long long mask_lds[kBwdThreads / 64];
+  __shared__ __attribute__((aligned(16))) DkvVisit visit_lds[kDkvMaxVisits];
+  __shared__ unsigned long long mask_lds[kDkvMaxVisits][1 + kBwdThreads / 64];  // active tiles; per wave: unmasked ones
   // With D = 128 the accumulators (128 registers), K and V (64) and the products in flight do
   // not fit in 256 registers.  The compiler would spill to scratch memory, and a scratch
   // reload waits for every outstanding global load, i.e. for the tiles requested a step
@@ -126,38 +148,54 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
   const int c = lane & 31;
   const int h = lane >> 5;
 
-  // ---- which (row, kv head, key tile) ------------------------------------------
-  // the key tiles of a row share its Q/dO tiles: keep them on one XCD
-  int wg = xcd_logical_id(blockIdx.x, p.dkv_xcd_group, p.n_dkv_items);
-  if (wg < 0) return;
+  // ---- which (kv block, 128-key tile, kv head), and the rows that attend to it ------------
   // Integer division runs on the vector unit, so its (uniform) results sit in vector registers
   // and drag every address derived from them there too: each tile load then costs three vector
   // instructions to rebuild a scalar base.  readfirstlane puts the indices back on the scalar unit.
-  const int kt = __builtin_amdgcn_readfirstlane(wg % p.kv_tiles_per_row);
+  int wg = xcd_logical_id(blockIdx.x, p.dkv_xcd_group, p.n_dkv_items);
+  if (wg < 0) return;
+  const int tile_no = __builtin_amdgcn_readfirstlane(wg % p.kv_tiles_per_row);
   wg /= p.kv_tiles_per_row;
   const int kv_head = __builtin_amdgcn_readfirstlane(wg % p.n_heads_kv);
-  const int bi = __builtin_amdgcn_readfirstlane(wg / p.n_heads_kv);
-  const int b = __builtin_amdgcn_readfirstlane(p.row_order ? p.row_order[bi] : bi);
-  const int q_begin = p.cu_seqlens_q[b];
-  const int seqlen_q = p.cu_seqlens_q[b + 1] - q_begin;
-  const int seqlen_kv = p.cu_seqlens_kv[b + 1] - p.cu_seqlens_kv[b];
-  const int k0 = kt * BN;
-  if (k0 >= seqlen_kv) return;
-  // A wave whose 32 keys lie past the row's keys (seqlen_kv need not be a multiple of 128) still
-  // loads its share of every tile and meets every barrier; its arithmetic is switched off and it
-  // stores nothing.  Its K/V addresses fall back to the tile's first keys so that they stay valid.
-  const int kw = k0 + w * 32;
-  const bool has_keys = kw < seqlen_kv;
-  const int kv_or_beyond = kw + c < seqlen_kv ? kw + c : 0x7fffffff;  // this lane's key, for the range tests
-  const int kw_safe = has_keys ? kw : k0;
-  const int blk = __builtin_amdgcn_readfirstlane(kw_safe / p.block_size);
+  const int item = __builtin_amdgcn_readfirstlane(wg / p.n_heads_kv);
+  const bool grouped = p.dkv_groups != nullptr;
+  const int32_t* grp = p.dkv_groups + (grouped ? (int64_t)item * kDkvGroupInts : 0);
+  const int n_visits = grouped ? grp[5] : 1;
+  // lane v looks up visit v
+  int row = 0, k_row = tile_no * BN;  // the row, and the row's position of the tile's first key
+  if (!grouped) row = p.row_order ? p.row_order[item] : item;
+  else if (lane < n_visits) {
+    const int32_t* vis = p.dkv_visits + 2 * ((int64_t)grp[4] + lane);
+    row = vis[0];
+    k_row += vis[1] * p.block_size;
+  }
+  DkvVisit mine = {};
+  if (lane < n_visits) {
+    const int q_begin = p.cu_seqlens_q[row], kv_begin = p.cu_seqlens_kv[row];
+    mine.q_begin = q_begin;
+    mine.seqlen_q = p.cu_seqlens_q[row + 1] - q_begin;
+    mine.seqlen_kv = p.cu_seqlens_kv[row + 1] - kv_begin;
+    mine.q_entry = p.q_block_table[row];
+    mine.out_entry = p.out_block_table[row];
+    mine.ds_tile0 = kv_begin / 64 + row;
+    mine.k_row = k_row;
+    mine.row = row;
+  }
+  if (!grouped && tile_no * BN >= __builtin_amdgcn_readfirstlane(mine.seqlen_kv)) return;
+  if (w == 0 && lane < n_visits) visit_lds[lane] = mine;
+  // A wave whose 32 keys lie past the row's keys (seqlen_kv need not be a multiple of 128; a grouped
+  // launch has whole blocks only) still loads its share of every tile and meets every barrier; its
+  // arithmetic is switched off and it stores nothing.  Its K/V addresses fall back to the tile's
+  // first keys so that they stay valid.
+  const int kw_tile = tile_no * BN + w * 32;  // from the first key of the row's keys (of the block, in a group)
+  const bool has_keys = grouped || kw_tile < __builtin_amdgcn_readfirstlane(mine.seqlen_kv);
+  const int kw_safe = has_keys ? kw_tile : tile_no * BN;
+  const int blk = grouped ? 0 : __builtin_amdgcn_readfirstlane(kw_safe / p.block_size);
   const int tok0 = kw_safe - blk * p.block_size;
+  const int64_t table_at = grouped ? 0 : (int64_t)__builtin_amdgcn_readfirstlane(row) * p.max_kv_blocks + blk;
   const int group = p.n_heads_q / p.n_heads_kv;
   const int64_t q_row_stride = (int64_t)p.n_heads_q * D;
-  const int q_slot = p.q_block_table[b];
-  const int o_slot = p.out_block_table[b];
-  const int n_q_tiles = (seqlen_q + BM - 1) / BM;  // rows past seqlen_q stay inside the padded block
-  const int64_t kv_tile_off = (int64_t)p.kv_block_table[(int64_t)b * p.max_kv_blocks + blk] * p.kv_slot_stride +
+  const int64_t kv_tile_off = (int64_t)(grouped ? grp[0] : p.kv_block_table[table_at]) * p.kv_slot_stride +
                               (int64_t)tok0 * p.kv_token_stride + (int64_t)kv_head * D;
 
   // ---- K, V of this wave's 32 keys as B operands (lane = key, slots = dims) ------
@@ -174,6 +212,34 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
     for (int j = 0; j < VL; ++j) v_park[w][j][lane] = *reinterpret_cast<const u32x4*>(vp + (KS - VL + j) * 16);
   }
 
+  // ---- per visit: which 64-query tiles of its row see the keys (the same for every head) ------
+  // bit qt of `act`: some query of tile qt sees some of the workgroup's 128 keys; of the wave's
+  // `unm`: every query of it sees all of the wave's 32.  Taken once from the per-tile hulls, so the
+  // loop never waits for a table.  (No query sees a key past the row's last one.)  The waves share
+  // the visits out among them.
+  for (int v = w; v < n_visits; v += kBwdThreads / 64) {
+    const int vrow = __builtin_amdgcn_readlane(row, v), k0 = __builtin_amdgcn_readlane(mine.k_row, v);
+    const int n_tiles = (__builtin_amdgcn_readlane(mine.seqlen_q, v) + BM - 1) / BM;
+    i32x4 h0 = {0x7fffffff, 0, 0x7fffffff, 0}, h1 = {0x7fffffff, 0, 0x7fffffff, 0};
+    if (lane < n_tiles) {
+      const i32x4* hu = reinterpret_cast<const i32x4*>(p.hull + ((int64_t)vrow * p.q_tiles_per_row + lane) * 8);
+      h0 = hu[0];
+      h1 = hu[1];
+    }
+    const unsigned long long a = __ballot((k0 < h0[1] && k0 + BN > h0[0]) || (k0 < h0[3] && k0 + BN > h0[2]));
+    unsigned long long u[kBwdThreads / 64];
+#pragma unroll
+    for (int i = 0; i < kBwdThreads / 64; ++i) {
+      const int kw = k0 + i * 32;
+      u[i] = __ballot((h1[0] <= kw && kw + 32 <= h1[1]) || (h1[2] <= kw && kw + 32 <= h1[3]));
+    }
+    if (lane == 0) {
+      mask_lds[v][0] = a;
+#pragma unroll
+      for (int i = 0; i < kBwdThreads / 64; ++i) mask_lds[v][1 + i] = u[i];
+    }
+  }
+
   // dK^T and dV^T of this wave's keys: (all dims) x (32 keys), complete when the loop ends
   f32x16 dk_acc[DT], dv_acc[DT];
 #pragma unroll
@@ -184,37 +250,13 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
       dv_acc[dt][i] = 0.0f;
     }
 
-  const int32_t* hull_row = p.hull + (int64_t)b * p.q_tiles_per_row * 8;
   // loop-invariant per-lane pieces of the addresses used in the loop
   const int row_rd = Tile::row_base(c, h);
   const int col_rd = Tile::col_base(lane, true);
-  const uint16_t* q_base = reinterpret_cast<const uint16_t*>(p.q) + (int64_t)q_slot * p.q_slot_stride;
-  const uint16_t* do_base = reinterpret_cast<const uint16_t*>(p.dout) + (int64_t)o_slot * p.out_slot_stride;
   const uint32_t tiles_at = lds_address(&tiles[0][0]);
-
-  // ---- which 64-query tiles of the row see this wave's keys (the same for every head) ------
-  // bit qt of `act_w`: some row of tile qt sees some of the wave's keys; of `unm_w`: every row sees
-  // all of them.  Taken once from the per-tile hulls, so the loop never waits for a table.  The
-  // workgroup walks the tiles any of its waves needs (`act_mask`); a wave sits out the others.
-  unsigned long long act_w, unm_w;
-  {
-    bool a = false, u = false;
-    if (has_keys && lane < n_q_tiles) {
-      const int32_t* hu = hull_row + lane * 8;
-      a = (kw < hu[1] && kw + 32 > hu[0]) || (kw < hu[3] && kw + 32 > hu[2]);
-      u = (hu[4] <= kw && kw + 32 <= hu[5]) || (hu[6] <= kw && kw + 32 <= hu[7]);
-    }
-    act_w = __ballot(a);
-    unm_w = __ballot(u);
-    if (lane == 0) mask_lds[w] = act_w;
-  }
   __syncthreads();
-  const unsigned long long act = mask_lds[0] | mask_lds[1] | mask_lds[2] | mask_lds[3];
-  const uint32_t act_lo = __builtin_amdgcn_readfirstlane((uint32_t)act);
-  const uint32_t act_hi = __builtin_amdgcn_readfirstlane((uint32_t)(act >> 32));
-  const unsigned long long act_mask = ((unsigned long long)act_hi << 32) | act_lo;
 
-  // Everything step (head, qt) reads is requested a step ahead, straight into LDS stage st
+  // Everything step (visit, head, qt) reads is requested a step ahead, straight into LDS stage st
   // and with nothing held in registers meanwhile: the Q and dO tiles, and one value per
   // query of the range planes (waves 0 and 1), lse (wave 2) and delta (wave 3).  Queries
   // past seqlen_q read the last valid query's values; they are masked where they are used.
@@ -225,66 +267,99 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
   constexpr int NL = 2 * Tile::LPW;
   const uint64_t group_step = uniform64(Tile::group_global_step(q_row_stride));
   static_assert(NL <= KS, "a sub-step carries half of the tile loads, one per two k-steps of its first phase");
-  auto request_tile = [&](int idx, int head, int qt, int st) {
-    const int64_t off = (int64_t)qt * BM * q_row_stride + (int64_t)head * D;
-    const bool is_do = idx >= Tile::LPW;
-    Tile::load_group(tiles_at + (2 * st + (is_do ? 1 : 0)) * (Tile::SIZE * 2), (is_do ? do_base : q_base) + off, goff0,
-                     q_row_stride, w, is_do ? idx - Tile::LPW : idx);
-  };
   // Per-query values of a step, two dword loads per wave and no branches: wave 0 requests the
   // first range's starts and ends, wave 1 the second range's (the first's again, into planes
   // nobody reads, when there is one range), wave 2 the LSEs and wave 3 the deltas (each twice,
   // to the same place).  What depends on the wave's role is fixed here, once.
   const bool role_rng = w < 2, role_lse = w == 2;
   const int sc_plane = p.n_ranges == 2 ? 2 * w : 0;
-  const char* sc_base0 = role_rng   ? reinterpret_cast<const char*>(p.attn_range + (int64_t)sc_plane * p.total_q + q_begin)
-                         : role_lse ? reinterpret_cast<const char*>(p.lse2 + (int64_t)q_begin * p.n_heads_q)
-                                    : reinterpret_cast<const char*>(p.delta + (int64_t)q_begin * p.n_heads_q);
+  const char* sc_base0 = role_rng   ? reinterpret_cast<const char*>(p.attn_range + (int64_t)sc_plane * p.total_q)
+                         : role_lse ? reinterpret_cast<const char*>(p.lse2)
+                                    : reinterpret_cast<const char*>(p.delta);
   const int64_t sc_head_bytes = role_rng ? 0 : 4;
   const int64_t sc_second_bytes = role_rng ? (int64_t)p.total_q * 4 : 0;
   const int sc_query_bytes = role_rng ? 4 : p.n_heads_q * 4;
   const uint32_t sc_at0 = role_rng ? rng_at + (2 * w * BM) * 4 : role_lse ? lse_at : delta_at;
   const uint32_t sc_at_stage = role_rng ? 4 * BM * 4 : BM * 4, sc_at_second = role_rng ? BM * 4 : 0;
-  auto request_scalars = [&](int head, int qt, int st) {
-    const int ql = min(qt * BM + lane, seqlen_q - 1);
-    const char* base = sc_base0 + head * sc_head_bytes;
-    const uint32_t at = sc_at0 + st * sc_at_stage, voff = (uint32_t)(ql * sc_query_bytes);
-    load_async_dword(at, voff, base);
-    load_async_dword(at + sc_at_second, voff, base + sc_second_bytes);
-  };
 
+  // What the loop knows of the visit whose tiles are requested next, ...
+  const uint16_t *q_base = nullptr, *do_base = nullptr;
+  const char* sc_base = nullptr;
+  int req_seqlen_q = 0;
+  auto visit_field = [&](int v, int i) { return __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(&visit_lds[v])[i]); };
+  // (kernel arguments that only a change of visit needs are loaded then, through an opaque pointer:
+  // kept through the loop they push its own scalars out of the scalar registers)
+  auto begin_requests = [&](int v) {
+    KernArgs<AttnBwdParams>& p = fresh_kernel_args<AttnBwdParams>();
+    q_base = reinterpret_cast<const uint16_t*>(p.q) + (int64_t)visit_field(v, DkvVisit::kQEntry) * p.q_slot_stride;
+    do_base = reinterpret_cast<const uint16_t*>(p.dout) + (int64_t)visit_field(v, DkvVisit::kOutEntry) * p.out_slot_stride;
+    sc_base = sc_base0 + (int64_t)visit_field(v, DkvVisit::kQBegin) * sc_query_bytes;
+    req_seqlen_q = visit_field(v, DkvVisit::kSeqlenQ);
+  };
+  // ... and of the one whose step is multiplied.
+  int seqlen_q = 0, kv_or_beyond = 0;  // kv_or_beyond: this lane's key, for the range tests
+  unsigned long long unm_w = 0;
   // dS pieces (WRITE_DS).  The workspace holds the rows one after another; row b starts at 64-key
   // tile cu_seqlens_kv[b] / 64 + b (room for a last, partial tile of every row before it) and is laid
   // out [head][32-query chunk][64-key tile]: the pieces that a wave of the dQ kernel reads one after
   // another lie one after another (ordered by key tile first, they were 4 MiB apart at 32 heads and
   // 1024-token blocks, every one in a memory page of its own).  ds_lane: the lane's 16 bytes within a
-  // [key][query half] plane of a piece.
-  const int ds_row_tiles = (seqlen_kv + 63) / 64;
-  const uint64_t ds_row_base = ((uint64_t)(p.cu_seqlens_kv[b] / 64) + b) * p.n_heads_q * p.subs_per_row;
-  const int ds_tile_local = 2 * kt + (w >> 1);
-  const uint64_t ds_chunk_bytes = has_keys ? (uint64_t)ds_row_tiles << 12 : 4096;  // from a 32-query chunk to the next
+  // [key][query half] plane of a piece.  (A wave whose 32 keys lie past the row's last key has no
+  // piece -- its 64-key half tile would be the next row's first, or lie past the end of the
+  // workspace -- and writes its zeros into a spare piece behind the last one instead, with a row of
+  // no tiles: no branch around the stores.)
+  uint64_t ds_visit = 0;
+  uint32_t ds_row_tiles = 0;  // pieces from a 32-query chunk to the next
   const int ds_lane = (w & 1) * 128 + 2 * c + h;
+  auto begin_visit = [&](int v) {
+    KernArgs<AttnBwdParams>& p = fresh_kernel_args<AttnBwdParams>();
+    const int seqlen_kv = visit_field(v, DkvVisit::kSeqlenKv), kw = visit_field(v, DkvVisit::kKRow) + w * 32;
+    seqlen_q = visit_field(v, DkvVisit::kSeqlenQ);
+    kv_or_beyond = kw + c < seqlen_kv ? kw + c : 0x7fffffff;
+    unm_w = uniform64(mask_lds[v][1 + w]);
+    if constexpr (WRITE_DS) {
+      ds_row_tiles = has_keys ? (seqlen_kv + 63) / 64 : 0;
+      const uint64_t piece = (uint64_t)visit_field(v, DkvVisit::kDsTile0) * p.n_heads_q * p.subs_per_row +
+                             (uint64_t)(kv_head * group) * p.subs_per_row * ds_row_tiles + (kw >> 6);
+      ds_visit = uniform64(reinterpret_cast<uint64_t>(p.ds) + ((has_keys ? piece : (uint64_t)p.ds_pieces) << 12));
+    }
+  };
+  auto next_active = [&](int v) {  // the first visit from v on with an active tile, or n_visits
+    while (v < n_visits && uniform64(mask_lds[v][0]) == 0) ++v;
+    return v;
+  };
+  auto request_scalars = [&](int head, int qt, int st) {
+    const int ql = min(qt * BM + lane, req_seqlen_q - 1);
+    const char* base = sc_base + head * sc_head_bytes;
+    const uint32_t at = sc_at0 + st * sc_at_stage, voff = (uint32_t)(ql * sc_query_bytes);
+    load_async_dword(at, voff, base);
+    load_async_dword(at + sc_at_second, voff, base + sc_second_bytes);
+  };
 
-  // steps: (q head of the group) x (active 64-query tile)
-  int hg = 0;
-  unsigned long long rem = act_mask;  // tiles of head hg still to do
+  // steps: (visit) x (q head of the group) x (active 64-query tile)
+  int visit = next_active(0), hg = 0;
+  unsigned long long act_mask = 0, rem = 0;  // active tiles of the visit; tiles of head hg still to do
   int st = 0;
-  if (act_mask != 0 && group > 0) {
-    request_scalars(kv_head * group, __builtin_ctzll(rem), 0);
+  if (visit < n_visits) {
+    act_mask = rem = uniform64(mask_lds[visit][0]);
+    begin_requests(visit);
+    begin_visit(visit);
+    const int qt = __builtin_ctzll(rem), head = kv_head * group;
+    request_scalars(head, qt, 0);
+    const int64_t off = (int64_t)qt * BM * q_row_stride + (int64_t)head * D;
 #pragma unroll
-    for (int i = 0; i < NL; ++i) request_tile(i, kv_head * group, __builtin_ctzll(rem), 0);
+    for (int i = 0; i < NL; ++i) {
+      const bool is_do = i >= Tile::LPW;
+      Tile::load_group(tiles_at + (is_do ? 1 : 0) * (Tile::SIZE * 2), (is_do ? do_base : q_base) + off, goff0, q_row_stride, w,
+                       is_do ? i - Tile::LPW : i);
+    }
   }
   if constexpr (WRITE_DS) wait_loads();  // (the wait at the top of a step counts on two stores behind the tile loads)
-  while (act_mask != 0 && hg < group) {
+  while (visit < n_visits) {
     const int qt = __builtin_ctzll(rem);
     const bool unmasked = (unm_w >> qt) & 1;
     rem &= rem - 1;
-    int hg_next = hg;
-    if (rem == 0) {
-      rem = act_mask;
-      ++hg_next;
-    }
-    const bool more = hg_next < group;
+    int hg_next = hg, visit_next = visit;
 
     if constexpr (WRITE_DS) {
       // The tiles and scalars of this step were requested before the previous step's last two
@@ -296,12 +371,24 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();  // this step's tiles and scalars are in LDS; the previous step is fully consumed
     }
+    if (rem == 0) {
+      rem = act_mask;
+      if (++hg_next == group) {
+        visit_next = next_active(visit + 1);
+        if (visit_next < n_visits) {
+          hg_next = 0;
+          act_mask = rem = uniform64(mask_lds[visit_next][0]);
+          begin_requests(visit_next);
+        }
+      }
+    }
+    const bool more = visit_next < n_visits;
     // The next step's tiles are requested one load at a time between the matrix instructions of
     // the first phases below: a burst here would hold the wave at its last load until the memory
     // pipeline has taken them all.  They are issued unconditionally, so that the step has no
     // branches around them: the last step requests its own tiles once more, into the stage nobody
     // reads any more.
-    const int head_next = more ? kv_head * group + hg_next : kv_head * group + hg;
+    const int head_next = kv_head * group + (more ? hg_next : hg);
     const int qt_next = more ? __builtin_ctzll(rem) : qt;
     const uint16_t* q_lds = tiles[2 * st];
     const uint16_t* do_lds = tiles[2 * st + 1];
@@ -312,15 +399,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
     const uint64_t next_do = uniform64(reinterpret_cast<uint64_t>(do_base + off_next));
     const uint32_t next_at = __builtin_amdgcn_readfirstlane(Tile::group_lds_at(tiles_at + 2 * (st ^ 1) * (Tile::SIZE * 2), w, 0));
     // where this step's dS goes: the pieces of (this wave's 64-key half tile, head, the step's two 32-query sub-tiles)
-    // (a wave whose 32 keys lie past the row's last key has no piece -- its 64-key half tile would be
-    // the next row's first, or lie past the end of the workspace -- and writes its zeros into two
-    // spare pieces behind the last one instead: no branch around the stores)
-    const uint64_t ds_step =
-        WRITE_DS ? uniform64(reinterpret_cast<uint64_t>(p.ds) +
-                             (((has_keys ? ds_row_base + ((uint64_t)(kv_head * group + hg) * p.subs_per_row + 2 * qt) * ds_row_tiles + ds_tile_local
-                                         : (uint64_t)p.ds_pieces))
-                              << 12))
-                 : 0;
+    const uint64_t ds_step = WRITE_DS ? uniform64(ds_visit + (((uint64_t)(hg * p.subs_per_row + 2 * qt) * ds_row_tiles) << 12)) : 0;
+    const uint64_t ds_chunk_bytes = (uint64_t)ds_row_tiles << 12;
 
     // One sub-step = this wave's 32 keys against 32 of the step's 64 queries (QI = 0, 1).
     // (A real loop, not unrolled: one copy of the body keeps the register allocation of a single
@@ -339,7 +419,6 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
         // the four queries of an accumulator register group are consecutive: their range planes
         // come in 16-byte reads, requested together before the comparisons.  With one range the
         // second range's planes hold the first's again (see request_scalars): the union is the same.
-        typedef int i32x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           i32x4 rs[4];
@@ -466,15 +545,32 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
     __builtin_amdgcn_s_setprio(kPrioVector);
     st ^= 1;
     hg = hg_next;
+    if (visit_next != visit) {
+      visit = visit_next;
+      if (visit < n_visits) begin_visit(visit);
+    }
   }
 
   // ---- dK and dV of the wave's keys are complete: scale, round, store ---------------------
   wait_loads();  // the last step's (unused) requests must land before the workgroup's LDS is released
   if (!has_keys) return;
-  const int64_t off = (int64_t)p.dkv_block_table[(int64_t)b * p.max_kv_blocks + blk] * p.dkv_slot_stride +
-                      (int64_t)(tok0 + c) * p.dkv_token_stride + (int64_t)kv_head * D + 4 * h;
-  uint16_t* dv_dst = reinterpret_cast<uint16_t*>(p.dv) + off;
-  uint16_t* dk_dst = reinterpret_cast<uint16_t*>(p.dk) + off;
+  // a group's result goes to a slot of dk/dv or, where nothing else is added to it, to the caller's
+  // unpadded tensor, of which only the block's own tokens may be written
+  KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
+  int entry, in_unpadded = 0;
+  if (args.dkv_groups != nullptr) {
+    const int32_t* grp = args.dkv_groups + (int64_t)item * kDkvGroupInts;
+    entry = grp[1];
+    in_unpadded = grp[3];
+    if (tok0 + c >= grp[2]) return;
+  } else {
+    entry = args.dkv_block_table[(int64_t)visit_field(0, DkvVisit::kRow) * args.max_kv_blocks + blk];
+  }
+  const int64_t off = (int64_t)entry * (in_unpadded ? args.dkv2_entry_stride : args.dkv_slot_stride) +
+                      (int64_t)(tok0 + c) * (in_unpadded ? args.dkv2_token_stride : args.dkv_token_stride) + (int64_t)kv_head * D + 4 * h;
+  uint16_t* dv_dst = reinterpret_cast<uint16_t*>(in_unpadded ? args.dv2 : args.dv) + off;
+  uint16_t* dk_dst = reinterpret_cast<uint16_t*>(in_unpadded ? args.dk2 : args.dk) + off;
+  const float scale = args.scale;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -482,8 +578,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
       const int i = 4 * g;
       u32x2 v4 = {pack2<DTYPE>(dv_acc[dt][i], dv_acc[dt][i + 1]), pack2<DTYPE>(dv_acc[dt][i + 2], dv_acc[dt][i + 3])};
       *reinterpret_cast<u32x2*>(dv_dst + dt * 32 + 8 * g) = v4;
-      u32x2 k4 = {pack2<DTYPE>(dk_acc[dt][i] * p.scale, dk_acc[dt][i + 1] * p.scale),
-                  pack2<DTYPE>(dk_acc[dt][i + 2] * p.scale, dk_acc[dt][i + 3] * p.scale)};
+      u32x2 k4 = {pack2<DTYPE>(dk_acc[dt][i] * scale, dk_acc[dt][i + 1] * scale),
+                  pack2<DTYPE>(dk_acc[dt][i + 2] * scale, dk_acc[dt][i + 3] * scale)};
       *reinterpret_cast<u32x2*>(dk_dst + dt * 32 + 8 * g) = k4;
     }
 }
@@ -856,7 +952,17 @@ extern "C" size_t dcp_attn_bwd_workspace_bytes(int batch, int total_q, int block
          (bwd_fused_available() ? bwd_fused_extra_workspace_bytes(batch, block_size, n_heads_q, head_dim) : 0);
 }
 
-// Both entry points: argument checks, workspace carving, the four launches.
+// The groups of rows a dcp_attn_bwd_grouped call names.
+struct DkvGrouping {
+  const int32_t* groups;
+  int n_groups;
+  const int32_t* visits;
+  void* dk2;
+  void* dv2;
+  int64_t entry_stride, token_stride;
+};
+
+// All entry points: argument checks, workspace carving, the launches.
 static int attn_bwd_launch(const void* dout, const void* q, const void* k, const void* v,
                            const void* out, const float* lse, void* dq, void* dk, void* dv,
                            void* workspace, size_t workspace_bytes, const int32_t* cu_seqlens_q,
@@ -869,7 +975,8 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
                            int64_t kv_token_stride, int64_t dkv_slot_stride,
                            int64_t dkv_token_stride, int64_t q_slot_stride, int64_t out_slot_stride,
                            int64_t dq_slot_stride, int64_t lse_head_stride, int64_t lse_slot_stride,
-                           int64_t total_kv, float softmax_scale, int dtype, void* stream, bool allow_fused) {
+                           int64_t total_kv, float softmax_scale, int dtype, void* stream, bool allow_fused,
+                           const DkvGrouping* grouping = nullptr) {
   if (dtype != DCP_DTYPE_BF16 && dtype != DCP_DTYPE_FP16)
     return fail(DCP_ERR_UNSUPPORTED, "attn_bwd: dtype %d unsupported (bf16 and fp16 only)", dtype);
   if (head_dim != 64 && head_dim != 128)
@@ -904,7 +1011,15 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
   // partial sums; otherwise the two-kernel one, which needs the base workspace only.
   const size_t base = bwd_base_workspace_bytes(batch, total_q, block_size, n_heads_q);
   const size_t extra = bwd_fused_extra_workspace_bytes(batch, block_size, n_heads_q, head_dim);
-  const bool fused = allow_fused && head_dim == 128 && bwd_fused_available() && workspace_bytes >= base + extra;
+  if (grouping) {
+    DCP_REQUIRE(grouping->groups && grouping->visits && grouping->n_groups > 0, "attn_bwd_grouped: no groups");
+    DCP_REQUIRE(block_size % kDkvBN == 0, "attn_bwd_grouped: block_size %d must be a multiple of %d", block_size, kDkvBN);
+    DCP_REQUIRE(!grouping->dk2 == !grouping->dv2 && (!grouping->dk2 || (grouping->entry_stride > 0 && grouping->token_stride > 0 &&
+                grouping->entry_stride % 4 == 0 && grouping->token_stride % 4 == 0)) &&
+                    ((reinterpret_cast<uintptr_t>(grouping->dk2) | reinterpret_cast<uintptr_t>(grouping->dv2)) & 7) == 0,
+                "attn_bwd_grouped: the unpadded dk/dv must be 8-byte aligned, with strides that are multiples of 4 elements");
+  }
+  const bool fused = allow_fused && !grouping && head_dim == 128 && bwd_fused_available() && workspace_bytes >= base + extra;
   // The backward through dS in memory where it is selected, the caller said how many keys the rows
   // have in all and the workspace holds the dS pieces.
   const size_t ds_bytes = bwd_ds_workspace_bytes(total_kv, batch, block_size, n_heads_q);
@@ -974,8 +1089,14 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
   p.lse_slot_stride = lse_slot_stride;
   p.q_tiles_per_row = (block_size + kBwdBM - 1) / kBwdBM;
   p.dq_tiles_per_row = (block_size + kDqBM - 1) / kDqBM;
-  p.kv_tiles_per_row = (int)(((int64_t)max_kv_blocks * block_size + kDkvBN - 1) / kDkvBN);
-  p.n_dkv_items = (int64_t)batch * n_heads_kv * p.kv_tiles_per_row;
+  p.dkv_groups = grouping ? grouping->groups : nullptr;
+  p.dkv_visits = grouping ? grouping->visits : nullptr;
+  p.dk2 = grouping ? grouping->dk2 : nullptr;
+  p.dv2 = grouping ? grouping->dv2 : nullptr;
+  p.dkv2_entry_stride = grouping ? grouping->entry_stride : 0;
+  p.dkv2_token_stride = grouping ? grouping->token_stride : 0;
+  p.kv_tiles_per_row = grouping ? block_size / kDkvBN : (int)(((int64_t)max_kv_blocks * block_size + kDkvBN - 1) / kDkvBN);
+  p.n_dkv_items = (int64_t)(grouping ? grouping->n_groups : batch) * n_heads_kv * p.kv_tiles_per_row;
   p.n_dq_items = (int64_t)batch * n_heads_q * p.dq_tiles_per_row;
   p.dkv_xcd_group = p.kv_tiles_per_row;
   p.dq_xcd_group = p.dq_tiles_per_row * (n_heads_q / n_heads_kv);
@@ -1031,6 +1152,32 @@ extern "C" int dcp_attn_bwd_strided(const void* dout, const void* q, const void*
                          n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride, dkv_slot_stride,
                          dkv_token_stride, q_slot_stride, out_slot_stride, dq_slot_stride, lse_head_stride,
                          lse_slot_stride, total_kv, softmax_scale, dtype, stream, true);
+}
+
+extern "C" int dcp_attn_bwd_grouped(const void* dout, const void* q, const void* k, const void* v,
+                                    const void* out, const float* lse, void* dq, void* dk, void* dv,
+                                    void* workspace, size_t workspace_bytes, const int32_t* cu_seqlens_q,
+                                    const int32_t* cu_seqlens_kv, const int32_t* attn_range, int n_ranges,
+                                    const int32_t* q_block_table, const int32_t* kv_block_table,
+                                    const int32_t* out_block_table, const int32_t* dq_block_table,
+                                    const int32_t* dkv_block_table, const int32_t* row_order, int batch,
+                                    int max_kv_blocks, int total_q, int block_size, int n_heads_q,
+                                    int n_heads_kv, int head_dim, int64_t kv_slot_stride,
+                                    int64_t kv_token_stride, int64_t dkv_slot_stride,
+                                    int64_t dkv_token_stride, int64_t q_slot_stride, int64_t out_slot_stride,
+                                    int64_t dq_slot_stride, int64_t lse_head_stride, int64_t lse_slot_stride,
+                                    int64_t total_kv, const int32_t* dkv_groups, int n_groups,
+                                    const int32_t* dkv_visits, void* dk_unpadded, void* dv_unpadded,
+                                    int64_t unpadded_entry_stride, int64_t unpadded_token_stride,
+                                    float softmax_scale, int dtype, void* stream) {
+  const DkvGrouping grouping = {dkv_groups, n_groups, dkv_visits, dk_unpadded, dv_unpadded, unpadded_entry_stride,
+                                unpadded_token_stride};
+  return attn_bwd_launch(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
+                         cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table,
+                         dq_block_table, dkv_block_table, row_order, batch, max_kv_blocks, total_q, block_size,
+                         n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride, dkv_slot_stride,
+                         dkv_token_stride, q_slot_stride, out_slot_stride, dq_slot_stride, lse_head_stride,
+                         lse_slot_stride, total_kv, softmax_scale, dtype, stream, true, &grouping);
 }
 
 extern "C" int dcp_attn_bwd_select(int mode) { return bwd_select(mode); }

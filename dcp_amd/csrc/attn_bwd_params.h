@@ -56,13 +56,20 @@ struct AttnBwdParams {
   int64_t dq_slot_stride;
   int64_t lse_head_stride;
   int64_t lse_slot_stride;
+  // the dK/dV kernel over groups of rows (null: one row at a time, dK/dV into dkv_block_table's slots)
+  const int32_t* dkv_groups;  // [n_dkv_groups][kDkvGroupInts], see dcp_attn_bwd_grouped
+  const int32_t* dkv_visits;  // [..][2]: row, index of the block in the row's kv_block_table
+  void* dk2;                  // where groups marked unpadded go
+  void* dv2;
+  int64_t dkv2_entry_stride;
+  int64_t dkv2_token_stride;
   int dkv_xcd_group;     // dK/dV work items sharing one Q/dO stream (the key tiles of a row)
   int dq_xcd_group;      // dQ work items sharing one K/V stream
   int64_t n_dkv_items;   // batch * n_heads_kv * kv_tiles_per_row
   int64_t n_dq_items;    // batch * n_heads_q * dq_tiles_per_row
   int q_tiles_per_row;   // ceil(block_size / 64): query tiles of the dK/dV kernel
   int dq_tiles_per_row;  // ceil(block_size / 128): query tiles of the dQ kernel
-  int kv_tiles_per_row;  // ceil(max_kv_blocks * block_size / 128): key tiles of the dK/dV kernel
+  int kv_tiles_per_row;  // key tiles of a dK/dV row (ceil(max_kv_blocks * block_size / 128)), or of a group's block
   float scale;
   float scale_log2;
 };
@@ -75,6 +82,8 @@ constexpr int kPrioMatrix = 2, kPrioVector = 0;
 constexpr int kBwdBM = 64;
 constexpr int kBwdBN = 64;
 constexpr int kBwdThreads = 256;
+constexpr int kDkvGroupInts = 8;
+constexpr int kDkvMaxVisits = DCP_ATTN_BWD_MAX_VISITS;
 constexpr int kTicketInts = 16;  // one counter per XCD (the rest unused)
 
 // The backward through dS in memory: prepare (hulls, -delta, lse2), the dK/dV kernel writing dS, the

@@ -307,6 +307,7 @@ def _flash_attn_varlen_backward(
     workspace: Optional[torch.Tensor] = None,
     row_order: Optional[torch.Tensor] = None,
     block_size: Optional[int] = None,
+    dkv_groups: Optional[tuple] = None,
 ):
     """Writes dQ into ``dq`` (slots ``dq_block_table``) and dK/dV into
     ``dk``/``dv`` (one slot per (row, kv block), ``dkv_block_table``).
@@ -325,6 +326,9 @@ def _flash_attn_varlen_backward(
     each be the unpadded tensor, addressed by token offsets in its block table.  q and dout must
     then be readable for 64 tokens past the last row's queries (the dK/dV kernel loads whole
     64-query tiles).  dk/dv are always paged.
+    ``dkv_groups`` (extension): ``(groups, visits, dk_unpadded, dv_unpadded)`` -- dK/dV of a kv block
+    added over groups of rows in the kernel (``dcp_attn_bwd_grouped`` in ``dcp_hip.h`` describes the
+    two int32 tables ``[n, 8]`` and ``[m, 2]``); the unpadded tensors are ``[tokens, n_heads_kv, D]``.
     """
     _check_plain(dropout_p, causal, window_size_left, window_size_right, softcap, alibi_slopes)
     if attn_range is None or q_block_table is None or kv_block_table is None \
@@ -353,6 +357,8 @@ def _flash_attn_varlen_backward(
                   dict(kv_block_table=kv_block_table, dkv_block_table=dkv_block_table))
     if softmax_scale is None:
         softmax_scale = head_dim ** (-0.5)
+    if dkv_groups is not None and head_dim not in KERNEL_HEAD_DIMS:
+        raise ValueError(f"dkv_groups: head size {head_dim} is not one of {KERNEL_HEAD_DIMS}")
     if head_dim not in KERNEL_HEAD_DIMS:
         # as in the forward: zero-padded copies at the next kernel head size; the gradients'
         # padded columns come out zero and are dropped, slots this call leaves alone are carried
@@ -378,8 +384,17 @@ def _flash_attn_varlen_backward(
     ws_bytes = workspace.numel() * workspace.element_size()
     if not workspace.is_contiguous() or ws_bytes < need:
         raise ValueError(f"workspace must be contiguous with at least {need} bytes")
+    name, grouping = "dcp_attn_bwd_strided", ()
+    if dkv_groups is not None:
+        groups, visits, dk_unpadded, dv_unpadded = dkv_groups
+        if groups.dim() != 2 or groups.shape[1] != 8 or visits.dim() != 2 or visits.shape[1] != 2:
+            raise ValueError(f"dkv_groups: tables must be [n, 8] and [m, 2], got {tuple(groups.shape)}, {tuple(visits.shape)}")
+        unpadded_entry, unpadded_token = _kv_strides(dk_unpadded, dv_unpadded, "unpadded dk/dv")
+        name = "dcp_attn_bwd_grouped"
+        grouping = (_i32(groups, "dkv_groups").data_ptr(), groups.shape[0], _i32(visits, "dkv_visits").data_ptr(),
+                    dk_unpadded.data_ptr(), dv_unpadded.data_ptr(), unpadded_entry, unpadded_token)
     _lib.call(
-        "dcp_attn_bwd_strided",
+        name,
         dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
         softmax_lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
         workspace.data_ptr(), ws_bytes,
@@ -396,6 +411,6 @@ def _flash_attn_varlen_backward(
         n_heads_q, n_heads_kv, head_dim,
         kv_slot_stride, kv_token_stride, dkv_slot_stride, dkv_token_stride,
         q_entry, out_entry, dq_entry, lse_head_stride, lse_entry, int(total_k or 0),
-        float(softmax_scale), dtype_code(q.dtype), _stream(),
+        *grouping, float(softmax_scale), dtype_code(q.dtype), _stream(),
     )
     return dq, dk, dv, None

@@ -1,0 +1,167 @@
+"""Which dK/dV replicas of a plan the backward kernel adds up itself.
+
+A plan gives every (attention row, kv block) pair a private dK/dV block and adds the replicas of a
+kv block with ``SumInstr`` ops afterwards (reference ``dcp/core/scheduler.py:1365-1700,1764-1940``).
+The key-outer kernel holds dK/dV of 128 keys in registers, so rows of one launch that attend to the
+same kv block can be visited one after the other by the workgroup that holds its keys
+(``dcp_attn_bwd_grouped``): K and V are loaded once, the replicas are added in fp32 without being
+rounded and written first, and a sum whose sources have all been added that way is not run.
+
+``analyse`` looks at the instruction list only and changes nothing in the plan.  It takes replicas
+together that one ``SumInstr`` op reads and nothing else does; what that op still has to add are the
+groups' first slots and whatever other sources it has (blocks received from other devices, ...).
+"""
+
+from __future__ import annotations
+
+from collections import Counter, defaultdict
+from dataclasses import dataclass, field
+from typing import Dict, List, Optional, Set, Tuple
+
+from dcp_amd.core.instructions import (
+    AttnBackwardInstr,
+    AttnReductionInstr,
+    BufferBlock,
+    BufferType,
+    CommLaunchInstr,
+    CommType,
+    ExecutionPlan,
+    MemcpyInstr,
+    SumInstr,
+)
+from dcp_amd.runtime.flash_attention.direct import DirectPlan
+
+MAX_VISITS = 32  # DCP_ATTN_BWD_MAX_VISITS
+
+
+@dataclass
+class Group:
+    """Rows of one launch that attend to one kv block: ``(row, position in the row's kv blocks)``."""
+
+    visits: List[Tuple[int, int]]
+    dst: BufferBlock  # a BUFFER_dKV slot, or the LOCAL_dKV block the sum would have been scattered to
+
+
+@dataclass
+class DkvGroups:
+    # AttnBackwardInstr -> its groups, the ones with the most visits first
+    groups: Dict[int, List[Group]] = field(default_factory=dict)
+    # SumInstr -> positions of the ops that are not run
+    skip_ops: Dict[int, Set[int]] = field(default_factory=dict)
+    # SumInstr -> op position -> the sources the op still adds
+    sources: Dict[int, Dict[int, List[BufferBlock]]] = field(default_factory=dict)
+
+
+def visits_per_group(n_visits: int, tiles_per_visit: int, n_slots: int) -> int:
+    """How many rows a workgroup may visit.  Longer groups save prologues, K/V loads and replicas;
+    but a launch is as long as its longest workgroup, and too few of them leave the device idle: with
+    two of the longest groups' work per workgroup slot of the device, handed out longest first, the
+    slots end within a fraction of a group of each other.  Measured, dK/dV kernel plus replica sums
+    (us) with 0.5 / 1 / 2 / 4 / 8 such groups per slot and with one row per group: 32768 tokens, 8
+    heads in one-head blocks of 512 tokens 864 / 904 / 873 / 881 / 937, 1193; 16384 tokens, 16 heads,
+    blocks of 256 931 / 942 / 949 / 973 / 1012, 1690; 65536 tokens, 32 heads in four-head blocks of 1024
+    8282 / 8226 / 8330 / 8340 / 8374, 8544."""
+    return max(1, min(MAX_VISITS, int(n_visits * tiles_per_visit / n_slots / 2)))
+
+
+def _visit_order(counts: List[int]):
+    """In which order a group visits its rows, as a sort key over row numbers.  Workgroups that run at
+    the same time should read the same Q and dO.  With a causal mask every kv block of a sequence is
+    seen by its last row: last row first (against first row first 8.29 to 8.50 ms for the dK/dV
+    kernel on 65536 causal tokens).  With a sliding window most kv blocks are seen by the same number
+    of rows, each by the next ones in turn; taken modulo that number, neighbouring blocks visit a row
+    at the same time (131072 tokens, window 4096: 16.6 against 17.1 ms)."""
+    number, times = Counter(counts).most_common(1)[0]
+    if number > 2 and 2 * times > len(counts):
+        return lambda visit: (visit[0] % number, -visit[0])
+    return lambda visit: -visit[0]
+
+
+def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_block: int, n_slots: int) -> DkvGroups:
+    result = DkvGroups()
+    instrs = plan.instructions
+    limits = {idx: visits_per_group(sum(map(len, instr.dkv_block_table)), tiles_per_block * n_heads_kv, n_slots)
+              for idx, instr in enumerate(instrs) if isinstance(instr, AttnBackwardInstr)}
+    if all(limit == 1 for limit in limits.values()):
+        return result
+    # who wrote a BUFFER_dKV slot last -- (instruction, row, position), if a backward kernel did -- and
+    # which sum op reads what it wrote (None: something else does, or more than one op)
+    written: Dict[int, Optional[Tuple[int, int, int]]] = {}
+    reader: Dict[Tuple[int, int, int], Optional[Tuple[int, int]]] = {}
+    dkv = BufferType.BUFFER_dKV
+
+    def reads(blocks, who=None):
+        for block in blocks:
+            if block.buffer_type == dkv:
+                replica = written.get(block.index)
+                if replica is not None:
+                    reader[replica] = None if replica in reader else who
+
+    def writes(block: BufferBlock):
+        if block.buffer_type == dkv:
+            written[block.index] = None
+
+    for idx, instr in enumerate(instrs):
+        if isinstance(instr, AttnBackwardInstr):
+            for row, blocks in enumerate(instr.dkv_block_table):
+                for pos, block in enumerate(blocks):
+                    written[block.index] = (idx, row, pos)
+        elif isinstance(instr, SumInstr):
+            for pos, op in enumerate(instr.ops):
+                reads(op.src_buffers, (idx, pos))
+            for op in instr.ops:
+                writes(op.dst_buffer)
+        elif isinstance(instr, MemcpyInstr):
+            for src, dst in instr.src_dst_pairs:
+                if src.buffer_type == dkv or dst.buffer_type == dkv:
+                    reads((src,))
+                    writes(dst)
+        elif isinstance(instr, CommLaunchInstr):
+            for op in instr.comm_ops:
+                # (a receive lands at the wait at the latest: the slot is the exchange's from here on)
+                if op.comm_type == CommType.SEND:
+                    reads((op.buffer_block,))
+                else:
+                    writes(op.buffer_block)
+        elif isinstance(instr, AttnReductionInstr):
+            for op in instr.ops:
+                for blocks in op.src_buffers:
+                    reads(blocks)
+
+    for idx, instr in enumerate(instrs):
+        if limits.get(idx, 1) == 1:  # the launch does without groups
+            continue
+        # rows to take together: the same kv block, added by the same op and read by nothing else
+        together: Dict[tuple, List[Tuple[int, int]]] = defaultdict(list)
+        for row, (kv_blocks, dkv_blocks) in enumerate(zip(instr.kv_block_table, instr.dkv_block_table)):
+            for pos, (kv_block, dkv_block) in enumerate(zip(kv_blocks, dkv_blocks)):
+                op = reader.get((idx, row, pos))
+                together[(row, pos) if op is None else (op, kv_block.index, dkv_block.n_tokens)].append((row, pos))
+        limit = limits[idx]
+        groups: List[Group] = []
+        order = _visit_order([len(v) for v in together.values()]) if together else None
+        for key, visits in together.items():
+            visits.sort(key=order)
+            slot = lambda v: instr.dkv_block_table[v[0]][v[1]]
+            if len(key) == 2:
+                groups += [Group([v], slot(v)) for v in visits]
+                continue
+            j, op_pos = key[0]
+            op = instrs[j].ops[op_pos]
+            dst = direct.redirect_ops.get(j, {}).get(op_pos, op.dst_buffer if instrs[j].output_is_unpadded else None)
+            if (len(visits) <= limit and len(visits) == len(op.src_buffers) and dst is not None
+                    and dst.buffer_type == BufferType.LOCAL_dKV and dst.n_tokens == slot(visits[0]).n_tokens):
+                groups.append(Group(visits, dst))
+                result.skip_ops.setdefault(j, set()).add(op_pos)
+                continue
+            n_groups = -(-len(visits) // limit)
+            bounds = [len(visits) * i // n_groups for i in range(n_groups + 1)]
+            chunks = [visits[a:b] for a, b in zip(bounds, bounds[1:])]
+            groups += [Group(chunk, slot(chunk[0])) for chunk in chunks]
+            gone = {slot(v).index for chunk in chunks for v in chunk[1:]}
+            ops = result.sources.setdefault(j, {})
+            ops[op_pos] = [b for b in ops.get(op_pos, op.src_buffers)
+                           if not (b.buffer_type == BufferType.BUFFER_dKV and b.index in gone)]
+        groups.sort(key=lambda g: -len(g.visits))
+        result.groups[idx] = groups
+    return result

@@ -323,6 +323,53 @@ int dcp_attn_bwd_strided(const void* dout, const void* q, const void* k,
                          void* stream);
 
 /*
+ * dcp_attn_bwd_strided that adds dK/dV of a kv block over several rows in the
+ * kernel, in fp32, instead of leaving one private dK/dV block per (row, kv
+ * block).  A group is a kv block with up to DCP_ATTN_BWD_MAX_VISITS of the
+ * rows that list it:
+ *   dkv_groups int32 [n_groups][8]: the block's k/v table entry; where its dK/dV
+ *     goes (a table entry); tokens to store; 0 = into dk/dv (a slot), 1 = into
+ *     dk_unpadded/dv_unpadded (entry and token strides in elements); the first
+ *     of its visits; their number; two unused words
+ *   dkv_visits int32 [..][2]: a row, and the position of the group's block in
+ *     the row's kv_block_table
+ * Every (row, position) with keys belongs to exactly one group (a plan's
+ * replicas that are not added up form groups of one); dkv_block_table is
+ * not read.  Rows must hold whole blocks (key counts that are multiples of
+ * block_size) and block_size must be a multiple of 128.  A group's tokens are
+ * written whole (zeros where no query attends).  Launch order of the groups:
+ * as listed, so the ones with the most visits should come first.  The one-pass
+ * backward has no such form (the two-kernel one runs where it is selected).
+ * No counterpart in the reference, which sums replicas with a SumInstr
+ * (dcp/core/scheduler.py:1764-1940).
+ */
+#define DCP_ATTN_BWD_MAX_VISITS 32
+int dcp_attn_bwd_grouped(const void* dout, const void* q, const void* k,
+                         const void* v, const void* out, const float* lse,
+                         void* dq, void* dk, void* dv, void* workspace,
+                         size_t workspace_bytes, const int32_t* cu_seqlens_q,
+                         const int32_t* cu_seqlens_kv,
+                         const int32_t* attn_range, int n_ranges,
+                         const int32_t* q_block_table,
+                         const int32_t* kv_block_table,
+                         const int32_t* out_block_table,
+                         const int32_t* dq_block_table,
+                         const int32_t* dkv_block_table,
+                         const int32_t* row_order, int batch, int max_kv_blocks,
+                         int total_q, int block_size, int n_heads_q,
+                         int n_heads_kv, int head_dim, int64_t kv_slot_stride,
+                         int64_t kv_token_stride, int64_t dkv_slot_stride,
+                         int64_t dkv_token_stride, int64_t q_slot_stride,
+                         int64_t out_slot_stride, int64_t dq_slot_stride,
+                         int64_t lse_head_stride, int64_t lse_slot_stride,
+                         int64_t total_kv, const int32_t* dkv_groups,
+                         int n_groups, const int32_t* dkv_visits,
+                         void* dk_unpadded, void* dv_unpadded,
+                         int64_t unpadded_entry_stride,
+                         int64_t unpadded_token_stride, float softmax_scale,
+                         int dtype, void* stream);
+
+/*
  * Bytes of scratch dcp_attn_bwd needs for these sizes: rowsum(dO*O) and the
  * base-2 log-sum-exp (total_q*n_heads_q floats each), the per-(row, 64-query
  * tile) range hulls and the dQ kernel's work counters.  No counterpart in the reference (its

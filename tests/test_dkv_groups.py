@@ -1,0 +1,143 @@
+"""Which dK/dV replicas the backward kernel adds itself (``dkv_groups.analyse``): every (row, kv block)
+of a launch in exactly one group, a group's rows attend to one kv block, and group results plus what
+the sums still read are the replicas the plan adds, each exactly once (CPU).  On the GPU: grouped
+launches against dense attention and against the plan's own replicas, at group sizes from one row to
+more than the kernel takes at once."""
+
+from collections import Counter
+
+import pytest
+import torch
+
+from dcp_amd.core.instructions import AttnBackwardInstr, BufferType, SumInstr
+from dcp_amd.runtime.flash_attention import dkv_groups
+from dcp_amd.runtime.flash_attention.direct import DirectPlan, analyse as analyse_direct
+from tests.plan_cases import check_against_truth, dense_truth, make_case, make_multi_case, run_executor, run_multi_executor, scaled_err
+
+PLANS = {
+    # blocks with 1 to 9 rows, several q head blocks per kv head; ragged last blocks
+    "causal_gqa": dict(seqlens=[1100, 300, 1, 129], block_size=128, n_heads=8, n_groups=2, head_dim=128, head_block=2, qkv_scale=0.5),
+    # two partials per row: one backward launch per partial, one sum over both
+    "split": dict(seqlens=[900, 130], block_size=128, n_heads=4, n_groups=2, head_dim=64, head_block=1, n_kv_groups=2,
+                  kv_split="contiguous", qkv_scale=0.5),
+    # two ranges per query: key tiles of the sink block that most rows do not see (visits without a step)
+    "lambda": dict(seqlens=[1500, 130], block_size=256, n_heads=4, n_groups=1, head_dim=128, head_block=2, mask="lambda",
+                   mask_kwargs=dict(n_starting=16, l_pretrain=300), qkv_scale=0.5),
+    # no grouped queries: a visit of one head's tiles
+    "mha_fp16": dict(seqlens=[1300, 70], block_size=128, n_heads=3, n_groups=3, head_dim=64, head_block=3, dtype="fp16", qkv_scale=0.5),
+    # 41 rows for the first block: more than a group holds
+    "many_rows": dict(seqlens=[41 * 128 - 5], block_size=128, n_heads=2, n_groups=2, head_dim=128, head_block=2, qkv_scale=0.5),
+}
+
+
+def _check_groups(plan, found, slots_written_once=True):
+    instrs = plan.instructions
+    written = Counter()  # (instr, row, pos) -> times its dK/dV is part of a group
+    for idx, instr in enumerate(instrs):
+        if not isinstance(instr, AttnBackwardInstr):
+            continue
+        if idx not in found.groups:
+            continue
+        for g in found.groups[idx]:
+            assert 1 <= len(g.visits) <= dkv_groups.MAX_VISITS
+            assert len({instr.kv_block_table[r][p].index for r, p in g.visits}) == 1
+            written.update((idx, r, p) for r, p in g.visits)
+            if g.dst.buffer_type == BufferType.BUFFER_dKV:
+                assert g.dst.index == instr.dkv_block_table[g.visits[0][0]][g.visits[0][1]].index
+        pairs = {(idx, r, p) for r, row in enumerate(instr.kv_block_table) for p in range(len(row))}
+        assert set(k for k in written if k[0] == idx) == pairs
+        sizes = [len(g.visits) for g in found.groups[idx]]
+        assert sizes == sorted(sizes, reverse=True)
+    assert all(n == 1 for n in written.values())
+    if not slots_written_once:
+        return
+    # every replica reaches the sum that adds it exactly once
+    members = {g.dst.index: Counter(instrs[i].dkv_block_table[r][p].index for r, p in g.visits)
+               for i, gs in found.groups.items() for g in gs if g.dst.buffer_type == BufferType.BUFFER_dKV}
+    local = [Counter(instrs[i].dkv_block_table[r][p].index for r, p in g.visits)
+             for i, gs in found.groups.items() for g in gs if g.dst.buffer_type == BufferType.LOCAL_dKV]
+    for j, instr in enumerate(instrs):
+        for pos, op in enumerate(instr.ops if isinstance(instr, SumInstr) else []):
+            want = Counter(b.index for b in op.src_buffers)
+            if pos in found.skip_ops.get(j, ()):
+                assert want in local
+                continue
+            left = found.sources.get(j, {}).get(pos)
+            if left is None:
+                continue
+            got = Counter()
+            for b in left:
+                got.update(members.get(b.index, Counter([b.index])))
+            assert got == want
+
+
+@pytest.mark.parametrize("limit", [1, 3, 32])
+@pytest.mark.parametrize("direct", [False, True])
+@pytest.mark.parametrize("name", list(PLANS))
+def test_every_replica_is_added_once(monkeypatch, name, direct, limit):
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: limit)
+    plan = make_case(**PLANS[name])["bw"]
+    d = analyse_direct(plan) if direct else DirectPlan()
+    found = dkv_groups.analyse(plan, d, 1, 1, 512)
+    _check_groups(plan, found)
+    if limit == 1:
+        assert not found.groups
+    else:
+        assert any(len(g.visits) > 1 for gs in found.groups.values() for g in gs)
+
+
+def test_exchanged_replicas_are_left_alone(monkeypatch):
+    """A dK/dV slot that is sent to another device is read by the exchange and keeps its own slot."""
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+    case = make_multi_case(n_nodes=1, n_devices_per_node=2, seqlens=[700, 330], block_size=128, n_heads=4, n_groups=2, head_dim=64,
+                           head_block=2, n_stages=2)
+    for plan in case["bw"]:
+        found = dkv_groups.analyse(plan, DirectPlan(), 1, 1, 512)
+        _check_groups(plan, found, slots_written_once=False)
+
+
+def test_group_size_rule():
+    """One row per group where the launch does not fill the device several times over, never more
+    than the kernel takes."""
+    assert dkv_groups.visits_per_group(60, 8, 512) == 1
+    assert dkv_groups.visits_per_group(10 ** 6, 8, 512) == dkv_groups.MAX_VISITS
+    assert 1 < dkv_groups.visits_per_group(2544, 8, 512) < dkv_groups.MAX_VISITS
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("limit", [2, 32])
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("name", list(PLANS))
+def test_grouped_backward_matches_dense_attention(gpu, monkeypatch, name, mode, limit):
+    from dcp_amd import _lib
+
+    lib = _lib.load()
+    case = make_case(**PLANS[name])
+    before = lib.dcp_attn_bwd_select(mode)
+    try:
+        monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 1)
+        single, _ = run_executor(case, backward=True)
+        monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: limit)
+        grouped, ex = run_executor(case, backward=True, poison=200.0)
+        monkeypatch.setenv("DCP_DIRECT_LOCAL", "0")
+        as_written, _ = run_executor(case, backward=True)
+    finally:
+        lib.dcp_attn_bwd_select(before)
+    assert any(len(g.visits) == min(limit, 2) or len(g.visits) > 2 for gs in ex._dkv_groups.groups.values() for g in gs)
+    check_against_truth(grouped, dense_truth(case, backward=True))
+    same_dq = torch.equal(grouped[2], single[2])  # dQ does not depend on the grouping
+    same_as_written = torch.equal(grouped[3], as_written[3]) and torch.equal(grouped[2], as_written[2])
+    assert same_dq and same_as_written
+
+
+@pytest.mark.gpu
+def test_grouped_backward_with_an_exchange(gpu, monkeypatch):
+    case = make_multi_case(n_nodes=1, n_devices_per_node=2, seqlens=[700, 330], block_size=128, n_heads=4, n_groups=2, head_dim=128,
+                           head_block=2, n_stages=2)
+    single, _ = run_multi_executor(case, backward=True)
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+    grouped, _ = run_multi_executor(case, backward=True, repeats=2)
+    # unscaled inputs and partials that cross the exchange rounded: the bound of the exchange tests
+    err = scaled_err(grouped[3].float().numpy(), dense_truth(case, backward=True)[3])
+    same_dq = torch.equal(grouped[2], single[2])
+    assert same_dq and err <= 4e-2
