@@ -25,6 +25,11 @@ SIGNATURES = {
     "dcp_last_error": [],
     "dcp_profile_enable": [_I],
     "dcp_profile_report": [c_char_p, c_size_t],
+    "dcp_record_begin": [],
+    "dcp_record_end": [],
+    "dcp_record_size": [_P],
+    "dcp_record_run": [_P, _I, _I, _P],
+    "dcp_record_free": [_P],
     "dcp_fused_copy_varlen": [_P, _P, _P, _P, _P, _P, _P, _I, _L, _I, _P],
     "dcp_fused_copy_varlen_dkv": [_P, _P, _P, _I, _I, _I, _I, _P],
     "dcp_fused_copy_varlen_lse": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
@@ -76,12 +81,39 @@ def load():
         for name, argtypes in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.argtypes = argtypes
-            fn.restype = {"dcp_last_error": c_char_p, "dcp_attn_bwd_workspace_bytes": c_size_t,
+            fn.restype = {"dcp_last_error": c_char_p, "dcp_record_begin": c_void_p, "dcp_record_free": None, "dcp_attn_bwd_workspace_bytes": c_size_t,
                           "dcp_attn_fwd_workspace_bytes": c_size_t,
                           "dcp_attn_bwd_static_scratch_bytes": c_size_t,
                           "dcp_attn_bwd_workspace_bytes_kv": c_size_t}.get(name, c_int)
         _lib = lib
     return _lib
+
+
+class Recording:
+    """Library calls made on this thread between ``begin()`` and ``end()``, kept so that ``run`` can make
+    them again in one call.  ``keep`` holds what their pointers point to."""
+
+    def __init__(self, *keep):
+        self._list = None
+        self.keep = keep
+
+    def begin(self) -> bool:
+        """False if this thread is recording already (nothing is recorded then)."""
+        self._list = load().dcp_record_begin()
+        return self._list is not None
+
+    def end(self) -> None:
+        load().dcp_record_end()
+
+    def size(self) -> int:
+        return load().dcp_record_size(self._list)
+
+    def run(self, begin: int, end: int, stream: int) -> None:
+        call("dcp_record_run", self._list, begin, end, stream)
+
+    def __del__(self):
+        if self._list is not None and _lib is not None:
+            _lib.dcp_record_free(self._list)
 
 
 def profile_enable(on: bool) -> None:

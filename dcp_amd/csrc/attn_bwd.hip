@@ -52,6 +52,7 @@
 #include <mutex>
 
 #include "attn_bwd_params.h"
+#include "record.h"
 
 namespace dcp {
 
@@ -1123,6 +1124,10 @@ extern "C" int dcp_attn_bwd(const void* dout, const void* q, const void* k, cons
                             int64_t kv_token_stride, int64_t dkv_slot_stride,
                             int64_t dkv_token_stride, int n_out_slots, float softmax_scale,
                             int dtype, void* stream) {
+  DCP_RECORDED(dcp_attn_bwd(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
+      cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table, dq_block_table,
+      dkv_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim,
+      kv_slot_stride, kv_token_stride, dkv_slot_stride, dkv_token_stride, n_out_slots, softmax_scale, dtype, stream));
   DCP_REQUIRE(batch == 0 || n_out_slots > 0, "attn_bwd: empty block tables");
   const int64_t slot = (int64_t)block_size * n_heads_q * head_dim;
   return attn_bwd_launch(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
@@ -1146,6 +1151,11 @@ extern "C" int dcp_attn_bwd_strided(const void* dout, const void* q, const void*
                                     int64_t dkv_token_stride, int64_t q_slot_stride, int64_t out_slot_stride,
                                     int64_t dq_slot_stride, int64_t lse_head_stride, int64_t lse_slot_stride,
                                     int64_t total_kv, float softmax_scale, int dtype, void* stream) {
+  DCP_RECORDED(dcp_attn_bwd_strided(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
+      cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table, dq_block_table,
+      dkv_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim,
+      kv_slot_stride, kv_token_stride, dkv_slot_stride, dkv_token_stride, q_slot_stride, out_slot_stride,
+      dq_slot_stride, lse_head_stride, lse_slot_stride, total_kv, softmax_scale, dtype, stream));
   return attn_bwd_launch(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
                          cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table,
                          dq_block_table, dkv_block_table, row_order, batch, max_kv_blocks, total_q, block_size,
@@ -1170,6 +1180,12 @@ extern "C" int dcp_attn_bwd_grouped(const void* dout, const void* q, const void*
                                     const int32_t* dkv_visits, void* dk_unpadded, void* dv_unpadded,
                                     int64_t unpadded_entry_stride, int64_t unpadded_token_stride,
                                     float softmax_scale, int dtype, void* stream) {
+  DCP_RECORDED(dcp_attn_bwd_grouped(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
+      cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table, dq_block_table,
+      dkv_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim,
+      kv_slot_stride, kv_token_stride, dkv_slot_stride, dkv_token_stride, q_slot_stride, out_slot_stride,
+      dq_slot_stride, lse_head_stride, lse_slot_stride, total_kv, dkv_groups, n_groups, dkv_visits, dk_unpadded,
+      dv_unpadded, unpadded_entry_stride, unpadded_token_stride, softmax_scale, dtype, stream));
   const DkvGrouping grouping = {dkv_groups, n_groups, dkv_visits, dk_unpadded, dv_unpadded, unpadded_entry_stride,
                                 unpadded_token_stride};
   return attn_bwd_launch(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
@@ -1243,6 +1259,10 @@ extern "C" int dcp_attn_bwd_static(const void* dout, const void* q, const void* 
                                    int64_t kv_slot_stride, int64_t kv_token_stride, int64_t dkv_slot_stride,
                                    int64_t dkv_token_stride, int n_out_slots, float softmax_scale, int dtype,
                                    void* stream) {
+  DCP_RECORDED(dcp_attn_bwd_static(dout, q, k, v, out, lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_kv, attn_range,
+      n_ranges, q_block_table, kv_block_table, out_block_table, dq_block_table, dkv_block_table, row_order, batch,
+      max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride,
+      dkv_slot_stride, dkv_token_stride, n_out_slots, softmax_scale, dtype, stream));
   (void)head_dim;
   const size_t need = bwd_base_workspace_bytes(batch, total_q, block_size, n_heads_q);  // the two-kernel backward's
   DCP_REQUIRE(need <= (size_t)DCP_ATTN_BWD_STATIC_SCRATCH_BYTES,

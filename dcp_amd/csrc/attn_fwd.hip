@@ -36,6 +36,7 @@
 #include <algorithm>
 
 #include "attn_common.h"
+#include "record.h"
 
 namespace dcp {
 
@@ -620,6 +621,10 @@ extern "C" int dcp_attn_fwd(const void* q, const void* k, const void* v, void* o
                             int64_t kv_slot_stride, int64_t kv_token_stride, int n_out_slots,
                             float softmax_scale, int dtype, void* workspace, size_t workspace_bytes,
                             void* stream) {
+  DCP_RECORDED(dcp_attn_fwd(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table,
+      kv_block_table, out_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv,
+      head_dim, kv_slot_stride, kv_token_stride, n_out_slots, softmax_scale, dtype, workspace, workspace_bytes,
+      stream));
   DCP_REQUIRE(batch == 0 || n_out_slots > 0, "attn_fwd: empty block tables");
   const int64_t slot = (int64_t)block_size * n_heads_q * head_dim;
   return dcp_attn_fwd_strided(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table,
@@ -639,6 +644,10 @@ extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v,
                                     int64_t out_slot_stride, int64_t lse_head_stride, int64_t lse_slot_stride,
                                     int merged_form, float softmax_scale, int dtype, void* workspace,
                                     size_t workspace_bytes, void* stream) {
+  DCP_RECORDED(dcp_attn_fwd_strided(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges,
+      q_block_table, kv_block_table, out_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q,
+      n_heads_kv, head_dim, kv_slot_stride, kv_token_stride, q_slot_stride, out_slot_stride, lse_head_stride,
+      lse_slot_stride, merged_form, softmax_scale, dtype, workspace, workspace_bytes, stream));
   if (dtype != DCP_DTYPE_BF16 && dtype != DCP_DTYPE_FP16)
     return fail(DCP_ERR_UNSUPPORTED, "attn_fwd: dtype %d unsupported (bf16 and fp16 only)", dtype);
   if (head_dim != 64 && head_dim != 128)

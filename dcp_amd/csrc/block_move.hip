@@ -11,6 +11,7 @@
 // executor gather (ragged, two sizes in one launch) take 0.31 ms per launch
 // with 4 KiB chunks against 0.23 with 16 KiB.
 #include "common.h"
+#include "record.h"
 
 namespace dcp {
 
@@ -136,6 +137,8 @@ extern "C" int dcp_fused_copy_varlen(const int64_t* src_ptrs, const int32_t* src
                                      const int32_t* dst_offsets, const int32_t* dst_strides,
                                      const int32_t* n_elements, int n_ptrs, int64_t block_numel,
                                      int elem_size, void* stream) {
+  DCP_RECORDED(dcp_fused_copy_varlen(src_ptrs, src_offsets, src_strides, dst_ptrs, dst_offsets, dst_strides,
+      n_elements, n_ptrs, block_numel, elem_size, stream));
   DCP_REQUIRE(elem_size == 2 || elem_size == 4, "copy: unsupported element size %d", elem_size);
   DCP_REQUIRE(n_ptrs >= 0 && block_numel >= 0, "copy: negative size");
   if (n_ptrs == 0 || block_numel == 0) return DCP_OK;
@@ -149,6 +152,8 @@ extern "C" int dcp_fused_copy_varlen(const int64_t* src_ptrs, const int32_t* src
 extern "C" int dcp_fused_copy_varlen_dkv(const int64_t* src_ptrs, const int64_t* dst_ptrs,
                                          const int32_t* n_tokens, int n_ptrs, int max_n_tokens,
                                          int per_token_size, int elem_size, void* stream) {
+  DCP_RECORDED(dcp_fused_copy_varlen_dkv(src_ptrs, dst_ptrs, n_tokens, n_ptrs, max_n_tokens, per_token_size,
+      elem_size, stream));
   DCP_REQUIRE(elem_size == 2 || elem_size == 4, "dkv copy: unsupported element size %d",
               elem_size);
   DCP_REQUIRE(n_ptrs >= 0 && max_n_tokens >= 0 && per_token_size >= 0, "dkv copy: negative size");
@@ -166,6 +171,8 @@ extern "C" int dcp_fused_copy_varlen_lse(const int64_t* src_ptrs,
                                          const int32_t* dst_head_strides, const int32_t* n_tokens,
                                          int n_ptrs, int head_block_size, int max_n_tokens,
                                          int elem_size, void* stream) {
+  DCP_RECORDED(dcp_fused_copy_varlen_lse(src_ptrs, src_token_offsets, src_head_strides, dst_ptrs, dst_token_offsets,
+      dst_head_strides, n_tokens, n_ptrs, head_block_size, max_n_tokens, elem_size, stream));
   DCP_REQUIRE(elem_size == 2 || elem_size == 4, "lse copy: unsupported element size %d",
               elem_size);
   DCP_REQUIRE(n_ptrs >= 0 && head_block_size >= 0 && max_n_tokens >= 0,

@@ -5,6 +5,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "record.h"
 
 namespace dcp {
 
@@ -681,6 +682,9 @@ extern "C" int dcp_update_out_lse(const void* src_out, void* dst_out, const floa
                                   int64_t src_lse_head_stride, int64_t dst_lse_head_stride,
                                   int head_dim, int max_n_blocks_per_op, int dtype,
                                   void* stream) {
+  DCP_RECORDED(dcp_update_out_lse(src_out, dst_out, src_lse, dst_lse, n_head, src_block_table, dst_token_offsets,
+      n_tokens_per_block, block_lengths, n_red_ops, block_size, out_block_stride, out_token_stride, lse_block_stride,
+      lse_token_stride, src_lse_head_stride, dst_lse_head_stride, head_dim, max_n_blocks_per_op, dtype, stream));
   DCP_REQUIRE(max_n_blocks_per_op <= 64, "Too many blocks for reduction (%d > 64)",
               max_n_blocks_per_op);
   DCP_REQUIRE(max_n_blocks_per_op >= 1, "merge: max_n_blocks_per_op must be positive");
@@ -714,6 +718,8 @@ extern "C" int dcp_blockwise_sum(const int64_t* src_ptrs, const int32_t* src_off
                                  const int32_t* dst_strides, const int32_t* n_elements,
                                  int n_sums, int max_n_ops_per_block, int64_t block_numel,
                                  int dtype, void* stream) {
+  DCP_RECORDED(dcp_blockwise_sum(src_ptrs, src_offsets, src_strides, n_ops_per_block, dst_ptrs, dst_offsets,
+      dst_strides, n_elements, n_sums, max_n_ops_per_block, block_numel, dtype, stream));
   const int esize = dtype_size(dtype);
   if (esize == 0) return fail(DCP_ERR_UNSUPPORTED, "Unsupported dtype: %d", dtype);
   DCP_REQUIRE(n_sums >= 0 && block_numel >= 0 && max_n_ops_per_block >= 1, "sum: bad size");

@@ -1,0 +1,50 @@
+// Recorded launches (record.h): the list and its entry points.
+#include "record.h"
+
+#include <vector>
+
+#include "common.h"
+
+namespace dcp {
+
+struct RecordedCalls {
+  std::vector<std::function<int(void*)>> calls;
+};
+
+namespace {
+thread_local RecordedCalls* t_recording = nullptr;
+thread_local bool t_suspended = false;
+}  // namespace
+
+RecordedCalls* current_recording() { return t_suspended ? nullptr : t_recording; }
+void record_call(RecordedCalls* list, std::function<int(void*)> call) { list->calls.push_back(std::move(call)); }
+void suspend_recording(bool suspended) { t_suspended = suspended; }
+
+}  // namespace dcp
+
+using dcp::RecordedCalls;
+
+extern "C" void* dcp_record_begin(void) {
+  if (dcp::t_recording != nullptr) return nullptr;
+  dcp::t_recording = new RecordedCalls;
+  return dcp::t_recording;
+}
+
+extern "C" int dcp_record_end(void) {
+  DCP_REQUIRE(dcp::t_recording != nullptr, "record_end: this thread is not recording");
+  dcp::t_recording = nullptr;
+  return DCP_OK;
+}
+
+extern "C" int dcp_record_size(const void* list) { return list ? (int)static_cast<const RecordedCalls*>(list)->calls.size() : 0; }
+
+extern "C" int dcp_record_run(const void* list, int begin, int end, void* stream) {
+  DCP_REQUIRE(list != nullptr, "record_run: null list");
+  const auto& calls = static_cast<const RecordedCalls*>(list)->calls;
+  DCP_REQUIRE(begin >= 0 && begin <= end && end <= (int)calls.size(), "record_run: calls %d to %d of %zu", begin, end, calls.size());
+  for (int i = begin; i < end; ++i)
+    if (const int status = calls[i](stream)) return status;
+  return DCP_OK;
+}
+
+extern "C" void dcp_record_free(void* list) { delete static_cast<RecordedCalls*>(list); }

@@ -8,7 +8,8 @@
  *  - `stream` is a hipStream_t passed as void* (NULL = the null stream); all
  *    work is enqueued on it and nothing synchronises with the host;
  *  - the library borrows memory for the duration of a launch: it allocates
- *    nothing and keeps no pointer;
+ *    nothing and keeps no pointer (a caller's own list of recorded calls
+ *    aside, see dcp_record_begin);
  *  - return value 0 = launched, nonzero = rejected before any launch (argument
  *    error); dcp_last_error() then returns a message for the calling thread;
  *  - dtype codes follow the reference's wire integers
@@ -52,6 +53,24 @@ const char* dcp_last_error(void);
  */
 void dcp_profile_enable(int on);
 int dcp_profile_report(char* buffer, size_t capacity);
+
+/*
+ * Recorded calls, for callers that repeat a fixed sequence (a prepared plan).
+ * Between dcp_record_begin and dcp_record_end every call of an entry point
+ * below that takes a stream, made on this thread, is launched as usual and also
+ * added with its arguments to the list dcp_record_begin returned (NULL if the
+ * thread is recording already).  dcp_record_run makes calls [begin, end) of a
+ * list again, in order, on `stream`, and returns the first nonzero status.  The
+ * arguments are kept as they were given: the caller keeps the memory they point
+ * to alive and in place for as long as it runs the list.  A list may be run
+ * from several threads; nothing in it changes.  No counterpart in the reference
+ * (its executor walks the instructions in Python at every call).
+ */
+void* dcp_record_begin(void);
+int dcp_record_end(void);
+int dcp_record_size(const void* list);
+int dcp_record_run(const void* list, int begin, int end, void* stream);
+void dcp_record_free(void* list);
 
 /*
  * Block gather / scatter through pointer tables.
