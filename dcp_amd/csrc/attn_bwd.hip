@@ -618,6 +618,7 @@ __device__ __forceinline__ void attn_bwd_dq_item(KernArgs<AttnBwdParams>& p, int
   __shared__ int slot_lds[kSlotTableCap];
 
   int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (per item: what is derived from it is not kept through the item before)
   const int w = tid >> 6;
   const int lane = tid & 63;
   const int c = lane & 31;
@@ -874,34 +875,28 @@ __device__ __forceinline__ void attn_bwd_dq_item(KernArgs<AttnBwdParams>& p, int
     }
 }
 
-// Persistent, like the forward kernel: as many workgroups as the device holds, each taking the
-// next item of its XCD (workgroup b sits on XCD b % 8; the query tiles and grouped heads of a row
-// share its K/V and stay on one XCD) from a ticket counter in the workspace, which the hull
-// kernel zeroes before every launch.  2.7 % on the causal benchmark, 0.8 % with a lambda mask
-// (whose items are all alike, so there is little dispatch imbalance to recover).
+// Persistent, like the forward kernel (the counters are zeroed by the hull kernel).  2.7 % on the causal
+// benchmark, 0.8 % with a lambda mask (whose items are all alike, so there is little dispatch
+// imbalance to recover).
 template <int DTYPE, int D>
 __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dq_kernel(const AttnBwdParams p) {
   __shared__ int ticket_lds;
-  const int x = blockIdx.x % kNumXcd;
-  const int64_t n_streams = (p.n_dq_items + p.dq_xcd_group - 1) / p.dq_xcd_group;
-  const int64_t n_x = n_streams > x ? (n_streams - x + kNumXcd - 1) / kNumXcd * p.dq_xcd_group : 0;
   while (true) {
-    if (threadIdx.x == 0) ticket_lds = atomicAdd(&p.tickets[x], 1);
-    __syncthreads();
-    const int i = __builtin_amdgcn_readfirstlane(ticket_lds);
-    if (i >= n_x) break;
-    const int64_t item = (x + kNumXcd * (int64_t)(i / p.dq_xcd_group)) * p.dq_xcd_group + i % p.dq_xcd_group;
-    if (item < p.n_dq_items) attn_bwd_dq_item<DTYPE, D>(fresh_kernel_args<AttnBwdParams>(), (int)item);
-    __syncthreads();  // the next item reuses the LDS tables and tiles, and the ticket's place
+    KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
+    const int item = next_item({args.dq_tickets, args.n_dq_items, args.dq_xcd_group}, &ticket_lds);
+    if (item < 0) break;
+    attn_bwd_dq_item<DTYPE, D>(args, item);
+    if (fresh_kernel_args<AttnBwdParams>().dq_tickets == nullptr) break;
   }
 }
 
 template <int DTYPE, int D>
-static int launch_bwd(const AttnBwdParams& p, hipStream_t stream) {
+static int launch_bwd(AttnBwdParams p, hipStream_t stream) {
   const int64_t n_dkv = xcd_grid_size(p.n_dkv_items, p.dkv_xcd_group);
   DCP_REQUIRE(n_dkv < ((int64_t)1 << 31) && p.n_dq_items < ((int64_t)1 << 31), "attn_bwd: grid too large");
   // as many workgroups as the device holds at once (two per CU), a multiple of the XCD count
   const int64_t n_dq = std::min<int64_t>(xcd_grid_size(p.n_dq_items, 1), xcd_grid_size(2 * (int64_t)device_cu_count(), 1));
+  p.dq_tickets = p.n_dq_items > n_dq ? p.tickets : nullptr;
   {
     KernelTimer timer("bwd_tile_hull_kernel", stream);
     hipLaunchKernelGGL(bwd_tile_hull_kernel, dim3(p.batch * p.q_tiles_per_row), dim3(64), 0, stream, p);
@@ -1046,6 +1041,7 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
   p.hull = reinterpret_cast<int32_t*>(ws);
   ws += align256((size_t)batch * ((block_size + kBwdBM - 1) / kBwdBM) * 8 * sizeof(int32_t));
   p.tickets = reinterpret_cast<int*>(ws);
+  p.dq_tickets = nullptr;  // (the launchers say)
   ws += align256(kTicketInts * sizeof(int32_t));
   p.subs_per_row = (block_size + 31) / 32;
   p.head_dim = head_dim;

@@ -275,21 +275,16 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   }
 }
 
-// persistent, like the recomputing dQ kernel: per-XCD tickets in the workspace (zeroed by the prepare kernel)
+// persistent, like the recomputing dQ kernel (the counters are zeroed by the prepare kernel)
 template <int DTYPE, int D, int HH>
 __global__ __launch_bounds__(kDsThreads, 1) void attn_bwd_dq_ds_kernel(const AttnBwdParams p) {
   __shared__ int ticket_lds;
-  const int x = blockIdx.x % kNumXcd;
-  const int64_t n_streams = (p.n_dq_items + p.dq_xcd_group - 1) / p.dq_xcd_group;
-  const int64_t n_x = n_streams > x ? (n_streams - x + kNumXcd - 1) / kNumXcd * p.dq_xcd_group : 0;
   while (true) {
-    if (threadIdx.x == 0) ticket_lds = atomicAdd(&p.tickets[x], 1);
-    __syncthreads();
-    const int i = __builtin_amdgcn_readfirstlane(ticket_lds);
-    if (i >= n_x) break;
-    const int64_t item = (x + kNumXcd * (int64_t)(i / p.dq_xcd_group)) * p.dq_xcd_group + i % p.dq_xcd_group;
-    if (item < p.n_dq_items) attn_bwd_dq_ds_item<DTYPE, D, HH>(fresh_kernel_args<AttnBwdParams>(), (int)item);
-    __syncthreads();
+    KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
+    const int item = next_item({args.dq_tickets, args.n_dq_items, args.dq_xcd_group}, &ticket_lds);
+    if (item < 0) break;
+    attn_bwd_dq_ds_item<DTYPE, D, HH>(args, item);
+    if (fresh_kernel_args<AttnBwdParams>().dq_tickets == nullptr) break;
   }
 }
 
@@ -313,6 +308,7 @@ int launch_bwd_through_ds(const AttnBwdParams& p, int dtype, hipStream_t stream)
   q.dq_xcd_group = q.dq_tiles_per_row * (per_kv / hh);
   DCP_REQUIRE(q.n_dq_items < ((int64_t)1 << 31), "attn_bwd: grid too large");
   const int64_t n_dq = std::min<int64_t>(xcd_grid_size(q.n_dq_items, 1), xcd_grid_size((int64_t)device_cu_count(), 1));
+  q.dq_tickets = q.n_dq_items > n_dq ? p.tickets : nullptr;
   KernelTimer timer("attn_bwd_dq_ds_kernel", stream);
   const dim3 grid((unsigned)n_dq), block(kDsThreads);
 #define DCP_DQ_DS_LAUNCH(DT, HD, HH) hipLaunchKernelGGL((attn_bwd_dq_ds_kernel<DT, HD, HH>), grid, block, 0, stream, q)

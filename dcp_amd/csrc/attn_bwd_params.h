@@ -19,6 +19,7 @@ struct AttnBwdParams {
   float* lse2;       // [total_q, H]: lse * log2(e); both written by the dQ kernel, read by the dK/dV kernel
   int32_t* hull;     // [batch * q_tiles_per_row, 8]
   int* tickets;      // work-item counters of the persistent dQ kernel (kTicketInts); zeroed by the hull kernel
+  int* dq_tickets;   // the same where the dQ kernel has more items than workgroups, else null
   // the one-pass backward only (attn_bwd_fused.hip):
   float* dq_part;    // [batch * n_heads_q * subs_per_row][4096]: partial dQ of a (row, head, 32-query) chunk, fp32
   int* chain;        // [batch * n_heads_q * subs_per_row][4]: links of the chunk's chain done so far, per wave

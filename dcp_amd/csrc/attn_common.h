@@ -313,6 +313,60 @@ inline int64_t xcd_grid_size(int64_t total, int group) {
   return (total + per_super - 1) / per_super * per_super;
 }
 
+// Work items of a persistent kernel (as many workgroups as the device holds, each taking item after
+// item).  Workgroup b sits on XCD b % 8; the items that stream the same tiles (`group` of them with
+// consecutive ids: stream s) belong to XCD s % 8 and are handed out in id order through one ticket
+// counter per XCD.  An XCD that has run out takes from the one with the most items left: streams are
+// not equally long, and a launch with fewer than a few hundred streams need not even have the same
+// number of them on every XCD.
+struct ItemQueue {
+  int* tickets;     // kNumXcd counters, zero before the launch; null: one item per workgroup, item = workgroup id
+  int64_t n_items;  // a multiple of group
+  int group;
+};
+// The workgroup's next item, or -1.  `box`: a word of LDS.  Contains the barriers that separate one
+// item's use of LDS from the next one's.  (Without tickets the workgroup's only item, at every call.)
+__device__ __forceinline__ int next_item(const ItemQueue& queue, int* box) {
+  if (queue.tickets == nullptr) {
+    // as many workgroups as items: whole streams by XCD as long as every XCD gets one more, the rest
+    // item by item over all of them
+    const int w = blockIdx.x, group = queue.group;
+    if (w >= queue.n_items) return -1;
+    const int in_turns = (int)(queue.n_items / (kNumXcd * group)) * kNumXcd * group;
+    if (w >= in_turns) return w;
+    const int i = w / kNumXcd;
+    return __builtin_amdgcn_readfirstlane((w % kNumXcd + kNumXcd * (i / group)) * group + i % group);
+  }
+  __syncthreads();  // everybody has read the last ticket and is done with the last item's LDS
+  if (threadIdx.x == 0) {
+    const int group = queue.group, n_streams = (int)(queue.n_items / group);
+    const int own = blockIdx.x % kNumXcd;
+    auto items_of = [&](int x) { return n_streams > x ? (n_streams - x + kNumXcd - 1) / kNumXcd * group : 0; };
+    int x = own, found = -1;
+    while (true) {
+      const int i = atomicAdd(&queue.tickets[x], 1);
+      if (i < items_of(x)) {
+        const int s = i / group;
+        found = (x + kNumXcd * s) * group + (i - s * group);
+        break;
+      }
+      // (the counters only grow, so every round either takes an item or finds one queue fewer to ask)
+      int most = 0;
+      for (int y = 0; y < kNumXcd; ++y) {
+        const int left = items_of(y) - __hip_atomic_load(&queue.tickets[y], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (left > most) {
+          most = left;
+          x = y;
+        }
+      }
+      if (most == 0) break;
+    }
+    *box = found;
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(*box);
+}
+
 // A persistent kernel's item body reads the kernel arguments through a pointer to the
 // kernel-argument segment that is made opaque once per item, so that the compiler loads each
 // field where the item uses it.  Read through the kernel's by-value parameter, every field an

@@ -74,7 +74,7 @@ struct AttnFwdParams {
   int xcd_group;     // work items per shared K/V stream
   int64_t n_items;   // batch * n_heads_q * q_tiles_per_row
   float scale_log2;  // softmax_scale * log2(e)
-  int* tickets;      // kNumXcd item counters, zeroed before the launch
+  int* tickets;      // of the item queue, zeroed before the launch; null: one item per workgroup
 };
 
 // Wave priority by phase: the two waves of a SIMD come from different workgroups and drift
@@ -101,7 +101,7 @@ constexpr float kMaxTileSum = 16384.0f;
 // serves twice the arithmetic; the wave then needs the whole register file (one workgroup
 // per CU, accumulators in the AGPR half).
 template <int DTYPE, int D, int QB>
-__device__ __forceinline__ void attn_fwd_item(const AttnFwdParams& p, int item) {
+__device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int item) {
   constexpr int BN = kFwdBN;
   constexpr int BM = 128 * QB;
   constexpr int KS = D / 16;  // k-steps of S^T = K Q^T
@@ -575,30 +575,22 @@ __device__ __forceinline__ void attn_fwd_item(const AttnFwdParams& p, int item) 
 }
 
 // The kernel is persistent: the launch has (at most) as many workgroups as the device holds at
-// once and each keeps taking the next work item of its XCD until none is left.  A grid of one
+// once and each keeps taking the next work item until none is left (ItemQueue).  A grid of one
 // workgroup per item loses a tenth of the device to dispatch: workgroup ids are dealt to the 8
 // XCDs strictly in turn, so an XCD with a free slot waits until every XCD before it in the turn
 // has taken its workgroup (13 us between two workgroups of a CU slot on average, against 100 us
-// of work), and the last, unevenly long items leave slots empty at the end.
-//
-// Workgroup b sits on XCD b % 8.  The items that stream the same K/V (the query tiles and grouped
-// heads of a row, `xcd_group` of them with consecutive ids) stay on one XCD: stream s belongs to
-// XCD s % 8, and an XCD's items are handed out in id order (rows come longest first) through one
-// ticket counter per XCD in `p.tickets`, which a one-wave kernel zeroes on the stream just before.
+// of work), and the last, unevenly long items leave slots empty at the end.  Rows come longest first;
+// the counters are zeroed by a one-wave kernel on the stream just before.  A launch whose items all
+// fit on the device at once needs no queue and no such kernel.
 template <int DTYPE, int D, int QB>
 __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(const AttnFwdParams p) {
   __shared__ int ticket_lds;
-  const int x = blockIdx.x % kNumXcd;
-  const int64_t n_streams = (p.n_items + p.xcd_group - 1) / p.xcd_group;
-  const int64_t n_x = n_streams > x ? (n_streams - x + kNumXcd - 1) / kNumXcd * p.xcd_group : 0;  // items of this XCD
   while (true) {
-    if (threadIdx.x == 0) ticket_lds = atomicAdd(&p.tickets[x], 1);
-    __syncthreads();
-    const int i = __builtin_amdgcn_readfirstlane(ticket_lds);
-    if (i >= n_x) break;
-    const int64_t item = (x + kNumXcd * (int64_t)(i / p.xcd_group)) * p.xcd_group + i % p.xcd_group;
-    if (item < p.n_items) attn_fwd_item<DTYPE, D, QB>(p, (int)item);
-    __syncthreads();  // the next item reuses the LDS tables and tiles, and the ticket's place
+    KernArgs<AttnFwdParams>& args = fresh_kernel_args<AttnFwdParams>();
+    const int item = next_item({args.tickets, args.n_items, args.xcd_group}, &ticket_lds);
+    if (item < 0) break;
+    attn_fwd_item<DTYPE, D, QB>(args, item);
+    if (fresh_kernel_args<AttnFwdParams>().tickets == nullptr) break;
   }
 }
 
@@ -713,9 +705,9 @@ extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v,
   DCP_REQUIRE(p.n_items < ((int64_t)1 << 31), "attn_fwd: too many work items");
   // as many workgroups as the device holds at once (two per CU), a multiple of the XCD count
   const int64_t n_wg = std::min<int64_t>(xcd_grid_size(p.n_items, 1), xcd_grid_size(2 * (int64_t)device_cu_count(), 1));
-  p.tickets = reinterpret_cast<int*>(workspace);
+  p.tickets = p.n_items > n_wg ? reinterpret_cast<int*>(workspace) : nullptr;
   dim3 grid((unsigned)n_wg), block(kFwdThreads);
-  hipLaunchKernelGGL(attn_fwd_reset_tickets_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, p.tickets);
+  if (p.tickets) hipLaunchKernelGGL(attn_fwd_reset_tickets_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, p.tickets);
   KernelTimer timer("attn_fwd_kernel", stream);
 #define DCP_FWD(DT, HD) \
   hipLaunchKernelGGL((attn_fwd_kernel<DT, HD, 1>), grid, block, 0, (hipStream_t)stream, p)

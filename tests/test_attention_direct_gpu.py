@@ -242,3 +242,31 @@ def test_arbitrary_ranges(gpu, seed, d, bs, hq, hkv):
     pr = _paged_rows(gpu, rows, bs, hq=hq, hkv=hkv, d=d, seed=seed)
     worst = _check_direct(pr, _run_direct(pr))
     assert worst["out"] <= OUT_TOL and worst["lse"] <= LSE_TOL and worst["dq"] <= GRAD_TOL and worst["dkv"] <= GRAD_TOL, worst
+
+
+# The persistent kernels' item queue: launches whose items all fit on the device at once (whole streams
+# per XCD, a remainder of streams dealt item by item, fewer items than XCDs), and launches with more
+# items than workgroups but fewer streams than XCDs, which all but two XCDs' workgroups have to take
+# from the others.
+QUEUE_CASES = {
+    "one_item": dict(seqlens=[40], block_size=64, n_heads=1, n_groups=1, head_dim=64, head_block=1),
+    "three_streams": dict(seqlens=[300], block_size=128, n_heads=4, n_groups=1, head_dim=128, head_block=4),
+    "nineteen_streams": dict(seqlens=[19 * 64 - 3], block_size=64, n_heads=2, n_groups=2, head_dim=64, head_block=1, n_kv_groups=2),
+    "two_streams_of_512_items": dict(seqlens=[2100, 300], block_size=2048, n_heads=32, n_groups=1, head_dim=64, head_block=32),
+}
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("name", list(QUEUE_CASES))
+def test_every_item_of_a_launch_is_taken_once(gpu, name, mode):
+    from dcp_amd import _lib
+    from tests.plan_cases import check_against_truth, dense_truth, make_case, run_executor
+
+    case = make_case(**QUEUE_CASES[name], qkv_scale=0.5)
+    lib = _lib.load()
+    before = lib.dcp_attn_bwd_select(mode)
+    try:
+        res, _ = run_executor(case, backward=True)
+    finally:
+        lib.dcp_attn_bwd_select(before)
+    check_against_truth(res, dense_truth(case, backward=True))
