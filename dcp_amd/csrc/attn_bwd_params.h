@@ -19,6 +19,7 @@ struct AttnBwdParams {
   float* lse2;       // [total_q, H]: lse * log2(e); both written by the dQ kernel, read by the dK/dV kernel
   int32_t* hull;     // [batch * q_tiles_per_row, 8]
   int* tickets;      // work-item counters of the persistent dQ kernel (kTicketInts); zeroed by the hull kernel
+  int* dkv_tickets;
   int* dq_tickets;   // the same where the dQ kernel has more items than workgroups, else null
   // the one-pass backward only (attn_bwd_fused.hip):
   float* dq_part;    // [batch * n_heads_q * subs_per_row][4096]: partial dQ of a (row, head, 32-query) chunk, fp32
@@ -91,7 +92,7 @@ constexpr int kTicketInts = 16;  // one counter per XCD (the rest unused)
 // dQ kernel that reads it back (attn_bwd_ds.hip); the pieces it is made of live in three files.
 int launch_bwd_through_ds(const AttnBwdParams& p, int dtype, hipStream_t stream);
 int launch_bwd_prepare(const AttnBwdParams& p, int dtype, hipStream_t stream);
-int launch_bwd_dkv_writing_ds(const AttnBwdParams& p, int dtype, hipStream_t stream);
+int launch_bwd_dkv_writing_ds(AttnBwdParams p, int dtype, hipStream_t stream);
 size_t bwd_ds_workspace_bytes(int64_t total_kv, int batch, int block_size, int n_heads_q);
 
 // The one-pass backward (prepare + fused kernel) for head size 128; p.hull, p.delta, p.lse2,

@@ -77,6 +77,52 @@ def _visit_order(counts: List[int]):
     return lambda visit: -visit[0]
 
 
+def _chunk_sizes(n_visits: int, limit: int) -> List[int]:
+    """How a kv block with more rows than a group may visit is split: whole groups, then what is left in
+    halves down to an eighth of one.  Groups of one size end together and leave the device idle for up
+    to a group's time; small ones, handed out last, fill that (98304 tokens, shared prefixes, up to 150
+    rows a block: dK/dV kernel and sums 28.2 ms in equal parts of up to 32, 27.5 this way)."""
+    sizes = [limit] * (n_visits // limit - 1)
+    left = n_visits - sum(sizes)  # between one and two groups
+    smallest = max(1, limit // 8)
+    while left > 0:
+        size = min(limit, max(smallest, (left + 1) // 2))
+        sizes.append(min(size, left))
+        left -= sizes[-1]
+    return sizes
+
+
+def _components(kv_table) -> Dict[int, Tuple[int, int]]:
+    """kv block -> (component, rank in it), two blocks being in one component if some row attends to
+    both: the blocks of a sequence's kv head.  In order of first appearance."""
+    parent: Dict[int, int] = {}
+
+    def root(x):
+        while parent[x] != x:
+            parent[x] = x = parent[parent[x]]
+        return x
+
+    for blocks in kv_table:
+        first = blocks[0].index
+        if first not in parent:
+            parent[first] = first
+        r = root(first)
+        for block in blocks[1:]:
+            i = block.index
+            if i not in parent:
+                parent[i] = r
+            elif parent[i] != r and root(i) != r:
+                parent[root(i)] = r
+    numbers: Dict[int, int] = {}
+    ranks: Counter = Counter()
+    found = {}
+    for i in parent:
+        r = root(i)
+        found[i] = (numbers.setdefault(r, len(numbers)), ranks[r])
+        ranks[r] += 1
+    return found
+
+
 def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_block: int, n_slots: int) -> DkvGroups:
     result = DkvGroups()
     instrs = plan.instructions
@@ -154,14 +200,25 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
                 groups.append(Group(visits, dst))
                 result.skip_ops.setdefault(j, set()).add(op_pos)
                 continue
-            n_groups = -(-len(visits) // limit)
-            bounds = [len(visits) * i // n_groups for i in range(n_groups + 1)]
-            chunks = [visits[a:b] for a, b in zip(bounds, bounds[1:])]
+            chunks, at = [], 0
+            for size in _chunk_sizes(len(visits), limit) if len(visits) > limit else [len(visits)]:
+                chunks.append(visits[at : at + size])
+                at += size
             groups += [Group(chunk, slot(chunk[0])) for chunk in chunks]
             gone = {slot(v).index for chunk in chunks for v in chunk[1:]}
             ops = result.sources.setdefault(j, {})
             ops[op_pos] = [b for b in ops.get(op_pos, op.src_buffers)
                            if not (b.buffer_type == BufferType.BUFFER_dKV and b.index in gone)]
-        groups.sort(key=lambda g: -len(g.visits))
+        # longest first; among equals the same block of every sequence and head together: consecutive
+        # groups go to the XCDs in turn, so that the blocks of one head, whose rows are the same, meet on
+        # one XCD at about the same time (131072 tokens, window 4096, 8 kv heads: 15.6 -> 15.3 ms)
+        component = _components(instr.kv_block_table)
+
+        def place(group: Group):
+            row, pos = group.visits[0]
+            number, rank = component[instr.kv_block_table[row][pos].index]
+            return (-len(group.visits), rank, number)
+
+        groups.sort(key=place)
         result.groups[idx] = groups
     return result
