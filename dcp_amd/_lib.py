@@ -35,6 +35,7 @@ SIGNATURES = {
     "dcp_fused_copy_varlen_lse": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "dcp_update_out_lse": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _L, _L, _L, _L, _L, _L, _I, _I, _I, _P],
     "dcp_blockwise_sum": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _L, _I, _P],
+    "dcp_blockwise_sum_fp32_sources": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _L, _I, _P],
     "dcp_attn_fwd": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _L, _L, _I, _F, _I, _P, c_size_t, _P],
     "dcp_attn_fwd_workspace_bytes": [],
     "dcp_attn_bwd": [_P] * 10 + [c_size_t] + [_P] * 3 + [_I] + [_P] * 6 + [_I] * 7 + [_L] * 4 + [_I, _F, _I, _P],
@@ -42,7 +43,7 @@ SIGNATURES = {
                             + [_I, _F, _I, _P, c_size_t, _P],
     "dcp_attn_bwd_strided": [_P] * 10 + [c_size_t] + [_P] * 3 + [_I] + [_P] * 6 + [_I] * 7 + [_L] * 10 + [_F, _I, _P],
     "dcp_attn_bwd_grouped": [_P] * 10 + [c_size_t] + [_P] * 3 + [_I] + [_P] * 6 + [_I] * 7 + [_L] * 10
-                            + [_P, _I, _P, _P, _P, _L, _L, _F, _I, _P],
+                            + [_P, _I, _P, _P, _P, _L, _L, _P, _F, _I, _P],
     "dcp_attn_bwd_workspace_bytes_kv": [_I, _I, _L, _I, _I, _I],
     "dcp_attn_bwd_workspace_bytes": [_I, _I, _I, _I, _I],
     "dcp_attn_bwd_static": [_P] * 9 + [_P] * 3 + [_I] + [_P] * 6 + [_I] * 7 + [_L] * 4 + [_I, _F, _I, _P],

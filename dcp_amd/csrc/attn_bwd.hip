@@ -60,7 +60,8 @@ namespace dcp {
 // rows with a non-empty range; hull[4..7] = the intersection (core) of the
 // rows' ranges, empty as soon as one row has an empty range.
 __global__ __launch_bounds__(64) void bwd_tile_hull_kernel(const AttnBwdParams p) {
-  if (blockIdx.x == 0 && threadIdx.x < kTicketInts) p.tickets[threadIdx.x] = 0;  // for the dQ kernel that follows
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < 2 * kTicketInts; i += 64) p.tickets[i] = 0;  // for the kernels that follow
   const int b = blockIdx.x / p.q_tiles_per_row;
   const int qt = blockIdx.x - b * p.q_tiles_per_row;
   const int q_begin = p.cu_seqlens_q[b];
@@ -155,12 +156,16 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   // and drag every address derived from them there too: each tile load then costs three vector
   // instructions to rebuild a scalar base.  readfirstlane puts the indices back on the scalar unit.
   const int tile_no = __builtin_amdgcn_readfirstlane(wg % p.kv_tiles_per_row);
-  wg /= p.kv_tiles_per_row;
-  const int kv_head = __builtin_amdgcn_readfirstlane(wg % p.n_heads_kv);
-  const int item = __builtin_amdgcn_readfirstlane(wg / p.n_heads_kv);
+  const int kv_head = __builtin_amdgcn_readfirstlane(wg / p.kv_tiles_per_row % p.n_heads_kv);
+  const int item = __builtin_amdgcn_readfirstlane(wg / p.kv_tiles_per_row / p.n_heads_kv);
   const bool grouped = p.dkv_groups != nullptr;
   const int32_t* grp = p.dkv_groups + (grouped ? (int64_t)item * kDkvGroupInts : 0);
   const int n_visits = grouped ? grp[5] : 1;
+  const int group = p.n_heads_q / p.n_heads_kv;
+  // the part of the rows' queries this workgroup takes: q heads [hg_begin, hg_end) of the kv head's,
+  // every tile_parts-th 64-query tile
+  const int hg_begin = grouped ? grp[6] & 0xffff : 0, hg_end = grouped && grp[6] != 0 ? grp[6] >> 16 : group;
+  const int tile_parts = grouped ? grp[7] & 0xffff : 0, tile_part = grouped ? grp[7] >> 16 : 0;
   // lane v looks up visit v
   int row = 0, k_row = tile_no * BN;  // the row, and the row's position of the tile's first key
   if (!grouped) row = p.row_order ? p.row_order[item] : item;
@@ -193,7 +198,6 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   const int blk = grouped ? 0 : __builtin_amdgcn_readfirstlane(kw_safe / p.block_size);
   const int tok0 = kw_safe - blk * p.block_size;
   const int64_t table_at = grouped ? 0 : (int64_t)__builtin_amdgcn_readfirstlane(row) * p.max_kv_blocks + blk;
-  const int group = p.n_heads_q / p.n_heads_kv;
   const int64_t q_row_stride = (int64_t)p.n_heads_q * D;
   const int64_t kv_tile_off = (int64_t)(grouped ? grp[0] : p.kv_block_table[table_at]) * p.kv_slot_stride +
                               (int64_t)tok0 * p.kv_token_stride + (int64_t)kv_head * D;
@@ -221,7 +225,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     const int vrow = __builtin_amdgcn_readlane(row, v), k0 = __builtin_amdgcn_readlane(mine.k_row, v);
     const int n_tiles = (__builtin_amdgcn_readlane(mine.seqlen_q, v) + BM - 1) / BM;
     i32x4 h0 = {0x7fffffff, 0, 0x7fffffff, 0}, h1 = {0x7fffffff, 0, 0x7fffffff, 0};
-    if (lane < n_tiles) {
+    if (lane < n_tiles && (tile_parts == 0 || lane % tile_parts == tile_part)) {
       const i32x4* hu = reinterpret_cast<const i32x4*>(p.hull + ((int64_t)vrow * p.q_tiles_per_row + lane) * 8);
       h0 = hu[0];
       h1 = hu[1];
@@ -276,7 +280,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   const char* sc_base0 = role_rng   ? reinterpret_cast<const char*>(p.attn_range + (int64_t)sc_plane * p.total_q)
                          : role_lse ? reinterpret_cast<const char*>(p.lse2)
                                     : reinterpret_cast<const char*>(p.delta);
-  const int64_t sc_head_bytes = role_rng ? 0 : 4;
+  const int sc_head_bytes = role_rng ? 0 : 4;
   const int64_t sc_second_bytes = role_rng ? (int64_t)p.total_q * 4 : 0;
   const int sc_query_bytes = role_rng ? 4 : p.n_heads_q * 4;
   const uint32_t sc_at0 = role_rng ? rng_at + (2 * w * BM) * 4 : role_lse ? lse_at : delta_at;
@@ -297,7 +301,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     req_seqlen_q = visit_field(v, DkvVisit::kSeqlenQ);
   };
   // ... and of the one whose step is multiplied.
-  int seqlen_q = 0, kv_or_beyond = 0;  // kv_or_beyond: this lane's key, for the range tests
+  int seqlen_q = 0;
   unsigned long long unm_w = 0;
   // dS pieces (WRITE_DS).  The workspace holds the rows one after another; row b starts at 64-key
   // tile cu_seqlens_kv[b] / 64 + b (room for a last, partial tile of every row before it) and is laid
@@ -313,11 +317,10 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   const int ds_lane = (w & 1) * 128 + 2 * c + h;
   auto begin_visit = [&](int v) {
     KernArgs<AttnBwdParams>& p = fresh_kernel_args<AttnBwdParams>();
-    const int seqlen_kv = visit_field(v, DkvVisit::kSeqlenKv), kw = visit_field(v, DkvVisit::kKRow) + w * 32;
     seqlen_q = visit_field(v, DkvVisit::kSeqlenQ);
-    kv_or_beyond = kw + c < seqlen_kv ? kw + c : 0x7fffffff;
     unm_w = uniform64(mask_lds[v][1 + w]);
     if constexpr (WRITE_DS) {
+      const int seqlen_kv = visit_field(v, DkvVisit::kSeqlenKv), kw = visit_field(v, DkvVisit::kKRow) + w * 32;
       ds_row_tiles = has_keys ? (seqlen_kv + 63) / 64 : 0;
       const uint64_t piece = (uint64_t)visit_field(v, DkvVisit::kDsTile0) * p.n_heads_q * p.subs_per_row +
                              (uint64_t)(kv_head * group) * p.subs_per_row * ds_row_tiles + (kw >> 6);
@@ -329,7 +332,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     return v;
   };
   auto request_scalars = [&](int head, int qt, int st) {
-    const int ql = min(qt * BM + lane, req_seqlen_q - 1);
+    const int ql = min(qt * BM + lane_here(), req_seqlen_q - 1);
     const char* base = sc_base + head * sc_head_bytes;
     const uint32_t at = sc_at0 + st * sc_at_stage, voff = (uint32_t)(ql * sc_query_bytes);
     load_async_dword(at, voff, base);
@@ -337,14 +340,14 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   };
 
   // steps: (visit) x (q head of the group) x (active 64-query tile)
-  int visit = next_active(0), hg = 0;
+  int visit = next_active(0), hg = hg_begin;
   unsigned long long act_mask = 0, rem = 0;  // active tiles of the visit; tiles of head hg still to do
   int st = 0;
   if (visit < n_visits) {
     act_mask = rem = uniform64(mask_lds[visit][0]);
     begin_requests(visit);
     begin_visit(visit);
-    const int qt = __builtin_ctzll(rem), head = kv_head * group;
+    const int qt = __builtin_ctzll(rem), head = kv_head * group + hg_begin;
     request_scalars(head, qt, 0);
     const int64_t off = (int64_t)qt * BM * q_row_stride + (int64_t)head * D;
 #pragma unroll
@@ -373,10 +376,10 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     }
     if (rem == 0) {
       rem = act_mask;
-      if (++hg_next == group) {
+      if (++hg_next == hg_end) {
         visit_next = next_active(visit + 1);
         if (visit_next < n_visits) {
-          hg_next = 0;
+          hg_next = hg_begin;
           act_mask = rem = uniform64(mask_lds[visit_next][0]);
           begin_requests(visit_next);
         }
@@ -416,6 +419,8 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
 #pragma unroll
         for (int i = 0; i < 16; ++i) s_acc[i] = 0.0f;
       } else {
+        const int my_key = visit_lds[visit].k_row + w * 32 + (lane_here() & 31);
+        const int kv_or_beyond = my_key < visit_lds[visit].seqlen_kv ? my_key : 0x7fffffff;  // this lane's key, for the range tests
         // the four queries of an accumulator register group are consecutive: their range planes
         // come in 16-byte reads, requested together before the comparisons.  With one range the
         // second range's planes hold the first's again (see request_scalars): the union is the same.
@@ -553,24 +558,49 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
 
   // ---- dK and dV of the wave's keys are complete: scale, round, store ---------------------
   wait_loads();  // the last step's (unused) requests must land before the workgroup's LDS is released
-  if (!has_keys) return;
-  // a group's result goes to a slot of dk/dv or, where nothing else is added to it, to the caller's
-  // unpadded tensor, of which only the block's own tokens may be written
+  // (what the loop did not need is worked out from the item's number again)
   KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
-  int entry, in_unpadded = 0;
+  asm volatile("" : "+s"(wg));
+  const int out_item = __builtin_amdgcn_readfirstlane(wg / args.kv_tiles_per_row / args.n_heads_kv);
+  const int out_head = __builtin_amdgcn_readfirstlane(wg / args.kv_tiles_per_row % args.n_heads_kv);
+  const int out_key = __builtin_amdgcn_readfirstlane(wg % args.kv_tiles_per_row) * BN + w * 32;
+  // a group's result goes to a slot of dk/dv; or, where nothing else is added to it, to the caller's
+  // unpadded tensor, of which only the block's own tokens may be written; or it is partial
+  int entry, where = 0, token = out_key + c;
   if (args.dkv_groups != nullptr) {
-    const int32_t* grp = args.dkv_groups + (int64_t)item * kDkvGroupInts;
+    const int32_t* grp = args.dkv_groups + (int64_t)out_item * kDkvGroupInts;
     entry = grp[1];
-    in_unpadded = grp[3];
-    if (tok0 + c >= grp[2]) return;
+    where = grp[3];
+    if (token >= grp[2]) return;
   } else {
+    if (out_key >= visit_field(0, DkvVisit::kSeqlenKv)) return;  // a wave without keys
+    const int blk = __builtin_amdgcn_readfirstlane(out_key / args.block_size);
     entry = args.dkv_block_table[(int64_t)visit_field(0, DkvVisit::kRow) * args.max_kv_blocks + blk];
+    token -= blk * args.block_size;
   }
-  const int64_t off = (int64_t)entry * (in_unpadded ? args.dkv2_entry_stride : args.dkv_slot_stride) +
-                      (int64_t)(tok0 + c) * (in_unpadded ? args.dkv2_token_stride : args.dkv_token_stride) + (int64_t)kv_head * D + 4 * h;
-  uint16_t* dv_dst = reinterpret_cast<uint16_t*>(in_unpadded ? args.dv2 : args.dv) + off;
-  uint16_t* dk_dst = reinterpret_cast<uint16_t*>(in_unpadded ? args.dk2 : args.dk) + off;
   const float scale = args.scale;
+  if (where == 2) {  // a part's share, to be added to the other parts' by a sum kernel
+    const int64_t head_row = (int64_t)args.n_heads_kv * D;
+    float* dst = args.dkv_partials + ((int64_t)entry * args.block_size + token) * (2 * head_row) + (int64_t)out_head * D + 4 * h;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 k4, v4;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          k4[r] = dk_acc[dt][4 * g + r] * scale;
+          v4[r] = dv_acc[dt][4 * g + r];
+        }
+        *reinterpret_cast<f32x4*>(dst + dt * 32 + 8 * g) = k4;
+        *reinterpret_cast<f32x4*>(dst + head_row + dt * 32 + 8 * g) = v4;
+      }
+    return;
+  }
+  const int64_t off = (int64_t)entry * (where ? args.dkv2_entry_stride : args.dkv_slot_stride) +
+                      (int64_t)(token) * (where ? args.dkv2_token_stride : args.dkv_token_stride) + (int64_t)out_head * D + 4 * h;
+  uint16_t* dv_dst = reinterpret_cast<uint16_t*>(where ? args.dv2 : args.dv) + off;
+  uint16_t* dk_dst = reinterpret_cast<uint16_t*>(where ? args.dk2 : args.dk) + off;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -591,12 +621,17 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
 template <int DTYPE, int D, bool WRITE_DS>
 __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const AttnBwdParams p) {
   __shared__ int ticket_lds;
+  int item = 0;
+  {
+    KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
+    item = first_item({args.dkv_tickets, kTicketStride, args.n_dkv_items, args.dkv_xcd_group});
+  }
   while (true) {
     KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
-    const int item = next_item({args.dkv_tickets, args.n_dkv_items, args.dkv_xcd_group}, &ticket_lds);
+    if (item < 0) item = next_item({args.dkv_tickets, kTicketStride, args.n_dkv_items, args.dkv_xcd_group}, &ticket_lds);
     if (item < 0) break;
     attn_bwd_dkv_item<DTYPE, D, WRITE_DS>(args, item);
-    if (fresh_kernel_args<AttnBwdParams>().dkv_tickets == nullptr) break;
+    item = -1;
   }
 }
 
@@ -896,12 +931,17 @@ __device__ __forceinline__ void attn_bwd_dq_item(KernArgs<AttnBwdParams>& p, int
 template <int DTYPE, int D>
 __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dq_kernel(const AttnBwdParams p) {
   __shared__ int ticket_lds;
+  int item = 0;
+  {
+    KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
+    item = first_item({args.dq_tickets, kTicketStride, args.n_dq_items, args.dq_xcd_group});
+  }
   while (true) {
     KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
-    const int item = next_item({args.dq_tickets, args.n_dq_items, args.dq_xcd_group}, &ticket_lds);
+    if (item < 0) item = next_item({args.dq_tickets, kTicketStride, args.n_dq_items, args.dq_xcd_group}, &ticket_lds);
     if (item < 0) break;
     attn_bwd_dq_item<DTYPE, D>(args, item);
-    if (fresh_kernel_args<AttnBwdParams>().dq_tickets == nullptr) break;
+    item = -1;
   }
 }
 
@@ -909,7 +949,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dq_kernel(const AttnB
 static int64_t dkv_grid(AttnBwdParams& p) {
   const int64_t resident = xcd_grid_size((p.head_dim == 128 ? 2 : 3) * (int64_t)device_cu_count(), 1);
   const int64_t n = xcd_grid_size(p.n_dkv_items, 1);
-  p.dkv_tickets = p.dkv_groups != nullptr && n > resident ? p.tickets + kNumXcd : nullptr;
+  p.dkv_tickets = p.dkv_groups != nullptr && n > resident ? p.tickets + kTicketInts : nullptr;
   return p.dkv_tickets ? resident : n;
 }
 
@@ -961,7 +1001,7 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 static size_t bwd_base_workspace_bytes(int batch, int total_q, int block_size, int n_heads_q) {
   const size_t q_tiles = (size_t)batch * ((block_size + kBwdBM - 1) / kBwdBM);
   return 2 * align256((size_t)total_q * n_heads_q * sizeof(float)) + align256(q_tiles * 8 * sizeof(int32_t)) +
-         align256(kTicketInts * sizeof(int32_t));
+         align256(2 * kTicketInts * sizeof(int32_t));
 }
 
 extern "C" size_t dcp_attn_bwd_workspace_bytes(int batch, int total_q, int block_size, int n_heads_q,
@@ -979,6 +1019,7 @@ struct DkvGrouping {
   void* dk2;
   void* dv2;
   int64_t entry_stride, token_stride;
+  float* partials;
 };
 
 // All entry points: argument checks, workspace carving, the launches.
@@ -1035,8 +1076,9 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
     DCP_REQUIRE(block_size % kDkvBN == 0, "attn_bwd_grouped: block_size %d must be a multiple of %d", block_size, kDkvBN);
     DCP_REQUIRE(!grouping->dk2 == !grouping->dv2 && (!grouping->dk2 || (grouping->entry_stride > 0 && grouping->token_stride > 0 &&
                 grouping->entry_stride % 4 == 0 && grouping->token_stride % 4 == 0)) &&
-                    ((reinterpret_cast<uintptr_t>(grouping->dk2) | reinterpret_cast<uintptr_t>(grouping->dv2)) & 7) == 0,
-                "attn_bwd_grouped: the unpadded dk/dv must be 8-byte aligned, with strides that are multiples of 4 elements");
+                    ((reinterpret_cast<uintptr_t>(grouping->dk2) | reinterpret_cast<uintptr_t>(grouping->dv2)) & 7) == 0 &&
+                    (reinterpret_cast<uintptr_t>(grouping->partials) & 15) == 0,
+                "attn_bwd_grouped: the partials must be 16-byte aligned, the unpadded dk/dv must be 8-byte aligned, with strides that are multiples of 4 elements");
   }
   const bool fused = allow_fused && !grouping && head_dim == 128 && bwd_fused_available() && workspace_bytes >= base + extra;
   // The backward through dS in memory where it is selected, the caller said how many keys the rows
@@ -1065,7 +1107,7 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
   ws += align256((size_t)batch * ((block_size + kBwdBM - 1) / kBwdBM) * 8 * sizeof(int32_t));
   p.tickets = reinterpret_cast<int*>(ws);
   p.dq_tickets = p.dkv_tickets = nullptr;  // (the launchers say)
-  ws += align256(kTicketInts * sizeof(int32_t));
+  ws += align256(2 * kTicketInts * sizeof(int32_t));
   p.subs_per_row = (block_size + 31) / 32;
   p.head_dim = head_dim;
   p.dq_part = nullptr;
@@ -1113,6 +1155,7 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
   p.dkv_visits = grouping ? grouping->visits : nullptr;
   p.dk2 = grouping ? grouping->dk2 : nullptr;
   p.dv2 = grouping ? grouping->dv2 : nullptr;
+  p.dkv_partials = grouping ? grouping->partials : nullptr;
   p.dkv2_entry_stride = grouping ? grouping->entry_stride : 0;
   p.dkv2_token_stride = grouping ? grouping->token_stride : 0;
   p.kv_tiles_per_row = grouping ? block_size / kDkvBN : (int)(((int64_t)max_kv_blocks * block_size + kDkvBN - 1) / kDkvBN);
@@ -1197,16 +1240,17 @@ extern "C" int dcp_attn_bwd_grouped(const void* dout, const void* q, const void*
                                     int64_t dq_slot_stride, int64_t lse_head_stride, int64_t lse_slot_stride,
                                     int64_t total_kv, const int32_t* dkv_groups, int n_groups,
                                     const int32_t* dkv_visits, void* dk_unpadded, void* dv_unpadded,
-                                    int64_t unpadded_entry_stride, int64_t unpadded_token_stride,
+                                    int64_t unpadded_entry_stride, int64_t unpadded_token_stride, float* partials,
                                     float softmax_scale, int dtype, void* stream) {
   DCP_RECORDED(dcp_attn_bwd_grouped(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
       cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table, dq_block_table,
       dkv_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim,
       kv_slot_stride, kv_token_stride, dkv_slot_stride, dkv_token_stride, q_slot_stride, out_slot_stride,
       dq_slot_stride, lse_head_stride, lse_slot_stride, total_kv, dkv_groups, n_groups, dkv_visits, dk_unpadded,
-      dv_unpadded, unpadded_entry_stride, unpadded_token_stride, softmax_scale, dtype, stream));
+      dv_unpadded, unpadded_entry_stride, unpadded_token_stride, partials,
+      softmax_scale, dtype, stream));
   const DkvGrouping grouping = {dkv_groups, n_groups, dkv_visits, dk_unpadded, dv_unpadded, unpadded_entry_stride,
-                                unpadded_token_stride};
+                                unpadded_token_stride, partials};
   return attn_bwd_launch(dout, q, k, v, out, lse, dq, dk, dv, workspace, workspace_bytes, cu_seqlens_q,
                          cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table,
                          dq_block_table, dkv_block_table, row_order, batch, max_kv_blocks, total_q, block_size,

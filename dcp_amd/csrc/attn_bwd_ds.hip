@@ -279,12 +279,17 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
 template <int DTYPE, int D, int HH>
 __global__ __launch_bounds__(kDsThreads, 1) void attn_bwd_dq_ds_kernel(const AttnBwdParams p) {
   __shared__ int ticket_lds;
+  int item = 0;
+  {
+    KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
+    item = first_item({args.dq_tickets, kTicketStride, args.n_dq_items, args.dq_xcd_group});
+  }
   while (true) {
     KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
-    const int item = next_item({args.dq_tickets, args.n_dq_items, args.dq_xcd_group}, &ticket_lds);
+    if (item < 0) item = next_item({args.dq_tickets, kTicketStride, args.n_dq_items, args.dq_xcd_group}, &ticket_lds);
     if (item < 0) break;
     attn_bwd_dq_ds_item<DTYPE, D, HH>(args, item);
-    if (fresh_kernel_args<AttnBwdParams>().dq_tickets == nullptr) break;
+    item = -1;
   }
 }
 

@@ -78,7 +78,8 @@ __global__ __launch_bounds__(kBwdThreads) void bwd_prepare_kernel(const AttnBwdP
   const int b = blockIdx.x / p.q_tiles_per_row;
   const int qt = blockIdx.x - b * p.q_tiles_per_row;
   if (blockIdx.x == 0 && tid == 0 && p.fault != nullptr) *p.fault = 0;
-  if (blockIdx.x == 0 && tid < kTicketInts) p.tickets[tid] = 0;  // for a persistent dQ kernel that follows
+  if (blockIdx.x == 0)
+    for (int i = tid; i < 2 * kTicketInts; i += kBwdThreads) p.tickets[i] = 0;  // for the kernels that follow
   const int q_begin = p.cu_seqlens_q[b];
   const int seqlen_q = p.cu_seqlens_q[b + 1] - q_begin;
   const int seqlen_kv = p.cu_seqlens_kv[b + 1] - p.cu_seqlens_kv[b];

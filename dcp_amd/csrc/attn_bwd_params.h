@@ -18,9 +18,9 @@ struct AttnBwdParams {
   float* delta;      // [total_q, H]: MINUS rowsum(dO * O)
   float* lse2;       // [total_q, H]: lse * log2(e); both written by the dQ kernel, read by the dK/dV kernel
   int32_t* hull;     // [batch * q_tiles_per_row, 8]
-  int* tickets;      // work-item counters of the persistent dQ kernel (kTicketInts); zeroed by the hull kernel
-  int* dkv_tickets;
-  int* dq_tickets;   // the same where the dQ kernel has more items than workgroups, else null
+  int* tickets;      // counters of the dQ and the dK/dV kernel's item queues (2 kTicketInts); zeroed by the hull / prepare kernel
+  int* dkv_tickets;  // the dK/dV kernel's where it has more items than workgroups, else null
+  int* dq_tickets;   // the dQ kernel's likewise
   // the one-pass backward only (attn_bwd_fused.hip):
   float* dq_part;    // [batch * n_heads_q * subs_per_row][4096]: partial dQ of a (row, head, 32-query) chunk, fp32
   int* chain;        // [batch * n_heads_q * subs_per_row][4]: links of the chunk's chain done so far, per wave
@@ -63,6 +63,7 @@ struct AttnBwdParams {
   const int32_t* dkv_visits;  // [..][2]: row, index of the block in the row's kv_block_table
   void* dk2;                  // where groups marked unpadded go
   void* dv2;
+  float* dkv_partials;        // where groups marked partial go
   int64_t dkv2_entry_stride;
   int64_t dkv2_token_stride;
   int dkv_xcd_group;     // dK/dV work items sharing one Q/dO stream (the key tiles of a row)
@@ -84,9 +85,10 @@ constexpr int kPrioMatrix = 2, kPrioVector = 0;
 constexpr int kBwdBM = 64;
 constexpr int kBwdBN = 64;
 constexpr int kBwdThreads = 256;
+constexpr int kTicketStride = 32;  // a counter per cache line
+constexpr int kTicketInts = kNumXcd * kTicketStride;
 constexpr int kDkvGroupInts = 8;
 constexpr int kDkvMaxVisits = DCP_ATTN_BWD_MAX_VISITS;
-constexpr int kTicketInts = 16;  // one counter per XCD (the rest unused)
 
 // The backward through dS in memory: prepare (hulls, -delta, lse2), the dK/dV kernel writing dS, the
 // dQ kernel that reads it back (attn_bwd_ds.hip); the pieces it is made of live in three files.

@@ -154,6 +154,14 @@ __device__ __forceinline__ void load_async_dword(uint32_t lds_at, uint32_t lane_
                : "memory");
 }
 
+// The lane's number, worked out where it is used: unlike one derived from threadIdx.x, which the compiler
+// keeps in a register of its own through every loop around.
+__device__ __forceinline__ int lane_here() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
+}
+
 // A 64-bit value that every lane holds alike, moved to scalar registers.
 __device__ __forceinline__ uint64_t uniform64(uint64_t a) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
@@ -319,33 +327,41 @@ inline int64_t xcd_grid_size(int64_t total, int group) {
 // counter per XCD.  An XCD that has run out takes from the one with the most items left: streams are
 // not equally long, and a launch with fewer than a few hundred streams need not even have the same
 // number of them on every XCD.
+//
+// A workgroup's first item is fixed by its number: with every workgroup of the launch drawing its first
+// ticket from counters in one cache line, the line went around the XCDs' caches for each of them,
+// 45 us for 768 workgroups.
 struct ItemQueue {
-  int* tickets;     // kNumXcd counters, zero before the launch; null: one item per workgroup, item = workgroup id
+  int* tickets;     // kNumXcd counters, zero before the launch; null: one item per workgroup
+  int stride;       // ints from one counter to the next
   int64_t n_items;  // a multiple of group
   int group;
 };
-// The workgroup's next item, or -1.  `box`: a word of LDS.  Contains the barriers that separate one
-// item's use of LDS from the next one's.  (Without tickets the workgroup's only item, at every call.)
+__device__ __forceinline__ int items_of_xcd(int n_streams, int group, int x) {
+  return n_streams > x ? (n_streams - x + kNumXcd - 1) / kNumXcd * group : 0;
+}
+// The workgroup's first item, or -1 (with a queue, next_item may still have one).
+__device__ __forceinline__ int first_item(const ItemQueue& queue) {
+  const int w = blockIdx.x, group = queue.group, x = w % kNumXcd, i = w / kNumXcd;
+  const int item = __builtin_amdgcn_readfirstlane((x + kNumXcd * (i / group)) * group + i % group);
+  if (queue.tickets != nullptr) return i < items_of_xcd((int)(queue.n_items / group), group, x) ? item : -1;
+  // as many workgroups as items: whole streams by XCD as long as every XCD gets one more, the rest
+  // item by item over all of them
+  if (w >= queue.n_items) return -1;
+  return w < (int)(queue.n_items / (kNumXcd * group)) * kNumXcd * group ? item : w;
+}
+// Its next item, or -1.  `box`: a word of LDS.  Contains the barriers that separate one item's use of LDS
+// from the next one's.
 __device__ __forceinline__ int next_item(const ItemQueue& queue, int* box) {
-  if (queue.tickets == nullptr) {
-    // as many workgroups as items: whole streams by XCD as long as every XCD gets one more, the rest
-    // item by item over all of them
-    const int w = blockIdx.x, group = queue.group;
-    if (w >= queue.n_items) return -1;
-    const int in_turns = (int)(queue.n_items / (kNumXcd * group)) * kNumXcd * group;
-    if (w >= in_turns) return w;
-    const int i = w / kNumXcd;
-    return __builtin_amdgcn_readfirstlane((w % kNumXcd + kNumXcd * (i / group)) * group + i % group);
-  }
+  if (queue.tickets == nullptr) return -1;
   __syncthreads();  // everybody has read the last ticket and is done with the last item's LDS
   if (threadIdx.x == 0) {
     const int group = queue.group, n_streams = (int)(queue.n_items / group);
-    const int own = blockIdx.x % kNumXcd;
-    auto items_of = [&](int x) { return n_streams > x ? (n_streams - x + kNumXcd - 1) / kNumXcd * group : 0; };
-    int x = own, found = -1;
+    const int n_first = gridDim.x / kNumXcd;  // items of every XCD that went out as first ones
+    int x = blockIdx.x % kNumXcd, found = -1;
     while (true) {
-      const int i = atomicAdd(&queue.tickets[x], 1);
-      if (i < items_of(x)) {
+      const int i = n_first + atomicAdd(&queue.tickets[x * queue.stride], 1);
+      if (i < items_of_xcd(n_streams, group, x)) {
         const int s = i / group;
         found = (x + kNumXcd * s) * group + (i - s * group);
         break;
@@ -353,7 +369,8 @@ __device__ __forceinline__ int next_item(const ItemQueue& queue, int* box) {
       // (the counters only grow, so every round either takes an item or finds one queue fewer to ask)
       int most = 0;
       for (int y = 0; y < kNumXcd; ++y) {
-        const int left = items_of(y) - __hip_atomic_load(&queue.tickets[y], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int taken = n_first + __hip_atomic_load(&queue.tickets[y * queue.stride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int left = items_of_xcd(n_streams, group, y) - taken;
         if (left > most) {
           most = left;
           x = y;

@@ -82,6 +82,8 @@ struct AttnFwdParams {
 // (2-3 % on the kernel), and the fused phase, whose vector work is the longer chain, outranks
 // the dense one (another 1.5 %; the other way round it was 1.5 % slower).
 constexpr int kPrioControl = 0, kPrioFused = 2, kPrioDense = 1;
+constexpr int kFwdTicketStride = 8;  // (the workspace is small: two cache lines of counters)
+constexpr int kFwdTicketInts = kNumXcd * kFwdTicketStride;
 constexpr int kFwdBN = 64;
 constexpr int kFwdThreads = 256;
 // The running maximum of a row is only raised (and O^T rescaled) when the tile's maximum
@@ -585,24 +587,29 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
 template <int DTYPE, int D, int QB>
 __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(const AttnFwdParams p) {
   __shared__ int ticket_lds;
+  int item = 0;
+  {
+    KernArgs<AttnFwdParams>& args = fresh_kernel_args<AttnFwdParams>();
+    item = first_item({args.tickets, kFwdTicketStride, args.n_items, args.xcd_group});
+  }
   while (true) {
     KernArgs<AttnFwdParams>& args = fresh_kernel_args<AttnFwdParams>();
-    const int item = next_item({args.tickets, args.n_items, args.xcd_group}, &ticket_lds);
+    if (item < 0) item = next_item({args.tickets, kFwdTicketStride, args.n_items, args.xcd_group}, &ticket_lds);
     if (item < 0) break;
     attn_fwd_item<DTYPE, D, QB>(args, item);
-    if (fresh_kernel_args<AttnFwdParams>().tickets == nullptr) break;
+    item = -1;
   }
 }
 
 __global__ void attn_fwd_reset_tickets_kernel(int* tickets) {
-  if (threadIdx.x < kNumXcd) tickets[threadIdx.x] = 0;
+  if (threadIdx.x < kFwdTicketInts) tickets[threadIdx.x] = 0;
 }
 
 }  // namespace dcp
 
 using namespace dcp;
 
-extern "C" size_t dcp_attn_fwd_workspace_bytes(void) { return 16 * sizeof(int32_t); }
+extern "C" size_t dcp_attn_fwd_workspace_bytes(void) { return kFwdTicketInts * sizeof(int32_t); }
 
 extern "C" int dcp_attn_fwd(const void* q, const void* k, const void* v, void* out, float* lse,
                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
@@ -707,7 +714,7 @@ extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v,
   const int64_t n_wg = std::min<int64_t>(xcd_grid_size(p.n_items, 1), xcd_grid_size(2 * (int64_t)device_cu_count(), 1));
   p.tickets = p.n_items > n_wg ? reinterpret_cast<int*>(workspace) : nullptr;
   dim3 grid((unsigned)n_wg), block(kFwdThreads);
-  if (p.tickets) hipLaunchKernelGGL(attn_fwd_reset_tickets_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, p.tickets);
+  if (p.tickets) hipLaunchKernelGGL(attn_fwd_reset_tickets_kernel, dim3(1), dim3(kFwdTicketInts), 0, (hipStream_t)stream, p.tickets);
   KernelTimer timer("attn_fwd_kernel", stream);
 #define DCP_FWD(DT, HD) \
   hipLaunchKernelGGL((attn_fwd_kernel<DT, HD, 1>), grid, block, 0, (hipStream_t)stream, p)

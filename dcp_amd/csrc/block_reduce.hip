@@ -587,7 +587,9 @@ static int launch_merge(const void* src_out, void* dst_out, const float* src_lse
 constexpr int kSumThreads = 64;
 constexpr int kSumUnroll = 1;
 
-template <int DTYPE, int THREADS, int kSumUnroll>
+// SRC: type of the sources, DTYPE or fp32 (partial sums that have not been rounded yet; a single one is
+// rounded, not copied).
+template <int DTYPE, int SRC, int THREADS, int kSumUnroll>
 __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
     const int64_t* __restrict__ src_ptrs, const int32_t* __restrict__ src_offsets,
     const int32_t* __restrict__ src_strides, const int32_t* __restrict__ n_ops_per_block,
@@ -595,7 +597,9 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
     const int32_t* __restrict__ dst_strides, const int32_t* __restrict__ n_elements,
     int max_n_ops_per_block, int chunks_per_sum) {
   typedef typename Elem<DTYPE>::raw raw;
+  typedef typename Elem<SRC>::raw src_raw;
   constexpr int VN = Vec16<DTYPE>::N;
+  constexpr int WORDS = VN / Vec16<SRC>::N;  // 16-byte words of a source per word of the result
   const int s = blockIdx.x / chunks_per_sum;
   const int64_t n_elem = n_elements[s];
   const int64_t chunk_elems = (int64_t)THREADS * VN * kSumUnroll;
@@ -605,7 +609,7 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
 
   const int n_ops = n_ops_per_block[s];
   const int32_t* offs = src_offsets + (int64_t)s * max_n_ops_per_block;
-  const raw* src = reinterpret_cast<const raw*>(src_ptrs[s]);
+  const src_raw* src = reinterpret_cast<const src_raw*>(src_ptrs[s]);
   const int64_t src_stride = src_strides[s];
   raw* dst = reinterpret_cast<raw*>(dst_ptrs[s]) + (int64_t)dst_offsets[s] * dst_strides[s];
 
@@ -627,8 +631,8 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
 #pragma unroll
       for (int k = 0; k < VN; ++k) acc[u][k] = 0.0f;
     }
-    if (begin < vec_end && n_ops == 1) {  // a single source: the scatter-back, copied bit for bit
-      const raw* row = src + offs[0] * src_stride;
+    if (begin < vec_end && n_ops == 1 && SRC == DTYPE) {  // a single source: the scatter-back, copied bit for bit
+      const src_raw* row = src + offs[0] * src_stride;
       u32x4 bits[kSumUnroll];
 #pragma unroll
       for (int u = 0; u < kSumUnroll; ++u) bits[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + pos[u]));
@@ -637,19 +641,28 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
         if (live[u]) __builtin_nontemporal_store(bits[u], reinterpret_cast<u32x4*>(dst + pos[u]));
     } else if (begin < vec_end) {
       for (int j0 = 0; j0 < n_ops; j0 += 4) {
-        u32x4 bits[4][kSumUnroll];
+        u32x4 bits[4][kSumUnroll][WORDS];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const raw* row = src + offs[min(j0 + q, n_ops - 1)] * src_stride;  // tail: re-read the last source
+          const src_raw* row = src + offs[min(j0 + q, n_ops - 1)] * src_stride;  // tail: re-read the last source
 #pragma unroll
           for (int u = 0; u < kSumUnroll; ++u)
-            bits[q][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + pos[u]));
+#pragma unroll
+            for (int k = 0; k < WORDS; ++k)
+              bits[q][u][k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + pos[u]) + k);
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           if (j0 + q >= n_ops) break;
 #pragma unroll
-          for (int u = 0; u < kSumUnroll; ++u) fma_vec16<DTYPE>(acc[u], 1.0f, bits[q][u]);
+          for (int u = 0; u < kSumUnroll; ++u) {
+            if constexpr (WORDS == 1) {
+              fma_vec16<SRC>(acc[u], 1.0f, bits[q][u][0]);
+            } else {
+#pragma unroll
+              for (int k = 0; k < VN; ++k) acc[u][k] += __uint_as_float(bits[q][u][k / 4][k % 4]);
+            }
+          }
         }
       }
 #pragma unroll
@@ -658,12 +671,14 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
     }
   }
   for (int64_t i = vec_end + threadIdx.x; i < end; i += THREADS) {
-    if (n_ops == 1) {
-      dst[i] = src[offs[0] * src_stride + i];
-      continue;
+    if constexpr (SRC == DTYPE) {
+      if (n_ops == 1) {
+        dst[i] = src[offs[0] * src_stride + i];
+        continue;
+      }
     }
     float acc = 0.0f;
-    for (int j = 0; j < n_ops; ++j) acc += Elem<DTYPE>::load(src[offs[j] * src_stride + i]);
+    for (int j = 0; j < n_ops; ++j) acc += Elem<SRC>::load(src[offs[j] * src_stride + i]);
     dst[i] = Elem<DTYPE>::store(acc);
   }
 }
@@ -712,14 +727,10 @@ extern "C" int dcp_update_out_lse(const void* src_out, void* dst_out, const floa
 #undef DCP_MERGE_ARGS
 }
 
-extern "C" int dcp_blockwise_sum(const int64_t* src_ptrs, const int32_t* src_offsets,
-                                 const int32_t* src_strides, const int32_t* n_ops_per_block,
-                                 const int64_t* dst_ptrs, const int32_t* dst_offsets,
-                                 const int32_t* dst_strides, const int32_t* n_elements,
-                                 int n_sums, int max_n_ops_per_block, int64_t block_numel,
-                                 int dtype, void* stream) {
-  DCP_RECORDED(dcp_blockwise_sum(src_ptrs, src_offsets, src_strides, n_ops_per_block, dst_ptrs, dst_offsets,
-      dst_strides, n_elements, n_sums, max_n_ops_per_block, block_numel, dtype, stream));
+static int blockwise_sum(const int64_t* src_ptrs, const int32_t* src_offsets, const int32_t* src_strides,
+                         const int32_t* n_ops_per_block, const int64_t* dst_ptrs, const int32_t* dst_offsets,
+                         const int32_t* dst_strides, const int32_t* n_elements, int n_sums, int max_n_ops_per_block,
+                         int64_t block_numel, int dtype, bool fp32_sources, void* stream) {
   const int esize = dtype_size(dtype);
   if (esize == 0) return fail(DCP_ERR_UNSUPPORTED, "Unsupported dtype: %d", dtype);
   DCP_REQUIRE(n_sums >= 0 && block_numel >= 0 && max_n_ops_per_block >= 1, "sum: bad size");
@@ -733,21 +744,38 @@ extern "C" int dcp_blockwise_sum(const int64_t* src_ptrs, const int32_t* src_off
               (long long)block_numel);
   dim3 grid((unsigned)(chunks * n_sums));
   KernelTimer timer("blockwise_sum_kernel", stream);
-#define DCP_SUM_LAUNCH(DT)                                                                          \
-  hipLaunchKernelGGL((blockwise_sum_kernel<DT, kSumThreads, kSumUnroll>), grid, dim3(kSumThreads), 0, \
-                     (hipStream_t)stream, src_ptrs, src_offsets, src_strides, n_ops_per_block,      \
-                     dst_ptrs, dst_offsets, dst_strides, n_elements, max_n_ops_per_block, (int)chunks)
-  switch (dtype) {
-    case DCP_DTYPE_BF16:
-      DCP_SUM_LAUNCH(DCP_DTYPE_BF16);
-      break;
-    case DCP_DTYPE_FP16:
-      DCP_SUM_LAUNCH(DCP_DTYPE_FP16);
-      break;
-    default:
-      DCP_SUM_LAUNCH(DCP_DTYPE_FP32);
-      break;
-  }
-#undef DCP_SUM_LAUNCH
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kSumThreads), 0, (hipStream_t)stream, src_ptrs, src_offsets, src_strides,
+                       n_ops_per_block, dst_ptrs, dst_offsets, dst_strides, n_elements, max_n_ops_per_block, (int)chunks);
+  };
+  if (dtype == DCP_DTYPE_FP32) launch(blockwise_sum_kernel<DCP_DTYPE_FP32, DCP_DTYPE_FP32, kSumThreads, kSumUnroll>);
+  else if (dtype == DCP_DTYPE_BF16 && fp32_sources) launch(blockwise_sum_kernel<DCP_DTYPE_BF16, DCP_DTYPE_FP32, kSumThreads, kSumUnroll>);
+  else if (dtype == DCP_DTYPE_BF16) launch(blockwise_sum_kernel<DCP_DTYPE_BF16, DCP_DTYPE_BF16, kSumThreads, kSumUnroll>);
+  else if (fp32_sources) launch(blockwise_sum_kernel<DCP_DTYPE_FP16, DCP_DTYPE_FP32, kSumThreads, kSumUnroll>);
+  else launch(blockwise_sum_kernel<DCP_DTYPE_FP16, DCP_DTYPE_FP16, kSumThreads, kSumUnroll>);
   return check_launch("blockwise_sum_kernel");
+}
+
+extern "C" int dcp_blockwise_sum(const int64_t* src_ptrs, const int32_t* src_offsets,
+                                 const int32_t* src_strides, const int32_t* n_ops_per_block,
+                                 const int64_t* dst_ptrs, const int32_t* dst_offsets,
+                                 const int32_t* dst_strides, const int32_t* n_elements,
+                                 int n_sums, int max_n_ops_per_block, int64_t block_numel,
+                                 int dtype, void* stream) {
+  DCP_RECORDED(dcp_blockwise_sum(src_ptrs, src_offsets, src_strides, n_ops_per_block, dst_ptrs, dst_offsets,
+      dst_strides, n_elements, n_sums, max_n_ops_per_block, block_numel, dtype, stream));
+  return blockwise_sum(src_ptrs, src_offsets, src_strides, n_ops_per_block, dst_ptrs, dst_offsets, dst_strides, n_elements,
+                       n_sums, max_n_ops_per_block, block_numel, dtype, false, stream);
+}
+
+extern "C" int dcp_blockwise_sum_fp32_sources(const int64_t* src_ptrs, const int32_t* src_offsets,
+                                              const int32_t* src_strides, const int32_t* n_ops_per_block,
+                                              const int64_t* dst_ptrs, const int32_t* dst_offsets,
+                                              const int32_t* dst_strides, const int32_t* n_elements,
+                                              int n_sums, int max_n_ops_per_block, int64_t block_numel,
+                                              int dtype, void* stream) {
+  DCP_RECORDED(dcp_blockwise_sum_fp32_sources(src_ptrs, src_offsets, src_strides, n_ops_per_block, dst_ptrs, dst_offsets,
+      dst_strides, n_elements, n_sums, max_n_ops_per_block, block_numel, dtype, stream));
+  return blockwise_sum(src_ptrs, src_offsets, src_strides, n_ops_per_block, dst_ptrs, dst_offsets, dst_strides, n_elements,
+                       n_sums, max_n_ops_per_block, block_numel, dtype, true, stream);
 }

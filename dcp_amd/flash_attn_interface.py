@@ -326,9 +326,10 @@ def _flash_attn_varlen_backward(
     each be the unpadded tensor, addressed by token offsets in its block table.  q and dout must
     then be readable for 64 tokens past the last row's queries (the dK/dV kernel loads whole
     64-query tiles).  dk/dv are always paged.
-    ``dkv_groups`` (extension): ``(groups, visits, dk_unpadded, dv_unpadded)`` -- dK/dV of a kv block
-    added over groups of rows in the kernel (``dcp_attn_bwd_grouped`` in ``dcp_hip.h`` describes the
-    two int32 tables ``[n, 8]`` and ``[m, 2]``); the unpadded tensors are ``[tokens, n_heads_kv, D]``.
+    ``dkv_groups`` (extension): ``(groups, visits, dk_unpadded, dv_unpadded, partials)`` -- dK/dV of a kv
+    block added over groups of rows in the kernel (``dcp_attn_bwd_grouped`` in ``dcp_hip.h`` describes
+    the two int32 tables ``[n, 8]`` and ``[m, 2]``); the unpadded tensors are ``[tokens, n_heads_kv, D]``,
+    the partials (or None) a contiguous fp32 tensor.
     """
     _check_plain(dropout_p, causal, window_size_left, window_size_right, softcap, alibi_slopes)
     if attn_range is None or q_block_table is None or kv_block_table is None \
@@ -386,13 +387,16 @@ def _flash_attn_varlen_backward(
         raise ValueError(f"workspace must be contiguous with at least {need} bytes")
     name, grouping = "dcp_attn_bwd_strided", ()
     if dkv_groups is not None:
-        groups, visits, dk_unpadded, dv_unpadded = dkv_groups
+        groups, visits, dk_unpadded, dv_unpadded, partials = dkv_groups
+        if partials is not None and (partials.dtype != torch.float32 or not partials.is_contiguous()):
+            raise ValueError("dkv_groups: the partials must be contiguous float32")
         if groups.dim() != 2 or groups.shape[1] != 8 or visits.dim() != 2 or visits.shape[1] != 2:
             raise ValueError(f"dkv_groups: tables must be [n, 8] and [m, 2], got {tuple(groups.shape)}, {tuple(visits.shape)}")
         unpadded_entry, unpadded_token = _kv_strides(dk_unpadded, dv_unpadded, "unpadded dk/dv")
         name = "dcp_attn_bwd_grouped"
         grouping = (_i32(groups, "dkv_groups").data_ptr(), groups.shape[0], _i32(visits, "dkv_visits").data_ptr(),
-                    dk_unpadded.data_ptr(), dv_unpadded.data_ptr(), unpadded_entry, unpadded_token)
+                    dk_unpadded.data_ptr(), dv_unpadded.data_ptr(), unpadded_entry, unpadded_token,
+                    0 if partials is None else partials.data_ptr())
     _lib.call(
         name,
         dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),

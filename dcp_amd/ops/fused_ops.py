@@ -323,9 +323,11 @@ def fused_blockwise_sum(
     block_size: int,
     triton_block_size: int,
     require_cached: bool = False,
+    fp32_sources: bool = False,
 ):
     """``dst[s] = sum_j src[s][j]`` over ``n_elements[s]`` elements (reference
-    ``fused_ops.py:1288-1360``); accumulated in fp32."""
+    ``fused_ops.py:1288-1360``); accumulated in fp32.  ``fp32_sources`` (extension): the sources are
+    fp32 whatever ``dtype``, the destinations' type, is."""
     assert block_size % triton_block_size == 0
     code = dtype_code(dtype if isinstance(dtype, str) else str(dtype))
     if src_offsets.dim() != 2 or src_offsets.shape[1] != max_n_ops_per_block:
@@ -334,7 +336,7 @@ def fused_blockwise_sum(
             f"{tuple(src_offsets.shape)}"
         )
     _lib.call(
-        "dcp_blockwise_sum",
+        "dcp_blockwise_sum_fp32_sources" if fp32_sources else "dcp_blockwise_sum",
         _i64(src_ptrs, "src_ptrs"),
         _i32(src_offsets, "src_offsets"),
         _i32(src_strides, "src_strides"),

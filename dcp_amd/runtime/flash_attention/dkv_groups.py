@@ -7,6 +7,10 @@ same kv block can be visited one after the other by the workgroup that holds its
 (``dcp_attn_bwd_grouped``): K and V are loaded once, the replicas are added in fp32 without being
 rounded and written first, and a sum whose sources have all been added that way is not run.
 
+Where a plan is so small that its (row, kv block) pairs leave most of the device idle, the opposite: a
+pair's queries are split over several workgroups (``Group.heads``, ``Group.tiles``), whose shares are
+left in fp32 and added, and rounded once, by the sum that would have added the replicas.
+
 ``analyse`` looks at the instruction list only and changes nothing in the plan.  It takes replicas
 together that one ``SumInstr`` op reads and nothing else does; what that op still has to add are the
 groups' first slots and whatever other sources it has (blocks received from other devices, ...).
@@ -14,9 +18,10 @@ groups' first slots and whatever other sources it has (blocks received from othe
 
 from __future__ import annotations
 
+import math
 from collections import Counter, defaultdict
 from dataclasses import dataclass, field
-from typing import Dict, List, Optional, Set, Tuple
+from typing import Dict, List, Optional, Set, Tuple, Union
 
 from dcp_amd.core.instructions import (
     AttnBackwardInstr,
@@ -39,7 +44,11 @@ class Group:
     """Rows of one launch that attend to one kv block: ``(row, position in the row's kv blocks)``."""
 
     visits: List[Tuple[int, int]]
-    dst: BufferBlock  # a BUFFER_dKV slot, or the LOCAL_dKV block the sum would have been scattered to
+    # a BUFFER_dKV slot, or the LOCAL_dKV block the sum would have been scattered to, or the number of a
+    # partial (fp32, a block each)
+    dst: Union[BufferBlock, int]
+    heads: Tuple[int, int] = (0, 0)  # of each kv head's q heads [begin, end); (0, 0): all
+    tiles: Tuple[int, int] = (0, 0)  # (n, i): every n-th 64-query tile from the i-th on; (0, 0): all
 
 
 @dataclass
@@ -50,6 +59,9 @@ class DkvGroups:
     skip_ops: Dict[int, Set[int]] = field(default_factory=dict)
     # SumInstr -> op position -> the sources the op still adds
     sources: Dict[int, Dict[int, List[BufferBlock]]] = field(default_factory=dict)
+    # SumInstr -> op position -> the partials the op adds instead
+    partials: Dict[int, Dict[int, List[int]]] = field(default_factory=dict)
+    n_partials: int = 0
 
 
 def visits_per_group(n_visits: int, tiles_per_visit: int, n_slots: int) -> int:
@@ -60,8 +72,19 @@ def visits_per_group(n_visits: int, tiles_per_visit: int, n_slots: int) -> int:
     (us) with 0.5 / 1 / 2 / 4 / 8 such groups per slot and with one row per group: 32768 tokens, 8
     heads in one-head blocks of 512 tokens 864 / 904 / 873 / 881 / 937, 1193; 16384 tokens, 16 heads,
     blocks of 256 931 / 942 / 949 / 973 / 1012, 1690; 65536 tokens, 32 heads in four-head blocks of 1024
-    8282 / 8226 / 8330 / 8340 / 8374, 8544."""
-    return max(1, min(MAX_VISITS, int(n_visits * tiles_per_visit / n_slots / 2)))
+    8282 / 8226 / 8330 / 8340 / 8374, 8544.  (Rounded up: 8192 tokens, 32 heads, 3.1 pairs per slot, in
+    groups of up to 2 rows 479, one by one 523.)"""
+    return max(1, min(MAX_VISITS, math.ceil(n_visits * tiles_per_visit / n_slots / 2)))
+
+
+def parts_per_visit(n_visits: int, tiles_per_visit: int, n_slots: int, n_heads: int, n_q_tiles: int) -> Tuple[int, int]:
+    """Into how many parts the queries of a (row, kv block) pair are split, by heads and by 64-query
+    tiles, so that the launch comes to one workgroup per slot of the device; parts of fewer than four
+    steps are not worth their start."""
+    steps = n_heads * n_q_tiles
+    parts = min(n_slots // max(1, n_visits * tiles_per_visit), steps // 4)
+    by_heads = max(1, min(parts, n_heads))
+    return by_heads, max(1, min(parts // by_heads, n_q_tiles))
 
 
 def _visit_order(counts: List[int]):
@@ -123,17 +146,24 @@ def _components(kv_table) -> Dict[int, Tuple[int, int]]:
     return found
 
 
-def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_block: int, n_slots: int) -> DkvGroups:
+def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_block: int, n_slots: int,
+            q_heads_per_kv_head: int = 1) -> DkvGroups:
     result = DkvGroups()
     instrs = plan.instructions
-    limits = {idx: visits_per_group(sum(map(len, instr.dkv_block_table)), tiles_per_block * n_heads_kv, n_slots)
-              for idx, instr in enumerate(instrs) if isinstance(instr, AttnBackwardInstr)}
-    if all(limit == 1 for limit in limits.values()):
+    limits, parts = {}, {}
+    for idx, instr in enumerate(instrs):
+        if isinstance(instr, AttnBackwardInstr):
+            n_visits = sum(map(len, instr.dkv_block_table))
+            limits[idx] = visits_per_group(n_visits, tiles_per_block * n_heads_kv, n_slots)
+            parts[idx] = (1, 1) if limits[idx] > 1 else parts_per_visit(
+                n_visits, tiles_per_block * n_heads_kv, n_slots, q_heads_per_kv_head, 2 * tiles_per_block)
+    if all(limit == 1 for limit in limits.values()) and all(p == (1, 1) for p in parts.values()):
         return result
     # who wrote a BUFFER_dKV slot last -- (instruction, row, position), if a backward kernel did -- and
     # which sum op reads what it wrote (None: something else does, or more than one op)
     written: Dict[int, Optional[Tuple[int, int, int]]] = {}
     reader: Dict[Tuple[int, int, int], Optional[Tuple[int, int]]] = {}
+    replicas_of: Dict[Tuple[int, int], List[Tuple[int, int, int]]] = defaultdict(list)  # what a sum op reads of that kind
     dkv = BufferType.BUFFER_dKV
 
     def reads(blocks, who=None):
@@ -142,6 +172,7 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
                 replica = written.get(block.index)
                 if replica is not None:
                     reader[replica] = None if replica in reader else who
+                    replicas_of[who].append(replica)
 
     def writes(block: BufferBlock):
         if block.buffer_type == dkv:
@@ -173,6 +204,28 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
             for op in instr.ops:
                 for blocks in op.src_buffers:
                     reads(blocks)
+
+    # sum ops all of whose sources can be left as partials
+    in_parts = {idx for idx, p in parts.items() if p != (1, 1)}
+    split_ops = {who for who, replicas in replicas_of.items() if who is not None and in_parts
+                 and len(replicas) == len(instrs[who[0]].ops[who[1]].src_buffers)
+                 and all(r[0] in in_parts and reader[r] == who for r in replicas)}
+    for idx in sorted(in_parts):
+        by_heads, by_tiles = parts[idx]
+        groups = []
+        for row, dkv_blocks in enumerate(instrs[idx].dkv_block_table):
+            for pos, block in enumerate(dkv_blocks):
+                who = reader.get((idx, row, pos))
+                if who not in split_ops:
+                    groups.append(Group([(row, pos)], block))
+                    continue
+                for i in range(by_heads):
+                    heads = (q_heads_per_kv_head * i // by_heads, q_heads_per_kv_head * (i + 1) // by_heads)
+                    for j in range(by_tiles):
+                        groups.append(Group([(row, pos)], result.n_partials, heads, (by_tiles, j) if by_tiles > 1 else (0, 0)))
+                        result.partials.setdefault(who[0], {}).setdefault(who[1], []).append(result.n_partials)
+                        result.n_partials += 1
+        result.groups[idx] = groups
 
     for idx, instr in enumerate(instrs):
         if limits.get(idx, 1) == 1:  # the launch does without groups

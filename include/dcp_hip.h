@@ -172,6 +172,18 @@ int dcp_blockwise_sum(const int64_t* src_ptrs, const int32_t* src_offsets,
                       const int32_t* n_elements, int n_sums,
                       int max_n_ops_per_block, int64_t block_numel, int dtype,
                       void* stream);
+/*
+ * The same with fp32 sources whatever the destination's type `dtype`
+ * (src_strides in fp32 elements): partial sums that have not been rounded yet,
+ * as dcp_attn_bwd_grouped leaves them.  A single source is rounded.
+ */
+int dcp_blockwise_sum_fp32_sources(
+    const int64_t* src_ptrs, const int32_t* src_offsets,
+    const int32_t* src_strides, const int32_t* n_ops_per_block,
+    const int64_t* dst_ptrs, const int32_t* dst_offsets,
+    const int32_t* dst_strides, const int32_t* n_elements, int n_sums,
+    int max_n_ops_per_block, int64_t block_numel, int dtype, void* stream);
+
 
 /*
  * Range-masked, paged, variable-length attention forward.
@@ -344,15 +356,19 @@ int dcp_attn_bwd_strided(const void* dout, const void* q, const void* k,
 /*
  * dcp_attn_bwd_strided that adds dK/dV of a kv block over several rows in the
  * kernel, in fp32, instead of leaving one private dK/dV block per (row, kv
- * block).  A group is a kv block with up to DCP_ATTN_BWD_MAX_VISITS of the
- * rows that list it:
+ * block), or splits the work of one over several workgroups.  A group is a kv
+ * block with up to DCP_ATTN_BWD_MAX_VISITS of the rows that list it, or a part
+ * of the queries of these rows:
  *   dkv_groups int32 [n_groups][8]: the block's k/v table entry; where its dK/dV
- *     goes (a table entry); tokens to store; 0 = into dk/dv (a slot), 1 = into
- *     dk_unpadded/dv_unpadded (entry and token strides in elements); the first
- *     of its visits; their number; two unused words
+ *     goes (an entry); tokens to store; which memory that is: 0 = dk/dv (a
+ *     slot), 1 = dk_unpadded/dv_unpadded (entry and token strides in elements),
+ *     2 = partials, fp32 [..][block_size][dK, dV][n_heads_kv][head_dim]; the
+ *     first of its visits; their number; the part's q heads of each kv head's
+ *     (begin + 65536 * end, 0 = all of them); the part's 64-query tiles (number
+ *     of parts + 65536 * part: every so many tiles, 0 = all of them)
  *   dkv_visits int32 [..][2]: a row, and the position of the group's block in
  *     the row's kv_block_table
- * Every (row, position) with keys belongs to exactly one group (a plan's
+ * Every (query, row, position) with keys belongs to exactly one group (a plan's
  * replicas that are not added up form groups of one); dkv_block_table is
  * not read.  Rows must hold whole blocks (key counts that are multiples of
  * block_size) and block_size must be a multiple of 128.  A group's tokens are
@@ -385,8 +401,8 @@ int dcp_attn_bwd_grouped(const void* dout, const void* q, const void* k,
                          int n_groups, const int32_t* dkv_visits,
                          void* dk_unpadded, void* dv_unpadded,
                          int64_t unpadded_entry_stride,
-                         int64_t unpadded_token_stride, float softmax_scale,
-                         int dtype, void* stream);
+                         int64_t unpadded_token_stride, float* partials,
+                         float softmax_scale, int dtype, void* stream);
 
 /*
  * Bytes of scratch dcp_attn_bwd needs for these sizes: rowsum(dO*O) and the

@@ -96,12 +96,51 @@ def test_exchanged_replicas_are_left_alone(monkeypatch):
         _check_groups(plan, found, slots_written_once=False)
 
 
+@pytest.mark.parametrize("parts", [(1, 2), (2, 1), (3, 4)])
+@pytest.mark.parametrize("name", ["causal_gqa", "split", "lambda"])
+def test_parts_cover_every_head_and_tile_once(monkeypatch, name, parts):
+    """A plan whose pairs are split: each pair's parts cover the q heads of its kv head and the 64-query
+    tiles exactly once, every partial is added by exactly one sum, the one that adds the replica."""
+    monkeypatch.setattr(dkv_groups, "parts_per_visit", lambda *a: parts)
+    kw = PLANS[name]
+    plan, bs = make_case(**kw)["bw"], kw["block_size"]
+    n_heads, n_tiles = 5, bs // 64
+    found = dkv_groups.analyse(plan, analyse_direct(plan), 1, bs // 128, 512, n_heads)
+    added = [p for ops in found.partials.values() for op in ops.values() for p in op]
+    assert sorted(added) == list(range(found.n_partials))
+    for idx, groups in found.groups.items():
+        instr = plan.instructions[idx]
+        seen, of_pair = {}, {}
+        for g in groups:
+            (pair,) = g.visits
+            assert isinstance(g.dst, int)
+            heads = range(*g.heads) if g.heads != (0, 0) else range(n_heads)
+            n, i = g.tiles
+            cells = [(h, t) for h in heads for t in range(n_tiles) if n == 0 or t % n == i]
+            assert not set(cells) & seen.setdefault(pair, set())
+            seen[pair].update(cells)
+            of_pair.setdefault(pair, []).append(g.dst)
+        assert set(seen) == {(r, p) for r, row in enumerate(instr.kv_block_table) for p in range(len(row))}
+        assert all(len(cells) == n_heads * n_tiles for cells in seen.values())
+        for (row, pos), partials in of_pair.items():
+            slot = instr.dkv_block_table[row][pos].index
+            (op,) = [(j, k) for j, i in enumerate(plan.instructions) if isinstance(i, SumInstr)
+                     for k, o in enumerate(i.ops) if any(b.buffer_type == BufferType.BUFFER_dKV and b.index == slot for b in o.src_buffers)
+                     and k in found.partials.get(j, {})]
+            assert set(partials) <= set(found.partials[op[0]][op[1]])
+
+
 def test_group_size_rule():
     """One row per group where the launch does not fill the device several times over, never more
     than the kernel takes."""
     assert dkv_groups.visits_per_group(60, 8, 512) == 1
     assert dkv_groups.visits_per_group(10 ** 6, 8, 512) == dkv_groups.MAX_VISITS
     assert 1 < dkv_groups.visits_per_group(2544, 8, 512) < dkv_groups.MAX_VISITS
+    # and parts of a row only where the rows are fewer than half the device's workgroups
+    assert dkv_groups.parts_per_visit(6, 4, 512, 4, 8) == (4, 2)
+    assert dkv_groups.parts_per_visit(24, 8, 512, 5, 16) == (2, 1)
+    assert dkv_groups.parts_per_visit(40, 8, 512, 5, 16) == (1, 1)
+    assert dkv_groups.parts_per_visit(1, 2, 512, 1, 4) == (1, 1)
 
 
 @pytest.mark.gpu
@@ -128,6 +167,32 @@ def test_grouped_backward_matches_dense_attention(gpu, monkeypatch, name, mode, 
     same_dq = torch.equal(grouped[2], single[2])  # dQ does not depend on the grouping
     same_as_written = torch.equal(grouped[3], as_written[3]) and torch.equal(grouped[2], as_written[2])
     assert same_dq and same_as_written
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("parts", [(1, 1), (1, 2), (2, 1), (2, 3)])
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("name", ["causal_gqa", "split", "lambda", "mha_fp16"])
+def test_backward_in_parts_matches_dense_attention(gpu, monkeypatch, name, mode, parts):
+    """Parts without a single visible key, of one head, of every third tile; two launches that add to one sum."""
+    from dcp_amd import _lib
+
+    monkeypatch.setattr(dkv_groups, "parts_per_visit", lambda *a: (min(parts[0], a[3]), min(parts[1], a[4])))
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 1)
+    lib = _lib.load()
+    case = make_case(**PLANS[name])
+    before = lib.dcp_attn_bwd_select(mode)
+    try:
+        direct, ex = run_executor(case, backward=True, poison=200.0)
+        monkeypatch.setenv("DCP_DIRECT_LOCAL", "0")
+        as_written, _ = run_executor(case, backward=True)
+    finally:
+        lib.dcp_attn_bwd_select(before)
+    split = parts[1] > 1 or parts[0] > 1 and name in ("causal_gqa", "lambda")  # (the others have one q head per kv head in a block)
+    assert (ex._dkv_groups.n_partials > 0) == split
+    check_against_truth(direct, dense_truth(case, backward=True))
+    same = torch.equal(direct[3], as_written[3]) and torch.equal(direct[2], as_written[2])
+    assert same
 
 
 @pytest.mark.gpu
