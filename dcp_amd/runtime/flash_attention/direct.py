@@ -71,101 +71,115 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
     if any(isinstance(i, (CommLaunchInstr, CommWaitInstr, BarrierInstr)) for i in instrs):
         return result
 
-    # A slot that holds a copy of a local block: (buffer type, slot) -> (memcpy index, pair position, source)
-    origin: Dict[Tuple[str, int], Tuple[int, int, BufferBlock]] = {}
-    # per copied pair: does every reader address it through an operand that can go to the source?
-    pair_readers: Dict[Tuple[int, int], List[bool]] = defaultdict(list)
+    # A slot that holds a copy of a local block of the matching type: buffer type -> slot -> (memcpy
+    # index, pair position, index and tokens of the local block)
+    origin: Dict[str, Dict[int, Tuple[int, int, int, int]]] = defaultdict(dict)
     all_pairs: Set[Tuple[int, int]] = set()
-    # kernel outputs: (buffer type, slot) -> producer, and the readers of each produced block
-    produced: Dict[Tuple[str, int], tuple] = {}
+    # copied pairs with a reader that does not address them through an operand that can go to the source
+    blocked: Set[Tuple[int, int]] = set()
+    # results that a scatter may take from their slot: buffer type -> slot -> producer; and the readers of each
+    produced: Dict[str, Dict[int, tuple]] = defaultdict(dict)
     readers: Dict[tuple, list] = defaultdict(list)
 
-    def local_blocks(idx: int, blocks: List[BufferBlock]):
-        """The local blocks behind ``blocks`` if every one of them is a fresh copy of the matching
-        LOCAL_* type; the copied pairs get a reader each, direct or not."""
-        hits = [origin.get((blk.buffer_type, blk.index)) for blk in blocks]
-        ok = all(h is not None and h[2].buffer_type == _LOCAL_OF.get(blk.buffer_type) and h[2].n_tokens == blk.n_tokens
-                 for h, blk in zip(hits, blocks))
-        for h in hits:
-            if h is not None:
-                pair_readers[(h[0], h[1])].append(ok)
-        return [h[2].index for h in hits] if ok else None
+    # (The tables hold a block per (row, kv block) pair: tens of thousands in a long plan, and a plan is
+    # executed once or a few times.  So the loops over them look a block up once and build nothing.)
+    def local_rows(buffer_type: str, table):
+        """Per row the indices of the local blocks behind its blocks, if every one of them is a fresh copy
+        of the matching LOCAL_* type; otherwise the copies among them have a reader in their slot."""
+        found = origin[buffer_type].get
+        rows = []
+        for row in table:
+            indices = []
+            for blk in row:
+                h = found(blk.index)
+                if h is None or h[3] != blk.n_tokens or blk.buffer_type != buffer_type:
+                    for r in table:
+                        for b in r:
+                            read_in_slot(b)
+                    return None
+                indices.append(h[2])
+            rows.append(indices)
+        return rows
 
-    def overwritten(blk: BufferBlock):
-        origin.pop((blk.buffer_type, blk.index), None)
-        produced.pop((blk.buffer_type, blk.index), None)
+    def read_in_slot(blk: BufferBlock):
+        h = origin[blk.buffer_type].get(blk.index)
+        if h is not None:
+            blocked.add((h[0], h[1]))
+
+    def overwritten(buffer_type: str, index: int):
+        origin[buffer_type].pop(index, None)
+        produced[buffer_type].pop(index, None)
 
     candidates: Dict[int, Dict[str, list]] = defaultdict(dict)
     for idx, instr in enumerate(instrs):
         if isinstance(instr, MemcpyInstr):
             for pos, (src, dst) in enumerate(instr.src_dst_pairs):
-                overwritten(dst)
-                if _LOCAL_OF.get(dst.buffer_type) == src.buffer_type:
-                    origin[(dst.buffer_type, dst.index)] = (idx, pos, src)
+                dst_type, slot = dst.buffer_type, dst.index
+                produced[dst_type].pop(slot, None)
+                if _LOCAL_OF.get(dst_type) == src.buffer_type:
+                    origin[dst_type][slot] = (idx, pos, src.index, src.n_tokens)
                     all_pairs.add((idx, pos))
+                else:
+                    origin[dst_type].pop(slot, None)
         elif isinstance(instr, (AttnInstr, AttnBackwardInstr)):
-            q_local = local_blocks(idx, [row[0] for row in instr.q_block_table])
-            kv_rows = [local_blocks(idx, list(row)) for row in instr.kv_block_table]
+            q_local = local_rows(BufferType.BUFFER_Q, [row[:1] for row in instr.q_block_table])
+            kv_local = local_rows(BufferType.BUFFER_KV, instr.kv_block_table)
             if q_local is not None:
-                candidates[idx]["q"] = q_local
-            if all(r is not None for r in kv_rows):
-                candidates[idx]["kv"] = kv_rows
-            elif any(r is not None for r in kv_rows):  # some rows could, the launch as a whole cannot
-                for row in instr.kv_block_table:
-                    for blk in row:
-                        h = origin.get((blk.buffer_type, blk.index))
-                        if h is not None:
-                            pair_readers[(h[0], h[1])].append(False)
+                candidates[idx]["q"] = [r[0] for r in q_local]
+            if kv_local is not None:
+                candidates[idx]["kv"] = kv_local
             if isinstance(instr, AttnInstr):
                 for b, row in enumerate(instr.out_block_table):
                     for t in (BufferType.BUFFER_OUT, BufferType.BUFFER_LSE):
-                        overwritten(BufferBlock(t, row[0].index, row[0].n_tokens))
-                    produced[(BufferType.BUFFER_OUT, row[0].index)] = ("out", idx, b)
+                        overwritten(t, row[0].index)
+                    produced[BufferType.BUFFER_OUT][row[0].index] = ("out", idx, b)
             else:
                 # out, lse and dout of a row share the slot number: all three must be copies of the same local block
-                per_type = [local_blocks(idx, [BufferBlock(t, row[0].index, row[0].n_tokens) for row in instr.out_block_table])
-                            for t in (BufferType.BUFFER_OUT, BufferType.BUFFER_LSE, BufferType.BUFFER_dOUT)]
-                if all(x is not None for x in per_type) and per_type[0] == per_type[1] == per_type[2]:
-                    candidates[idx]["out"] = per_type[0]
+                types = (BufferType.BUFFER_OUT, BufferType.BUFFER_LSE, BufferType.BUFFER_dOUT)
+                hits = [[origin[t].get(row[0].index) for row in instr.out_block_table] for t in types]
+                tokens = [row[0].n_tokens for row in instr.out_block_table]
+                local = [[h[2] for h in per_type] if all(h is not None and h[3] == n for h, n in zip(per_type, tokens)) else None
+                         for per_type in hits]
+                if local[0] is not None and local[0] == local[1] == local[2]:
+                    candidates[idx]["out"] = local[0]
                 else:
-                    for t in (BufferType.BUFFER_OUT, BufferType.BUFFER_LSE, BufferType.BUFFER_dOUT):
-                        for row in instr.out_block_table:
-                            h = origin.get((t, row[0].index))
-                            if h is not None:
-                                pair_readers[(h[0], h[1])].append(False)
+                    blocked.update((h[0], h[1]) for per_type in hits for h in per_type if h is not None)
                 for b, row in enumerate(instr.dq_block_table):
-                    overwritten(row[0])
-                    produced[(row[0].buffer_type, row[0].index)] = ("dq", idx, b)
-                for b, row in enumerate(instr.dkv_block_table):
-                    for blk in row:
-                        overwritten(blk)
-                        produced[(blk.buffer_type, blk.index)] = ("dkv", idx, b)
+                    overwritten(row[0].buffer_type, row[0].index)
+                    produced[row[0].buffer_type][row[0].index] = ("dq", idx, b)
+                # (who wrote a dK/dV replica is not asked for: none of them is moved to where it is read)
+                if any(produced.values()) or any(origin.values()):
+                    for row in instr.dkv_block_table:
+                        for blk in row:
+                            if produced[blk.buffer_type] or origin[blk.buffer_type]:
+                                overwritten(blk.buffer_type, blk.index)
         elif isinstance(instr, AttnReductionInstr):
             for pos, op in enumerate(instr.ops):
                 for src_out, src_lse in op.src_buffers:
-                    for blk in (src_out, src_lse):
-                        h = origin.get((blk.buffer_type, blk.index))
-                        if h is not None:
-                            pair_readers[(h[0], h[1])].append(False)
-                    who = produced.get((src_out.buffer_type, src_out.index))
+                    read_in_slot(src_out)
+                    read_in_slot(src_lse)
+                    who = produced[src_out.buffer_type].get(src_out.index)
                     if who is not None:
                         readers[who].append((idx, pos, len(op.src_buffers), bool(instr.output_is_unpadded)))
                 if not instr.output_is_unpadded:
                     for blk in op.dst_buffer:
-                        overwritten(blk)
-                    produced[(op.dst_buffer[0].buffer_type, op.dst_buffer[0].index)] = ("merged", idx, pos)
+                        overwritten(blk.buffer_type, blk.index)
+                    produced[op.dst_buffer[0].buffer_type][op.dst_buffer[0].index] = ("merged", idx, pos)
         elif isinstance(instr, SumInstr):
+            unpadded = bool(instr.output_is_unpadded)
             for pos, op in enumerate(instr.ops):
                 for blk in op.src_buffers:
-                    h = origin.get((blk.buffer_type, blk.index))
-                    if h is not None:
-                        pair_readers[(h[0], h[1])].append(False)
-                    who = produced.get((blk.buffer_type, blk.index))
-                    if who is not None:
-                        readers[who].append((idx, pos, len(op.src_buffers), bool(instr.output_is_unpadded)))
-                if not instr.output_is_unpadded:
-                    overwritten(op.dst_buffer)
-                    produced[(op.dst_buffer.buffer_type, op.dst_buffer.index)] = ("summed", idx, pos)
+                    of_type = produced[blk.buffer_type]
+                    if of_type:
+                        who = of_type.get(blk.index)
+                        if who is not None:
+                            readers[who].append((idx, pos, len(op.src_buffers), unpadded))
+                    if origin[blk.buffer_type]:
+                        read_in_slot(blk)
+                if not unpadded:
+                    dst = op.dst_buffer
+                    overwritten(dst.buffer_type, dst.index)
+                    produced[dst.buffer_type][dst.index] = ("summed", idx, pos)
         else:  # an instruction this analysis does not know: leave the plan alone
             return DirectPlan()
 
@@ -207,7 +221,6 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
                     result.skip_ops.setdefault(hit[0], set()).add(hit[1])
 
     result.operands = {idx: ops for idx, ops in candidates.items() if ops}
-    for key in all_pairs:
-        if all(pair_readers.get(key, [])):  # (a slot nobody reads is not worth filling either)
-            result.skip_pairs.setdefault(key[0], set()).add(key[1])
+    for idx, pos in all_pairs - blocked:  # (a slot nobody reads is not worth filling either)
+        result.skip_pairs.setdefault(idx, set()).add(pos)
     return result

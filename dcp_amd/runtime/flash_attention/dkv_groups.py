@@ -115,7 +115,7 @@ def _chunk_sizes(n_visits: int, limit: int) -> List[int]:
     return sizes
 
 
-def _components(kv_table) -> Dict[int, Tuple[int, int]]:
+def _components(kv_rows: List[List[int]]) -> Dict[int, Tuple[int, int]]:
     """kv block -> (component, rank in it), two blocks being in one component if some row attends to
     both: the blocks of a sequence's kv head.  In order of first appearance."""
     parent: Dict[int, int] = {}
@@ -125,16 +125,17 @@ def _components(kv_table) -> Dict[int, Tuple[int, int]]:
             parent[x] = x = parent[parent[x]]
         return x
 
-    for blocks in kv_table:
-        first = blocks[0].index
+    known = parent.get
+    for blocks in kv_rows:
+        first = blocks[0]
         if first not in parent:
             parent[first] = first
         r = root(first)
-        for block in blocks[1:]:
-            i = block.index
-            if i not in parent:
+        for i in blocks:
+            up = known(i)
+            if up is None:
                 parent[i] = r
-            elif parent[i] != r and root(i) != r:
+            elif up != r and root(i) != r:
                 parent[root(i)] = r
     numbers: Dict[int, int] = {}
     ranks: Counter = Counter()
@@ -144,6 +145,31 @@ def _components(kv_table) -> Dict[int, Tuple[int, int]]:
         found[i] = (numbers.setdefault(r, len(numbers)), ranks[r])
         ranks[r] += 1
     return found
+
+
+class _Visits:
+    """Every (row, kv block) pair of the plan's backward instructions, numbered.  (Tens of thousands in a
+    long plan, and a plan is executed once or a few times: the analysis works on these numbers and on
+    flat lists, and looks at a block once.)"""
+
+    def __init__(self, instrs):
+        self.begin: Dict[int, int] = {}  # instruction -> its first visit
+        self.row: List[int] = []
+        self.pos: List[int] = []
+        self.slot: List[BufferBlock] = []  # the pair's dK/dV replica
+        for idx, instr in enumerate(instrs):
+            if isinstance(instr, AttnBackwardInstr):
+                self.begin[idx] = len(self.row)
+                for row, blocks in enumerate(instr.dkv_block_table):
+                    self.row += [row] * len(blocks)
+                    self.pos += range(len(blocks))
+                    self.slot += blocks
+
+    def of(self, idx: int, instr: AttnBackwardInstr) -> range:
+        return range(self.begin[idx], self.begin[idx] + sum(map(len, instr.dkv_block_table)))
+
+
+_UNREAD, _ELSEWHERE = -1, -2  # readers of a replica: none; other than one sum op
 
 
 def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_block: int, n_slots: int,
@@ -159,33 +185,37 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
                 n_visits, tiles_per_block * n_heads_kv, n_slots, q_heads_per_kv_head, 2 * tiles_per_block)
     if all(limit == 1 for limit in limits.values()) and all(p == (1, 1) for p in parts.values()):
         return result
-    # who wrote a BUFFER_dKV slot last -- (instruction, row, position), if a backward kernel did -- and
-    # which sum op reads what it wrote (None: something else does, or more than one op)
-    written: Dict[int, Optional[Tuple[int, int, int]]] = {}
-    reader: Dict[Tuple[int, int, int], Optional[Tuple[int, int]]] = {}
-    replicas_of: Dict[Tuple[int, int], List[Tuple[int, int, int]]] = defaultdict(list)  # what a sum op reads of that kind
+    visits = _Visits(instrs)
+    row_of, pos_of, slot_of = visits.row, visits.pos, visits.slot
+    # which visit wrote a BUFFER_dKV slot last, if a backward kernel did, and which sum op reads what it wrote
+    written: Dict[int, int] = {}
+    reader = [_UNREAD] * len(row_of)
+    sum_ops: List[Tuple[int, int]] = []  # the sum ops, numbered as in `reader`: (instruction, position)
+    replicas_of: Dict[int, List[int]] = defaultdict(list)  # what a sum op reads of that kind
     dkv = BufferType.BUFFER_dKV
+    in_parts = {idx for idx, p in parts.items() if p != (1, 1)}
 
-    def reads(blocks, who=None):
+    def reads(blocks, who=_ELSEWHERE):
         for block in blocks:
             if block.buffer_type == dkv:
                 replica = written.get(block.index)
                 if replica is not None:
-                    reader[replica] = None if replica in reader else who
-                    replicas_of[who].append(replica)
+                    reader[replica] = who if reader[replica] == _UNREAD else _ELSEWHERE
+                    if in_parts:
+                        replicas_of[who].append(replica)
 
     def writes(block: BufferBlock):
         if block.buffer_type == dkv:
-            written[block.index] = None
+            written.pop(block.index, None)
 
     for idx, instr in enumerate(instrs):
         if isinstance(instr, AttnBackwardInstr):
-            for row, blocks in enumerate(instr.dkv_block_table):
-                for pos, block in enumerate(blocks):
-                    written[block.index] = (idx, row, pos)
+            mine = visits.of(idx, instr)
+            written.update(zip([block.index for block in slot_of[mine.start : mine.stop]], mine))
         elif isinstance(instr, SumInstr):
             for pos, op in enumerate(instr.ops):
-                reads(op.src_buffers, (idx, pos))
+                reads(op.src_buffers, len(sum_ops))
+                sum_ops.append((idx, pos))
             for op in instr.ops:
                 writes(op.dst_buffer)
         elif isinstance(instr, MemcpyInstr):
@@ -206,70 +236,71 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
                     reads(blocks)
 
     # sum ops all of whose sources can be left as partials
-    in_parts = {idx for idx, p in parts.items() if p != (1, 1)}
-    split_ops = {who for who, replicas in replicas_of.items() if who is not None and in_parts
-                 and len(replicas) == len(instrs[who[0]].ops[who[1]].src_buffers)
-                 and all(r[0] in in_parts and reader[r] == who for r in replicas)}
+    splittable = {v for idx in in_parts for v in visits.of(idx, instrs[idx])}
+    split_ops = {who for who, replicas in replicas_of.items() if who >= 0
+                 and len(replicas) == len(instrs[sum_ops[who][0]].ops[sum_ops[who][1]].src_buffers)
+                 and all(v in splittable and reader[v] == who for v in replicas)}
     for idx in sorted(in_parts):
         by_heads, by_tiles = parts[idx]
         groups = []
-        for row, dkv_blocks in enumerate(instrs[idx].dkv_block_table):
-            for pos, block in enumerate(dkv_blocks):
-                who = reader.get((idx, row, pos))
-                if who not in split_ops:
-                    groups.append(Group([(row, pos)], block))
-                    continue
-                for i in range(by_heads):
-                    heads = (q_heads_per_kv_head * i // by_heads, q_heads_per_kv_head * (i + 1) // by_heads)
-                    for j in range(by_tiles):
-                        groups.append(Group([(row, pos)], result.n_partials, heads, (by_tiles, j) if by_tiles > 1 else (0, 0)))
-                        result.partials.setdefault(who[0], {}).setdefault(who[1], []).append(result.n_partials)
-                        result.n_partials += 1
+        for v in visits.of(idx, instrs[idx]):
+            who, pair = reader[v], (row_of[v], pos_of[v])
+            if who not in split_ops:
+                groups.append(Group([pair], slot_of[v]))
+                continue
+            j, op_pos = sum_ops[who]
+            for i in range(by_heads):
+                heads = (q_heads_per_kv_head * i // by_heads, q_heads_per_kv_head * (i + 1) // by_heads)
+                for k in range(by_tiles):
+                    groups.append(Group([pair], result.n_partials, heads, (by_tiles, k) if by_tiles > 1 else (0, 0)))
+                    result.partials.setdefault(j, {}).setdefault(op_pos, []).append(result.n_partials)
+                    result.n_partials += 1
         result.groups[idx] = groups
 
     for idx, instr in enumerate(instrs):
         if limits.get(idx, 1) == 1:  # the launch does without groups
             continue
+        mine = visits.of(idx, instr)
+        kv_rows = [[block.index for block in row] for row in instr.kv_block_table]
+        kv_of = [i for row in kv_rows for i in row]
         # rows to take together: the same kv block, added by the same op and read by nothing else
-        together: Dict[tuple, List[Tuple[int, int]]] = defaultdict(list)
-        for row, (kv_blocks, dkv_blocks) in enumerate(zip(instr.kv_block_table, instr.dkv_block_table)):
-            for pos, (kv_block, dkv_block) in enumerate(zip(kv_blocks, dkv_blocks)):
-                op = reader.get((idx, row, pos))
-                together[(row, pos) if op is None else (op, kv_block.index, dkv_block.n_tokens)].append((row, pos))
+        alone: List[int] = []
+        together: Dict[Tuple[int, int, int], List[int]] = defaultdict(list)
+        for v, kv_block in zip(mine, kv_of):
+            if reader[v] < 0:
+                alone.append(v)
+            else:
+                together[reader[v], kv_block, slot_of[v].n_tokens].append(v)
         limit = limits[idx]
-        groups: List[Group] = []
-        order = _visit_order([len(v) for v in together.values()]) if together else None
-        for key, visits in together.items():
-            visits.sort(key=order)
-            slot = lambda v: instr.dkv_block_table[v[0]][v[1]]
-            if len(key) == 2:
-                groups += [Group([v], slot(v)) for v in visits]
-                continue
-            j, op_pos = key[0]
+        groups: List[Group] = [Group([(row_of[v], pos_of[v])], slot_of[v]) for v in alone]
+        if together or alone:
+            order = _visit_order([len(t) for t in together.values()] + [1] * len(alone))
+        for (who, _, _), taken in together.items():
+            taken.sort(key=lambda v: order((row_of[v], pos_of[v])))
+            j, op_pos = sum_ops[who]
             op = instrs[j].ops[op_pos]
             dst = direct.redirect_ops.get(j, {}).get(op_pos, op.dst_buffer if instrs[j].output_is_unpadded else None)
-            if (len(visits) <= limit and len(visits) == len(op.src_buffers) and dst is not None
-                    and dst.buffer_type == BufferType.LOCAL_dKV and dst.n_tokens == slot(visits[0]).n_tokens):
-                groups.append(Group(visits, dst))
+            if (len(taken) <= limit and len(taken) == len(op.src_buffers) and dst is not None
+                    and dst.buffer_type == BufferType.LOCAL_dKV and dst.n_tokens == slot_of[taken[0]].n_tokens):
+                groups.append(Group([(row_of[v], pos_of[v]) for v in taken], dst))
                 result.skip_ops.setdefault(j, set()).add(op_pos)
                 continue
-            chunks, at = [], 0
-            for size in _chunk_sizes(len(visits), limit) if len(visits) > limit else [len(visits)]:
-                chunks.append(visits[at : at + size])
+            gone, at = set(), 0
+            for size in _chunk_sizes(len(taken), limit) if len(taken) > limit else [len(taken)]:
+                chunk = taken[at : at + size]
                 at += size
-            groups += [Group(chunk, slot(chunk[0])) for chunk in chunks]
-            gone = {slot(v).index for chunk in chunks for v in chunk[1:]}
+                groups.append(Group([(row_of[v], pos_of[v]) for v in chunk], slot_of[chunk[0]]))
+                gone.update([slot_of[v].index for v in chunk[1:]])
             ops = result.sources.setdefault(j, {})
-            ops[op_pos] = [b for b in ops.get(op_pos, op.src_buffers)
-                           if not (b.buffer_type == BufferType.BUFFER_dKV and b.index in gone)]
+            ops[op_pos] = [b for b in ops.get(op_pos, op.src_buffers) if b.buffer_type != dkv or b.index not in gone]
         # longest first; among equals the same block of every sequence and head together: consecutive
         # groups go to the XCDs in turn, so that the blocks of one head, whose rows are the same, meet on
         # one XCD at about the same time (131072 tokens, window 4096, 8 kv heads: 15.6 -> 15.3 ms)
-        component = _components(instr.kv_block_table)
+        component = _components(kv_rows)
 
         def place(group: Group):
             row, pos = group.visits[0]
-            number, rank = component[instr.kv_block_table[row][pos].index]
+            number, rank = component[kv_rows[row][pos]]
             return (-len(group.visits), rank, number)
 
         groups.sort(key=place)

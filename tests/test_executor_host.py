@@ -1,7 +1,9 @@
 """Handler registry and instruction loop of the abstract executor (no GPU):
 the error behaviour of the reference's dcp/core/executor.py."""
 
+import numpy as np
 import pytest
+import torch
 
 from dcp_amd.core.executor import DCPExecutor
 from dcp_amd.core.instructions import (
@@ -95,3 +97,35 @@ def test_blocks_share_a_launch_only_within_a_factor_of_four():
     assert c[1 << 22] == 1 << 22 and c[4096] == 4096 and c[16385] == 16385
     for n, top in c.items():
         assert n <= top <= 4 * n
+
+
+def test_padded_tables():
+    from dcp_amd.runtime.flash_attention.executor import _padded
+
+    for rows, width in (([[3, 4], [5], []], 2), ([[7]], 1), ([[1, 2, 3], [4]], 8), ([[], []], 1)):
+        assert _padded(rows, width).tolist() == [row + [-1] * (width - len(row)) for row in rows]
+
+
+@pytest.mark.gpu
+def test_tables_of_a_prepare_arrive_whole(gpu):
+    """Tables that fill a chunk to its last byte, exceed one, are empty, or do not fit their type."""
+    from dcp_amd.runtime.flash_attention import executor as ex
+
+    rng, upload = np.random.default_rng(0), ex._TableUpload()
+    ex._preparing.upload = upload
+    try:
+        with pytest.raises(OverflowError):
+            ex._dev([2 ** 31], torch.int32)
+        with pytest.raises(OverflowError):
+            ex._dev(np.asarray([-(2 ** 31) - 1]), torch.int32)
+        tables = []
+        for shape in ((5,), (0,), (3, 7), (upload.CHUNK // 4 - 64 * 3,), (1,), (upload.CHUNK // 4 + 1,), (2, 2, 9), (upload.CHUNK // 8,)):
+            for dtype, kind in ((torch.int32, np.int32), (torch.int64, np.int64)):
+                values = rng.integers(np.iinfo(kind).min, np.iinfo(kind).max, size=shape)
+                tables.append((values, ex._dev(values if len(tables) % 4 < 2 else values.tolist(), dtype), dtype))
+    finally:
+        ex._preparing.upload = None
+    upload.send()
+    for values, table, dtype in tables:
+        assert table.dtype == dtype and table.is_contiguous() and table.data_ptr() % 16 == 0
+        assert np.array_equal(table.cpu().numpy(), values)
