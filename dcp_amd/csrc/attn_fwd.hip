@@ -40,6 +40,12 @@
 
 namespace dcp {
 
+// Part `part` of `n_parts` of a row's keys: an equal share of the key tiles of each of the row's work
+// items.  n_parts > 1: the result goes to partial first_partial + part.
+struct FwdPart {
+  int row, part, n_parts, first_partial;
+};
+
 struct AttnFwdParams {
   const void* q;
   const void* k;
@@ -75,6 +81,10 @@ struct AttnFwdParams {
   int64_t n_items;   // batch * n_heads_q * q_tiles_per_row
   float scale_log2;  // softmax_scale * log2(e)
   int* tickets;      // of the item queue, zeroed before the launch; null: one item per workgroup
+  // rows in parts (dcp_attn_fwd_parts): a record per launch entry, which takes the place of a row
+  const FwdPart* parts;
+  float* partial_out;   // [partial][head][32-query block][D / 4][query][4]: O^T relative to the part's maximum
+  float* partial_sums;  // [partial][head][32-query block][query][2]: the maximum (log2 domain) and the sum of the weights
 };
 
 // Wave priority by phase: the two waves of a SIMD come from different workgroups and drift
@@ -102,7 +112,10 @@ constexpr float kMaxTileSum = 16384.0f;
 // K / V^T operand read from LDS feeds two matrix instructions and every tile brought into LDS
 // serves twice the arithmetic; the wave then needs the whole register file (one workgroup
 // per CU, accumulators in the AGPR half).
-template <int DTYPE, int D, int QB>
+// PARTS: the launch's rows are split along their keys.  A work item is a serial chain, a tile after the
+// other (1.2-1.5 us each with a workgroup alone on its CU), and a launch of few, uneven rows lasts as long as its longest:
+// see dcp_attn_fwd_parts.
+template <int DTYPE, int D, int QB, bool PARTS>
 __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int item) {
   constexpr int BN = kFwdBN;
   constexpr int BM = 128 * QB;
@@ -135,7 +148,8 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
   wg /= p.q_tiles_per_row;
   const int head = __builtin_amdgcn_readfirstlane(wg % p.n_heads_q);
   const int bi = __builtin_amdgcn_readfirstlane(wg / p.n_heads_q);
-  const int b = __builtin_amdgcn_readfirstlane(p.row_order ? p.row_order[bi] : bi);
+  const FwdPart part = PARTS ? p.parts[bi] : FwdPart{0, 0, 1, 0};
+  const int b = __builtin_amdgcn_readfirstlane(PARTS ? part.row : p.row_order ? p.row_order[bi] : bi);
   const int q_begin = p.cu_seqlens_q[b];
   const int seqlen_q = p.cu_seqlens_q[b + 1] - q_begin;
   const int seqlen_kv = p.cu_seqlens_kv[b + 1] - p.cu_seqlens_kv[b];
@@ -218,7 +232,12 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
   g_lo1 = __builtin_amdgcn_readfirstlane(g_lo1);
   g_hi1 = __builtin_amdgcn_readfirstlane(g_hi1);
   const TileRuns runs(g_lo0, g_hi0, g_lo1, g_hi1, BN);
-  const int n_tiles = runs.count();
+  int first_tile = 0, n_tiles = runs.count();  // where the item begins and ends in the tile list
+  const int partial = PARTS && part.n_parts > 1 ? part.first_partial + part.part : -1;  // where its result goes
+  if constexpr (PARTS) {
+    first_tile = __builtin_amdgcn_readfirstlane(n_tiles * part.part / part.n_parts);
+    n_tiles = __builtin_amdgcn_readfirstlane(n_tiles * (part.part + 1) / part.n_parts);
+  }
 
   // ---- running state ---------------------------------------------------------
   f32x16 o_acc[QB][DT];
@@ -519,8 +538,8 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
     v_off = cursor.off;
     cursor_next();
   };
-  if (n_tiles > 0) {
-    cursor.seek(runs, 0, tiles_per_block, slot_lds, kv_table, p.kv_slot_stride, tile_stride);
+  if (n_tiles > first_tile) {
+    cursor.seek(runs, first_tile, tiles_per_block, slot_lds, kv_table, p.kv_slot_stride, tile_stride);
     tile_cur = cursor.tile;
     fill_k = k_at0;
     fill_v = v_at0;
@@ -544,7 +563,7 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
       pending = true;
       anchored = cur_full;
     }
-    for (int j = 0; j < n_tiles; j += 2) {
+    for (int j = first_tile; j < n_tiles; j += 2) {
       iteration(j, s_a, s_b, k_lds1, k_at0, v_lds0, v_at1);
       if (__builtin_expect(j + 1 >= n_tiles, 0)) break;
       iteration(j + 1, s_b, s_a, k_lds0, k_at1, v_lds1, v_at0);
@@ -553,6 +572,30 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
   }
 
   // ---- epilogue ------------------------------------------------------------------
+  if constexpr (PARTS) {
+    if (partial >= 0) {
+      // 32 queries' 16-byte pieces side by side: whole 512-byte runs per store and half-wave
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        const float l_tot = halves_sum(l_run[qb]);
+        const int64_t block = ((int64_t)partial * p.n_heads_q + head) * (p.q_tiles_per_row * (BM / 32)) +
+                              qt * (BM / 32) + w * QB + qb;
+        f32x4* dst = reinterpret_cast<f32x4*>(p.partial_out) + block * (32 * D / 4) + h * 32 + c;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 o4 = {o_acc[qb][dt][4 * g], o_acc[qb][dt][4 * g + 1], o_acc[qb][dt][4 * g + 2], o_acc[qb][dt][4 * g + 3]};
+            dst[(dt * 4 + g) * 64] = o4;
+          }
+        if (h == 0) {
+          p.partial_sums[(block * 32 + c) * 2] = m_run[qb];
+          p.partial_sums[(block * 32 + c) * 2 + 1] = l_tot;
+        }
+      }
+      return;
+    }
+  }
   const int o_slot = p.out_block_table[b];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
@@ -584,7 +627,7 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
 // of work), and the last, unevenly long items leave slots empty at the end.  Rows come longest first;
 // the counters are zeroed by a one-wave kernel on the stream just before.  A launch whose items all
 // fit on the device at once needs no queue and no such kernel.
-template <int DTYPE, int D, int QB>
+template <int DTYPE, int D, int QB, bool PARTS>
 __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(const AttnFwdParams p) {
   __shared__ int ticket_lds;
   int item = 0;
@@ -596,13 +639,67 @@ __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(
     KernArgs<AttnFwdParams>& args = fresh_kernel_args<AttnFwdParams>();
     if (item < 0) item = next_item({args.tickets, kFwdTicketStride, args.n_items, args.xcd_group}, &ticket_lds);
     if (item < 0) break;
-    attn_fwd_item<DTYPE, D, QB>(args, item);
+    attn_fwd_item<DTYPE, D, QB, PARTS>(args, item);
     item = -1;
   }
 }
 
 __global__ void attn_fwd_reset_tickets_kernel(int* tickets) {
   if (threadIdx.x < kFwdTicketInts) tickets[threadIdx.x] = 0;
+}
+
+// Adds up the parts of the split rows: out = sum_i 2^(m_i - m) O_i / sum_i 2^(m_i - m) l_i, rounded once.
+// A workgroup takes 32 queries of one (row, head); a lane one query and D / 32 groups of four dims, so
+// that its reads of the partials are whole runs and a query's weights are the same for all of them.
+struct FwdSplit {
+  int row, n_parts, first_partial, unused;
+};
+constexpr int kMergePartsThreads = 256;
+template <int DTYPE, int D>
+__global__ __launch_bounds__(kMergePartsThreads) void attn_fwd_merge_parts_kernel(const AttnFwdParams p, const FwdSplit* splits) {
+  const int blocks_per_row = p.q_tiles_per_row * 4;
+  const int qb = blockIdx.x % blocks_per_row;
+  const int head = blockIdx.x / blocks_per_row % p.n_heads_q;
+  const FwdSplit split = splits[blockIdx.x / blocks_per_row / p.n_heads_q];
+  const int q_begin = p.cu_seqlens_q[split.row];
+  const int c = threadIdx.x & 31, q_local = qb * 32 + c;
+  if (q_local >= p.cu_seqlens_q[split.row + 1] - q_begin) return;
+  const int64_t block0 = ((int64_t)split.first_partial * p.n_heads_q + head) * blocks_per_row + qb;
+  const int64_t block_step = (int64_t)p.n_heads_q * blocks_per_row;
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  const f32x2* sums = reinterpret_cast<const f32x2*>(p.partial_sums) + block0 * 32 + c;
+  float m = -INFINITY;
+  for (int i = 0; i < split.n_parts; ++i) m = fmaxf(m, sums[i * block_step * 32][0]);
+  const float m_use = m == -INFINITY ? 0.0f : m;
+  constexpr int PER = 32 * D / 4 / kMergePartsThreads;
+  f32x4 acc[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) acc[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float l = 0.0f;
+  const f32x4* src = reinterpret_cast<const f32x4*>(p.partial_out) + block0 * (32 * D / 4) + threadIdx.x;
+  for (int i = 0; i < split.n_parts; ++i) {
+    const f32x2 ml = sums[i * block_step * 32];
+    const float weight = fast_exp2(ml[0] - m_use);  // a part without a visible key: exp2(-inf) = 0, and its O is 0
+    l += weight * ml[1];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const f32x4 o4 = src[i * block_step * (32 * D / 4) + k * kMergePartsThreads];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[k][r] += weight * o4[r];
+    }
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const int o_slot = p.out_block_table[split.row];
+  uint16_t* out = reinterpret_cast<uint16_t*>(p.out) + (int64_t)o_slot * p.out_slot_stride +
+                  ((int64_t)q_local * p.n_heads_q + head) * D + 4 * (threadIdx.x >> 5);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const u32x2 pk = {pack2<DTYPE>(acc[k][0] * inv, acc[k][1] * inv), pack2<DTYPE>(acc[k][2] * inv, acc[k][3] * inv)};
+    *reinterpret_cast<u32x2*>(out + k * (kMergePartsThreads / 8)) = pk;
+  }
+  if (threadIdx.x < 32)
+    p.lse[(int64_t)head * p.lse_head_stride + (int64_t)o_slot * p.lse_slot_stride + q_local] =
+        l > 0.0f ? (m + log2f(l)) * kLn2 : p.empty_lse;
 }
 
 }  // namespace dcp
@@ -633,20 +730,23 @@ extern "C" int dcp_attn_fwd(const void* q, const void* k, const void* v, void* o
                               workspace_bytes, stream);
 }
 
-extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v, void* out, float* lse,
-                                    const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
-                                    const int32_t* attn_range, int n_ranges, const int32_t* q_block_table,
-                                    const int32_t* kv_block_table, const int32_t* out_block_table,
-                                    const int32_t* row_order, int batch, int max_kv_blocks, int total_q,
-                                    int block_size, int n_heads_q, int n_heads_kv, int head_dim,
-                                    int64_t kv_slot_stride, int64_t kv_token_stride, int64_t q_slot_stride,
-                                    int64_t out_slot_stride, int64_t lse_head_stride, int64_t lse_slot_stride,
-                                    int merged_form, float softmax_scale, int dtype, void* workspace,
-                                    size_t workspace_bytes, void* stream) {
-  DCP_RECORDED(dcp_attn_fwd_strided(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges,
-      q_block_table, kv_block_table, out_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q,
-      n_heads_kv, head_dim, kv_slot_stride, kv_token_stride, q_slot_stride, out_slot_stride, lse_head_stride,
-      lse_slot_stride, merged_form, softmax_scale, dtype, workspace, workspace_bytes, stream));
+// What dcp_attn_fwd_parts adds to dcp_attn_fwd_strided.
+struct FwdParts {
+  const int32_t* parts = nullptr;
+  int n_entries = 0;
+  const int32_t* splits = nullptr;
+  int n_splits = 0, n_partials = 0;
+  float* partials = nullptr;
+  size_t partials_bytes = 0;
+};
+
+static int attn_fwd(const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu_seqlens_q,
+                    const int32_t* cu_seqlens_kv, const int32_t* attn_range, int n_ranges, const int32_t* q_block_table,
+                    const int32_t* kv_block_table, const int32_t* out_block_table, const int32_t* row_order, int batch,
+                    int max_kv_blocks, int total_q, int block_size, int n_heads_q, int n_heads_kv, int head_dim,
+                    int64_t kv_slot_stride, int64_t kv_token_stride, int64_t q_slot_stride, int64_t out_slot_stride,
+                    int64_t lse_head_stride, int64_t lse_slot_stride, int merged_form, float softmax_scale, int dtype,
+                    void* workspace, size_t workspace_bytes, const FwdParts& in_parts, void* stream) {
   if (dtype != DCP_DTYPE_BF16 && dtype != DCP_DTYPE_FP16)
     return fail(DCP_ERR_UNSUPPORTED, "attn_fwd: dtype %d unsupported (bf16 and fp16 only)", dtype);
   if (head_dim != 64 && head_dim != 128)
@@ -674,6 +774,16 @@ extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v,
                   workspace_bytes >= dcp_attn_fwd_workspace_bytes(),
               "attn_fwd: workspace of %zu bytes is missing or smaller than the %zu needed", workspace_bytes,
               dcp_attn_fwd_workspace_bytes());
+  if (in_parts.parts != nullptr) {
+    DCP_REQUIRE(in_parts.n_entries >= batch && in_parts.n_splits >= 0 && in_parts.n_splits <= batch && in_parts.n_partials >= 2 * in_parts.n_splits,
+                "attn_fwd: %d entries and %d partials of %d split rows do not fit %d rows", in_parts.n_entries, in_parts.n_partials,
+                in_parts.n_splits, batch);
+    const size_t queries = (size_t)((block_size + 127) / 128) * 128 * n_heads_q * in_parts.n_partials;
+    DCP_REQUIRE(in_parts.n_splits == 0 || (in_parts.splits && in_parts.partials && (reinterpret_cast<uintptr_t>(in_parts.partials) & 15) == 0 &&
+                                           in_parts.partials_bytes >= queries * (head_dim + 2) * sizeof(float)),
+                "attn_fwd: the partials are missing, not 16-byte aligned or smaller than the %zu bytes needed",
+                queries * (head_dim + 2) * sizeof(float));
+  }
   AttnFwdParams p;
   p.q = q;
   p.k = k;
@@ -707,7 +817,10 @@ extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v,
   const int bm = 128;
   p.q_tiles_per_row = (block_size + bm - 1) / bm;
   p.scale_log2 = softmax_scale * kLog2e;
-  p.n_items = (int64_t)batch * n_heads_q * p.q_tiles_per_row;
+  p.n_items = (int64_t)(in_parts.parts ? in_parts.n_entries : batch) * n_heads_q * p.q_tiles_per_row;
+  p.parts = reinterpret_cast<const FwdPart*>(in_parts.parts);
+  p.partial_out = in_parts.partials;
+  p.partial_sums = in_parts.partials + (size_t)in_parts.n_partials * n_heads_q * p.q_tiles_per_row * bm * head_dim;
   p.xcd_group = p.q_tiles_per_row * (n_heads_q / n_heads_kv);
   DCP_REQUIRE(p.n_items < ((int64_t)1 << 31), "attn_fwd: too many work items");
   // as many workgroups as the device holds at once (two per CU), a multiple of the XCD count
@@ -715,9 +828,11 @@ extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v,
   p.tickets = p.n_items > n_wg ? reinterpret_cast<int*>(workspace) : nullptr;
   dim3 grid((unsigned)n_wg), block(kFwdThreads);
   if (p.tickets) hipLaunchKernelGGL(attn_fwd_reset_tickets_kernel, dim3(1), dim3(kFwdTicketInts), 0, (hipStream_t)stream, p.tickets);
-  KernelTimer timer("attn_fwd_kernel", stream);
-#define DCP_FWD(DT, HD) \
-  hipLaunchKernelGGL((attn_fwd_kernel<DT, HD, 1>), grid, block, 0, (hipStream_t)stream, p)
+  auto launch = [&](auto kernel) {
+    KernelTimer timer("attn_fwd_kernel", stream);
+    hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, p);
+  };
+#define DCP_FWD(DT, HD) (p.parts ? launch(attn_fwd_kernel<DT, HD, 1, true>) : launch(attn_fwd_kernel<DT, HD, 1, false>))
   if (dtype == DCP_DTYPE_BF16) {
     if (head_dim == 128) DCP_FWD(DCP_DTYPE_BF16, 128);
     else DCP_FWD(DCP_DTYPE_BF16, 64);
@@ -726,5 +841,61 @@ extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v,
     else DCP_FWD(DCP_DTYPE_FP16, 64);
   }
 #undef DCP_FWD
-  return check_launch("attn_fwd_kernel");
+  const int status = check_launch("attn_fwd_kernel");
+  if (status != DCP_OK || in_parts.n_splits == 0) return status;
+  const int64_t merges = (int64_t)in_parts.n_splits * n_heads_q * p.q_tiles_per_row * (bm / 32);
+  DCP_REQUIRE(merges < ((int64_t)1 << 31), "attn_fwd: too many split rows");
+  auto merge = [&](auto kernel) {
+    KernelTimer timer("attn_fwd_merge_parts_kernel", stream);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)merges), dim3(kMergePartsThreads), 0, (hipStream_t)stream, p,
+                       reinterpret_cast<const FwdSplit*>(in_parts.splits));
+  };
+  if (dtype == DCP_DTYPE_BF16) {
+    if (head_dim == 128) merge(attn_fwd_merge_parts_kernel<DCP_DTYPE_BF16, 128>);
+    else merge(attn_fwd_merge_parts_kernel<DCP_DTYPE_BF16, 64>);
+  } else {
+    if (head_dim == 128) merge(attn_fwd_merge_parts_kernel<DCP_DTYPE_FP16, 128>);
+    else merge(attn_fwd_merge_parts_kernel<DCP_DTYPE_FP16, 64>);
+  }
+  return check_launch("attn_fwd_merge_parts_kernel");
 }
+
+extern "C" int dcp_attn_fwd_strided(const void* q, const void* k, const void* v, void* out, float* lse,
+                                    const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
+                                    const int32_t* attn_range, int n_ranges, const int32_t* q_block_table,
+                                    const int32_t* kv_block_table, const int32_t* out_block_table,
+                                    const int32_t* row_order, int batch, int max_kv_blocks, int total_q,
+                                    int block_size, int n_heads_q, int n_heads_kv, int head_dim,
+                                    int64_t kv_slot_stride, int64_t kv_token_stride, int64_t q_slot_stride,
+                                    int64_t out_slot_stride, int64_t lse_head_stride, int64_t lse_slot_stride,
+                                    int merged_form, float softmax_scale, int dtype, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  DCP_RECORDED(dcp_attn_fwd_strided(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges,
+      q_block_table, kv_block_table, out_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q,
+      n_heads_kv, head_dim, kv_slot_stride, kv_token_stride, q_slot_stride, out_slot_stride, lse_head_stride,
+      lse_slot_stride, merged_form, softmax_scale, dtype, workspace, workspace_bytes, stream));
+  return attn_fwd(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table,
+                  row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride,
+                  q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
+                  workspace_bytes, FwdParts{}, stream);
+}
+
+extern "C" int dcp_attn_fwd_parts(const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu_seqlens_q,
+                    const int32_t* cu_seqlens_kv, const int32_t* attn_range, int n_ranges, const int32_t* q_block_table,
+                    const int32_t* kv_block_table, const int32_t* out_block_table, const int32_t* row_order, int batch,
+                    int max_kv_blocks, int total_q, int block_size, int n_heads_q, int n_heads_kv, int head_dim,
+                    int64_t kv_slot_stride, int64_t kv_token_stride, int64_t q_slot_stride, int64_t out_slot_stride,
+                    int64_t lse_head_stride, int64_t lse_slot_stride, int merged_form, float softmax_scale, int dtype,
+                    void* workspace, size_t workspace_bytes, const int32_t* parts, int n_entries, const int32_t* splits,
+                    int n_splits, int n_partials, void* partials, size_t partials_bytes, void* stream) {
+  DCP_RECORDED(dcp_attn_fwd_parts(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table,
+      out_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride,
+      kv_token_stride, q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
+      workspace_bytes, parts, n_entries, splits, n_splits, n_partials, partials, partials_bytes, stream));
+  DCP_REQUIRE(parts != nullptr, "attn_fwd: no table of parts");
+  return attn_fwd(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table,
+                  row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride,
+                  q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
+                  workspace_bytes, FwdParts{parts, n_entries, splits, n_splits, n_partials, reinterpret_cast<float*>(partials), partials_bytes}, stream);
+}
+

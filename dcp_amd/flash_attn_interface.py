@@ -195,6 +195,7 @@ def _flash_attn_varlen_forward(
     workspace: Optional[torch.Tensor] = None,
     block_size: Optional[int] = None,
     merged_form: bool = False,
+    parts=None,
 ):
     """Writes the row outputs into ``out_`` / ``lse_`` in place and returns
     ``(out_, lse_, None, None)`` (the reference returns
@@ -213,6 +214,8 @@ def _flash_attn_varlen_forward(
     readable for ``block_size`` tokens from every table entry on (the kernel loads whole blocks).
     ``merged_form`` (extension): queries without a visible key get ``lse = -1`` (what the merge
     leaves for a row with no finite source) instead of ``+inf``.
+    ``parts`` (extension): ``(parts, splits, n_partials, partials)``, rows split along their keys
+    (``dcp_attn_fwd_parts``): int32 ``[entries, 4]`` and ``[split rows, 4]``, and fp32 scratch.
     """
     _check_plain(dropout_p, causal, window_size_left, window_size_right, softcap,
                  alibi_slopes, return_softmax)
@@ -247,15 +250,14 @@ def _flash_attn_varlen_forward(
             _widen(q, d, block_size), _widen(k, d, block_size), _widen(v, d, block_size), cu_seqlens_q, cu_seqlens_k, total_q, max_seqlen_q, max_seqlen_k,
             dropout_p, softmax_scale, attn_range=attn_range, q_block_table=q_block_table, kv_block_table=kv_block_table,
             out_block_table=out_block_table, out_=out_wide, lse_=lse_, row_order=row_order, workspace=workspace,
-            block_size=block_size, merged_form=merged_form)
+            block_size=block_size, merged_form=merged_form, parts=parts)
         out_.copy_(out_wide[..., :head_dim])
         return out_, lse_, None, None
     if workspace is None:
         workspace = forward_workspace(q.device)
     if workspace.dtype != torch.int32 or not workspace.is_contiguous():
         raise ValueError("workspace must be a contiguous int32 tensor from forward_workspace()")
-    _lib.call(
-        "dcp_attn_fwd_strided",
+    args = (
         q.data_ptr(), k.data_ptr(), v.data_ptr(), out_.data_ptr(), lse_.data_ptr(),
         _i32(cu_seqlens_q, "cu_seqlens_q").data_ptr(),
         _i32(cu_seqlens_k, "cu_seqlens_k").data_ptr(),
@@ -268,8 +270,16 @@ def _flash_attn_varlen_forward(
         n_heads_q, n_heads_kv, head_dim,
         kv_slot_stride, kv_token_stride, q_entry, out_entry, lse_head_stride, lse_entry,
         1 if merged_form else 0, float(softmax_scale), dtype_code(q.dtype),
-        workspace.data_ptr(), workspace.numel() * 4, _stream(),
+        workspace.data_ptr(), workspace.numel() * 4,
     )
+    if parts is None:
+        _lib.call("dcp_attn_fwd_strided", *args, _stream())
+    else:
+        entries, splits, n_partials, partials = parts
+        if entries.shape[1:] != (4,) or splits.shape[1:] != (4,) or partials.dtype != torch.float32 or not partials.is_contiguous():
+            raise ValueError("parts: [entries, 4] and [split rows, 4] tables and contiguous fp32 scratch expected")
+        _lib.call("dcp_attn_fwd_parts", *args, _i32(entries, "parts").data_ptr(), entries.shape[0], _i32(splits, "splits").data_ptr(),
+                  splits.shape[0], int(n_partials), partials.data_ptr(), partials.numel() * 4, _stream())
     return out_, lse_, None, None
 
 

@@ -281,6 +281,37 @@ int dcp_attn_fwd_strided(const void* q, const void* k, const void* v, void* out,
                          void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * dcp_attn_fwd_strided for launches of few, uneven rows: rows may be split along
+ * their keys, so that the launch does not last as long as its longest row.
+ * `parts` ([n_entries][4] int32: row, part, number of parts n, first partial)
+ * takes the place of row_order: an entry computes an equal share of the key tiles
+ * of every (head, query tile) of its row; every row appears with parts 0..n-1.
+ * Entries with n = 1 write out and lse.  The others leave fp32 sums in partial
+ * `first partial` + part of `partials` (16-byte aligned, n_partials *
+ * ceil(block_size / 128) * 128 * n_heads_q * (head_dim + 2) floats, contents
+ * overwritten; partials of a launch are not shared), and a second kernel adds
+ * the parts of the rows that `splits` lists ([n_splits][4]: row, n, first
+ * partial, 0) and rounds once.  No counterpart in the reference.
+ */
+int dcp_attn_fwd_parts(const void* q, const void* k, const void* v, void* out,
+                       float* lse, const int32_t* cu_seqlens_q,
+                       const int32_t* cu_seqlens_kv, const int32_t* attn_range,
+                       int n_ranges, const int32_t* q_block_table,
+                       const int32_t* kv_block_table,
+                       const int32_t* out_block_table,
+                       const int32_t* row_order, int batch, int max_kv_blocks,
+                       int total_q, int block_size, int n_heads_q,
+                       int n_heads_kv, int head_dim, int64_t kv_slot_stride,
+                       int64_t kv_token_stride, int64_t q_slot_stride,
+                       int64_t out_slot_stride, int64_t lse_head_stride,
+                       int64_t lse_slot_stride, int merged_form,
+                       float softmax_scale, int dtype, void* workspace,
+                       size_t workspace_bytes, const int32_t* parts,
+                       int n_entries, const int32_t* splits, int n_splits,
+                       int n_partials, void* partials, size_t partials_bytes,
+                       void* stream);
+
+/*
  * Range-masked, paged, variable-length attention backward.
  * Replaces dcp_flash_attn._flash_attn_varlen_backward as called by
  * _wrapped_flash_attn_varlen_backward (executor.py:256-337) from
