@@ -47,6 +47,7 @@ constexpr int kDsThreads = 64 * kDsWaves;
 constexpr int kDsBM = 32 * kDsWaves;  // queries per workgroup
 constexpr int kDsBN = 64;             // keys per tile
 constexpr int kDsStages = 3;
+constexpr int kDsFewItems = 4;        // per CU, see launch_bwd_through_ds
 
 // HH: q heads per work item (1, or 2 of the same kv head).  With two, a K tile brought into LDS
 // serves both heads' pieces: the sequence of steps is (tile 0, head 0), (tile 0, head 1), (tile 1,
@@ -306,7 +307,13 @@ int launch_bwd_through_ds(const AttnBwdParams& p, int dtype, hipStream_t stream)
   // this dQ kernel's work items: (row, one or two q heads of a kv head, 256-query tile); the tiles and
   // heads that share a K stay on one XCD
   const int per_kv = p.n_heads_q / p.n_heads_kv;
-  const int hh = per_kv % 2 == 0 ? 2 : 1;  // (four heads' accumulators do not fit the 256 registers of a wave)
+  // One head per item where that gives at most kDsFewItems items per CU: with two, half as many and twice
+  // as long, the launch is bound by its longest rows and not by the stream of dS (backward of 4096 tokens,
+  // 8 heads, 144 one-head items: 160 us with two heads, 132 with one; 8192 tokens, 16 heads, 544 items:
+  // 441 and 397; 1088 items, two ranges per query: 658 and 666).  (Four heads' accumulators do not fit
+  // the 256 registers of a wave.)
+  const int64_t one_head_items = (int64_t)p.batch * p.n_heads_q * ((p.block_size + kDsBM - 1) / kDsBM);
+  const int hh = per_kv % 2 == 0 && one_head_items > kDsFewItems * (int64_t)device_cu_count() ? 2 : 1;
   AttnBwdParams q = p;
   q.dq_tiles_per_row = (p.block_size + kDsBM - 1) / kDsBM;
   q.n_dq_items = (int64_t)p.batch * (p.n_heads_q / hh) * q.dq_tiles_per_row;
