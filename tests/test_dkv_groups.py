@@ -143,6 +143,11 @@ def test_group_size_rule():
     assert dkv_groups.parts_per_visit(1, 2, 512, 1, 4) == (1, 1)
 
 
+@pytest.mark.parametrize("pairs,rows", [(0.99, 1), (1.19, 2), (2.38, 3), (3.12, 3), (3.53, 4), (7.75, 8), (8.1, 8), (15.9, 8), (25, 13), (80, 32)])
+def test_rows_per_group_by_pairs_per_slot(pairs, rows):
+    assert dkv_groups.visits_per_group(round(pairs * 512), 1, 512) == rows
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("limit", [2, 32])
 @pytest.mark.parametrize("mode", [0, 2])
