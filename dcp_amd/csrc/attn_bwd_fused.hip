@@ -59,6 +59,7 @@ constexpr int kFusedBM = 32;              // queries per step
 constexpr int kFusedBN = 128;             // keys per workgroup
 constexpr int kDsStride = 36;             // elements per key row of the dS exchange (32 queries + 8 bytes)
 constexpr int kChunkFloats = 4096;        // one chunk of partial dQ: 32 queries x 128 dims
+constexpr int kPrepareRound = 4;          // (query, head) pairs a lane of the prepare kernel has in flight
 constexpr int kSpinLimit = 1 << 20;       // polls of a chain counter before a wave gives up (and raises the fault flag)
 
 // Key tiles (128 keys) that see a 64-query tile, from the tile's range hull: two runs of tile
@@ -70,6 +71,11 @@ __device__ __forceinline__ TileRuns chain_runs(const int32_t* hull) {
 
 // ---------------------------------------------------------------------------
 // prepare: hulls, -delta, lse2, counters
+//
+// Bound by the reads of out and dO.  A workgroup per (row, 64-query tile) is too few of them for a short
+// plan (88 at 5120 tokens, four rounds of loads each), so that a tile's (query, head) pairs are dealt to
+// gridDim.y workgroups then; the first of them does what is done once per tile.  5120 tokens, 8 heads of
+// size 64: 9.1 -> 5.3 us; at 8192 workgroups (65536 tokens, 32 heads) one each, 1.07 GB in 235 us.
 // ---------------------------------------------------------------------------
 template <int DTYPE, int D>
 __global__ __launch_bounds__(kBwdThreads) void bwd_prepare_kernel(const AttnBwdParams p) {
@@ -77,13 +83,14 @@ __global__ __launch_bounds__(kBwdThreads) void bwd_prepare_kernel(const AttnBwdP
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int b = blockIdx.x / p.q_tiles_per_row;
   const int qt = blockIdx.x - b * p.q_tiles_per_row;
-  if (blockIdx.x == 0 && tid == 0 && p.fault != nullptr) *p.fault = 0;
-  if (blockIdx.x == 0)
+  const bool first = blockIdx.y == 0;
+  if (blockIdx.x == 0 && first && tid == 0 && p.fault != nullptr) *p.fault = 0;
+  if (blockIdx.x == 0 && first)
     for (int i = tid; i < 2 * kTicketInts; i += kBwdThreads) p.tickets[i] = 0;  // for the kernels that follow
   const int q_begin = p.cu_seqlens_q[b];
   const int seqlen_q = p.cu_seqlens_q[b + 1] - q_begin;
   const int seqlen_kv = p.cu_seqlens_kv[b + 1] - p.cu_seqlens_kv[b];
-  if (wave == 0) {
+  if (wave == 0 && first) {
     const int ql = qt * kBwdBM + lane;
     int s0 = 0, l0 = 0, s1 = 0, l1 = 0;
     if (ql < seqlen_q) {
@@ -132,9 +139,9 @@ __global__ __launch_bounds__(kBwdThreads) void bwd_prepare_kernel(const AttnBwdP
   const int sub_lane = lane % LPP;
   // (four positions per round, all their words requested before anything is stored: the stores could
   // alias the loads as far as the compiler knows, so it would not move a load above one itself)
-  constexpr int U = 4;
+  constexpr int U = kPrepareRound;
   constexpr int STEP = (kBwdThreads / 64) * PPW;
-  for (int pair0 = wave * PPW; pair0 < n_q * H; pair0 += U * STEP) {
+  for (int pair0 = blockIdx.y * (U * STEP) + wave * PPW; pair0 < n_q * H; pair0 += gridDim.y * (U * STEP)) {
     u32x4 o[U], g[U];
     float l[U];
     bool live[U];
@@ -664,7 +671,13 @@ size_t bwd_fused_extra_workspace_bytes(int batch, int block_size, int n_heads_q,
 
 int launch_bwd_prepare(const AttnBwdParams& p, int dtype, hipStream_t stream) {
   KernelTimer timer("bwd_prepare_kernel", stream);
-  const dim3 grid(p.batch * p.q_tiles_per_row), block(kBwdThreads);
+  // workgroups for eight per CU, none without a round of its own (the one-pass backward's work per tile
+  // needs the tile's hull in every workgroup: one)
+  const int64_t tiles = (int64_t)p.batch * p.q_tiles_per_row;
+  const int pairs_per_round = kPrepareRound * kBwdThreads / (p.head_dim / 8);
+  const int rounds = (kBwdBM * p.n_heads_q + pairs_per_round - 1) / pairs_per_round;
+  const int split = p.chain != nullptr ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rounds, 8 * (int64_t)device_cu_count() / tiles));
+  const dim3 grid((unsigned)tiles, split), block(kBwdThreads);
   if (dtype == DCP_DTYPE_BF16) {
     if (p.head_dim == 128) hipLaunchKernelGGL((bwd_prepare_kernel<DCP_DTYPE_BF16, 128>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((bwd_prepare_kernel<DCP_DTYPE_BF16, 64>), grid, block, 0, stream, p);

@@ -80,3 +80,24 @@ def test_executor_recomputes_when_ds_would_not_fit_the_workspace_limit(gpu, monk
     assert "attn_bwd_dq_kernel" in ran_small and "attn_bwd_dq_ds_kernel" not in ran_small, ran_small
     assert scaled_err(ds[3].float().numpy(), small[3].float().numpy()) <= GRAD_TOL
     assert np.abs(ds[2].float().numpy() - small[2].float().numpy()).max() <= GRAD_TOL
+
+
+@pytest.mark.parametrize("kw", [
+    dict(n_heads=4, n_groups=1, head_dim=128, head_block=4),
+    dict(n_heads=6, n_groups=1, head_dim=64, head_block=6, mask="lambda", mask_kwargs=dict(n_starting=16, l_pretrain=150)),
+    dict(n_heads=5, n_groups=1, head_dim=128, head_block=5, dtype="fp16"),
+], ids=["two_heads_per_item", "two_heads_two_ranges", "five_heads"])
+def test_many_short_rows(gpu, kw):
+    """Launches of more than four one-head dQ items per CU, which take two heads per item where a kv head
+    has an even number of them, and whose prepare kernel deals a tile's pairs to fewer workgroups than
+    it has rounds of loads; short ragged rows, a partly filled last key tile."""
+    from dcp_amd import _lib
+
+    case = make_case(seqlens=[100, 33, 300, 129] * 60, block_size=128, qkv_scale=0.5, **kw)
+    lib = _lib.load()
+    before = lib.dcp_attn_bwd_select(2)
+    try:
+        result, _ = run_executor(case, backward=True, poison=200.0)
+    finally:
+        lib.dcp_attn_bwd_select(before)
+    check_against_truth(result, dense_truth(case, backward=True))
