@@ -49,5 +49,8 @@ def test_split_forward_matches_dense_attention(gpu, monkeypatch, name, share):
     assert ex._fwd_partials is not None
     check_against_truth(split, dense_truth(case, backward=False))
     assert torch.equal(split[0], as_written[0])
+    monkeypatch.delenv("DCP_DIRECT_LOCAL")
+    replayed, _ = run_executor(case, backward=False, use_graph=True)
+    assert torch.equal(split[0], replayed[0]) and torch.equal(split[1], replayed[1])
     # the merged LSE of two launches goes through the merge kernel as written and directly
     np.testing.assert_allclose(split[1].float().cpu().numpy(), whole[1].float().cpu().numpy(), rtol=2e-6, atol=2e-6)
