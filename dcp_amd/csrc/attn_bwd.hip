@@ -188,10 +188,10 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   }
   if (!grouped && tile_no * BN >= __builtin_amdgcn_readfirstlane(mine.seqlen_kv)) return;
   if (w == 0 && lane < n_visits) visit_lds[lane] = mine;
-  // A wave whose 32 keys lie past the row's keys (seqlen_kv need not be a multiple of 128; a grouped
-  // launch has whole blocks only) still loads its share of every tile and meets every barrier; its
-  // arithmetic is switched off and it stores nothing.  Its K/V addresses fall back to the tile's
-  // first keys so that they stay valid.
+  // A wave whose 32 keys lie past the row's keys (seqlen_kv need not be a multiple of 128) still loads its
+  // share of every tile and meets every barrier; its keys are masked and it stores no dK/dV.  Its
+  // K/V addresses fall back to the tile's first keys so that they stay valid.  (A group's K/V are the
+  // kv block's, whole: which of its keys a row has is asked per visit.)
   const int kw_tile = tile_no * BN + w * 32;  // from the first key of the row's keys (of the block, in a group)
   const bool has_keys = grouped || kw_tile < __builtin_amdgcn_readfirstlane(mine.seqlen_kv);
   const int kw_safe = has_keys ? kw_tile : tile_no * BN;
@@ -308,10 +308,11 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   // out [head][32-query chunk][64-key tile]: the pieces that a wave of the dQ kernel reads one after
   // another lie one after another (ordered by key tile first, they were 4 MiB apart at 32 heads and
   // 1024-token blocks, every one in a memory page of its own).  ds_lane: the lane's 16 bytes within a
-  // [key][query half] plane of a piece.  (A wave whose 32 keys lie past the row's last key has no
-  // piece -- its 64-key half tile would be the next row's first, or lie past the end of the
+  // [key][query half] plane of a piece.  (A wave whose 64-key half tile begins past the row's last
+  // key has no piece -- it would be one of the next 32-query chunk's, or lie past the end of the
   // workspace -- and writes its zeros into a spare piece behind the last one instead, with a row of
-  // no tiles: no branch around the stores.)
+  // no tiles: no branch around the stores.  The zeros of a wave without keys beside one with some
+  // are the other half of that one's piece, which the dQ kernel reads whole.)
   uint64_t ds_visit = 0;
   uint32_t ds_row_tiles = 0;  // pieces from a 32-query chunk to the next
   const int ds_lane = (w & 1) * 128 + 2 * c + h;
@@ -321,10 +322,11 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     unm_w = uniform64(mask_lds[v][1 + w]);
     if constexpr (WRITE_DS) {
       const int seqlen_kv = visit_field(v, DkvVisit::kSeqlenKv), kw = visit_field(v, DkvVisit::kKRow) + w * 32;
-      ds_row_tiles = has_keys ? (seqlen_kv + 63) / 64 : 0;
+      const bool has_piece = (kw & ~63) < seqlen_kv;
+      ds_row_tiles = has_piece ? (seqlen_kv + 63) / 64 : 0;
       const uint64_t piece = (uint64_t)visit_field(v, DkvVisit::kDsTile0) * p.n_heads_q * p.subs_per_row +
                              (uint64_t)(kv_head * group) * p.subs_per_row * ds_row_tiles + (kw >> 6);
-      ds_visit = uniform64(reinterpret_cast<uint64_t>(p.ds) + ((has_keys ? piece : (uint64_t)p.ds_pieces) << 12));
+      ds_visit = uniform64(reinterpret_cast<uint64_t>(p.ds) + ((has_piece ? piece : (uint64_t)p.ds_pieces) << 12));
     }
   };
   auto next_active = [&](int v) {  // the first visit from v on with an active tile, or n_visits

@@ -109,7 +109,7 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
     g[3] = max(g[3], __builtin_amdgcn_readfirstlane(hu[3]));
   }
   TileRuns runs(g[0], g[1], g[2], g[3], 128);
-  // as runs of 64-key tiles, none past the row's last key (its key count is a multiple of 64)
+  // as runs of 64-key tiles, none past the one that holds the row's last key
   const int last64 = (seqlen_kv + BN - 1) / BN;
   runs.a0 *= 2;
   runs.b0 = min(runs.b0 * 2, last64);

@@ -401,8 +401,8 @@ int dcp_attn_bwd_strided(const void* dout, const void* q, const void* k,
  *     the row's kv_block_table
  * Every (query, row, position) with keys belongs to exactly one group (a plan's
  * replicas that are not added up form groups of one); dkv_block_table is
- * not read.  Rows must hold whole blocks (key counts that are multiples of
- * block_size) and block_size must be a multiple of 128.  A group's tokens are
+ * not read.  block_size must be a multiple of 128; a row's last block may be
+ * partly filled (its key count need not be a multiple).  A group's tokens are
  * written whole (zeros where no query attends).  Launch order of the groups:
  * as listed, so the ones with the most visits should come first.  The one-pass
  * backward has no such form (the two-kernel one runs where it is selected).

@@ -211,3 +211,51 @@ def test_grouped_backward_with_an_exchange(gpu, monkeypatch):
     err = scaled_err(grouped[3].float().numpy(), dense_truth(case, backward=True)[3])
     same_dq = torch.equal(grouped[2], single[2])
     assert same_dq and err <= 4e-2
+
+
+def _with_exact_key_counts(case):
+    """The case's backward plan with the rows' key counts taken from their blocks' tokens: a row whose last
+    block is ragged ends inside it.  How many rows that are."""
+    n = 0
+    for instr in case["bw"].instructions:
+        if isinstance(instr, AttnBackwardInstr):
+            exact = [sum(block.n_tokens for block in row) for row in instr.kv_block_table]
+            n += sum(a != b for a, b in zip(exact, instr.seqlens_kv))
+            instr.seqlens_kv = exact
+    return n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("limit", [1, 2, 32])
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("name", ["causal_gqa", "split", "lambda"])
+def test_rows_that_end_inside_a_block(gpu, monkeypatch, name, mode, limit):
+    """Key counts that are no multiples of the block size, nor of the 64 keys of a dS piece: the masked keys of
+    whole blocks contribute exact zeros, so the results are those of whole blocks bit for bit.  The
+    backward's scratch holds NaNs before."""
+    from dcp_amd import _lib
+    from dcp_amd.runtime.flash_attention.executor import AttentionExecutor
+
+    prepare = AttentionExecutor.prepare
+
+    def with_nans_in_scratch(self, forward=True):
+        prepare(self, forward)
+        if self._bwd_workspace is not None:
+            self._bwd_workspace.fill_(255)
+
+    monkeypatch.setattr(AttentionExecutor, "prepare", with_nans_in_scratch)
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: limit)
+    monkeypatch.setattr(dkv_groups, "parts_per_visit", lambda *a: (1, 1))
+    lib = _lib.load()
+    case = make_case(**PLANS[name])
+    before = lib.dcp_attn_bwd_select(mode)
+    try:
+        whole, _ = run_executor(case, backward=True)
+        assert _with_exact_key_counts(case) > 0
+        exact, ex = run_executor(case, backward=True, poison=200.0)
+    finally:
+        lib.dcp_attn_bwd_select(before)
+    assert bool(ex._dkv_groups.groups) == (limit > 1)
+    check_against_truth(exact, dense_truth(case, backward=True))
+    same_dq, same_dkv = torch.equal(exact[2], whole[2]), torch.equal(exact[3], whole[3])
+    assert same_dq and same_dkv
