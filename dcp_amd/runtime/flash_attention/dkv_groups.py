@@ -25,11 +25,14 @@ from typing import Dict, List, Optional, Set, Tuple, Union
 
 from dcp_amd.core.instructions import (
     AttnBackwardInstr,
+    AttnInstr,
     AttnReductionInstr,
+    BarrierInstr,
     BufferBlock,
     BufferType,
     CommLaunchInstr,
     CommType,
+    CommWaitInstr,
     ExecutionPlan,
     MemcpyInstr,
     SumInstr,
@@ -176,11 +179,16 @@ class _Visits:
 
 _UNREAD, _ELSEWHERE = -1, -2  # readers of a replica: none; other than one sum op
 
+# the instructions whose reads and writes of BUFFER_dKV slots `analyse` follows
+_KNOWN = {AttnInstr, AttnBackwardInstr, AttnReductionInstr, BarrierInstr, CommLaunchInstr, CommWaitInstr, MemcpyInstr, SumInstr}
+
 
 def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_block: int, n_slots: int,
             q_heads_per_kv_head: int = 1) -> DkvGroups:
     result = DkvGroups()
     instrs = plan.instructions
+    if not _KNOWN.issuperset(map(type, instrs)):  # an instruction of another kind may read any replica
+        return result
     limits, parts = {}, {}
     for idx, instr in enumerate(instrs):
         if isinstance(instr, AttnBackwardInstr):

@@ -96,6 +96,19 @@ def test_exchanged_replicas_are_left_alone(monkeypatch):
         _check_groups(plan, found, slots_written_once=False)
 
 
+@pytest.mark.parametrize("parts", [(1, 1), (2, 1)])
+def test_a_plan_with_an_unknown_instruction_is_left_alone(monkeypatch, parts):
+    """An instruction of a kind the analysis does not know may read any replica."""
+    monkeypatch.setattr(dkv_groups, "parts_per_visit", lambda *a: parts)
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 1 if parts != (1, 1) else 32)
+    plan = make_case(**PLANS["causal_gqa"])["bw"]
+    assert dkv_groups.analyse(plan, DirectPlan(), 1, 1, 512, 2).groups
+    for at in (0, len(plan.instructions) // 2, len(plan.instructions)):
+        other = make_case(**PLANS["causal_gqa"])["bw"]
+        other.instructions.insert(at, object())
+        assert dkv_groups.analyse(other, DirectPlan(), 1, 1, 512, 2) == dkv_groups.DkvGroups()
+
+
 @pytest.mark.parametrize("parts", [(1, 2), (2, 1), (3, 4)])
 @pytest.mark.parametrize("name", ["causal_gqa", "split", "lambda"])
 def test_parts_cover_every_head_and_tile_once(monkeypatch, name, parts):
