@@ -135,6 +135,8 @@ def _components(kv_rows: List[List[int]]) -> Dict[int, Tuple[int, int]]:
 
     known = parent.get
     for blocks in kv_rows:
+        if not blocks:  # a row that attends to nothing
+            continue
         first = blocks[0]
         if first not in parent:
             parent[first] = first

@@ -96,6 +96,32 @@ def test_exchanged_replicas_are_left_alone(monkeypatch):
         _check_groups(plan, found, slots_written_once=False)
 
 
+def _without_keys_of_a_row(plan):
+    """Leaves a row of the backward plan (the first of one kv block) nothing to attend to, and takes its
+    replica from the sum.  The slots that are gone."""
+    gone = set()
+    for instr in plan.instructions:
+        if isinstance(instr, AttnBackwardInstr):
+            row = next(r for r, blocks in enumerate(instr.kv_block_table) if len(blocks) == 1)
+            gone.update(b.index for b in instr.dkv_block_table[row])
+            instr.kv_block_table[row], instr.dkv_block_table[row], instr.seqlens_kv[row] = [], [], 0
+        elif isinstance(instr, SumInstr):
+            for op in instr.ops:
+                if op.src_buffers[0].buffer_type == BufferType.BUFFER_dKV and len(op.src_buffers) > 1:
+                    op.src_buffers = [b for b in op.src_buffers if b.index not in gone]
+    return gone
+
+
+@pytest.mark.parametrize("limit", [3, 32])
+def test_a_row_without_kv_blocks(monkeypatch, limit):
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: limit)
+    plan = make_case(**PLANS["causal_gqa"])["bw"]
+    assert _without_keys_of_a_row(plan)
+    found = dkv_groups.analyse(plan, analyse_direct(plan), 1, 1, 512)
+    assert found.groups
+    _check_groups(plan, found)
+
+
 @pytest.mark.parametrize("parts", [(1, 1), (2, 1)])
 def test_a_plan_with_an_unknown_instruction_is_left_alone(monkeypatch, parts):
     """An instruction of a kind the analysis does not know may read any replica."""
@@ -272,3 +298,26 @@ def test_rows_that_end_inside_a_block(gpu, monkeypatch, name, mode, limit):
     check_against_truth(exact, dense_truth(case, backward=True))
     same_dq, same_dkv = torch.equal(exact[2], whole[2]), torch.equal(exact[3], whole[3])
     assert same_dq and same_dkv
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [0, 2])
+def test_grouped_backward_of_a_row_without_kv_blocks(gpu, monkeypatch, mode):
+    from dcp_amd import _lib
+
+    lib = _lib.load()
+    case = make_case(**PLANS["causal_gqa"])
+    assert _without_keys_of_a_row(case["bw"])
+    monkeypatch.setattr(dkv_groups, "parts_per_visit", lambda *a: (1, 1))
+    before = lib.dcp_attn_bwd_select(mode)
+    try:
+        monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 1)
+        single, _ = run_executor(case, backward=True)
+        monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+        grouped, ex = run_executor(case, backward=True, poison=200.0)
+    finally:
+        lib.dcp_attn_bwd_select(before)
+    assert ex._dkv_groups.groups
+    same_dq = torch.equal(grouped[2], single[2])
+    # nine replicas of about one, each rounded to bf16 (2^-9) before the plan's own sum adds them
+    assert same_dq and scaled_err(grouped[3].float().numpy(), single[3].float().numpy()) <= 2e-2
