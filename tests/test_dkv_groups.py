@@ -122,6 +122,37 @@ def test_a_row_without_kv_blocks(monkeypatch, limit):
     _check_groups(plan, found)
 
 
+def _executor_without_a_device(monkeypatch, plan, run=None, prep=None):
+    """An executor that can be asked for its groups on a machine without a GPU; ``run`` and ``prep``: handlers
+    that take the place of this package's, by instruction type."""
+    from types import SimpleNamespace
+
+    from dcp_amd.core.executor import HandlerTable
+    from dcp_amd.runtime.flash_attention import executor as module
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: SimpleNamespace(multi_processor_count=256))
+    ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
+    ex.fabric, ex.execution_plan, ex._direct = None, plan, DirectPlan()
+    ex.buffer_per_token_shape = {t: info.per_token_shape for t, info in plan.buffer_info.items()}
+    ex._handlers, ex._prep_handlers = HandlerTable("run"), HandlerTable("prep")
+    for kind, name in ((AttnBackwardInstr, "attn_bw"), (SumInstr, "sum")):
+        ex._handlers.register(kind, (run or {}).get(kind, getattr(module, f"_handle_{name}")))
+        ex._prep_handlers.register(kind, (prep or {}).get(kind, getattr(module, f"_prepare_{name}")))
+    return ex
+
+
+@pytest.mark.parametrize("table", ["run", "prep"])
+@pytest.mark.parametrize("kind", [AttnBackwardInstr, SumInstr])
+def test_no_groups_where_a_handler_is_the_callers_own(monkeypatch, table, kind):
+    """The plug-in surface: an own handler writes and adds every replica, as the plan says."""
+    plan = make_case(**PLANS["causal_gqa"])["bw"]
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+    assert _executor_without_a_device(monkeypatch, plan)._group_dkv_replicas().groups
+    own = {kind: lambda e, i: None}
+    assert _executor_without_a_device(monkeypatch, plan, **{table: own})._group_dkv_replicas() == dkv_groups.DkvGroups()
+
+
 @pytest.mark.parametrize("parts", [(1, 1), (2, 1)])
 def test_a_plan_with_an_unknown_instruction_is_left_alone(monkeypatch, parts):
     """An instruction of a kind the analysis does not know may read any replica."""
@@ -321,3 +352,50 @@ def test_grouped_backward_of_a_row_without_kv_blocks(gpu, monkeypatch, mode):
     same_dq = torch.equal(grouped[2], single[2])
     # nine replicas of about one, each rounded to bf16 (2^-9) before the plan's own sum adds them
     assert same_dq and scaled_err(grouped[3].float().numpy(), single[3].float().numpy()) <= 2e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [AttnBackwardInstr, SumInstr])
+def test_handlers_of_the_callers_own_find_every_replica(gpu, monkeypatch, kind):
+    """A caller's own backward that writes the replicas, and a caller's own sum that reads them."""
+    from dcp_amd.runtime.flash_attention import executor as module
+
+    case = make_case(**PLANS["causal_gqa"])
+    with monkeypatch.context() as m:
+        m.setattr(dkv_groups, "visits_per_group", lambda *a: 1)
+        m.setattr(dkv_groups, "parts_per_visit", lambda *a: (1, 1))
+        want, _ = run_executor(case, backward=True)
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+    theirs = {AttnBackwardInstr: module._handle_attn_bw, SumInstr: module._handle_sum}[kind]
+    seen = []
+
+    def own(ex, instr):
+        seen.append(ex.instr_index)
+        if kind is AttnBackwardInstr:
+            theirs(ex, instr)
+            return
+        cu, bs = ex.execution_plan.local_cu_seqlens, ex.buffer_block_sizes
+        for op in instr.ops:  # the plan's sum in torch: added in fp32 in the plan's order, rounded once
+            n, dst = op.dst_buffer.n_tokens, op.dst_buffer
+            total = sum(ex.buffers[b.buffer_type].view(-1, bs[b.buffer_type], *ex.buffer_per_token_shape[b.buffer_type])[b.index, :n].float()
+                        for b in op.src_buffers)
+            to = ex.buffers[dst.buffer_type]
+            if instr.output_is_unpadded:
+                to[cu[dst.index] : cu[dst.index] + n] = total.to(to.dtype)
+            else:
+                to.view(-1, bs[dst.buffer_type], *ex.buffer_per_token_shape[dst.buffer_type])[dst.index, :n] = total.to(to.dtype)
+
+    monkeypatch.setattr(module, "get_executor", _with_own_handler(module.get_executor, kind, own))
+    monkeypatch.setenv("DCP_DIRECT_LOCAL", "0")  # (its sums may leave out scatters, which an own handler makes)
+    got, ex = run_executor(case, backward=True)
+    assert seen and not ex._dkv_groups.groups
+    assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3])
+
+
+def _with_own_handler(get_executor, kind, own):
+    def make(*args, **kw):
+        ex = get_executor(*args, **kw)
+        ex._handlers._by_type[kind] = own
+        return ex
+
+    return make
