@@ -133,7 +133,7 @@ def _executor_without_a_device(monkeypatch, plan, run=None, prep=None):
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: SimpleNamespace(multi_processor_count=256))
     ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
-    ex.fabric, ex.execution_plan, ex._direct = None, plan, DirectPlan()
+    ex.fabric, ex.execution_plan, ex._direct, ex.dkv_groups = None, plan, DirectPlan(), True
     ex.buffer_per_token_shape = {t: info.per_token_shape for t, info in plan.buffer_info.items()}
     ex._handlers, ex._prep_handlers = HandlerTable("run"), HandlerTable("prep")
     for kind, name in ((AttnBackwardInstr, "attn_bw"), (SumInstr, "sum")):
@@ -151,6 +151,13 @@ def test_no_groups_where_a_handler_is_the_callers_own(monkeypatch, table, kind):
     assert _executor_without_a_device(monkeypatch, plan)._group_dkv_replicas().groups
     own = {kind: lambda e, i: None}
     assert _executor_without_a_device(monkeypatch, plan, **{table: own})._group_dkv_replicas() == dkv_groups.DkvGroups()
+
+
+def test_groups_can_be_turned_off(monkeypatch):
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+    ex = _executor_without_a_device(monkeypatch, make_case(**PLANS["causal_gqa"])["bw"])
+    ex.dkv_groups = False
+    assert ex._group_dkv_replicas() == dkv_groups.DkvGroups()
 
 
 @pytest.mark.parametrize("parts", [(1, 1), (2, 1)])
@@ -399,3 +406,35 @@ def _with_own_handler(get_executor, kind, own):
         return ex
 
     return make
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(PLANS))
+def test_plan_as_written(gpu, monkeypatch, name):
+    """Without groups dK/dV are the sums of the rounded replicas the plan asks for, whether or not copies
+    are left out, and every replica is in its slot."""
+    from collections import defaultdict
+
+    case = make_case(**PLANS[name])
+    grouped, _ = run_executor(case, backward=True)
+    monkeypatch.setenv("DCP_DKV_GROUPS", "0")
+    direct, ex = run_executor(case, backward=True)
+    assert not ex.dkv_groups and not ex._dkv_groups.groups
+    monkeypatch.setenv("DCP_DIRECT_LOCAL", "0")
+    as_written, ex = run_executor(case, backward=True, poison=200.0)
+    assert torch.equal(direct[2], as_written[2]) and torch.equal(direct[3], as_written[3])
+    assert torch.equal(grouped[2], as_written[2])  # (dQ does not depend on the grouping)
+    assert scaled_err(grouped[3].float().numpy(), as_written[3].float().numpy()) <= 2e-2
+    cu, slots, written = case["bw"].local_cu_seqlens, ex.buffers["BufferdKV"], defaultdict(int)
+    for instr in case["bw"].instructions:
+        if isinstance(instr, AttnBackwardInstr):
+            for row in instr.dkv_block_table:
+                for block in row:
+                    written[block.index] += 1
+        for op in instr.ops if isinstance(instr, SumInstr) else []:
+            src, dst = op.src_buffers, op.dst_buffer
+            if dst.buffer_type != BufferType.LOCAL_dKV or not all(written[b.index] == 1 for b in src):
+                continue
+            total = sum(slots[b.index, : dst.n_tokens].float() for b in src)
+            got = ex.buffers["LocaldKV"][cu[dst.index] : cu[dst.index] + dst.n_tokens]
+            assert torch.equal(got, total.to(got.dtype))
