@@ -160,6 +160,18 @@ def test_groups_can_be_turned_off(monkeypatch):
     assert ex._group_dkv_replicas() == dkv_groups.DkvGroups()
 
 
+def test_no_groups_in_plans_without_a_backward_or_its_tensor(monkeypatch):
+    """Plans that have dK/dV slots but no backward launch (and no dQ), or no LOCAL_dKV."""
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+    sums = make_case(**PLANS["causal_gqa"])["bw"]
+    sums.instructions = [i for i in sums.instructions if isinstance(i, SumInstr)]
+    del sums.buffer_info[BufferType.BUFFER_dQ]
+    assert _executor_without_a_device(monkeypatch, sums)._group_dkv_replicas() == dkv_groups.DkvGroups()
+    slots_only = make_case(**PLANS["causal_gqa"])["bw"]
+    del slots_only.buffer_info[BufferType.LOCAL_dKV]
+    assert _executor_without_a_device(monkeypatch, slots_only)._group_dkv_replicas() == dkv_groups.DkvGroups()
+
+
 @pytest.mark.parametrize("parts", [(1, 1), (2, 1)])
 def test_a_plan_with_an_unknown_instruction_is_left_alone(monkeypatch, parts):
     """An instruction of a kind the analysis does not know may read any replica."""
