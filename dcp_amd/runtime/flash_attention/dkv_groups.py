@@ -207,7 +207,8 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
     reader = [_UNREAD] * len(row_of)
     sum_ops: List[Tuple[int, int]] = []  # the sum ops, numbered as in `reader`: (instruction, position)
     replicas_of: Dict[int, List[int]] = defaultdict(list)  # what a sum op reads of that kind
-    dkv = BufferType.BUFFER_dKV
+    dkv, local_dkv = followed = (BufferType.BUFFER_dKV, BufferType.LOCAL_dKV)
+    named: Counter = Counter()  # how often the plan names a LOCAL_dKV block
     in_parts = {idx for idx, p in parts.items() if p != (1, 1)}
 
     def reads(blocks, who=_ELSEWHERE):
@@ -218,10 +219,14 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
                     reader[replica] = who if reader[replica] == _UNREAD else _ELSEWHERE
                     if in_parts:
                         replicas_of[who].append(replica)
+            elif block.buffer_type == local_dkv:
+                named[block.index] += 1
 
     def writes(block: BufferBlock):
         if block.buffer_type == dkv:
             written.pop(block.index, None)
+        elif block.buffer_type == local_dkv:
+            named[block.index] += 1
 
     for idx, instr in enumerate(instrs):
         if isinstance(instr, AttnBackwardInstr):
@@ -235,7 +240,7 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
                 writes(op.dst_buffer)
         elif isinstance(instr, MemcpyInstr):
             for src, dst in instr.src_dst_pairs:
-                if src.buffer_type == dkv or dst.buffer_type == dkv:
+                if src.buffer_type in followed or dst.buffer_type in followed:
                     reads((src,))
                     writes(dst)
         elif isinstance(instr, CommLaunchInstr):
@@ -249,6 +254,8 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
             for op in instr.ops:
                 for blocks in op.src_buffers:
                     reads(blocks)
+                for block in op.dst_buffer:
+                    writes(block)
 
     # sum ops all of whose sources can be left as partials
     splittable = {v for idx in in_parts for v in visits.of(idx, instrs[idx])}
@@ -296,7 +303,8 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
             op = instrs[j].ops[op_pos]
             dst = direct.redirect_ops.get(j, {}).get(op_pos, op.dst_buffer if instrs[j].output_is_unpadded else None)
             if (len(taken) <= limit and len(taken) == len(op.src_buffers) and dst is not None
-                    and dst.buffer_type == BufferType.LOCAL_dKV and dst.n_tokens == slot_of[taken[0]].n_tokens):
+                    and dst.buffer_type == local_dkv and dst.n_tokens == slot_of[taken[0]].n_tokens
+                    and named[dst.index] == 1):  # (the launch writes it earlier than the sum would)
                 groups.append(Group([(row_of[v], pos_of[v]) for v in taken], dst))
                 result.skip_ops.setdefault(j, set()).add(op_pos)
                 continue

@@ -9,7 +9,7 @@ from collections import Counter
 import pytest
 import torch
 
-from dcp_amd.core.instructions import AttnBackwardInstr, BufferType, SumInstr
+from dcp_amd.core.instructions import AttnBackwardInstr, BufferBlock, BufferType, MemcpyInstr, SumInstr, SumOp
 from dcp_amd.runtime.flash_attention import dkv_groups
 from dcp_amd.runtime.flash_attention.direct import DirectPlan, analyse as analyse_direct
 from tests.plan_cases import check_against_truth, dense_truth, make_case, make_multi_case, run_executor, run_multi_executor, scaled_err
@@ -170,6 +170,26 @@ def test_no_groups_in_plans_without_a_backward_or_its_tensor(monkeypatch):
     slots_only = make_case(**PLANS["causal_gqa"])["bw"]
     del slots_only.buffer_info[BufferType.LOCAL_dKV]
     assert _executor_without_a_device(monkeypatch, slots_only)._group_dkv_replicas() == dkv_groups.DkvGroups()
+
+
+@pytest.mark.parametrize("how", ["written", "read"])
+def test_a_local_block_named_twice_is_left_to_its_sums(monkeypatch, how):
+    """The launch writes LOCAL_dKV earlier than the sum would: not if the plan does anything else with the
+    block, here between the two."""
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+
+    def local_blocks(plan):
+        found = dkv_groups.analyse(plan, analyse_direct(plan), 1, 1, 512)
+        _check_groups(plan, found)
+        return {g.dst.index: g.dst for gs in found.groups.values() for g in gs if g.dst.buffer_type == BufferType.LOCAL_dKV}
+
+    plan = make_case(**PLANS["causal_gqa"])["bw"]
+    before = local_blocks(plan)
+    block = next(iter(before.values()))
+    slot = BufferBlock(BufferType.BUFFER_dKV, 10 ** 6, block.n_tokens)
+    between = next(i for i, instr in enumerate(plan.instructions) if isinstance(instr, AttnBackwardInstr)) + 1
+    plan.instructions.insert(between, SumInstr([SumOp([slot], block)], True) if how == "written" else MemcpyInstr([(block, slot)]))
+    assert set(local_blocks(plan)) == set(before) - {block.index}
 
 
 @pytest.mark.parametrize("parts", [(1, 1), (2, 1)])
