@@ -9,7 +9,17 @@ from collections import Counter
 import pytest
 import torch
 
-from dcp_amd.core.instructions import AttnBackwardInstr, BufferBlock, BufferType, MemcpyInstr, SumInstr, SumOp
+from dcp_amd.core.instructions import (
+    AttnBackwardInstr,
+    BufferBlock,
+    BufferType,
+    CommLaunchInstr,
+    CommOp,
+    CommType,
+    MemcpyInstr,
+    SumInstr,
+    SumOp,
+)
 from dcp_amd.runtime.flash_attention import dkv_groups
 from dcp_amd.runtime.flash_attention.direct import DirectPlan, analyse as analyse_direct
 from tests.plan_cases import check_against_truth, dense_truth, make_case, make_multi_case, run_executor, run_multi_executor, scaled_err
@@ -30,45 +40,67 @@ PLANS = {
 }
 
 
-def _check_groups(plan, found, slots_written_once=True):
+def _check_groups(plan, found):
+    """Every (row, kv block) pair of a grouped launch is in exactly one group; and, walking the plan once as
+    written and once with the groups: whatever reads a dK/dV slot other than a sum finds in it what the plan
+    put there, and every sum adds the same replicas (or is left out where its replicas went together)."""
     instrs = plan.instructions
-    written = Counter()  # (instr, row, pos) -> times its dK/dV is part of a group
+    as_written, with_groups = {}, {}  # slot -> the (instr, row, pos) replicas or other writes added up in it
+    local = []  # what groups put into LOCAL_dKV
+
+    def put(block, what):
+        if block.buffer_type == BufferType.BUFFER_dKV:
+            as_written[block.index] = with_groups[block.index] = Counter([what])
+
+    def same(block):
+        if block.buffer_type == BufferType.BUFFER_dKV:
+            assert with_groups.get(block.index) == as_written.get(block.index)
+
+    def total(slots, blocks):
+        blocks = [b for b in blocks if b.buffer_type == BufferType.BUFFER_dKV]
+        assert all(b.index in slots for b in blocks)
+        return sum((slots[b.index] for b in blocks), Counter())
+
     for idx, instr in enumerate(instrs):
-        if not isinstance(instr, AttnBackwardInstr):
-            continue
-        if idx not in found.groups:
-            continue
-        for g in found.groups[idx]:
-            assert 1 <= len(g.visits) <= dkv_groups.MAX_VISITS
-            assert len({instr.kv_block_table[r][p].index for r, p in g.visits}) == 1
-            written.update((idx, r, p) for r, p in g.visits)
-            if g.dst.buffer_type == BufferType.BUFFER_dKV:
-                assert g.dst.index == instr.dkv_block_table[g.visits[0][0]][g.visits[0][1]].index
-        pairs = {(idx, r, p) for r, row in enumerate(instr.kv_block_table) for p in range(len(row))}
-        assert set(k for k in written if k[0] == idx) == pairs
-        sizes = [len(g.visits) for g in found.groups[idx]]
-        assert sizes == sorted(sizes, reverse=True)
-    assert all(n == 1 for n in written.values())
-    if not slots_written_once:
-        return
-    # every replica reaches the sum that adds it exactly once
-    members = {g.dst.index: Counter(instrs[i].dkv_block_table[r][p].index for r, p in g.visits)
-               for i, gs in found.groups.items() for g in gs if g.dst.buffer_type == BufferType.BUFFER_dKV}
-    local = [Counter(instrs[i].dkv_block_table[r][p].index for r, p in g.visits)
-             for i, gs in found.groups.items() for g in gs if g.dst.buffer_type == BufferType.LOCAL_dKV]
-    for j, instr in enumerate(instrs):
-        for pos, op in enumerate(instr.ops if isinstance(instr, SumInstr) else []):
-            want = Counter(b.index for b in op.src_buffers)
-            if pos in found.skip_ops.get(j, ()):
-                assert want in local
+        if isinstance(instr, AttnBackwardInstr):
+            pairs = {(r, p): slot for r, row in enumerate(instr.dkv_block_table) for p, slot in enumerate(row)}
+            for (r, p), slot in pairs.items():
+                put(slot, (idx, r, p))
+            if idx not in found.groups:
                 continue
-            left = found.sources.get(j, {}).get(pos)
-            if left is None:
-                continue
-            got = Counter()
-            for b in left:
-                got.update(members.get(b.index, Counter([b.index])))
-            assert got == want
+            for slot in pairs.values():  # (the launch writes the groups' slots only)
+                with_groups.pop(slot.index, None)
+            groups = found.groups[idx]
+            assert sorted(v for g in groups for v in g.visits) == sorted(pairs)
+            assert [len(g.visits) for g in groups] == sorted((len(g.visits) for g in groups), reverse=True)
+            for g in groups:
+                assert 1 <= len(g.visits) <= dkv_groups.MAX_VISITS
+                assert len({instr.kv_block_table[r][p].index for r, p in g.visits}) == 1
+                added = Counter((idx, r, p) for r, p in g.visits)
+                if g.dst.buffer_type == BufferType.BUFFER_dKV:
+                    assert g.dst.index == pairs[g.visits[0]].index
+                    with_groups[g.dst.index] = added
+                else:
+                    local.append(added)
+        elif isinstance(instr, SumInstr):
+            for pos, op in enumerate(instr.ops):
+                want = total(as_written, op.src_buffers) if op.src_buffers[0].buffer_type == BufferType.BUFFER_dKV else Counter()
+                if pos in found.skip_ops.get(idx, ()):
+                    assert want in local
+                else:
+                    assert total(with_groups, found.sources.get(idx, {}).get(pos, op.src_buffers)) == want
+            for pos, op in enumerate(instr.ops):
+                put(op.dst_buffer, ("sum", idx, pos))
+        elif isinstance(instr, MemcpyInstr):
+            for pos, (src, dst) in enumerate(instr.src_dst_pairs):
+                same(src)
+                put(dst, ("copy", idx, pos))
+        elif isinstance(instr, CommLaunchInstr):
+            for pos, op in enumerate(instr.comm_ops):
+                if op.comm_type == CommType.SEND:
+                    same(op.buffer_block)
+                else:
+                    put(op.buffer_block, ("received", idx, pos))
 
 
 @pytest.mark.parametrize("limit", [1, 3, 32])
@@ -86,14 +118,45 @@ def test_every_replica_is_added_once(monkeypatch, name, direct, limit):
         assert any(len(g.visits) > 1 for gs in found.groups.values() for g in gs)
 
 
-def test_exchanged_replicas_are_left_alone(monkeypatch):
-    """A dK/dV slot that is sent to another device is read by the exchange and keeps its own slot."""
-    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+@pytest.mark.parametrize("limit", [2, 32])
+@pytest.mark.parametrize("n_stages", [None, 2])
+def test_every_replica_of_a_device_is_added_once(monkeypatch, n_stages, limit):
+    """Plans with an exchange: sums over replicas and blocks that were received, slots used again."""
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: limit)
     case = make_multi_case(n_nodes=1, n_devices_per_node=2, seqlens=[700, 330], block_size=128, n_heads=4, n_groups=2, head_dim=64,
-                           head_block=2, n_stages=2)
+                           head_block=2, n_stages=n_stages)
     for plan in case["bw"]:
         found = dkv_groups.analyse(plan, DirectPlan(), 1, 1, 512)
-        _check_groups(plan, found, slots_written_once=False)
+        _check_groups(plan, found)
+        assert any(len(g.visits) > 1 for gs in found.groups.values() for g in gs)
+
+
+@pytest.mark.parametrize("how", ["sent", "copied", "added_twice", "received"])
+def test_replicas_with_another_reader_are_left_alone(monkeypatch, how):
+    """A replica that is sent to another device, copied, added by a second sum, or whose slot a received block
+    takes, keeps a group and a slot of its own, and the sum still adds that slot."""
+    monkeypatch.setattr(dkv_groups, "visits_per_group", lambda *a: 32)
+    plan = make_case(**PLANS["causal_gqa"])["bw"]
+    at = next(i for i, instr in enumerate(plan.instructions) if isinstance(instr, AttnBackwardInstr))
+    group = next(g for g in dkv_groups.analyse(plan, analyse_direct(plan), 1, 1, 512).groups[at] if len(g.visits) > 3)
+    row, pos = group.visits[2]
+    slot = plan.instructions[at].dkv_block_table[row][pos]
+    elsewhere = BufferBlock(BufferType.BUFFER_dKV, 10 ** 6, slot.n_tokens)
+    plan.instructions.insert(at + 1, {
+        "sent": lambda: CommLaunchInstr("k", [CommOp(CommType.SEND, (0, 1), slot)], None),
+        "received": lambda: CommLaunchInstr("k", [CommOp(CommType.RECV, (0, 1), slot)], None),
+        "copied": lambda: MemcpyInstr([(slot, elsewhere)]),
+        "added_twice": lambda: SumInstr([SumOp([slot], elsewhere)], False),
+    }[how]())
+    found = dkv_groups.analyse(plan, analyse_direct(plan), 1, 1, 512)
+    _check_groups(plan, found)
+    (alone,) = [g for g in found.groups[at] if (row, pos) in g.visits]
+    assert alone.visits == [(row, pos)] and alone.dst == slot
+    adding = [(j, k) for j, i in enumerate(plan.instructions) if j > at + 1 and isinstance(i, SumInstr) for k, op in enumerate(i.ops)
+              if slot in op.src_buffers]
+    assert adding
+    for j, k in adding:
+        assert k not in found.skip_ops.get(j, ()) and slot in found.sources.get(j, {}).get(k, plan.instructions[j].ops[k].src_buffers)
 
 
 def _without_keys_of_a_row(plan):
@@ -186,7 +249,7 @@ def test_a_local_block_named_twice_is_left_to_its_sums(monkeypatch, how):
     plan = make_case(**PLANS["causal_gqa"])["bw"]
     before = local_blocks(plan)
     block = next(iter(before.values()))
-    slot = BufferBlock(BufferType.BUFFER_dKV, 10 ** 6, block.n_tokens)
+    slot = BufferBlock(BufferType.BUFFER_KV, 10 ** 6, block.n_tokens)
     between = next(i for i, instr in enumerate(plan.instructions) if isinstance(instr, AttnBackwardInstr)) + 1
     plan.instructions.insert(between, SumInstr([SumOp([slot], block)], True) if how == "written" else MemcpyInstr([(block, slot)]))
     assert set(local_blocks(plan)) == set(before) - {block.index}
