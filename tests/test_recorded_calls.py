@@ -44,6 +44,86 @@ def test_a_nested_call_is_recorded_once_and_errors_come_back():
         rec.run(0, 1, 0)
 
 
+class _Stream:
+    """Which pieces of work are over when the next piece on the stream begins."""
+
+    def __init__(self, name, handle=1):
+        self.name, self.cuda_stream, self.over, self.gone = name, handle, set(), False
+
+    def work(self, what):
+        self.over.add(what)
+
+    def wait_stream(self, other):
+        assert not other.gone, f"waits on {other.name}, which has been destroyed"
+        self.over |= other.over
+
+    def wait_event(self, event):
+        self.over |= event.over
+
+
+class _Event:
+    def record(self, stream):
+        self.over = set(stream.over)
+
+
+def _executor_on_streams(monkeypatch):
+    """An executor whose passes and copies are marks on streams like these (no GPU); ``use(stream)``
+    makes a stream the caller's."""
+    from dcp_amd.core.instructions import BufferType
+    from dcp_amd.runtime.flash_attention import executor as module
+
+    current = [None]
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: current[0])
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "Event", _Event)
+    ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
+    ex.main_stream = _Stream("main")
+    ex.main_stream.device_index = 0
+    ex._last_stream = ex._last_pass = ex.cuda_graph = None
+    ex.streams, ex._recorded_steps, ex._steps_of = {}, {}, (None, ())
+    ex.kernel_head_dim = ex.head_dim = 64
+
+    class Buffer:
+        def copy_(self, value):
+            current[0].work(value)
+
+    ex.buffers = {t: Buffer() for t in (BufferType.LOCAL_Q, BufferType.LOCAL_KV, BufferType.LOCAL_dOUT, BufferType.LOCAL_OUT,
+                                        BufferType.LOCAL_LSE, BufferType.LOCAL_dQ, BufferType.LOCAL_dKV)}
+    ex.init_buffers = lambda plan: None
+    monkeypatch.setattr(ex, "_replay", lambda plan, stream: stream.work(plan) or True)
+    return ex, lambda stream: current.__setitem__(0, stream)
+
+
+@pytest.mark.parametrize("handle", [0, 1])
+@pytest.mark.parametrize("then", ["execute", "begin", "inputs", "dout", "out_lse"])
+def test_what_follows_a_pass_on_another_stream_waits_for_it(monkeypatch, then, handle):
+    """Passes share buffers, so whatever runs kernels on them or writes them waits for the last pass, also if
+    that pass was on a stream that is gone by then."""
+    ex, use = _executor_on_streams(monkeypatch)
+    first, second = _Stream("first", handle), _Stream("second", 2)
+    use(first)
+    ex.execute("a pass", True)
+    first.gone = handle != 0
+    use(second)
+    {"execute": lambda: ex.execute("another", True), "begin": lambda: ex.begin("another"), "inputs": lambda: ex.init_forward_input("q", "kv"),
+     "dout": lambda: ex.init_backward_input("dout"), "out_lse": lambda: ex.set_local_out_lse("out", "lse")}[then]()
+    assert "a pass" in (ex.main_stream if then == "begin" else second).over
+
+
+def test_a_pass_in_steps_is_a_pass(monkeypatch):
+    ex, use = _executor_on_streams(monkeypatch)
+    first, second = _Stream("first"), _Stream("second", 2)
+    use(first)
+    ex.begin("a plan")
+    ex.main_stream.work("a step")
+    ex.finish()
+    first.gone = True
+    use(second)
+    ex.execute("another", True)
+    assert "a step" in second.over
+
+
 def _executors(case):
     from dcp_amd.runtime.flash_attention.executor import get_executor
 
@@ -122,3 +202,49 @@ def test_a_handler_of_the_callers_own_is_not_recorded(gpu):
     a, b = ex.forward(q, kv), ex.forward(q, kv)
     assert len(seen) == 4 and ex._recorded is None  # two attention instructions, two passes
     assert torch.equal(a[0], b[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("inputs_first", [False, True])
+def test_inputs_of_a_pass_on_another_stream_wait_for_the_last_one(gpu, inputs_first):
+    """A pass is held up on one stream while another stream gives the executor new inputs and runs it."""
+    case, other = make_case(**CASE), make_case(**CASE, seed=3)
+    ex = _executors(case)
+    inputs = [(c["layout"].to_local_q(c["q"]).cuda(), c["layout"].to_local_kv(c["kv"]).cuda()) for c in (case, other)]
+    want = [ex.forward(*x) for x in inputs]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(streams[0]):
+        if inputs_first:
+            ex.init_forward_input(*inputs[0])
+        torch.cuda._sleep(20_000_000)
+        got = [ex.forward(*inputs[0])] if not inputs_first else [tuple(t.clone() for t in ex.execute(case["fw"], True))]
+    with torch.cuda.stream(streams[1]):
+        got.append(ex.forward(*inputs[1]))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for g, w in zip(got, want) for a, b in zip(g, w))
+
+
+@pytest.mark.gpu
+def test_a_pass_in_steps_waits_for_the_last_pass(gpu):
+    from dcp_amd.runtime.flash_attention.fabric import execute_together
+
+    case = make_case(**CASE)
+    ex = _executors(case)
+    want = ex.forward(case["layout"].to_local_q(case["q"]).cuda(), case["layout"].to_local_kv(case["kv"]).cuda())
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for turn in range(2):  # (the second time the steps are recorded)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            torch.cuda._sleep(20_000_000)
+            ex.execute(case["fw"], True)
+            marker = torch.cuda.Event()
+            marker.record()
+        with torch.cuda.stream(streams[1]):
+            execute_together([ex])
+            out = ex.buffers["LocalOut"].clone()
+            done = torch.cuda.Event()
+            done.record()
+        done.synchronize()
+        assert marker.query()
+        assert torch.equal(out, want[0])
