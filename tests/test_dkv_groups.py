@@ -214,6 +214,9 @@ def test_no_groups_where_a_handler_is_the_callers_own(monkeypatch, table, kind):
     assert _executor_without_a_device(monkeypatch, plan)._group_dkv_replicas().groups
     own = {kind: lambda e, i: None}
     assert _executor_without_a_device(monkeypatch, plan, **{table: own})._group_dkv_replicas() == dkv_groups.DkvGroups()
+    ex = _executor_without_a_device(monkeypatch, plan)
+    monkeypatch.setattr(ex, "_execute_instruction", lambda instr: None)  # (runs them in its own way)
+    assert ex._group_dkv_replicas() == dkv_groups.DkvGroups()
 
 
 def test_groups_can_be_turned_off(monkeypatch):

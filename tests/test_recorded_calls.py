@@ -111,6 +111,39 @@ def test_what_follows_a_pass_on_another_stream_waits_for_it(monkeypatch, then, h
     assert "a pass" in (ex.main_stream if then == "begin" else second).over
 
 
+def _set(name, value):
+    return lambda ex: setattr(ex, name, value)
+
+
+@pytest.mark.parametrize("change", [_set("synchronous", True), _set("logger", object()),
+                                    _set("_execute_instruction", lambda instr: None), _set("init_buffers", lambda plan: None)],
+                         ids=["synchronous", "logger", "own_instruction_loop", "own_buffers"])
+def test_switches_set_after_the_first_pass_are_seen(monkeypatch, change):
+    """The recorded calls stand for a pass that is nothing but its handlers."""
+    from types import SimpleNamespace
+
+    from dcp_amd.runtime.flash_attention import executor as module
+
+    ran = []
+    calls = SimpleNamespace(run=lambda *a: ran.append(a))
+    ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
+    ex.synchronous, ex.logger, ex.buffers = False, None, {}
+    ex.main_stream = SimpleNamespace(cuda_stream=7)
+    ex._recorded, ex._recorded_steps = ("plan", (), calls, 3), {0: (calls, 2)}
+    ex.execution_plan = SimpleNamespace(instructions=["an instruction"])
+    assert ex._replay("plan", ex.main_stream) and ran == [(0, 3, 7)]
+    ex.execution_plan = SimpleNamespace(instructions=["an instruction"])
+    ex.step(0)
+    assert ran == [(0, 3, 7), (0, 2, 7)]
+    change(ex)
+    assert not ex._replay("plan", ex.main_stream)
+    seen = []
+    monkeypatch.setattr(torch.cuda, "stream", lambda stream: __import__("contextlib").nullcontext())
+    monkeypatch.setattr(ex, "_execute_instruction", seen.append)
+    ex.step(0)
+    assert seen == ["an instruction"] and len(ran) == 2
+
+
 def test_a_pass_in_steps_is_a_pass(monkeypatch):
     ex, use = _executor_on_streams(monkeypatch)
     first, second = _Stream("first"), _Stream("second", 2)
@@ -248,3 +281,18 @@ def test_a_pass_in_steps_waits_for_the_last_pass(gpu):
         done.synchronize()
         assert marker.query()
         assert torch.equal(out, want[0])
+
+
+@pytest.mark.gpu
+def test_a_synchronous_executor_synchronises_after_the_first_pass_too(gpu):
+    case = make_case(**CASE)
+    ex = _executors(case)
+    q, kv = case["layout"].to_local_q(case["q"]).cuda(), case["layout"].to_local_kv(case["kv"]).cuda()
+    want = ex.forward(q, kv)
+    assert ex._recorded is not None
+    waits = []
+    ex.register_synchronization_handler(lambda: (waits.append(1), torch.cuda.synchronize()))
+    ex.synchronous = True
+    got = ex.forward(q, kv)
+    assert len(waits) == len(case["fw"].instructions)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
