@@ -85,7 +85,9 @@ constexpr int kPrioMatrix = 2, kPrioVector = 0;
 constexpr int kBwdBM = 64;
 constexpr int kBwdBN = 64;
 constexpr int kBwdThreads = 256;
-constexpr int kTicketStride = 32;  // a counter per cache line
+// Both kernels' counters in the 256 bytes that the base workspace has always had for them (a cache line
+// each makes no difference: 65536 causal tokens, 32 heads, 11.40 ms either way).
+constexpr int kTicketStride = 4;
 constexpr int kTicketInts = kNumXcd * kTicketStride;
 constexpr int kDkvGroupInts = 8;
 constexpr int kDkvMaxVisits = DCP_ATTN_BWD_MAX_VISITS;

@@ -81,6 +81,7 @@ struct AttnFwdParams {
   int64_t n_items;   // batch * n_heads_q * q_tiles_per_row
   float scale_log2;  // softmax_scale * log2(e)
   int* tickets;      // of the item queue, zeroed before the launch; null: one item per workgroup
+  int ticket_stride;
   // rows in parts (dcp_attn_fwd_parts): a record per launch entry, which takes the place of a row
   const FwdPart* parts;
   float* partial_out;   // [partial][head][32-query block][D / 4][query][4]: O^T relative to the part's maximum
@@ -92,8 +93,9 @@ struct AttnFwdParams {
 // (2-3 % on the kernel), and the fused phase, whose vector work is the longer chain, outranks
 // the dense one (another 1.5 %; the other way round it was 1.5 % slower).
 constexpr int kPrioControl = 0, kPrioFused = 2, kPrioDense = 1;
-constexpr int kFwdTicketStride = 8;  // (the workspace is small: two cache lines of counters)
-constexpr int kFwdTicketInts = kNumXcd * kFwdTicketStride;
+// Ints from one counter of the item queue to the next, and in a workspace of the 64 bytes that used to be
+// all there was (65536 causal tokens, 32 heads: 3.75 and 3.77 ms).
+constexpr int kFwdTicketStride = 8, kFwdTicketStrideMin = DCP_ATTN_FWD_MIN_WORKSPACE_BYTES / (kNumXcd * 4);
 constexpr int kFwdBN = 64;
 constexpr int kFwdThreads = 256;
 // The running maximum of a row is only raised (and O^T rescaled) when the tile's maximum
@@ -633,19 +635,19 @@ __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(
   int item = 0;
   {
     KernArgs<AttnFwdParams>& args = fresh_kernel_args<AttnFwdParams>();
-    item = first_item({args.tickets, kFwdTicketStride, args.n_items, args.xcd_group});
+    item = first_item({args.tickets, args.ticket_stride, args.n_items, args.xcd_group});
   }
   while (true) {
     KernArgs<AttnFwdParams>& args = fresh_kernel_args<AttnFwdParams>();
-    if (item < 0) item = next_item({args.tickets, kFwdTicketStride, args.n_items, args.xcd_group}, &ticket_lds);
+    if (item < 0) item = next_item({args.tickets, args.ticket_stride, args.n_items, args.xcd_group}, &ticket_lds);
     if (item < 0) break;
     attn_fwd_item<DTYPE, D, QB, PARTS>(args, item);
     item = -1;
   }
 }
 
-__global__ void attn_fwd_reset_tickets_kernel(int* tickets) {
-  if (threadIdx.x < kFwdTicketInts) tickets[threadIdx.x] = 0;
+__global__ void attn_fwd_reset_tickets_kernel(int* tickets, int stride) {
+  if (threadIdx.x < kNumXcd) tickets[threadIdx.x * stride] = 0;
 }
 
 // Adds up the parts of the split rows: out = sum_i 2^(m_i - m) O_i / sum_i 2^(m_i - m) l_i, rounded once.
@@ -706,7 +708,7 @@ __global__ __launch_bounds__(kMergePartsThreads) void attn_fwd_merge_parts_kerne
 
 using namespace dcp;
 
-extern "C" size_t dcp_attn_fwd_workspace_bytes(void) { return kFwdTicketInts * sizeof(int32_t); }
+extern "C" size_t dcp_attn_fwd_workspace_bytes(void) { return kNumXcd * kFwdTicketStride * sizeof(int32_t); }
 
 extern "C" int dcp_attn_fwd(const void* q, const void* k, const void* v, void* out, float* lse,
                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
@@ -771,9 +773,9 @@ static int attn_fwd(const void* q, const void* k, const void* v, void* out, floa
                 reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(out)) & 15) == 0,
               "attn_fwd: q/k/v/out must be 16-byte aligned");
   DCP_REQUIRE(workspace && (reinterpret_cast<uintptr_t>(workspace) & 3) == 0 &&
-                  workspace_bytes >= dcp_attn_fwd_workspace_bytes(),
-              "attn_fwd: workspace of %zu bytes is missing or smaller than the %zu needed", workspace_bytes,
-              dcp_attn_fwd_workspace_bytes());
+                  workspace_bytes >= DCP_ATTN_FWD_MIN_WORKSPACE_BYTES,
+              "attn_fwd: workspace of %zu bytes is missing or smaller than the %d needed", workspace_bytes,
+              DCP_ATTN_FWD_MIN_WORKSPACE_BYTES);
   if (in_parts.parts != nullptr) {
     DCP_REQUIRE(in_parts.n_entries >= batch && in_parts.n_splits >= 0 && in_parts.n_splits <= batch && in_parts.n_partials >= 2 * in_parts.n_splits,
                 "attn_fwd: %d entries and %d partials of %d split rows do not fit %d rows", in_parts.n_entries, in_parts.n_partials,
@@ -826,8 +828,9 @@ static int attn_fwd(const void* q, const void* k, const void* v, void* out, floa
   // as many workgroups as the device holds at once (two per CU), a multiple of the XCD count
   const int64_t n_wg = std::min<int64_t>(xcd_grid_size(p.n_items, 1), xcd_grid_size(2 * (int64_t)device_cu_count(), 1));
   p.tickets = p.n_items > n_wg ? reinterpret_cast<int*>(workspace) : nullptr;
+  p.ticket_stride = workspace_bytes >= dcp_attn_fwd_workspace_bytes() ? kFwdTicketStride : kFwdTicketStrideMin;
   dim3 grid((unsigned)n_wg), block(kFwdThreads);
-  if (p.tickets) hipLaunchKernelGGL(attn_fwd_reset_tickets_kernel, dim3(1), dim3(kFwdTicketInts), 0, (hipStream_t)stream, p.tickets);
+  if (p.tickets) hipLaunchKernelGGL(attn_fwd_reset_tickets_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, p.tickets, p.ticket_stride);
   auto launch = [&](auto kernel) {
     KernelTimer timer("attn_fwd_kernel", stream);
     hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, p);

@@ -217,14 +217,17 @@ int dcp_blockwise_sum_fp32_sources(
  * masked there.  It must be finite, and small enough that its dot products with
  * q stay finite; the reference's kernels zero-fill such loads instead.  Query
  * rows past seqlen_q are not read.
- * `workspace`: caller-provided device scratch of at least
+ * `workspace`: caller-provided device scratch of
  * dcp_attn_fwd_workspace_bytes() bytes, 4-byte aligned, for the kernel's work
  * counters (the launch is persistent: its workgroups take (row, head, query
- * tile) items from per-XCD counters).  Its contents are overwritten (a small
+ * tile) items from per-XCD counters).  DCP_ATTN_FWD_MIN_WORKSPACE_BYTES are
+ * enough; the counters then share a cache line, half a percent of a long
+ * launch.  Its contents are overwritten (a small
  * kernel zeroes it on `stream` before the attention kernel); one workspace
  * serves any number of launches that follow each other on a stream or in a
  * captured graph, launches that may run at the same time need one each.
  */
+#define DCP_ATTN_FWD_MIN_WORKSPACE_BYTES 64
 size_t dcp_attn_fwd_workspace_bytes(void);
 int dcp_attn_fwd(const void* q, const void* k, const void* v, void* out,
                  float* lse, const int32_t* cu_seqlens_q,

@@ -63,6 +63,20 @@ def test_argument_errors_are_reported_without_a_launch(lib):
     assert lib.dcp_attn_bwd_workspace_bytes(2, 128, 64, 4, 128) >= 128 * 4 * 4 + 2 * 8 * 4
 
 
+def test_workspaces_have_the_sizes_callers_know(lib):
+    """A caller may have its buffers before it asks, for the backward two floats per (query, head), a hull of
+    32 bytes per 64-query tile, each rounded up to 256 bytes, and 256 bytes of counters.  A problem
+    that just fills the static entry point's scratch stays one."""
+    up = lambda n: -(-n // 256) * 256
+    for batch, bs, heads in ((1, 64, 1), (3, 128, 5), (508, 1024, 8)):
+        total_q = batch * bs
+        want = 2 * up(total_q * heads * 4) + up(batch * -(-bs // 64) * 32) + 256
+        assert lib.dcp_attn_bwd_workspace_bytes(batch, total_q, bs, heads, 64) == want
+    # 8 heads, 64-token rows: (64 * 64 + 32) bytes a row and the counters
+    rows = ((32 << 20) - 256) // (64 * 8 * 8 + 32) // 8 * 8
+    assert (32 << 20) - 8 * (64 * 8 * 8 + 32) < lib.dcp_attn_bwd_workspace_bytes(rows, rows * 64, 64, 8, 64) <= 32 << 20
+
+
 def test_backward_selection_and_its_workspace_size(lib):
     """dcp_attn_bwd_select returns the previous setting and only sets a known mode; the workspace the
     selected backward needs: the recomputing one the small scratch whatever the key count, the one

@@ -256,6 +256,24 @@ QUEUE_CASES = {
 }
 
 
+@pytest.mark.parametrize("name", list(QUEUE_CASES))
+def test_forward_with_the_smallest_workspace(gpu, monkeypatch, name):
+    """64 bytes of work counters, which is what the entry point needed at first, with and without a queue; what
+    lies behind them stays as it was."""
+    from dcp_amd.runtime.flash_attention import executor as module
+
+    case = make_case(**QUEUE_CASES[name], qkv_scale=0.5)
+    want, _ = run_executor(case, backward=False)
+    memory = torch.full((64,), 77, dtype=torch.int32, device=gpu)
+    monkeypatch.setattr(module, "forward_workspace", lambda: memory[:16])
+    got, _ = run_executor(case, backward=False)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert (memory[16:] == 77).all()
+    monkeypatch.setattr(module, "forward_workspace", lambda: memory[:15])
+    with pytest.raises(AssertionError, match="60 bytes"):
+        run_executor(case, backward=False)
+
+
 @pytest.mark.parametrize("mode", [0, 2])
 @pytest.mark.parametrize("name", list(QUEUE_CASES))
 def test_every_item_of_a_launch_is_taken_once(gpu, name, mode):
