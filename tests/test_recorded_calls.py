@@ -128,7 +128,8 @@ def test_switches_set_after_the_first_pass_are_seen(monkeypatch, change):
     calls = SimpleNamespace(run=lambda *a: ran.append(a))
     ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
     ex.synchronous, ex.logger, ex.buffers = False, None, {}
-    ex.main_stream = SimpleNamespace(cuda_stream=7)
+    ex.main_stream = SimpleNamespace(cuda_stream=7, device_index=0)
+    monkeypatch.setattr(torch.cuda, "device", lambda device: __import__("contextlib").nullcontext())
     ex._recorded, ex._recorded_steps = ("plan", (), calls, 3), {0: (calls, 2)}
     ex.execution_plan = SimpleNamespace(instructions=["an instruction"])
     assert ex._replay("plan", ex.main_stream) and ran == [(0, 3, 7)]
@@ -142,6 +143,30 @@ def test_switches_set_after_the_first_pass_are_seen(monkeypatch, change):
     monkeypatch.setattr(ex, "_execute_instruction", seen.append)
     ex.step(0)
     assert seen == ["an instruction"] and len(ran) == 2
+
+
+def test_a_recorded_step_runs_on_the_executors_device(monkeypatch):
+    """Whatever device is the caller's current one."""
+    from contextlib import contextmanager
+    from types import SimpleNamespace
+
+    from dcp_amd.runtime.flash_attention import executor as module
+
+    current, ran_on = [1], []
+
+    @contextmanager
+    def device(index):
+        before, current[0] = current[0], index
+        yield
+        current[0] = before
+
+    monkeypatch.setattr(torch.cuda, "device", device)
+    ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
+    ex.synchronous, ex.logger = False, None
+    ex.main_stream = SimpleNamespace(cuda_stream=7, device_index=0)
+    ex._recorded_steps = {0: (SimpleNamespace(run=lambda *a: ran_on.append(current[0])), 1)}
+    ex.step(0)
+    assert ran_on == [0] and current == [1]
 
 
 def test_a_pass_in_steps_is_a_pass(monkeypatch):
