@@ -44,6 +44,26 @@ def test_a_nested_call_is_recorded_once_and_errors_come_back():
         rec.run(0, 1, 0)
 
 
+def test_a_recording_keeps_what_its_calls_point_to():
+    import weakref
+
+    from dcp_amd.runtime.flash_attention import executor as module
+
+    ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
+    memory = [torch.zeros(4) for _ in range(4)]
+    ex._args_cache = {0: (memory[0],)}
+    ex._dkv_partials, ex._bwd_workspace, ex._fwd_partials = memory[1:]
+    alive = [weakref.ref(t) for t in memory]
+    recording = ex._recording()
+    recording.end()
+    ex._args_cache = {}
+    ex._dkv_partials = ex._bwd_workspace = ex._fwd_partials = None
+    memory.clear()
+    assert all(r() is not None for r in alive)
+    del recording
+    assert all(r() is None for r in alive)
+
+
 class _Stream:
     """Which pieces of work are over when the next piece on the stream begins."""
 
