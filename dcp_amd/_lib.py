@@ -101,12 +101,13 @@ class Recording:
         self.keep = keep
 
     def begin(self) -> bool:
-        """False if this thread is recording already (nothing is recorded then)."""
+        """False if this thread is recording already, or without host memory (nothing is recorded then)."""
         self._list = load().dcp_record_begin()
         return self._list is not None
 
-    def end(self) -> None:
-        load().dcp_record_end()
+    def end(self) -> bool:
+        """Is every call in the list (host memory may have run out)?"""
+        return load().dcp_record_end() == 0
 
     def size(self) -> int:
         return load().dcp_record_size(self._list)

@@ -1,6 +1,7 @@
 // Recorded launches (record.h): the list and its entry points.
 #include "record.h"
 
+#include <new>
 #include <vector>
 
 #include "common.h"
@@ -9,6 +10,7 @@ namespace dcp {
 
 struct RecordedCalls {
   std::vector<std::function<int(void*)>> calls;
+  bool whole = true;
 };
 
 namespace {
@@ -18,6 +20,7 @@ thread_local bool t_suspended = false;
 
 RecordedCalls* current_recording() { return t_suspended ? nullptr : t_recording; }
 void record_call(RecordedCalls* list, std::function<int(void*)> call) { list->calls.push_back(std::move(call)); }
+void recording_failed(RecordedCalls* list) { list->whole = false; }
 void suspend_recording(bool suspended) { t_suspended = suspended; }
 
 }  // namespace dcp
@@ -26,13 +29,15 @@ using dcp::RecordedCalls;
 
 extern "C" void* dcp_record_begin(void) {
   if (dcp::t_recording != nullptr) return nullptr;
-  dcp::t_recording = new RecordedCalls;
+  dcp::t_recording = new (std::nothrow) RecordedCalls;
   return dcp::t_recording;
 }
 
 extern "C" int dcp_record_end(void) {
   DCP_REQUIRE(dcp::t_recording != nullptr, "record_end: this thread is not recording");
+  const bool whole = dcp::t_recording->whole;
   dcp::t_recording = nullptr;
+  DCP_REQUIRE(whole, "record_end: a call could not be recorded, out of host memory");
   return DCP_OK;
 }
 
@@ -40,6 +45,7 @@ extern "C" int dcp_record_size(const void* list) { return list ? (int)static_cas
 
 extern "C" int dcp_record_run(const void* list, int begin, int end, void* stream) {
   DCP_REQUIRE(list != nullptr, "record_run: null list");
+  DCP_REQUIRE(static_cast<const RecordedCalls*>(list)->whole, "record_run: a call is missing from the list");
   const auto& calls = static_cast<const RecordedCalls*>(list)->calls;
   DCP_REQUIRE(begin >= 0 && begin <= end && end <= (int)calls.size(), "record_run: calls %d to %d of %zu", begin, end, calls.size());
   for (int i = begin; i < end; ++i)

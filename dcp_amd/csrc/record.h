@@ -11,15 +11,20 @@ namespace dcp {
 struct RecordedCalls;
 RecordedCalls* current_recording();  // of this thread; null while it does not record or is inside a recorded call
 void record_call(RecordedCalls* list, std::function<int(void*)> call);
+void recording_failed(RecordedCalls* list);  // a call could not be added
 void suspend_recording(bool suspended);
 
 // One per entry point, at its top.  Entry points that call each other record the outermost call.
 class RecordScope {
  public:
   template <typename F>
-  explicit RecordScope(F&& call) : list_(current_recording()) {
+  explicit RecordScope(F&& call) noexcept : list_(current_recording()) {
     if (list_ == nullptr) return;
-    record_call(list_, std::forward<F>(call));
+    try {
+      record_call(list_, std::forward<F>(call));
+    } catch (...) {  // no host memory: nothing is thrown at a C caller, the list is no good
+      recording_failed(list_);
+    }
     suspend_recording(true);
   }
   ~RecordScope() {

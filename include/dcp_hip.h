@@ -59,7 +59,8 @@ int dcp_profile_report(char* buffer, size_t capacity);
  * Between dcp_record_begin and dcp_record_end every call of an entry point
  * below that takes a stream, made on this thread, is launched as usual and also
  * added with its arguments to the list dcp_record_begin returned (NULL if the
- * thread is recording already).  dcp_record_run makes calls [begin, end) of a
+ * thread is recording already, or host memory has run out; where it runs out
+ * later, dcp_record_end says so and the list cannot be run).  dcp_record_run makes calls [begin, end) of a
  * list again, in order, on `stream`, and returns the first nonzero status.  The
  * arguments are kept as they were given: the caller keeps the memory they point
  * to alive and in place for as long as it runs the list.  A list may be run

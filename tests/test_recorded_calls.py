@@ -44,6 +44,20 @@ def test_a_nested_call_is_recorded_once_and_errors_come_back():
         rec.run(0, 1, 0)
 
 
+def test_recording_without_host_memory_throws_nothing_at_a_c_caller(tmp_path):
+    import subprocess
+    from pathlib import Path
+
+    from dcp_amd import _lib
+
+    root, program = Path(__file__).parent, tmp_path / "record_no_memory"
+    lib = Path(_lib.LIB_PATH).parent
+    subprocess.run(["g++", "-O1", "-std=c++17", f"-I{root.parent / 'include'}", str(root / "abi_host" / "record_no_memory.cpp"), "-o",
+                    str(program), f"-L{lib}", "-ldcp_hip", f"-Wl,-rpath,{lib}:/opt/rocm/lib", "-Wl,--allow-shlib-undefined"], check=True)
+    ran = subprocess.run([str(program)], capture_output=True, text=True, timeout=60)
+    assert ran.returncode == 0 and ran.stdout.strip() == "ok", ran.stdout + ran.stderr
+
+
 def test_a_recording_keeps_what_its_calls_point_to():
     import weakref
 
