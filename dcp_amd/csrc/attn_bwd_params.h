@@ -68,7 +68,7 @@ struct AttnBwdParams {
   int64_t dkv2_token_stride;
   int dkv_xcd_group;     // dK/dV work items sharing one Q/dO stream (the key tiles of a row)
   int dq_xcd_group;      // dQ work items sharing one K/V stream
-  int64_t n_dkv_items;   // batch * n_heads_kv * kv_tiles_per_row
+  int64_t n_dkv_items;   // (rows, or groups of rows) * n_heads_kv * kv_tiles_per_row
   int64_t n_dq_items;    // batch * n_heads_q * dq_tiles_per_row
   int q_tiles_per_row;   // ceil(block_size / 64): query tiles of the dK/dV kernel
   int dq_tiles_per_row;  // ceil(block_size / 128): query tiles of the dQ kernel

@@ -330,7 +330,9 @@ inline int64_t xcd_grid_size(int64_t total, int group) {
 //
 // A workgroup's first item is fixed by its number: with every workgroup of the launch drawing its first
 // ticket from counters in one cache line, the line went around the XCDs' caches for each of them,
-// 45 us for 768 workgroups.
+// 45 us for 768 workgroups.  That counts on the launch having the device to itself, as a plan's launches
+// have: next to another stream's kernel a workgroup may get its slot only when the others have drained the
+// counters, and then starts one of the longest items last.  (Results do not depend on it.)
 struct ItemQueue {
   int* tickets;     // kNumXcd counters, zero before the launch; null: one item per workgroup
   int stride;       // ints from one counter to the next

@@ -71,14 +71,16 @@ def visits_per_group(n_visits: int, tiles_per_visit: int, n_slots: int) -> int:
     """How many rows a workgroup may visit.  Longer groups save prologues, K/V loads and replicas;
     but a launch is as long as its longest workgroup, and too few of them leave the device idle.  Up
     to eight (row, kv block) pairs per workgroup slot of the device, groups of as many, so that (nearly) all
-    of them run at once; past that half as many, so that the slots, which take the longest groups first,
-    end within a fraction of a group of each other.  Measured, backward (us) with 1 / 2 / 3 / 4 / 6 / 8 rows
-    per group: 1.2 pairs per slot (4096 tokens, 32 heads) 266 / 249 / 303 / 358 / 357 / 358; 1.9 (4096
-    tokens, 8 heads of size 64) 95 / 80 / 80 / 84 / 95 / 101; 2.6 (20000 tokens, 8 heads) 547 / 514 / 509 /
-    532 / 616 / 716; 3.1 (8192 tokens, 32 heads) 902 / 848 / 840 / 880 / 975 / 980; 3.5 (16384 tokens, 16
-    heads) 627 / 576 / 565 / 558 / 639 / 724; 7.1 (8192 tokens, 8 one-head blocks) 332 / 252 / 237 / 235 / 237 /
-    232; 7.8 (16384 tokens, 32 heads) 2260 / 2193 / 2190 / 2161 / 2142 / 2146.  At 25 pairs per slot (32768 tokens, 8 one-head blocks), dK/dV kernel plus replica sums
-    904 in groups of 25 rows and 873 of 13; at 32 (65536 tokens, 32 heads) 8226 and 8330."""
+    of them run at once: rounded up to three, to the nearest past that (at 3.1 pairs three rows beat four by
+    5 %; between the points measured the choice is within a few percent either way).  Past eight half
+    as many, so that the slots, which take the longest groups first, end within a fraction of a group of
+    each other.  Measured, backward (us) with 1 / 2 / 3 / 4 / 6 / 8 rows per group: 1.2 pairs per slot (4096
+    tokens, 32 heads) 266 / 249 / 303 / 358 / 357 / 358; 1.9 (4096 tokens, 8 heads of size 64) 95 / 80 / 80 /
+    84 / 95 / 101; 2.6 (20000 tokens, 8 heads) 547 / 514 / 509 / 532 / 616 / 716; 3.1 (8192 tokens, 32 heads)
+    902 / 848 / 840 / 880 / 975 / 980; 3.5 (16384 tokens, 16 heads) 627 / 576 / 565 / 558 / 639 / 724; 7.1
+    (8192 tokens, 8 one-head blocks) 332 / 252 / 237 / 235 / 237 / 232; 7.8 (16384 tokens, 32 heads) 2260 / 2193 /
+    2190 / 2161 / 2142 / 2146.  At 25 pairs per slot (32768 tokens, 8 one-head blocks), dK/dV kernel plus
+    replica sums 904 in groups of 25 rows and 873 of 13; at 32 (65536 tokens, 32 heads) 8226 and 8330."""
     pairs = n_visits * tiles_per_visit / n_slots
     if pairs <= 8:
         return max(1, math.ceil(pairs) if pairs <= 3 else round(pairs))

@@ -306,7 +306,7 @@ def test_parts_cover_every_head_and_tile_once(monkeypatch, name, parts):
 
 
 def test_group_size_rule():
-    """One row per group where the launch does not fill the device several times over, never more
+    """One row per group where the launch does not fill the device once, more the more often it does, never more
     than the kernel takes."""
     assert dkv_groups.visits_per_group(60, 8, 512) == 1
     assert dkv_groups.visits_per_group(10 ** 6, 8, 512) == dkv_groups.MAX_VISITS
