@@ -100,9 +100,10 @@ class _Event:
         self.over = set(stream.over)
 
 
-def _executor_on_streams(monkeypatch):
-    """An executor whose passes and copies are marks on streams like these (no GPU); ``use(stream)``
-    makes a stream the caller's."""
+def _executor_on_streams(monkeypatch, replay=False):
+    """An executor whose passes (unless ``replay``) and copies are marks on streams like these, without a GPU;
+    ``use(stream)`` makes a stream the caller's."""
+    from dcp_amd.core.executor import HandlerTable
     from dcp_amd.core.instructions import BufferType
     from dcp_amd.runtime.flash_attention import executor as module
 
@@ -115,6 +116,7 @@ def _executor_on_streams(monkeypatch):
     ex.main_stream = _Stream("main")
     ex.main_stream.device_index = 0
     ex._last_stream = ex._last_pass = ex.cuda_graph = None
+    ex._handlers = HandlerTable("Instruction handler")
     ex.streams, ex._recorded_steps, ex._steps_of = {}, {}, (None, ())
     ex.kernel_head_dim = ex.head_dim = 64
 
@@ -124,8 +126,9 @@ def _executor_on_streams(monkeypatch):
 
     ex.buffers = {t: Buffer() for t in (BufferType.LOCAL_Q, BufferType.LOCAL_KV, BufferType.LOCAL_dOUT, BufferType.LOCAL_OUT,
                                         BufferType.LOCAL_LSE, BufferType.LOCAL_dQ, BufferType.LOCAL_dKV)}
-    ex.init_buffers = lambda plan: None
-    monkeypatch.setattr(ex, "_replay", lambda plan, stream: stream.work(plan) or True)
+    monkeypatch.setattr(module.AttentionExecutor, "init_buffers", lambda self, plan: None)
+    if not replay:
+        monkeypatch.setattr(ex, "_replay", lambda plan, stream: stream.work(plan) or True)
     return ex, lambda stream: current.__setitem__(0, stream)
 
 
@@ -154,26 +157,26 @@ def _set(name, value):
                          ids=["synchronous", "logger", "own_instruction_loop", "own_buffers"])
 def test_switches_set_after_the_first_pass_are_seen(monkeypatch, change):
     """The recorded calls stand for a pass that is nothing but its handlers."""
+    from contextlib import nullcontext
     from types import SimpleNamespace
 
-    from dcp_amd.runtime.flash_attention import executor as module
-
+    ex, use = _executor_on_streams(monkeypatch, replay=True)
+    use(_Stream("callers", 0))
     ran = []
     calls = SimpleNamespace(run=lambda *a: ran.append(a))
-    ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
     ex.synchronous, ex.logger, ex.buffers = False, None, {}
-    ex.main_stream = SimpleNamespace(cuda_stream=7, device_index=0)
-    monkeypatch.setattr(torch.cuda, "device", lambda device: __import__("contextlib").nullcontext())
-    ex._recorded, ex._recorded_steps = ("plan", (), calls, 3), {0: (calls, 2)}
-    ex.execution_plan = SimpleNamespace(instructions=["an instruction"])
-    assert ex._replay("plan", ex.main_stream) and ran == [(0, 3, 7)]
-    ex.execution_plan = SimpleNamespace(instructions=["an instruction"])
+    plan = SimpleNamespace(instructions=["an instruction"])
+    ex._recorded, ex._recorded_steps, ex._steps_of = (plan, (), calls, 3), {0: (calls, 2)}, (plan, ())
+    handle = ex.main_stream.cuda_stream
+    assert ex._replay(plan, ex.main_stream) and ran == [(0, 3, handle)]
+    ex.begin(plan)
     ex.step(0)
-    assert ran == [(0, 3, 7), (0, 2, 7)]
+    assert ran == [(0, 3, handle), (0, 2, handle)]
     change(ex)
-    assert not ex._replay("plan", ex.main_stream)
+    assert not ex._replay(plan, ex.main_stream)
     seen = []
-    monkeypatch.setattr(torch.cuda, "stream", lambda stream: __import__("contextlib").nullcontext())
+    ex.begin(plan)
+    monkeypatch.setattr(torch.cuda, "stream", lambda stream: nullcontext())
     monkeypatch.setattr(ex, "_execute_instruction", seen.append)
     ex.step(0)
     assert seen == ["an instruction"] and len(ran) == 2
@@ -184,8 +187,6 @@ def test_a_recorded_step_runs_on_the_executors_device(monkeypatch):
     from contextlib import contextmanager
     from types import SimpleNamespace
 
-    from dcp_amd.runtime.flash_attention import executor as module
-
     current, ran_on = [1], []
 
     @contextmanager
@@ -194,11 +195,13 @@ def test_a_recorded_step_runs_on_the_executors_device(monkeypatch):
         yield
         current[0] = before
 
+    ex, use = _executor_on_streams(monkeypatch)
     monkeypatch.setattr(torch.cuda, "device", device)
-    ex = module.AttentionExecutor.__new__(module.AttentionExecutor)
-    ex.synchronous, ex.logger = False, None
-    ex.main_stream = SimpleNamespace(cuda_stream=7, device_index=0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    use(_Stream("callers", 0))
+    ex.synchronous, ex.logger, ex.buffers, ex._steps_of = False, None, {}, ("plan", ())
     ex._recorded_steps = {0: (SimpleNamespace(run=lambda *a: ran_on.append(current[0])), 1)}
+    ex.begin("plan")
     ex.step(0)
     assert ran_on == [0] and current == [1]
 
