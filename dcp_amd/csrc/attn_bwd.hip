@@ -108,7 +108,8 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 // 32768 causal tokens of 8 heads and the sums of the replicas 150; with groups of up to 12 rows 850
 // and 23; at 64 steps a visit (four-head blocks of 1024 tokens, 65536 tokens, 32 heads) the kernel
 // takes the same time either way (8.3 ms: two workgroups per CU hide each other's prologues) and
-// the sums' 0.24 ms are saved.
+// the sums' 0.24 ms are saved.  The key tiles of a row then no longer run at the same time on one XCD,
+// and Q and dO come through L2 about four times as often (14.5 GB a launch instead of 3.6).
 // What the kernel needs to know of one row (a "visit" of it) while it holds a kv block's keys.
 struct DkvVisit {
   int q_begin, seqlen_q, seqlen_kv, q_entry, out_entry;
