@@ -46,6 +46,14 @@ struct FwdPart {
   int row, part, n_parts, first_partial;
 };
 
+// A work item's queries (dcp_attn_fwd_items): 128 of a row, or a part of them as in FwdPart.  The other entry points
+// have as many items for a row as its block has tiles, whether the row has queries for them or not, and a
+// workgroup that draws one without spends 1.5-2 us on it (4476 tokens in sequences of 290 tokens and blocks of
+// 1024, 8 heads of size 64: 528 of 832 items are like that, the launch takes 31.7 us with and 17.5 without them).
+struct FwdTile {
+  int row, q_tile, part_of, first_partial;  // part_of: part + 65536 * number of parts
+};
+
 struct AttnFwdParams {
   const void* q;
   const void* k;
@@ -84,6 +92,7 @@ struct AttnFwdParams {
   int ticket_stride;
   // rows in parts (dcp_attn_fwd_parts): a record per launch entry, which takes the place of a row
   const FwdPart* parts;
+  const FwdTile* tiles;  // the launch's items, one for all heads; null: all tiles of all rows
   float* partial_out;   // [partial][head][32-query block][D / 4][query][4]: O^T relative to the part's maximum
   float* partial_sums;  // [partial][head][32-query block][query][2]: the maximum (log2 domain) and the sum of the weights
 };
@@ -114,11 +123,13 @@ constexpr float kMaxTileSum = 16384.0f;
 // K / V^T operand read from LDS feeds two matrix instructions and every tile brought into LDS
 // serves twice the arithmetic; the wave then needs the whole register file (one workgroup
 // per CU, accumulators in the AGPR half).
-// PARTS: the launch's rows are split along their keys.  A work item is a serial chain, a tile after the
+// ITEMS: what the launch is over.  kFwdParts: its rows are split along their keys.  A work item is a serial chain, a tile after the
 // other (1.2-1.5 us each with a workgroup alone on its CU), and a launch of few, uneven rows lasts as long as its longest:
-// see dcp_attn_fwd_parts.
-template <int DTYPE, int D, int QB, bool PARTS>
+// see dcp_attn_fwd_parts.  kFwdTiles: its items are listed (FwdTile), as parts or whole.
+enum FwdItems { kFwdRows, kFwdParts, kFwdTiles };
+template <int DTYPE, int D, int QB, FwdItems ITEMS>
 __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int item) {
+  constexpr bool PARTS = ITEMS != kFwdRows;
   constexpr int BN = kFwdBN;
   constexpr int BM = 128 * QB;
   constexpr int KS = D / 16;  // k-steps of S^T = K Q^T
@@ -145,12 +156,21 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
   // Integer division runs on the vector unit, so its (uniform) results sit in vector registers
   // and drag every address derived from them there too: each tile load then costs three vector
   // instructions to rebuild a scalar base.  readfirstlane puts the indices back on the scalar unit.
-  int wg = item;
-  const int qt = __builtin_amdgcn_readfirstlane(wg % p.q_tiles_per_row);
-  wg /= p.q_tiles_per_row;
+  int wg = item, qt;
+  if constexpr (ITEMS != kFwdTiles) {
+    qt = __builtin_amdgcn_readfirstlane(wg % p.q_tiles_per_row);
+    wg /= p.q_tiles_per_row;
+  }
   const int head = __builtin_amdgcn_readfirstlane(wg % p.n_heads_q);
   const int bi = __builtin_amdgcn_readfirstlane(wg / p.n_heads_q);
-  const FwdPart part = PARTS ? p.parts[bi] : FwdPart{0, 0, 1, 0};
+  FwdPart part = {0, 0, 1, 0};
+  if constexpr (ITEMS == kFwdTiles) {
+    const FwdTile t = p.tiles[bi];
+    part = {t.row, t.part_of & 0xffff, t.part_of >> 16, t.first_partial};
+    qt = __builtin_amdgcn_readfirstlane(t.q_tile);
+  } else if constexpr (ITEMS == kFwdParts) {
+    part = p.parts[bi];
+  }
   const int b = __builtin_amdgcn_readfirstlane(PARTS ? part.row : p.row_order ? p.row_order[bi] : bi);
   const int q_begin = p.cu_seqlens_q[b];
   const int seqlen_q = p.cu_seqlens_q[b + 1] - q_begin;
@@ -629,7 +649,7 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
 // of work), and the last, unevenly long items leave slots empty at the end.  Rows come longest first;
 // the counters are zeroed by a one-wave kernel on the stream just before.  A launch whose items all
 // fit on the device at once needs no queue and no such kernel.
-template <int DTYPE, int D, int QB, bool PARTS>
+template <int DTYPE, int D, int QB, FwdItems ITEMS>
 __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(const AttnFwdParams p) {
   __shared__ int ticket_lds;
   int item = 0;
@@ -641,7 +661,7 @@ __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(
     KernArgs<AttnFwdParams>& args = fresh_kernel_args<AttnFwdParams>();
     if (item < 0) item = next_item({args.tickets, args.ticket_stride, args.n_items, args.xcd_group}, &ticket_lds);
     if (item < 0) break;
-    attn_fwd_item<DTYPE, D, QB, PARTS>(args, item);
+    attn_fwd_item<DTYPE, D, QB, ITEMS>(args, item);
     item = -1;
   }
 }
@@ -740,6 +760,7 @@ struct FwdParts {
   int n_splits = 0, n_partials = 0;
   float* partials = nullptr;
   size_t partials_bytes = 0;
+  const int32_t* tiles = nullptr;  // dcp_attn_fwd_items: n_entries of them instead of parts
 };
 
 static int attn_fwd(const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu_seqlens_q,
@@ -776,8 +797,10 @@ static int attn_fwd(const void* q, const void* k, const void* v, void* out, floa
                   workspace_bytes >= DCP_ATTN_FWD_MIN_WORKSPACE_BYTES,
               "attn_fwd: workspace of %zu bytes is missing or smaller than the %d needed", workspace_bytes,
               DCP_ATTN_FWD_MIN_WORKSPACE_BYTES);
-  if (in_parts.parts != nullptr) {
-    DCP_REQUIRE(in_parts.n_entries >= batch && in_parts.n_splits >= 0 && in_parts.n_splits <= batch && in_parts.n_partials >= 2 * in_parts.n_splits,
+  if (in_parts.tiles != nullptr)
+    DCP_REQUIRE(in_parts.n_entries > 0 && (reinterpret_cast<uintptr_t>(in_parts.tiles) & 15) == 0, "attn_fwd: no items, or not 16-byte aligned");
+  if (in_parts.parts != nullptr || in_parts.tiles != nullptr) {
+    DCP_REQUIRE((in_parts.tiles != nullptr || in_parts.n_entries >= batch) && in_parts.n_splits >= 0 && in_parts.n_splits <= batch && in_parts.n_partials >= 2 * in_parts.n_splits,
                 "attn_fwd: %d entries and %d partials of %d split rows do not fit %d rows", in_parts.n_entries, in_parts.n_partials,
                 in_parts.n_splits, batch);
     const size_t queries = (size_t)((block_size + 127) / 128) * 128 * n_heads_q * in_parts.n_partials;
@@ -819,11 +842,12 @@ static int attn_fwd(const void* q, const void* k, const void* v, void* out, floa
   const int bm = 128;
   p.q_tiles_per_row = (block_size + bm - 1) / bm;
   p.scale_log2 = softmax_scale * kLog2e;
-  p.n_items = (int64_t)(in_parts.parts ? in_parts.n_entries : batch) * n_heads_q * p.q_tiles_per_row;
+  p.tiles = reinterpret_cast<const FwdTile*>(in_parts.tiles);
+  p.n_items = (int64_t)(in_parts.parts || p.tiles ? in_parts.n_entries : batch) * n_heads_q * (p.tiles ? 1 : p.q_tiles_per_row);
   p.parts = reinterpret_cast<const FwdPart*>(in_parts.parts);
   p.partial_out = in_parts.partials;
   p.partial_sums = in_parts.partials + (size_t)in_parts.n_partials * n_heads_q * p.q_tiles_per_row * bm * head_dim;
-  p.xcd_group = p.q_tiles_per_row * (n_heads_q / n_heads_kv);
+  p.xcd_group = (p.tiles ? 1 : p.q_tiles_per_row) * (n_heads_q / n_heads_kv);
   DCP_REQUIRE(p.n_items < ((int64_t)1 << 31), "attn_fwd: too many work items");
   // as many workgroups as the device holds at once (two per CU), a multiple of the XCD count
   const int64_t n_wg = std::min<int64_t>(xcd_grid_size(p.n_items, 1), xcd_grid_size(2 * (int64_t)device_cu_count(), 1));
@@ -835,7 +859,9 @@ static int attn_fwd(const void* q, const void* k, const void* v, void* out, floa
     KernelTimer timer("attn_fwd_kernel", stream);
     hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, p);
   };
-#define DCP_FWD(DT, HD) (p.parts ? launch(attn_fwd_kernel<DT, HD, 1, true>) : launch(attn_fwd_kernel<DT, HD, 1, false>))
+#define DCP_FWD(DT, HD) (p.tiles   ? launch(attn_fwd_kernel<DT, HD, 1, kFwdTiles>)   \
+                         : p.parts ? launch(attn_fwd_kernel<DT, HD, 1, kFwdParts>) \
+                                   : launch(attn_fwd_kernel<DT, HD, 1, kFwdRows>))
   if (dtype == DCP_DTYPE_BF16) {
     if (head_dim == 128) DCP_FWD(DCP_DTYPE_BF16, 128);
     else DCP_FWD(DCP_DTYPE_BF16, 64);
@@ -900,5 +926,25 @@ extern "C" int dcp_attn_fwd_parts(const void* q, const void* k, const void* v, v
                   row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride,
                   q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
                   workspace_bytes, FwdParts{parts, n_entries, splits, n_splits, n_partials, reinterpret_cast<float*>(partials), partials_bytes}, stream);
+}
+
+
+extern "C" int dcp_attn_fwd_items(const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu_seqlens_q,
+                    const int32_t* cu_seqlens_kv, const int32_t* attn_range, int n_ranges, const int32_t* q_block_table,
+                    const int32_t* kv_block_table, const int32_t* out_block_table, const int32_t* row_order, int batch,
+                    int max_kv_blocks, int total_q, int block_size, int n_heads_q, int n_heads_kv, int head_dim,
+                    int64_t kv_slot_stride, int64_t kv_token_stride, int64_t q_slot_stride, int64_t out_slot_stride,
+                    int64_t lse_head_stride, int64_t lse_slot_stride, int merged_form, float softmax_scale, int dtype,
+                    void* workspace, size_t workspace_bytes, const int32_t* items, int n_items, const int32_t* splits,
+                    int n_splits, int n_partials, void* partials, size_t partials_bytes, void* stream) {
+  DCP_RECORDED(dcp_attn_fwd_items(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table,
+      out_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride,
+      kv_token_stride, q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
+      workspace_bytes, items, n_items, splits, n_splits, n_partials, partials, partials_bytes, stream));
+  DCP_REQUIRE(items != nullptr, "attn_fwd: no table of items");
+  return attn_fwd(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table,
+                  row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride,
+                  q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
+                  workspace_bytes, FwdParts{nullptr, n_items, splits, n_splits, n_partials, reinterpret_cast<float*>(partials), partials_bytes, items}, stream);
 }
 

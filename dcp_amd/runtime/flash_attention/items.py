@@ -1,0 +1,62 @@
+"""The work items of a forward launch whose rows are shorter than their blocks (``dcp_attn_fwd_items``).
+
+An item is 128 queries of a row and one head.  The kernel can count them from the block size alone, but a row
+shorter than its block then has items without queries, and each costs a workgroup a ticket and a chain of table
+reads.  Forward (us) without and with a table of the items there are, by the share of them: 0.37 (4476 tokens in
+sequences of 290, blocks of 1024, 8 heads of size 64) 32.8 / 17.5; 0.52 (3477 tokens, 16 heads) 31.2 / 20.5; 5323
+tokens in sequences of 67 in two partials, 40 heads, 67.6 / 57.5; 0.87 (5269 tokens, 40 heads) 151.2 / 150.4; 0.98
+(12678 tokens, 8 heads) 100.2 / 103.5.
+"""
+
+from __future__ import annotations
+
+from math import gcd
+from typing import Optional, Sequence
+
+import numpy as np
+
+N_XCD = 8
+MAX_SHARE = 0.8  # of the blocks' tiles: with more of them than that in use the table does not pay
+
+
+def deal_to_xcds(row: np.ndarray, n_kv_heads: int) -> np.ndarray:
+    """The order of items of rows ``row`` (rows' items together, rows in the order they should start in), as a
+    permutation.  Items go to the eight XCDs in turn, ``n_kv_heads`` streams each; the items of a row read the same
+    K and V, so that they take positions that one XCD (one L2) serves, while the rows are dealt to the
+    XCDs forth and back."""
+    lanes = N_XCD // gcd(N_XCD, n_kv_heads)
+    n = len(row)
+    if lanes == 1 or n == 0:
+        return np.arange(n)
+    starts = np.flatnonzero(np.concatenate(([True], row[1:] != row[:-1])))
+    turn = np.arange(len(starts)) % (2 * lanes)
+    lane = np.repeat(np.where(turn < lanes, turn, 2 * lanes - 1 - turn), np.diff(np.append(starts, n)))
+    by_lane = np.argsort(lane, kind="stable")
+    counts = np.bincount(lane, minlength=lanes)
+    place = np.empty(n, dtype=np.int64)  # of an item among its lane's
+    place[by_lane] = np.arange(n) - np.repeat(np.cumsum(counts) - counts, counts)
+    return np.argsort(place * lanes + lane, kind="stable")
+
+
+def pays(seqlens_q: Sequence[int], block_size: int, n_heads: int, n_slots: int, tile: int = 128) -> bool:
+    """Whether few enough of the tiles that the blocks have room for hold queries, and not all of them find a
+    workgroup slot at once (where they do, the table is only one more thing to read: 773 tokens of 8 heads
+    in blocks of 1024, 10.8 us without and 11.0 with it)."""
+    used, room = sum(-(-n // tile) for n in seqlens_q), len(seqlens_q) * -(-block_size // tile)
+    return 0 < used <= MAX_SHARE * room and room * n_heads > n_slots
+
+
+def forward_items(seqlens_q: Sequence[int], seqlens_kv: Sequence[int], n_kv_heads: int, tile: int = 128,
+                  parts: Optional[np.ndarray] = None) -> np.ndarray:
+    """The table: int32 ``[items, 4]``.  ``parts``: the entries of ``fwd_parts.split_rows``; else the rows, the
+    ones with the most keys first."""
+    if parts is None:
+        order = np.argsort(-np.asarray(seqlens_kv, dtype=np.int64), kind="stable")
+        parts = np.stack([order, 0 * order, 0 * order + 1, 0 * order], axis=1)
+    tiles = -(-np.asarray(seqlens_q, dtype=np.int64)[parts[:, 0]] // tile)
+    entry = np.repeat(np.arange(len(parts)), tiles)
+    # a row's last queries first: with a causal mask they see the most keys
+    q_tile = np.repeat(np.cumsum(tiles), tiles) - 1 - np.arange(len(entry))
+    order = deal_to_xcds(entry, n_kv_heads)
+    part = parts[entry[order]]
+    return np.stack([part[:, 0], q_tile[order], part[:, 1] + (part[:, 2] << 16), part[:, 3]], axis=1).astype(np.int32)

@@ -316,6 +316,32 @@ int dcp_attn_fwd_parts(const void* q, const void* k, const void* v, void* out,
                        void* stream);
 
 /*
+ * The same from a table of the work items there are, one per 128 queries of a row
+ * (or of a row's part):
+ *   items int32 [n_items][4], 16-byte aligned: a row; which 128 of its queries; part +
+ *     65536 * number of parts (65536 where the row is not split); first partial
+ * Every (row with queries, 128 of its queries, part) once, taken in this order and
+ * dealt to the XCDs in turn.  row_order is not read.  Tiles of a block for which a row
+ * has no queries are not listed, and cost nothing.
+ */
+int dcp_attn_fwd_items(const void* q, const void* k, const void* v, void* out,
+                       float* lse, const int32_t* cu_seqlens_q,
+                       const int32_t* cu_seqlens_kv, const int32_t* attn_range,
+                       int n_ranges, const int32_t* q_block_table,
+                       const int32_t* kv_block_table,
+                       const int32_t* out_block_table,
+                       const int32_t* row_order, int batch, int max_kv_blocks,
+                       int total_q, int block_size, int n_heads_q,
+                       int n_heads_kv, int head_dim, int64_t kv_slot_stride,
+                       int64_t kv_token_stride, int64_t q_slot_stride,
+                       int64_t out_slot_stride, int64_t lse_head_stride,
+                       int64_t lse_slot_stride, int merged_form,
+                       float softmax_scale, int dtype, void* workspace,
+                       size_t workspace_bytes, const int32_t* items, int n_items, const int32_t* splits, int n_splits,
+                       int n_partials, void* partials, size_t partials_bytes,
+                       void* stream);
+
+/*
  * Range-masked, paged, variable-length attention backward.
  * Replaces dcp_flash_attn._flash_attn_varlen_backward as called by
  * _wrapped_flash_attn_varlen_backward (executor.py:256-337) from

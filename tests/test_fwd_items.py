@@ -1,0 +1,59 @@
+"""Forward launches from a table of their work items: the table names every 128 queries of every row (or part of a row)
+once and keeps a row's on one XCD (CPU); results are those of the launch that counts the items itself (GPU)."""
+
+from math import gcd
+
+import numpy as np
+import pytest
+import torch
+
+from dcp_amd.runtime.flash_attention import executor, fwd_parts, items
+from tests.plan_cases import check_against_truth, dense_truth, make_case, run_executor
+from tests.test_dkv_groups import PLANS
+
+
+@pytest.mark.parametrize("n_kv_heads", [1, 2, 3, 8])
+@pytest.mark.parametrize("seqlens_q", [[1], [128, 129, 127, 1, 1024, 300] * 7, [5, 0, 260], list(range(1, 40))])
+def test_every_tile_once(seqlens_q, n_kv_heads):
+    rng = np.random.default_rng(0)
+    seqlens_kv = rng.integers(1, 4000, size=len(seqlens_q)).tolist()
+    table = items.forward_items(seqlens_q, seqlens_kv, n_kv_heads)
+    want = [(row, t, 65536, 0) for row, n in enumerate(seqlens_q) for t in range(-(-n // 128))]
+    assert sorted(map(tuple, table.tolist())) == want
+    # positions that come round to one XCD hold whole rows, until the first XCD's are out (three rounds at least, here)
+    lanes = 8 // gcd(8, n_kv_heads)
+    xcds = {}
+    for at, (row, *_) in enumerate(table[: 3 * lanes].tolist()):
+        xcds.setdefault(row, set()).add(at % lanes)
+    assert len(seqlens_q) < 39 or all(len(x) == 1 for x in xcds.values())
+
+
+def test_parts_of_rows():
+    seqlens_q, seqlens_kv = [300, 128, 64, 512], [4096, 640, 64, 2048]
+    parts = np.asarray([[0, 0, 2, 0], [0, 1, 2, 0], [3, 0, 1, 0], [1, 0, 1, 0], [2, 0, 1, 0]], dtype=np.int32)
+    table = items.forward_items(seqlens_q, seqlens_kv, 8, parts=parts)
+    want = [(row, t, i + (n << 16), f) for row, i, n, f in parts.tolist() for t in range(-(-seqlens_q[row] // 128))]
+    assert sorted(map(tuple, table.tolist())) == sorted(want)
+
+
+def test_rule():
+    pays = lambda seqlens, block_size, n_heads=32, n_slots=100: items.pays(seqlens, block_size, n_heads, n_slots)
+    assert not pays([], 1024) and not pays([0], 1024)
+    assert pays([290] * 9, 1024) and not pays([1000] * 9, 1024) and not pays([256] * 9, 256) and pays([100] * 9, 256)
+    assert not pays([290] * 9, 1024, 1) and not pays([290] * 9, 1024, 8, 9 * 8 * 8) and pays([290] * 9, 1024, 8, 9 * 8 * 8 - 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("share", [None, 2])
+@pytest.mark.parametrize("name", list(PLANS))
+def test_same_results(gpu, monkeypatch, name, share):
+    case = make_case(**PLANS[name])
+    if share:
+        monkeypatch.setattr(fwd_parts, "share_of_a_part", lambda *a: share)
+    counted, _ = run_executor(case, backward=False)
+    monkeypatch.setattr(executor, "items_pay", lambda *a: True)
+    listed, _ = run_executor(case, backward=False, poison=200.0)
+    assert torch.equal(counted[0], listed[0]) and torch.equal(counted[1], listed[1])
+    check_against_truth(listed, dense_truth(case, backward=False))
+    replayed, _ = run_executor(case, backward=False, use_graph=True)
+    assert torch.equal(listed[0], replayed[0]) and torch.equal(listed[1], replayed[1])
