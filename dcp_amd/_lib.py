@@ -29,6 +29,7 @@ SIGNATURES = {
     "dcp_record_end": [],
     "dcp_record_size": [_P],
     "dcp_record_run": [_P, _I, _I, _P],
+    "dcp_sequence_run": [_P, _I, _P],
     "dcp_record_free": [_P],
     "dcp_fused_copy_varlen": [_P, _P, _P, _P, _P, _P, _P, _I, _L, _I, _P],
     "dcp_fused_copy_varlen_dkv": [_P, _P, _P, _I, _I, _I, _I, _P],
@@ -120,6 +121,33 @@ class Recording:
     def __del__(self):
         if self._list is not None and _lib is not None:
             _lib.dcp_record_free(self._list)
+
+
+class _SequenceOp(ctypes.Structure):
+    _fields_ = [("kind", ctypes.c_int32), ("begin", ctypes.c_int32), ("end", ctypes.c_int32), ("on_caller", ctypes.c_int32),
+                ("list", c_void_p), ("event", c_void_p), ("stream", c_void_p)]
+
+
+class Sequence:
+    """Recorded calls on several streams with the events between them (``dcp_sequence_run``).  Streams and events are
+    torch's; a stream of None is the one the sequence is run from.  The caller keeps recordings, streams and
+    events alive."""
+
+    RUN, RECORD, WAIT = range(3)
+
+    def __init__(self, ops):
+        """``ops``: ``(RUN, recording, stream)`` or ``(RECORD or WAIT, event, stream)``."""
+        self._ops = (_SequenceOp * len(ops))()
+        for op, (kind, what, stream) in zip(self._ops, ops):
+            op.kind, op.on_caller = kind, stream is None
+            op.stream = None if stream is None else stream.cuda_stream
+            if kind == self.RUN:
+                op.list, op.end = what._list, what.size()
+            else:
+                op.event = what.cuda_event
+
+    def run(self, stream: int) -> None:
+        call("dcp_sequence_run", self._ops, len(self._ops), stream)
 
 
 def profile_enable(on: bool) -> None:

@@ -54,3 +54,21 @@ extern "C" int dcp_record_run(const void* list, int begin, int end, void* stream
 }
 
 extern "C" void dcp_record_free(void* list) { delete static_cast<RecordedCalls*>(list); }
+
+extern "C" int dcp_sequence_run(const dcp_sequence_op* ops, int n_ops, void* stream) {
+  DCP_REQUIRE(n_ops >= 0 && (n_ops == 0 || ops != nullptr), "sequence_run: no operations");
+  for (int i = 0; i < n_ops; ++i) {
+    const dcp_sequence_op& op = ops[i];
+    void* const on = op.on_caller ? stream : op.stream;
+    if (op.kind == DCP_SEQUENCE_RUN) {
+      if (const int status = dcp_record_run(op.list, op.begin, op.end, on)) return status;
+      continue;
+    }
+    DCP_REQUIRE((op.kind == DCP_SEQUENCE_RECORD || op.kind == DCP_SEQUENCE_WAIT) && op.event != nullptr,
+                "sequence_run: operation %d is of kind %d, event %p", i, op.kind, op.event);
+    const hipError_t e = op.kind == DCP_SEQUENCE_RECORD ? hipEventRecord((hipEvent_t)op.event, (hipStream_t)on)
+                                                        : hipStreamWaitEvent((hipStream_t)on, (hipEvent_t)op.event, 0);
+    if (e != hipSuccess) return dcp::fail(DCP_ERR_LAUNCH, "sequence_run: operation %d: %s", i, hipGetErrorString(e));
+  }
+  return DCP_OK;
+}

@@ -74,6 +74,24 @@ int dcp_record_run(const void* list, int begin, int end, void* stream);
 void dcp_record_free(void* list);
 
 /*
+ * Recorded calls of several lists on several streams, with the events between
+ * them, in one call: what the plans of several devices that share a GPU come to.
+ * Operation i launches calls [begin, end) of `list`, records `event` or makes
+ * `stream` wait for it (hipEvent_t, hipStream_t); with on_caller nonzero the
+ * operation's stream is the `stream` argument.  Stops at the first error.
+ */
+#define DCP_SEQUENCE_RUN 0
+#define DCP_SEQUENCE_RECORD 1
+#define DCP_SEQUENCE_WAIT 2
+typedef struct {
+  int32_t kind, begin, end, on_caller;
+  const void* list;
+  void* event;
+  void* stream;
+} dcp_sequence_op;
+int dcp_sequence_run(const dcp_sequence_op* ops, int n_ops, void* stream);
+
+/*
  * Block gather / scatter through pointer tables.
  * Replaces dcp.ops.fused_ops.fused_copy_{bf16,fp16,fp32}_varlen
  * (dcp/ops/fused_ops.py:842-864, 916-938, 1013-1035; kernels :290-335,
