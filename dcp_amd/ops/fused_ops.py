@@ -35,34 +35,34 @@ __all__ = [
 ]
 
 _DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+_DTYPE_CODE.update({str(k): v for k, v in _DTYPE_CODE.items()})
 
 
 def dtype_code(dtype) -> int:
     """Wire integer of a torch dtype (or of its ``str``)."""
-    if isinstance(dtype, str):
-        for k, v in _DTYPE_CODE.items():
-            if str(k) == dtype:
-                return v
+    code = _DTYPE_CODE.get(dtype)
+    if code is None:
         raise ValueError(f"Unsupported dtype: {dtype}")
-    if dtype not in _DTYPE_CODE:
-        raise ValueError(f"Unsupported dtype: {dtype}")
-    return _DTYPE_CODE[dtype]
+    return code
 
 
+# A small operator is as long as its call.  So the call asks torch for the stream's handle alone (a Stream object
+# costs 1.5 us), and a table that is as it should be passes in one expression: 9.0 -> 6.1 us a call (sum of four
+# partials of 3118 tokens, 5 heads: 9.3 -> 6.3 us; merge of three of 1635 tokens: 9.1 -> 6.2).
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _table(t: torch.Tensor, dtype: torch.dtype, name: str) -> int:
+    if isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda and t.is_contiguous():
+        return t.data_ptr()
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor, got {type(t).__name__}")
     if t.dtype != dtype:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
     if not t.is_cuda:
         raise ValueError(f"{name} must be a device tensor")
-    if not t.is_contiguous():
-        raise ValueError(f"{name} must be contiguous")
-    return t.data_ptr()
+    raise ValueError(f"{name} must be contiguous")
 
 
 def _i32(t, name):
@@ -89,7 +89,7 @@ def _copy_varlen(elem_size, src_ptrs, src_offsets, src_strides, dst_ptrs,
         _i32(dst_offsets, "dst_offsets"),
         _i32(dst_strides, "dst_strides"),
         _i32(n_elements, "n_elements"),
-        len(src_ptrs),
+        src_ptrs.size(0),
         int(block_size),
         elem_size,
         _stream(),
@@ -157,7 +157,7 @@ def _copy_dkv(elem_size, src_ptrs, dst_ptrs, n_tokens, max_n_tokens,
         _i64(src_ptrs, "src_ptrs"),
         _i64(dst_ptrs, "dst_ptrs"),
         _i32(n_tokens, "n_tokens"),
-        len(src_ptrs),
+        src_ptrs.size(0),
         int(max_n_tokens),
         int(per_token_size),
         elem_size,
@@ -198,7 +198,7 @@ def _copy_lse(elem_size, src_ptrs, src_token_offsets, src_head_strides,
         _i32(dst_token_offsets, "dst_token_offsets"),
         _i32(dst_head_strides, "dst_head_strides"),
         _i32(n_tokens, "n_tokens"),
-        len(src_ptrs),
+        src_ptrs.size(0),
         int(head_block_size),
         int(block_size),
         elem_size,
@@ -287,7 +287,7 @@ def flash_attn_update_out_lse(
         _i32(dst_token_offsets, "dst_token_offsets"),
         _i32(n_tokens_per_block, "n_tokens_per_block"),
         _i32(block_lengths, "block_lengths"),
-        len(block_lengths),
+        block_lengths.size(0),
         int(block_size),
         int(out_block_stride),
         int(out_token_stride),
@@ -329,8 +329,8 @@ def fused_blockwise_sum(
     ``fused_ops.py:1288-1360``); accumulated in fp32.  ``fp32_sources`` (extension): the sources are
     fp32 whatever ``dtype``, the destinations' type, is."""
     assert block_size % triton_block_size == 0
-    code = dtype_code(dtype if isinstance(dtype, str) else str(dtype))
-    if src_offsets.dim() != 2 or src_offsets.shape[1] != max_n_ops_per_block:
+    code = dtype_code(dtype if isinstance(dtype, (str, torch.dtype)) else str(dtype))
+    if src_offsets.dim() != 2 or src_offsets.size(1) != max_n_ops_per_block:
         raise ValueError(
             "src_offsets must be [n_sums, max_n_ops_per_block], got "
             f"{tuple(src_offsets.shape)}"
@@ -345,7 +345,7 @@ def fused_blockwise_sum(
         _i32(dst_offsets, "dst_offsets"),
         _i32(dst_strides, "dst_strides"),
         _i32(n_elements, "n_elements"),
-        len(src_ptrs),
+        src_ptrs.size(0),
         int(max_n_ops_per_block),
         int(block_size),
         code,
