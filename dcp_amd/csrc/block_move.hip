@@ -37,16 +37,23 @@ __global__ __launch_bounds__(kCopyThreads) void copy_varlen_kernel(
   constexpr int kCopyChunkBytes = kCopyThreads * 16 * kCopyUnroll;
   const int p = blockIdx.x / chunks_per_block;
   const int c = blockIdx.x - p * chunks_per_block;
-  const int64_t n_bytes = (int64_t)n_count[p] * elems_per_count * elem_size;
+  // In one-wave workgroups all the tables' words of the block in one trip, before anything depends on one of
+  // them: 4 MiB blocks 6.67 -> 6.77 TB/s (2 GiB there and back 1288 -> 1269 us).  Larger workgroups, of which the
+  // ones past a ragged block's end leave at once, are better off with its length alone first (blocks of up
+  // to 640 KiB, 16.5 us and 16.9 with all words).
+  const int32_t count = n_count[p];
+  const int64_t src_ptr = src_ptrs[p], dst_ptr = dst_ptrs[p];
+  const bool strided = src_offsets != nullptr;  // (no such columns: any table's word in their place, and no branch)
+  int32_t src_offset = (strided ? src_offsets : n_count)[p], src_stride = (strided ? src_strides : n_count)[p];
+  int32_t dst_offset = (strided ? dst_offsets : n_count)[p], dst_stride = (strided ? dst_strides : n_count)[p];
+  if constexpr (kCopyThreads == 64) read_together(count, src_ptr, dst_ptr, src_offset, src_stride, dst_offset, dst_stride);
+  if (!strided) src_offset = dst_offset = 0;
+  const int64_t n_bytes = (int64_t)count * elems_per_count * elem_size;
   const int64_t begin = (int64_t)c * kCopyChunkBytes;
   if (begin >= n_bytes) return;
   const int64_t end = min(begin + (int64_t)kCopyChunkBytes, n_bytes);
-
-  int64_t src_off = 0, dst_off = 0;
-  if (src_offsets) src_off = (int64_t)src_offsets[p] * src_strides[p] * elem_size;
-  if (dst_offsets) dst_off = (int64_t)dst_offsets[p] * dst_strides[p] * elem_size;
-  const char* src = reinterpret_cast<const char*>(src_ptrs[p]) + src_off;
-  char* dst = reinterpret_cast<char*>(dst_ptrs[p]) + dst_off;
+  const char* src = reinterpret_cast<const char*>(src_ptr) + (int64_t)src_offset * src_stride * elem_size;
+  char* dst = reinterpret_cast<char*>(dst_ptr) + (int64_t)dst_offset * dst_stride * elem_size;
 
   const bool aligned =
       ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0;

@@ -601,17 +601,25 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
   constexpr int VN = Vec16<DTYPE>::N;
   constexpr int WORDS = VN / Vec16<SRC>::N;  // 16-byte words of a source per word of the result
   const int s = blockIdx.x / chunks_per_sum;
-  const int64_t n_elem = n_elements[s];
+  // All the tables' words of the sum in one trip, up to four of its sources among them (as in copy_varlen_kernel):
+  // 8192 ragged tokens of 8 heads, three sources, 8.3 -> 8.0 us
+  const int32_t* offs = src_offsets + (int64_t)s * max_n_ops_per_block;
+  const int64_t src_ptr = src_ptrs[s], dst_ptr = dst_ptrs[s];
+  const int32_t n_elem = n_elements[s], n_ops = n_ops_per_block[s];
+  const int32_t src_step = src_strides[s], dst_offset = dst_offsets[s], dst_step = dst_strides[s];
+  int32_t first[4];  // (past the last source: the last one again)
+#pragma unroll
+  for (int q = 0; q < 4; ++q) first[q] = offs[min(q, max_n_ops_per_block - 1)];
+  read_together(src_ptr, dst_ptr, n_elem, n_ops, src_step, dst_offset, dst_step, first[0], first[1], first[2], first[3]);
+#pragma unroll
+  for (int q = 1; q < 4; ++q) first[q] = q < n_ops ? first[q] : first[q - 1];
   const int64_t chunk_elems = (int64_t)THREADS * VN * kSumUnroll;
   const int64_t begin = (int64_t)(blockIdx.x - s * chunks_per_sum) * chunk_elems;
   if (begin >= n_elem) return;
-  const int64_t end = min(begin + chunk_elems, n_elem);
-
-  const int n_ops = n_ops_per_block[s];
-  const int32_t* offs = src_offsets + (int64_t)s * max_n_ops_per_block;
-  const src_raw* src = reinterpret_cast<const src_raw*>(src_ptrs[s]);
-  const int64_t src_stride = src_strides[s];
-  raw* dst = reinterpret_cast<raw*>(dst_ptrs[s]) + (int64_t)dst_offsets[s] * dst_strides[s];
+  const int64_t end = min(begin + chunk_elems, (int64_t)n_elem);
+  const src_raw* src = reinterpret_cast<const src_raw*>(src_ptr);
+  const int64_t src_stride = src_step;
+  raw* dst = reinterpret_cast<raw*>(dst_ptr) + (int64_t)dst_offset * dst_step;
 
   const bool aligned = ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0 &&
                        (src_stride % VN) == 0;
@@ -632,7 +640,7 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
       for (int k = 0; k < VN; ++k) acc[u][k] = 0.0f;
     }
     if (begin < vec_end && n_ops == 1 && SRC == DTYPE) {  // a single source: the scatter-back, copied bit for bit
-      const src_raw* row = src + offs[0] * src_stride;
+      const src_raw* row = src + first[0] * src_stride;
       u32x4 bits[kSumUnroll];
 #pragma unroll
       for (int u = 0; u < kSumUnroll; ++u) bits[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + pos[u]));
@@ -644,7 +652,8 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
         u32x4 bits[4][kSumUnroll][WORDS];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const src_raw* row = src + offs[min(j0 + q, n_ops - 1)] * src_stride;  // tail: re-read the last source
+          // tail: re-read the last source
+          const src_raw* row = src + (j0 == 0 ? first[q] : offs[min(j0 + q, n_ops - 1)]) * src_stride;
 #pragma unroll
           for (int u = 0; u < kSumUnroll; ++u)
 #pragma unroll

@@ -126,4 +126,16 @@ inline int dtype_size(int dtype) {
   }
 }
 
+// Makes the loads of (wave-uniform) values that stand before it go out together and be waited for once.  Left to
+// itself the compiler moves each to where it is used first, which for a table's words is behind a branch on
+// another table's word: a trip to memory after the other.
+template <typename T>
+__device__ __forceinline__ void read_here(const T& value) {
+  asm volatile("" : : "s"(value));
+}
+template <typename... T>
+__device__ __forceinline__ void read_together(const T&... value) {
+  (read_here(value), ...);
+}
+
 }  // namespace dcp
