@@ -45,7 +45,7 @@ SIGNATURES = {
     "dcp_attn_fwd_parts": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I] + [_L] * 6
                           + [_I, _F, _I, _P, c_size_t, _P, _I, _P, _I, _I, _P, c_size_t, _P],
     "dcp_attn_fwd_items": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I] + [_L] * 6
-                          + [_I, _F, _I, _P, c_size_t, _P, _I, _P, _I, _I, _P, c_size_t, _P],
+                          + [_I, _F, _I, _P, c_size_t, _P, _I, _I, _P, _I, _I, _P, c_size_t, _P],
     "dcp_attn_bwd_strided": [_P] * 10 + [c_size_t] + [_P] * 3 + [_I] + [_P] * 6 + [_I] * 7 + [_L] * 10 + [_F, _I, _P],
     "dcp_attn_bwd_grouped": [_P] * 10 + [c_size_t] + [_P] * 3 + [_I] + [_P] * 6 + [_I] * 7 + [_L] * 10
                             + [_P, _I, _P, _P, _P, _L, _L, _P, _F, _I, _P],

@@ -649,6 +649,9 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
 // of work), and the last, unevenly long items leave slots empty at the end.  Rows come longest first;
 // the counters are zeroed by a one-wave kernel on the stream just before.  A launch whose items all
 // fit on the device at once needs no queue and no such kernel.
+// But the queue costs that kernel, 4-5 us, and a launch of little work per slot wins less by it: dcp_attn_fwd_items
+// takes a workgroup per item where it is told to (the caller knows the rows' lengths; figures at
+// one_workgroup_each of items.py).
 template <int DTYPE, int D, int QB, FwdItems ITEMS>
 __global__ __launch_bounds__(kFwdThreads, QB == 1 ? 2 : 1) void attn_fwd_kernel(const AttnFwdParams p) {
   __shared__ int ticket_lds;
@@ -761,6 +764,7 @@ struct FwdParts {
   float* partials = nullptr;
   size_t partials_bytes = 0;
   const int32_t* tiles = nullptr;  // dcp_attn_fwd_items: n_entries of them instead of parts
+  bool one_each = false;           // a workgroup per work item, whether the device holds them all at once or not
 };
 
 static int attn_fwd(const void* q, const void* k, const void* v, void* out, float* lse, const int32_t* cu_seqlens_q,
@@ -850,7 +854,8 @@ static int attn_fwd(const void* q, const void* k, const void* v, void* out, floa
   p.xcd_group = (p.tiles ? 1 : p.q_tiles_per_row) * (n_heads_q / n_heads_kv);
   DCP_REQUIRE(p.n_items < ((int64_t)1 << 31), "attn_fwd: too many work items");
   // as many workgroups as the device holds at once (two per CU), a multiple of the XCD count
-  const int64_t n_wg = std::min<int64_t>(xcd_grid_size(p.n_items, 1), xcd_grid_size(2 * (int64_t)device_cu_count(), 1));
+  const int64_t n_slots = xcd_grid_size(2 * (int64_t)device_cu_count(), 1);
+  const int64_t n_wg = in_parts.one_each ? xcd_grid_size(p.n_items, 1) : std::min<int64_t>(xcd_grid_size(p.n_items, 1), n_slots);
   p.tickets = p.n_items > n_wg ? reinterpret_cast<int*>(workspace) : nullptr;
   p.ticket_stride = workspace_bytes >= dcp_attn_fwd_workspace_bytes() ? kFwdTicketStride : kFwdTicketStrideMin;
   dim3 grid((unsigned)n_wg), block(kFwdThreads);
@@ -935,16 +940,16 @@ extern "C" int dcp_attn_fwd_items(const void* q, const void* k, const void* v, v
                     int max_kv_blocks, int total_q, int block_size, int n_heads_q, int n_heads_kv, int head_dim,
                     int64_t kv_slot_stride, int64_t kv_token_stride, int64_t q_slot_stride, int64_t out_slot_stride,
                     int64_t lse_head_stride, int64_t lse_slot_stride, int merged_form, float softmax_scale, int dtype,
-                    void* workspace, size_t workspace_bytes, const int32_t* items, int n_items, const int32_t* splits,
+                    void* workspace, size_t workspace_bytes, const int32_t* items, int n_items, int one_each, const int32_t* splits,
                     int n_splits, int n_partials, void* partials, size_t partials_bytes, void* stream) {
   DCP_RECORDED(dcp_attn_fwd_items(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table,
       out_block_table, row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride,
       kv_token_stride, q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
-      workspace_bytes, items, n_items, splits, n_splits, n_partials, partials, partials_bytes, stream));
-  DCP_REQUIRE(items != nullptr, "attn_fwd: no table of items");
+      workspace_bytes, items, n_items, one_each, splits, n_splits, n_partials, partials, partials_bytes, stream));
+  DCP_REQUIRE(items != nullptr || (n_items == 0 && n_splits == 0), "attn_fwd: %d items and %d split rows, but no table of items", n_items, n_splits);
   return attn_fwd(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_kv, attn_range, n_ranges, q_block_table, kv_block_table, out_block_table,
                   row_order, batch, max_kv_blocks, total_q, block_size, n_heads_q, n_heads_kv, head_dim, kv_slot_stride, kv_token_stride,
                   q_slot_stride, out_slot_stride, lse_head_stride, lse_slot_stride, merged_form, softmax_scale, dtype, workspace,
-                  workspace_bytes, FwdParts{nullptr, n_items, splits, n_splits, n_partials, reinterpret_cast<float*>(partials), partials_bytes, items}, stream);
+                  workspace_bytes, FwdParts{nullptr, n_items, splits, n_splits, n_partials, reinterpret_cast<float*>(partials), partials_bytes, items, one_each != 0}, stream);
 }
 

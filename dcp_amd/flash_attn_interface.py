@@ -197,6 +197,7 @@ def _flash_attn_varlen_forward(
     merged_form: bool = False,
     parts=None,
     items: Optional[torch.Tensor] = None,
+    one_each: bool = False,
 ):
     """Writes the row outputs into ``out_`` / ``lse_`` in place and returns
     ``(out_, lse_, None, None)`` (the reference returns
@@ -219,6 +220,7 @@ def _flash_attn_varlen_forward(
     (``dcp_attn_fwd_parts``): int32 ``[entries, 4]`` and ``[split rows, 4]``, and fp32 scratch.
     ``items`` (extension): the launch's work items, int32 ``[n, 4]`` (``dcp_attn_fwd_items``; with ``parts``, whose
     entries they then stand for).
+    ``one_each`` (extension, not with ``parts`` alone): a workgroup for every work item (``dcp_attn_fwd_items``).
     """
     _check_plain(dropout_p, causal, window_size_left, window_size_right, softcap,
                  alibi_slopes, return_softmax)
@@ -253,7 +255,7 @@ def _flash_attn_varlen_forward(
             _widen(q, d, block_size), _widen(k, d, block_size), _widen(v, d, block_size), cu_seqlens_q, cu_seqlens_k, total_q, max_seqlen_q, max_seqlen_k,
             dropout_p, softmax_scale, attn_range=attn_range, q_block_table=q_block_table, kv_block_table=kv_block_table,
             out_block_table=out_block_table, out_=out_wide, lse_=lse_, row_order=row_order, workspace=workspace,
-            block_size=block_size, merged_form=merged_form, parts=parts, items=items)
+            block_size=block_size, merged_form=merged_form, parts=parts, items=items, one_each=one_each)
         out_.copy_(out_wide[..., :head_dim])
         return out_, lse_, None, None
     if workspace is None:
@@ -277,17 +279,20 @@ def _flash_attn_varlen_forward(
     )
     if items is not None and (items.dim() != 2 or items.shape[1] != 4):
         raise ValueError(f"items must be [n, 4], got {tuple(items.shape)}")
-    if parts is None and items is None:
+    n_items, table = (0, 0) if items is None else (items.shape[0], _i32(items, "items").data_ptr())
+    if parts is None and items is None and not one_each:
         _lib.call("dcp_attn_fwd_strided", *args, _stream())
     elif parts is None:
-        _lib.call("dcp_attn_fwd_items", *args, _i32(items, "items").data_ptr(), items.shape[0], 0, 0, 0, 0, 0, _stream())
+        _lib.call("dcp_attn_fwd_items", *args, table, n_items, 1 if one_each else 0, 0, 0, 0, 0, 0, _stream())
     else:
         entries, splits, n_partials, partials = parts
         if entries.shape[1:] != (4,) or splits.shape[1:] != (4,) or partials.dtype != torch.float32 or not partials.is_contiguous():
             raise ValueError("parts: [entries, 4] and [split rows, 4] tables and contiguous fp32 scratch expected")
-        name, table = ("dcp_attn_fwd_parts", entries) if items is None else ("dcp_attn_fwd_items", items)
-        _lib.call(name, *args, _i32(table, "parts").data_ptr(), table.shape[0], _i32(splits, "splits").data_ptr(),
-                  splits.shape[0], int(n_partials), partials.data_ptr(), partials.numel() * 4, _stream())
+        sums = (_i32(splits, "splits").data_ptr(), splits.shape[0], int(n_partials), partials.data_ptr(), partials.numel() * 4)
+        if items is None:
+            _lib.call("dcp_attn_fwd_parts", *args, _i32(entries, "parts").data_ptr(), entries.shape[0], *sums, _stream())
+        else:
+            _lib.call("dcp_attn_fwd_items", *args, table, n_items, 1 if one_each else 0, *sums, _stream())
     return out_, lse_, None, None
 
 

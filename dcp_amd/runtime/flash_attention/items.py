@@ -17,6 +17,7 @@ import numpy as np
 
 N_XCD = 8
 MAX_SHARE = 0.8  # of the blocks' tiles: with more of them than that in use the table does not pay
+MAX_TILES_WITHOUT_QUEUE = 64  # per slot
 
 
 def deal_to_xcds(row: np.ndarray, n_kv_heads: int) -> np.ndarray:
@@ -44,6 +45,20 @@ def pays(seqlens_q: Sequence[int], block_size: int, n_heads: int, n_slots: int, 
     in blocks of 1024, 10.8 us without and 11.0 with it)."""
     used, room = sum(-(-n // tile) for n in seqlens_q), len(seqlens_q) * -(-block_size // tile)
     return 0 < used <= MAX_SHARE * room and room * n_heads > n_slots
+
+
+def one_workgroup_each(seqlens_q: Sequence[int], seqlens_kv: Sequence[int], n_heads: int, n_slots: int, tile: int = 128) -> bool:
+    """Whether a launch of more items than workgroup slots starts a workgroup for every item, instead of one per slot
+    that takes item after item from a queue.  The queue wins by what it takes out of the gaps between workgroups,
+    some 5 % of the launch, and costs a kernel that clears its counters, 4-5 us.  Forward (us) with and
+    without it, by key tiles (64) per slot: 36 and 27 (two launches; 15480 tokens, 8 heads) 200 / 183; 43 (12678
+    tokens, 8 heads) 103 / 96; 44 (18701 tokens) 81 / 75; 53 and 41 (two; 12926 tokens, size 64) 147 / 133; 53
+    (5323 tokens, 40 heads of 64) 57.8 / 46.1; 56 (7604 tokens, 40 heads) 119 / 112; 98 (5269 tokens, 40 heads) 151 /
+    154; 103 (16384 tokens, 16 heads) 196 / 205; 122 (28012 tokens, 32 heads) 336 / 367; 183 (32768 tokens, 8
+    heads) 338 / 354; 2297 (65536 tokens, 32 heads) 3744 / 4007."""
+    items = [-(-n // tile) for n in seqlens_q]
+    return (sum(items) * n_heads > n_slots
+            and sum(n * -(-k // 64) for n, k in zip(items, seqlens_kv)) * n_heads <= MAX_TILES_WITHOUT_QUEUE * n_slots)
 
 
 def forward_items(seqlens_q: Sequence[int], seqlens_kv: Sequence[int], n_kv_heads: int, tile: int = 128,

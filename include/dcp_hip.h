@@ -340,7 +340,10 @@ int dcp_attn_fwd_parts(const void* q, const void* k, const void* v, void* out,
  *     65536 * number of parts (65536 where the row is not split); first partial
  * Every (row with queries, 128 of its queries, part) once, taken in this order and
  * dealt to the XCDs in turn.  row_order is not read.  Tiles of a block for which a row
- * has no queries are not listed, and cost nothing.
+ * has no queries are not listed, and cost nothing.  items null (and n_items and
+ * n_splits 0): all tiles of the rows, as dcp_attn_fwd_strided.
+ *   one_each: nonzero = a workgroup for every item from the start (the workspace is then
+ *     not used); 0 = as many as the device holds at once, which take item after item.
  */
 int dcp_attn_fwd_items(const void* q, const void* k, const void* v, void* out,
                        float* lse, const int32_t* cu_seqlens_q,
@@ -355,7 +358,7 @@ int dcp_attn_fwd_items(const void* q, const void* k, const void* v, void* out,
                        int64_t out_slot_stride, int64_t lse_head_stride,
                        int64_t lse_slot_stride, int merged_form,
                        float softmax_scale, int dtype, void* workspace,
-                       size_t workspace_bytes, const int32_t* items, int n_items, const int32_t* splits, int n_splits,
+                       size_t workspace_bytes, const int32_t* items, int n_items, int one_each, const int32_t* splits, int n_splits,
                        int n_partials, void* partials, size_t partials_bytes,
                        void* stream);
 

@@ -43,6 +43,13 @@ def test_rule():
     assert not pays([290] * 9, 1024, 1) and not pays([290] * 9, 1024, 8, 9 * 8 * 8) and pays([290] * 9, 1024, 8, 9 * 8 * 8 - 1)
 
 
+def test_rule_of_the_queue():
+    each = items.one_workgroup_each
+    assert not each([], [], 8, 512) and not each([128] * 64, [640] * 64, 8, 512)  # all at once
+    assert each([128] * 65, [640] * 65, 8, 512) and each([100] * 65, [640] * 65, 8, 512)
+    assert each([128] * 128, [64 * 32] * 128, 8, 512) and not each([128] * 128, [64 * 32 + 1] * 128, 8, 512)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("share", [None, 2])
 @pytest.mark.parametrize("name", list(PLANS))
@@ -57,3 +64,19 @@ def test_same_results(gpu, monkeypatch, name, share):
     check_against_truth(listed, dense_truth(case, backward=False))
     replayed, _ = run_executor(case, backward=False, use_graph=True)
     assert torch.equal(listed[0], replayed[0]) and torch.equal(listed[1], replayed[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("listed", [False, True])
+@pytest.mark.parametrize("name", list(PLANS))
+def test_a_workgroup_each(gpu, monkeypatch, name, listed):
+    """More work items than slots, with and without the table: the launch without a queue, the same bits."""
+    case = make_case(**dict(PLANS[name], seqlens=PLANS[name]["seqlens"] * 40))
+    monkeypatch.setattr(executor, "one_workgroup_each", lambda *a: False)
+    monkeypatch.setattr(executor, "items_pay", lambda *a: listed)
+    queued, _ = run_executor(case, backward=False)
+    monkeypatch.setattr(executor, "one_workgroup_each", lambda *a: True)
+    each, _ = run_executor(case, backward=False, poison=200.0)
+    assert torch.equal(queued[0], each[0]) and torch.equal(queued[1], each[1])
+    replayed, _ = run_executor(case, backward=False, use_graph=True)
+    assert torch.equal(each[0], replayed[0]) and torch.equal(each[1], replayed[1])
