@@ -74,7 +74,7 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
     # A slot that holds a copy of a local block of the matching type: buffer type -> slot -> (memcpy
     # index, pair position, index and tokens of the local block)
     origin: Dict[str, Dict[int, Tuple[int, int, int, int]]] = defaultdict(dict)
-    all_pairs: Set[Tuple[int, int]] = set()
+    copied: Dict[int, Set[int]] = {}  # memcpy index -> positions of such copies
     # copied pairs with a reader that does not address them through an operand that can go to the source
     blocked: Set[Tuple[int, int]] = set()
     # results that a scatter may take from their slot: buffer type -> slot -> producer; and the readers of each
@@ -89,15 +89,13 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
         found = origin[buffer_type].get
         rows = []
         for row in table:
-            indices = []
-            for blk in row:
-                h = found(blk.index)
-                if h is None or h[3] != blk.n_tokens or blk.buffer_type != buffer_type:
-                    for r in table:
-                        for b in r:
-                            read_in_slot(b)
-                    return None
-                indices.append(h[2])
+            indices = [h[2] for blk in row if (h := found(blk.index)) is not None and h[3] == blk.n_tokens
+                       and blk.buffer_type == buffer_type]
+            if len(indices) != len(row):
+                for r in table:
+                    for b in r:
+                        read_in_slot(b)
+                return None
             rows.append(indices)
         return rows
 
@@ -106,6 +104,10 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
         if h is not None:
             blocked.add((h[0], h[1]))
 
+    def with_entries() -> Set[str]:
+        """The buffer types that have blocks in the tables; a block of another type needs no look."""
+        return {t for table in (origin, produced) for t, blocks in table.items() if blocks}
+
     def overwritten(buffer_type: str, index: int):
         origin[buffer_type].pop(index, None)
         produced[buffer_type].pop(index, None)
@@ -113,14 +115,21 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
     candidates: Dict[int, Dict[str, list]] = defaultdict(dict)
     for idx, instr in enumerate(instrs):
         if isinstance(instr, MemcpyInstr):
+            of_type = {}
+            fresh = copied[idx] = set()
             for pos, (src, dst) in enumerate(instr.src_dst_pairs):
-                dst_type, slot = dst.buffer_type, dst.index
-                produced[dst_type].pop(slot, None)
-                if _LOCAL_OF.get(dst_type) == src.buffer_type:
-                    origin[dst_type][slot] = (idx, pos, src.index, src.n_tokens)
-                    all_pairs.add((idx, pos))
-                else:
-                    origin[dst_type].pop(slot, None)
+                dst_type = dst.buffer_type
+                known = of_type.get(dst_type)
+                if known is None:
+                    known = of_type[dst_type] = _LOCAL_OF.get(dst_type), origin[dst_type], produced[dst_type]
+                local_type, copies, results = known
+                if results:
+                    results.pop(dst.index, None)
+                if src.buffer_type == local_type:
+                    copies[dst.index] = (idx, pos, src.index, src.n_tokens)
+                    fresh.add(pos)
+                elif copies:
+                    copies.pop(dst.index, None)
         elif isinstance(instr, (AttnInstr, AttnBackwardInstr)):
             q_local = local_rows(BufferType.BUFFER_Q, [row[:1] for row in instr.q_block_table])
             kv_local = local_rows(BufferType.BUFFER_KV, instr.kv_block_table)
@@ -148,10 +157,11 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
                     overwritten(row[0].buffer_type, row[0].index)
                     produced[row[0].buffer_type][row[0].index] = ("dq", idx, b)
                 # (who wrote a dK/dV replica is not asked for: none of them is moved to where it is read)
-                if any(produced.values()) or any(origin.values()):
+                known = with_entries()
+                if known:
                     for row in instr.dkv_block_table:
                         for blk in row:
-                            if produced[blk.buffer_type] or origin[blk.buffer_type]:
+                            if blk.buffer_type in known:
                                 overwritten(blk.buffer_type, blk.index)
         elif isinstance(instr, AttnReductionInstr):
             for pos, op in enumerate(instr.ops):
@@ -167,19 +177,19 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
                     produced[op.dst_buffer[0].buffer_type][op.dst_buffer[0].index] = ("merged", idx, pos)
         elif isinstance(instr, SumInstr):
             unpadded = bool(instr.output_is_unpadded)
+            known = with_entries()
             for pos, op in enumerate(instr.ops):
                 for blk in op.src_buffers:
-                    of_type = produced[blk.buffer_type]
-                    if of_type:
-                        who = of_type.get(blk.index)
+                    if blk.buffer_type in known:
+                        who = produced[blk.buffer_type].get(blk.index)
                         if who is not None:
                             readers[who].append((idx, pos, len(op.src_buffers), unpadded))
-                    if origin[blk.buffer_type]:
                         read_in_slot(blk)
                 if not unpadded:
                     dst = op.dst_buffer
                     overwritten(dst.buffer_type, dst.index)
                     produced[dst.buffer_type][dst.index] = ("summed", idx, pos)
+                    known.add(dst.buffer_type)
         else:  # an instruction this analysis does not know: leave the plan alone
             return DirectPlan()
 
@@ -221,6 +231,7 @@ def analyse(plan: ExecutionPlan) -> DirectPlan:
                     result.skip_ops.setdefault(hit[0], set()).add(hit[1])
 
     result.operands = {idx: ops for idx, ops in candidates.items() if ops}
-    for idx, pos in all_pairs - blocked:  # (a slot nobody reads is not worth filling either)
-        result.skip_pairs.setdefault(idx, set()).add(pos)
+    for idx, pos in blocked:
+        copied[idx].discard(pos)
+    result.skip_pairs = {idx: pairs for idx, pairs in copied.items() if pairs}  # (a slot nobody reads is not worth filling either)
     return result
