@@ -50,7 +50,7 @@ struct FwdPart {
 // A work item's queries (dcp_attn_fwd_items): 128 of a row, or a part of them as in FwdPart.  The other entry points
 // have as many items for a row as its block has tiles, whether the row has queries for them or not, and a
 // workgroup that draws one without spends 1.5-2 us on it (4476 tokens in sequences of 290 tokens and blocks of
-// 1024, 8 heads of size 64: 528 of 832 items are like that, the launch takes 31.7 us with and 17.5 without them).
+// 1024, 8 heads of size 64: 528 of 832 items are like that, the launch takes 31.6 us with and 13.9 without them).
 struct FwdTile {
   int row, q_tile, part_of, first_partial;  // part_of: part + 65536 * number of parts
 };

@@ -3,7 +3,7 @@
 A work item of the forward kernel -- 128 queries of one (row, head) -- walks its key tiles one after
 the other.  A launch whose items all find a workgroup slot at once lasts as long as its longest item,
 however idle the device is: 5120 tokens of 8 heads (352 items of 4 to 32 tiles on 512 slots, head size
-64) took 50 us, and take 30 in parts of up to 16 tiles and 5 for the kernel that adds them.
+64) take 31 us, and 26 in parts of up to 16 tiles, 5 of them for the kernel that adds those.
 """
 
 from __future__ import annotations

@@ -3,9 +3,9 @@
 An item is 128 queries of a row and one head.  The kernel can count them from the block size alone, but a row
 shorter than its block then has items without queries, and each costs a workgroup a ticket and a chain of table
 reads.  Forward (us) without and with a table of the items there are, by the share of them: 0.37 (4476 tokens in
-sequences of 290, blocks of 1024, 8 heads of size 64) 32.8 / 17.5; 0.52 (3477 tokens, 16 heads) 31.2 / 20.5; 5323
-tokens in sequences of 67 in two partials, 40 heads, 67.6 / 57.5; 0.87 (5269 tokens, 40 heads) 151.2 / 150.4; 0.98
-(12678 tokens, 8 heads) 100.2 / 103.5.
+sequences of 290, blocks of 1024, 8 heads of size 64) 31.6 / 13.9; 0.52 (3477 tokens, 16 heads) 32.1 / 16.8; 5323
+tokens in sequences of 67 in two partials, 40 heads, 76.9 / 44.9; 0.87 (5269 tokens, 40 heads) 149.9 / 149.6; 0.98
+(12678 tokens, 8 heads) between 100.2 / 103.5 and 95.9 / 94.7.
 """
 
 from __future__ import annotations
@@ -42,7 +42,7 @@ def deal_to_xcds(row: np.ndarray, n_kv_heads: int) -> np.ndarray:
 def pays(seqlens_q: Sequence[int], block_size: int, n_heads: int, n_slots: int, tile: int = 128) -> bool:
     """Whether few enough of the tiles that the blocks have room for hold queries, and not all of them find a
     workgroup slot at once (where they do, the table is only one more thing to read: 773 tokens of 8 heads
-    in blocks of 1024, 10.8 us without and 11.0 with it)."""
+    in blocks of 1024, 9.4 us without and 9.5 with it)."""
     used, room = sum(-(-n // tile) for n in seqlens_q), len(seqlens_q) * -(-block_size // tile)
     return 0 < used <= MAX_SHARE * room and room * n_heads > n_slots
 
@@ -51,11 +51,11 @@ def one_workgroup_each(seqlens_q: Sequence[int], seqlens_kv: Sequence[int], n_he
     """Whether a launch of more items than workgroup slots starts a workgroup for every item, instead of one per slot
     that takes item after item from a queue.  The queue wins by what it takes out of the gaps between workgroups,
     some 5 % of the launch, and costs a kernel that clears its counters, 4-5 us.  Forward (us) with and
-    without it, by key tiles (64) per slot: 36 and 27 (two launches; 15480 tokens, 8 heads) 200 / 183; 43 (12678
-    tokens, 8 heads) 103 / 96; 44 (18701 tokens) 81 / 75; 53 and 41 (two; 12926 tokens, size 64) 147 / 133; 53
-    (5323 tokens, 40 heads of 64) 57.8 / 46.1; 56 (7604 tokens, 40 heads) 119 / 112; 98 (5269 tokens, 40 heads) 151 /
-    154; 103 (16384 tokens, 16 heads) 196 / 205; 122 (28012 tokens, 32 heads) 336 / 367; 183 (32768 tokens, 8
-    heads) 338 / 354; 2297 (65536 tokens, 32 heads) 3744 / 4007."""
+    without it, by key tiles (64) per slot: 36 and 27 (two launches; 15480 tokens, 8 heads) 183 / 170; 43 (12678
+    tokens, 8 heads) 103 / 96; 44 (18701 tokens) 76 / 65; 53 and 41 (two; 12926 tokens, size 64) 145 / 129; 53
+    (5323 tokens, 40 heads of 64) 56.9 / 44.0; 56 (7604 tokens, 40 heads) 114 / 109; 98 (5269 tokens, 40 heads) 149 /
+    152; 103 (16384 tokens, 16 heads) 197 / 199; 122 (28012 tokens, 32 heads) 348 / 363; 183 (32768 tokens, 8
+    heads) 340 / 356; 2297 (65536 tokens, 32 heads) 3762 / 3933."""
     items = [-(-n // tile) for n in seqlens_q]
     return (sum(items) * n_heads > n_slots
             and sum(n * -(-k // 64) for n, k in zip(items, seqlens_kv)) * n_heads <= MAX_TILES_WITHOUT_QUEUE * n_slots)
