@@ -97,9 +97,8 @@ class RecordedTurns:
     and takes 1810, which are the kernels'.  Holds nothing of the executors; ``fits`` says whether all is still as it
     was.  The events are its own: a pass in turns makes new ones."""
 
-    def __init__(self, executors, plans, turns: List[Tuple[int, int]]):
+    def __init__(self, executors, turns: List[Tuple[int, int]]):
         self._executors = [weakref.ref(ex) for ex in executors]
-        self._plans = [weakref.ref(plan) for plan in plans]
         self._tokens = [ex.steps_token() for ex in executors]
         self._epoch = executors[0].fabric.epoch
         self._turns = turns
@@ -112,13 +111,13 @@ class RecordedTurns:
         """None where some instruction does more than the library's calls, or an executor is not one of this package's."""
         if not all(hasattr(ex, "turns_are_recordable") and ex.turns_are_recordable(plan) for ex, plan in zip(executors, plans)):
             return None
-        return RecordedTurns(executors, plans, turns)
+        return RecordedTurns(executors, turns)
 
     def fits(self, executors, plans) -> bool:
         return (len(executors) == len(self._executors)
                 and all(ref() is ex for ref, ex in zip(self._executors, executors))
-                and all(ref() is plan for ref, plan in zip(self._plans, plans))
                 and self._epoch == executors[0].fabric.epoch
+                # (the plans are those of the first pass where the token is the same and the steps are the plan's)
                 and all(ex.steps_token() == token and ex.turns_are_recordable(plan)
                         for ex, plan, token in zip(executors, plans, self._tokens))
                 and (self._sequence is not None or self._make(executors)))
