@@ -89,6 +89,15 @@ class LocalFabric:
         return min(self._barrier_arrivals) >= generation
 
 
+# what a pass in turns calls on the fabric
+_PASS_METHODS = {name: vars(LocalFabric)[name] for name in ("post", "posted", "take", "consumed", "set_consumed")}
+
+
+def methods_are(obj, methods) -> bool:
+    """Are these (name -> function) still what the object calls by these names, whatever a subclass or a caller did?"""
+    return all(getattr(getattr(obj, name), "__func__", None) is function for name, function in methods.items())
+
+
 class RecordedTurns:
     """What ``execute_together`` does in a pass, done again in one library call: the recorded calls of the devices'
     instructions on their streams and the events by which they wait for each other, in the order in which the
@@ -108,7 +117,10 @@ class RecordedTurns:
 
     @staticmethod
     def of(executors, plans, turns) -> Optional["RecordedTurns"]:
-        """None where some instruction does more than the library's calls, or an executor is not one of this package's."""
+        """None where some instruction does more than the library's calls, or where an executor or the fabric has methods of
+        the caller's own: a pass in turns calls them."""
+        if not methods_are(executors[0].fabric, _PASS_METHODS):
+            return None
         if not all(hasattr(ex, "turns_are_recordable") and ex.turns_are_recordable(plan) for ex, plan in zip(executors, plans)):
             return None
         return RecordedTurns(executors, turns)
@@ -116,7 +128,7 @@ class RecordedTurns:
     def fits(self, executors, plans) -> bool:
         return (len(executors) == len(self._executors)
                 and all(ref() is ex for ref, ex in zip(self._executors, executors))
-                and self._epoch == executors[0].fabric.epoch
+                and self._epoch == executors[0].fabric.epoch and methods_are(executors[0].fabric, _PASS_METHODS)
                 # (the plans are those of the first pass where the token is the same and the steps are the plan's)
                 and all(ex.steps_token() == token and ex.turns_are_recordable(plan)
                         for ex, plan, token in zip(executors, plans, self._tokens))

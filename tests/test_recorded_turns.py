@@ -73,8 +73,43 @@ def devices(monkeypatch):
     return executors
 
 
+def _counted(calls, inner):
+    def counted(*args):
+        calls.append(args)
+        return inner(*args)
+
+    return counted
+
+
 def test_passes_after_the_first_are_one_call(devices):
     """(Of plans of any type: these cannot be weakly referenced.)"""
     for turn in range(3):
         fabric.execute_together(devices)
         assert _Sequence.runs == turn
+
+
+@pytest.mark.parametrize("passes_before", [0, 2])
+@pytest.mark.parametrize("how", ["instance", "subclass", "class"])
+@pytest.mark.parametrize("name", ["begin", "step", "finish", "comm_ready", "post", "posted", "take", "consumed", "set_consumed"])
+def test_methods_of_the_callers_own_run_in_every_pass(devices, monkeypatch, name, how, passes_before):
+    """A pass in turns calls them, so a caller may put something of their own in their place, at the start or later."""
+    for _ in range(passes_before):
+        fabric.execute_together(devices)
+    targets, calls = [devices[0].fabric] if hasattr(fabric.LocalFabric, name) else devices, []
+    kind = type(targets[0])
+    if how == "instance":
+        for target in targets:
+            setattr(target, name, _counted(calls, getattr(target, name)))
+    elif how == "subclass":
+        own = type("Own", (kind,), {name: _counted(calls, getattr(kind, name))})
+        for target in targets:
+            target.__class__ = own
+    else:
+        monkeypatch.setattr(kind, name, _counted(calls, getattr(kind, name)))
+    _Sequence.runs = 0
+    fabric.execute_together(devices)
+    in_a_pass = len(calls)
+    assert in_a_pass > 0
+    for _ in range(2):
+        fabric.execute_together(devices)
+    assert len(calls) == 3 * in_a_pass and _Sequence.runs == 0
