@@ -132,7 +132,7 @@ class RecordedTurns:
                 # (the plans are those of the first pass where the token is the same and the steps are the plan's)
                 and all(ex.steps_token() == token and ex.turns_are_recordable(plan)
                         for ex, plan, token in zip(executors, plans, self._tokens))
-                and (self._sequence is not None or self._make(executors)))
+                and (self._sequence is not None or self._make(executors, plans)))
 
     def _event(self, stream) -> torch.cuda.Event:
         event = torch.cuda.Event()
@@ -140,9 +140,9 @@ class RecordedTurns:
         self._events.append(event)
         return event
 
-    def _make(self, executors) -> bool:
+    def _make(self, executors, plans) -> bool:
         RUN, RECORD, WAIT = _lib.Sequence.RUN, _lib.Sequence.RECORD, _lib.Sequence.WAIT
-        steps = [(rank, executors[rank].recorded_step(i)) for rank, i in self._turns]
+        steps = [(rank, executors[rank].recorded_step(plans[rank], i)) for rank, i in self._turns]
         launches = [(rank, step["key"]) for rank, step in steps if step and step["kind"] == "launch"]
         received = {(rank, step["key"]) for rank, step in steps if step and step["kind"] == "wait" and step["peers"]}
         if (any(step is None for _, step in steps) or len(set(launches)) < len(launches)

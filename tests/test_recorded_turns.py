@@ -113,3 +113,15 @@ def test_methods_of_the_callers_own_run_in_every_pass(devices, monkeypatch, name
     for _ in range(2):
         fabric.execute_together(devices)
     assert len(calls) == 3 * in_a_pass and _Sequence.runs == 0
+
+
+def test_a_pass_of_another_plan_between_the_first_and_the_second(devices):
+    """The calls are those of the plan that the devices run together, whatever a device ran by itself last."""
+    fabric.execute_together(devices)
+    for ex in devices:
+        ex.cuda_graph, ex._recorded, ex.return_values = None, None, {}
+        with pytest.raises(KeyError, match="LocalOut"):  # (what a pass returns: these executors have no buffers)
+            ex.execute(SimpleNamespace(instructions=[], buffer_info={}))
+    fabric.execute_together(devices)
+    assert _Sequence.runs == 1
+    assert [what for _, what in _Sequence.made[0]] == [ex._recorded_steps[0][0] for ex in devices]  # the two gathers
