@@ -219,7 +219,7 @@ def _flash_attn_varlen_forward(
     ``parts`` (extension): ``(parts, splits, n_partials, partials)``, rows split along their keys
     (``dcp_attn_fwd_parts``): int32 ``[entries, 4]`` and ``[split rows, 4]``, and fp32 scratch.
     ``items`` (extension): the launch's work items, int32 ``[n, 4]`` (``dcp_attn_fwd_items``; with ``parts``, whose
-    entries they then stand for).
+    entries they then stand for).  Without rows: no work, and nothing is launched or written.
     ``one_each`` (extension, not with ``parts`` alone): a workgroup for every work item (``dcp_attn_fwd_items``).
     """
     _check_plain(dropout_p, causal, window_size_left, window_size_right, softcap,
@@ -280,6 +280,8 @@ def _flash_attn_varlen_forward(
     if items is not None and (items.dim() != 2 or items.shape[1] != 4):
         raise ValueError(f"items must be [n, 4], got {tuple(items.shape)}")
     n_items, table = (0, 0) if items is None else (items.shape[0], _i32(items, "items").data_ptr())
+    if items is not None and n_items == 0 and (parts is None or parts[1].shape[0] == 0):
+        return out_, lse_, None, None  # (to the library a table without an address is none: all tiles of the rows)
     if parts is None and items is None and not one_each:
         _lib.call("dcp_attn_fwd_strided", *args, _stream())
     elif parts is None:

@@ -9,6 +9,7 @@ import torch
 
 from dcp_amd.runtime.flash_attention import executor, fwd_parts, items
 from tests.plan_cases import check_against_truth, dense_truth, make_case, run_executor
+from tests.test_attention_direct_gpu import _paged_rows
 from tests.test_dkv_groups import PLANS
 
 
@@ -80,3 +81,29 @@ def test_a_workgroup_each(gpu, monkeypatch, name, listed):
     assert torch.equal(queued[0], each[0]) and torch.equal(queued[1], each[1])
     replayed, _ = run_executor(case, backward=False, use_graph=True)
     assert torch.equal(each[0], replayed[0]) and torch.equal(each[1], replayed[1])
+
+
+def _rows(gpu):
+    """Four rows of up to 300 queries in blocks of 512 and 1 to 3 blocks of keys; four q heads, two kv heads."""
+    rng = np.random.default_rng(3)
+    rows = [(nq, nblk, np.stack([np.zeros(nq), rng.integers(1, nblk * 512, size=nq)])[None]) for nq, nblk in ((300, 3), (128, 1), (1, 2), (130, 1))]
+    return _paged_rows(gpu, rows, 512, 4, 2, 64, seed=2)
+
+
+def _forward(pr, **options):
+    from dcp_amd.flash_attn_interface import _flash_attn_varlen_forward
+
+    q, kv, slots = pr["q"], pr["kv"], pr["slots"]
+    out, lse = torch.full_like(q, 3.0), torch.full((q.shape[2], q.shape[0], pr["bs"]), 3.0, device=q.device)
+    _flash_attn_varlen_forward(q, kv[:, :, 0], kv[:, :, 1], pr["cu_q"], pr["cu_kv"], pr["total_q"], pr["bs"], pr["max_kv"] * pr["bs"], 0.0,
+                               q.shape[-1] ** -0.5, attn_range=pr["rng"], q_block_table=slots, kv_block_table=pr["kv_table"],
+                               out_block_table=slots, out_=out, lse_=lse, **options)
+    torch.cuda.synchronize()
+    return out, lse
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("one_each", [False, True])
+def test_an_empty_table_is_no_work(gpu, one_each):
+    out, lse = _forward(_rows(gpu), items=torch.zeros((0, 4), dtype=torch.int32, device=gpu), one_each=one_each)
+    assert (out == 3.0).all() and (lse == 3.0).all()
