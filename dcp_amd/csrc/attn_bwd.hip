@@ -423,6 +423,11 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       const RangePair ranges = {s0, max(e0 - s0, 0), s1, max(e1 - s1, 0)};
       const uint32_t closed = ranges.closed_window(visit_lds[visit].k_row + w * 32);
       closed_lds[w][q] = qt * BM + q < seqlen_q ? closed : 0xffffffffu;
+      // Other lanes of the wave read it below.  The LDS serves a wave's accesses in order, so nothing has to be
+      // waited for, but the compiler must not take the reads before the store: these emit no instruction.
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 
     // One sub-step = this wave's 32 keys against 32 of the step's 64 queries (QI = 0, 1).
