@@ -71,11 +71,13 @@ __global__ __launch_bounds__(64) void bwd_tile_hull_kernel(const AttnBwdParams p
   int s0 = 0, l0 = 0, s1 = 0, l1 = 0;
   if (ql < seqlen_q) {
     const int32_t* r = p.attn_range + q_begin + ql;
-    s0 = r[0];
-    l0 = max(min(r[p.total_q], seqlen_kv) - s0, 0);
+    const KeyRange range0 = key_range(r[0], r[p.total_q], seqlen_kv);
+    s0 = range0.start;
+    l0 = range0.len;
     if (p.n_ranges == 2) {
-      s1 = r[2 * (int64_t)p.total_q];
-      l1 = max(min(r[3 * (int64_t)p.total_q], seqlen_kv) - s1, 0);
+      const KeyRange range1 = key_range(r[2 * (int64_t)p.total_q], r[3 * (int64_t)p.total_q], seqlen_kv);
+      s1 = range1.start;
+      l1 = range1.len;
     }
   }
   const int big = 0x7fffffff;
@@ -418,9 +420,9 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     if (!unmasked) {
       const int q = lane_here(), seqlen_kv = visit_lds[visit].seqlen_kv;
       // (with one range the second range's planes hold the first's again: the union is the same)
-      const int s0 = rng_lds[st][0][q], e0 = min(rng_lds[st][1][q], seqlen_kv);
-      const int s1 = rng_lds[st][2][q], e1 = min(rng_lds[st][3][q], seqlen_kv);
-      const RangePair ranges = {s0, max(e0 - s0, 0), s1, max(e1 - s1, 0)};
+      const KeyRange range0 = key_range(rng_lds[st][0][q], rng_lds[st][1][q], seqlen_kv);
+      const KeyRange range1 = key_range(rng_lds[st][2][q], rng_lds[st][3][q], seqlen_kv);
+      const RangePair ranges = {range0.start, range0.len, range1.start, range1.len};
       const uint32_t closed = ranges.closed_window(visit_lds[visit].k_row + w * 32);
       closed_lds[w][q] = qt * BM + q < seqlen_q ? closed : 0xffffffffu;
       // Other lanes of the wave read it below.  The LDS serves a wave's accesses in order, so nothing has to be
@@ -740,13 +742,13 @@ __device__ __forceinline__ void attn_bwd_dq_item(KernArgs<AttnBwdParams>& p, int
   RangePair rng = {0, 0, 0, 0};
   if (q_valid) {
     const int32_t* r = p.attn_range + q_begin + q_local;
-    const int s0 = r[0], e0 = min(r[p.total_q], seqlen_kv);
-    rng.s0 = s0;
-    rng.len0 = max(e0 - s0, 0);
+    const KeyRange range0 = key_range(r[0], r[p.total_q], seqlen_kv);
+    rng.s0 = range0.start;
+    rng.len0 = range0.len;
     if (p.n_ranges == 2) {
-      const int s1 = r[2 * (int64_t)p.total_q], e1 = min(r[3 * (int64_t)p.total_q], seqlen_kv);
-      rng.s1 = s1;
-      rng.len1 = max(e1 - s1, 0);
+      const KeyRange range1 = key_range(r[2 * (int64_t)p.total_q], r[3 * (int64_t)p.total_q], seqlen_kv);
+      rng.s1 = range1.start;
+      rng.len1 = range1.len;
     }
   }
   const int big = 0x7fffffff;

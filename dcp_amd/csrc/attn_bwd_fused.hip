@@ -95,11 +95,13 @@ __global__ __launch_bounds__(kBwdThreads) void bwd_prepare_kernel(const AttnBwdP
     int s0 = 0, l0 = 0, s1 = 0, l1 = 0;
     if (ql < seqlen_q) {
       const int32_t* r = p.attn_range + q_begin + ql;
-      s0 = r[0];
-      l0 = max(min(r[p.total_q], seqlen_kv) - s0, 0);
+      const KeyRange range0 = key_range(r[0], r[p.total_q], seqlen_kv);
+      s0 = range0.start;
+      l0 = range0.len;
       if (p.n_ranges == 2) {
-        s1 = r[2 * (int64_t)p.total_q];
-        l1 = max(min(r[3 * (int64_t)p.total_q], seqlen_kv) - s1, 0);
+        const KeyRange range1 = key_range(r[2 * (int64_t)p.total_q], r[3 * (int64_t)p.total_q], seqlen_kv);
+        s1 = range1.start;
+        l1 = range1.len;
       }
     }
     const int big = 0x7fffffff;

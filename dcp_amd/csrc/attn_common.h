@@ -494,8 +494,19 @@ struct TileCursor {
   }
 };
 
+// The keys [start, end) of a row that has seqlen_kv of them: the first one and how many.  Both ends are cut
+// before the difference is taken, which does not fit an int where a range is open to the left or empty by way
+// of the type's lowest value; and a start below zero would name key tiles before the row's first.
+struct KeyRange {
+  int start, len;
+};
+__device__ __forceinline__ KeyRange key_range(int start, int end, int seqlen_kv) {
+  const int s = min(max(start, 0), seqlen_kv);
+  return {s, max(min(end, seqlen_kv), s) - s};
+}
+
 struct RangePair {
-  int s0, len0, s1, len1;  // start and (non-negative) length of each range
+  int s0, len0, s1, len1;  // of each range, see KeyRange
   __device__ __forceinline__ bool contains(int k) const {
     return ((unsigned)(k - s0) < (unsigned)len0) | ((unsigned)(k - s1) < (unsigned)len1);
   }

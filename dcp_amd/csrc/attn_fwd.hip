@@ -212,13 +212,13 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
     RangePair r4 = {0, 0, 0, 0};
     if (q_valid[qb]) {
       const int32_t* r = p.attn_range + q_begin + q_local[qb];
-      const int s0 = r[0], e0 = min(r[p.total_q], seqlen_kv);
-      r4.s0 = s0;
-      r4.len0 = max(e0 - s0, 0);
+      const KeyRange range0 = key_range(r[0], r[p.total_q], seqlen_kv);
+      r4.s0 = range0.start;
+      r4.len0 = range0.len;
       if (p.n_ranges == 2) {
-        const int s1 = r[2 * (int64_t)p.total_q], e1 = min(r[3 * (int64_t)p.total_q], seqlen_kv);
-        r4.s1 = s1;
-        r4.len1 = max(e1 - s1, 0);
+        const KeyRange range1 = key_range(r[2 * (int64_t)p.total_q], r[3 * (int64_t)p.total_q], seqlen_kv);
+        r4.s1 = range1.start;
+        r4.len1 = range1.len;
       }
     }
     rng[qb] = r4;

@@ -219,6 +219,8 @@ int dcp_blockwise_sum_fp32_sources(
  * attn_range is int32 [n_ranges, 2, total_q]: query token t (global index
  * cu_seqlens_q[b]+i) attends kv positions in the union of
  * [attn_range[r][0][t], attn_range[r][1][t]).
+ * (A range may begin before key 0 or end past the row's last key, at any value of
+ * its type: the keys that there are count.  One that does not end past its start is empty.)
  * Writes out ([n_out_slots, block_size, n_heads_q, head_dim]) at slot
  * out_block_table[b] and lse (fp32 [n_heads_q, n_out_slots, block_size]) at the
  * same slot.  Rows with no visible key: out = 0, lse = +inf.
