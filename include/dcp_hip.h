@@ -345,7 +345,8 @@ int dcp_attn_fwd_parts(const void* q, const void* k, const void* v, void* out,
  * has no queries are not listed, and cost nothing.  items null (and n_items and
  * n_splits 0): all tiles of the rows, as dcp_attn_fwd_strided.
  *   one_each: nonzero = a workgroup for every item from the start (the workspace is then
- *     not used); 0 = as many as the device holds at once, which take item after item.
+ *     not written, but must be there all the same); 0 = as many as the device holds at
+ *     once, which take item after item.
  */
 int dcp_attn_fwd_items(const void* q, const void* k, const void* v, void* out,
                        float* lse, const int32_t* cu_seqlens_q,

@@ -63,6 +63,67 @@ def test_argument_errors_are_reported_without_a_launch(lib):
     assert lib.dcp_attn_bwd_workspace_bytes(2, 128, 64, 4, 128) >= 128 * 4 * 4 + 2 * 8 * 4
 
 
+def _items_call(items=16, n_items=1, one_each=0, splits=0, n_splits=0, n_partials=0, partials=0, partials_bytes=0,
+                workspace=16, workspace_bytes=64):
+    """One row of 64-token blocks; the addresses are not read before the arguments have been checked."""
+    from dcp_amd import _lib
+
+    _lib.call("dcp_attn_fwd_items", *([16] * 8), 1, *([16] * 3), 0, 1, 1, 64, 64, 1, 1, 64, 64 * 64, 64, 64 * 64, 64 * 64, 64, 64, 0, 1.0, 0,
+              workspace, workspace_bytes, items, n_items, one_each, splits, n_splits, n_partials, partials, partials_bytes, 0)
+
+
+@pytest.mark.parametrize("wrong,message", [
+    (dict(items=24), "not 16-byte aligned"),
+    (dict(n_items=0), "no items"),
+    (dict(n_items=-1), "no items"),
+    (dict(items=0), "no table of items"),
+    (dict(items=0, n_items=0, splits=16, n_splits=1, n_partials=2, partials=16, partials_bytes=1 << 20), "no table of items"),
+    (dict(n_splits=1, n_partials=1), "do not fit"),
+    (dict(n_splits=2, n_partials=4), "do not fit"),
+    (dict(n_splits=-1), "do not fit"),
+    (dict(n_splits=1, n_partials=2), "partials are missing"),
+    (dict(splits=16, n_splits=1, n_partials=2, partials=24, partials_bytes=1 << 20), "partials are missing"),
+    (dict(splits=16, n_splits=1, n_partials=2, partials=16, partials_bytes=2 * 128 * 66 * 4 - 1), "partials are missing"),
+    (dict(workspace=0), "workspace"),
+    (dict(workspace=0, one_each=1), "workspace"),
+    (dict(workspace_bytes=63, one_each=1), "workspace"),
+])
+def test_tables_of_items_that_are_refused(lib, wrong, message):
+    with pytest.raises(AssertionError, match=message):
+        _items_call(**wrong)
+
+
+def test_sequences_that_are_refused(lib):
+    from dcp_amd import _lib
+
+    recording = _lib.Recording()
+    assert recording.begin()
+    _lib.call("dcp_fused_copy_varlen", 0, 0, 0, 0, 0, 0, 0, 0, 16, 2, 0)  # (nothing to copy: returns before it launches)
+    recording.end()
+    run = dict(kind=_lib.Sequence.RUN, list=recording._list, end=1)
+
+    def sequence(*ops):
+        _lib.call("dcp_sequence_run", (_lib._SequenceOp * len(ops))(*(_lib._SequenceOp(**op) for op in ops)), len(ops), 0)
+
+    sequence()
+    _lib.call("dcp_sequence_run", None, 0, 0)
+    sequence(run, dict(run, begin=1))
+    for ops, message in [
+        ([dict(run, list=None)], "null list"),
+        ([dict(run, end=2)], "calls 0 to 2 of 1"),
+        ([dict(run, begin=-1)], "calls -1 to 1 of 1"),
+        ([run, dict(kind=3, event=16)], "operation 1 is of kind 3"),
+        ([dict(kind=-1, event=16)], "operation 0 is of kind -1"),
+        ([dict(kind=_lib.Sequence.RECORD)], "operation 0 is of kind 1, event"),
+        ([run, run, dict(kind=_lib.Sequence.WAIT)], "operation 2 is of kind 2, event"),
+    ]:
+        with pytest.raises(AssertionError, match=message):
+            sequence(*ops)
+    for n_ops in (1, -1):
+        with pytest.raises(AssertionError, match="no operations"):
+            _lib.call("dcp_sequence_run", None, n_ops, 0)
+
+
 def test_workspaces_have_the_sizes_callers_know(lib):
     """A caller may have its buffers before it asks, for the backward two floats per (query, head), a hull of
     32 bytes per 64-query tile, each rounded up to 256 bytes, and 256 bytes of counters.  A problem

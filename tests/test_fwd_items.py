@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+from dcp_amd.core.instructions import AttnInstr
 from dcp_amd.runtime.flash_attention import executor, fwd_parts, items
 from tests.plan_cases import check_against_truth, dense_truth, make_case, run_executor
 from tests.test_attention_direct_gpu import _paged_rows
@@ -51,6 +52,11 @@ def test_rule_of_the_queue():
     assert each([128] * 128, [64 * 32] * 128, 8, 512) and not each([128] * 128, [64 * 32 + 1] * 128, 8, 512)
 
 
+def _launches(ex, case):
+    """The forward launches' parts, items and whether a workgroup is started for each."""
+    return [ex._args_cache[i][-4:-1] for i, instr in enumerate(case["fw"].instructions) if isinstance(instr, AttnInstr)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("share", [None, 2])
 @pytest.mark.parametrize("name", list(PLANS))
@@ -58,9 +64,13 @@ def test_same_results(gpu, monkeypatch, name, share):
     case = make_case(**PLANS[name])
     if share:
         monkeypatch.setattr(fwd_parts, "share_of_a_part", lambda *a: share)
-    counted, _ = run_executor(case, backward=False)
+    monkeypatch.setattr(executor, "items_pay", lambda *a: False)
+    counted, ex = run_executor(case, backward=False)
+    assert all(items is None for _, items, _ in _launches(ex, case))
     monkeypatch.setattr(executor, "items_pay", lambda *a: True)
-    listed, _ = run_executor(case, backward=False, poison=200.0)
+    listed, ex = run_executor(case, backward=False, poison=200.0)
+    assert all(items is not None for _, items, _ in _launches(ex, case))
+    assert share is None or any(parts is not None for parts, _, _ in _launches(ex, case))
     assert torch.equal(counted[0], listed[0]) and torch.equal(counted[1], listed[1])
     check_against_truth(listed, dense_truth(case, backward=False))
     replayed, _ = run_executor(case, backward=False, use_graph=True)
@@ -75,9 +85,14 @@ def test_a_workgroup_each(gpu, monkeypatch, name, listed):
     case = make_case(**dict(PLANS[name], seqlens=PLANS[name]["seqlens"] * 40))
     monkeypatch.setattr(executor, "one_workgroup_each", lambda *a: False)
     monkeypatch.setattr(executor, "items_pay", lambda *a: listed)
-    queued, _ = run_executor(case, backward=False)
+    queued, ex = run_executor(case, backward=False)
+    slots = 2 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    for instr in case["fw"].instructions:
+        assert not isinstance(instr, AttnInstr) or sum(-(-row[0].n_tokens // 128) for row in instr.q_block_table) * case["head_block"] > slots
+    assert all(parts is None and (items is not None) == listed and not one_each for parts, items, one_each in _launches(ex, case))
     monkeypatch.setattr(executor, "one_workgroup_each", lambda *a: True)
-    each, _ = run_executor(case, backward=False, poison=200.0)
+    each, ex = run_executor(case, backward=False, poison=200.0)
+    assert all(parts is None and (items is not None) == listed and one_each for parts, items, one_each in _launches(ex, case))
     assert torch.equal(queued[0], each[0]) and torch.equal(queued[1], each[1])
     replayed, _ = run_executor(case, backward=False, use_graph=True)
     assert torch.equal(each[0], replayed[0]) and torch.equal(each[1], replayed[1])
@@ -107,3 +122,24 @@ def _forward(pr, **options):
 def test_an_empty_table_is_no_work(gpu, one_each):
     out, lse = _forward(_rows(gpu), items=torch.zeros((0, 4), dtype=torch.int32, device=gpu), one_each=one_each)
     assert (out == 3.0).all() and (lse == 3.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("one_each", [False, True])
+def test_the_launch_is_its_table(gpu, one_each):
+    """Queries whose 128 are left out of the table are not written, the others are those of a launch without one."""
+    pr = _rows(gpu)
+    want = _forward(pr, one_each=one_each)
+    table = items.forward_items([nq for nq, _, _ in pr["rows"]], [nblk * 512 for _, nblk, _ in pr["rows"]], 2)
+    left_out = [(0, 1), (2, 0), (3, 0)]  # (row, which 128 of its queries)
+    table = table[[(row, tile) not in left_out for row, tile, _, _ in table.tolist()]]
+    got = _forward(pr, items=torch.from_numpy(table).to(gpu), one_each=one_each)
+    for row, (nq, _, _) in enumerate(pr["rows"]):
+        for tile in range(-(-nq // 128)):
+            here = slice(tile * 128, min(tile * 128 + 128, nq))
+            written = (want[0][row, here], want[1][:, row, here])
+            found = (got[0][row, here], got[1][:, row, here])
+            if (row, tile) in left_out:
+                assert all((t == 3.0).all() for t in found)
+            else:
+                assert all(torch.equal(a, b) for a, b in zip(found, written))

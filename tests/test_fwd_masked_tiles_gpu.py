@@ -40,3 +40,26 @@ def test_masked_tiles_after_whole_ones(gpu, d, hq, hkv, n_ranges, empty, scale):
     assert worst["out"] <= OUT_TOL and worst["lse"] <= (LSE_TOL if scale == 1.0 else 2e-3)
     if scale == 1.0:
         assert worst["dq"] <= GRAD_TOL and worst["dkv"] <= GRAD_TOL
+
+
+@pytest.mark.parametrize("n_ranges", [1, 2])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_a_query_that_is_not_finite_keeps_to_itself(gpu, value, n_ranges):
+    """The weights of its wave are checked and taken again at every tile; the queries beside it are as accurate as
+    ever, and one that sees nothing has out = 0 and lse = +inf whatever its q holds."""
+    rng, bs = np.random.default_rng(7), 128
+    rows = [(nq, nblk, _ranges(rng, nq, nblk * bs, n_ranges, 0.2)) for nq, nblk in ((128, 3), (70, 2))]
+    pr = _paged_rows(gpu, rows, bs, 4, 2, 128, seed=4)
+    want = _run_direct(pr, backward=False)
+    spoilt = [(b, i) for b, (nq, _, ranges) in enumerate(rows) for i in range(5, nq, 17) if (ranges[:, 1, i] > ranges[:, 0, i]).any()]
+    nothing = [(b, i) for b, (nq, _, ranges) in enumerate(rows) for i in range(nq) if not (ranges[:, 1, i] > ranges[:, 0, i]).any()]
+    assert spoilt and nothing
+    for b, i in spoilt + nothing:
+        pr["q"][b, i, :, ::3] = value
+    got = _run_direct(pr, backward=False)
+    for b, i in nothing:
+        assert (got[0][b, i] == 0).all() and np.isposinf(got[1][:, b, i]).all()
+    for b, i in spoilt:
+        got[0][b, i], got[1][:, b, i] = want[0][b, i], want[1][:, b, i]
+    worst = _check_direct(pr, got)
+    assert worst["out"] <= OUT_TOL and worst["lse"] <= LSE_TOL
