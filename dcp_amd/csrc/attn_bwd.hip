@@ -416,7 +416,8 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     // mask that the lanes, which hold a key each, read back for their sixteen queries at a time.  Every lane
     // testing its key against every query's ranges was ten instructions an element, 320 a step, behind 32
     // reads of LDS.  Backward, us: 5269 tokens in shared prefixes, 40 heads, 685 -> 522; 12678 tokens, 8 heads,
-    // 341 -> 293; 4128 tokens 128 -> 111; 131072 tokens, window 4096, 21930 -> 21740; 65536 causal 11400 -> 11340.
+    // 341 -> 293; 4128 tokens 128 -> 111; 131072 tokens, window 4096, 21930 -> 21740; 65536 causal 11440 -> 11370
+    // (runs of one build differ by 50).
     if (!unmasked) {
       const int q = lane_here(), seqlen_kv = visit_lds[visit].seqlen_kv;
       // (with one range the second range's planes hold the first's again: the union is the same)

@@ -206,7 +206,7 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
   RangePair rng[QB];
   const int big = 0x7fffffff;
   int w_lo0 = big, w_hi0 = 0, w_lo1 = big, w_hi1 = 0;            // hull: what any row of the wave can see
-  int core_lo0 = 0, core_hi0 = big, core_lo1 = 0, core_hi1 = big;  // core: what every row sees
+  int core_lo0 = 0, core_hi0 = big, core_lo1 = 0, core_hi1 = big;  // core: what every row sees that sees anything
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     RangePair r4 = {0, 0, 0, 0};
@@ -518,7 +518,7 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
   bool cur_full = false;           // list entry j lies inside every row's range
   bool raw = false;                // its S^T still lacks the range mask (the fast path multiplies without)
   bool pending = false;            // the maximum step of list entry j has been done already
-  bool anchored = false;           // every row of the wave has a (finite) reference maximum
+  bool anchored = false;           // every row of the wave that sees anything has a (finite) reference maximum
   auto iteration = [&](int j, f32x16 (&s_cur)[2][QB], f32x16 (&s_nxt)[2][QB], const uint16_t* k_nxt, uint32_t k_fill,
                        const uint16_t* v_cur, uint32_t v_fill) {
     __builtin_amdgcn_s_waitcnt(0);
@@ -531,9 +531,9 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
     const bool nxt_full = j + 1 < n_tiles && tile_is_full(tile_nxt);
     // Tiles that some rows see in part take the pipelined path too, and the mask is added to their S^T when it is
     // consumed (`raw`).  On the path below they cost a product, a maximum and a softmax one after the other, in every
-    // wave of a workgroup that meets at each tile.  Where many tiles are masked that was up to a third of the launch
-    // (32 000 tokens in short sequences, blocks of 1024: 84 -> 64 us; 4476 tokens in sequences of 290: 17.3 -> 13.5);
-    // under a causal mask over 64 k tokens, where few are, 3701 -> 3651.  The tests for it stay out of an iteration
+    // wave of a workgroup that meets at each tile.  Forward, us, without and with this: 1000 tokens 15.4 -> 13.7; 4476
+    // tokens in sequences of 290 17.3 -> 13.5; 32 000 tokens in short sequences, blocks of 1024, 73.8 -> 64.4; under a
+    // causal mask over 64 k tokens, where few tiles are masked, 3709 -> 3689.  The tests for it stay out of an iteration
     // between two whole tiles; a test of every row's reference in each iteration below cost 3-4 % of every launch.
     bool cur = true, nxt = nxt_full, fast = cur_full && nxt_full && anchored;
     if (__builtin_expect(!fast, 0)) {
@@ -547,7 +547,8 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
     }
     if (__builtin_expect(fast, 1)) {
       // The common case, decided by one test per iteration where this tile and the next are inside
-      // every row's range: the wave sees both and every row has a reference maximum.  The weights are taken relative
+      // every row's range: the wave sees both and every row has a reference maximum (one that sees nothing may not:
+      // its zero Q gives it weights of 1 against the 0 that softmax_max left in its m_use).  The weights are taken relative
       // to that reference WITHOUT looking at the tile's own maximum first ...
       if (!pending) {
 #pragma unroll

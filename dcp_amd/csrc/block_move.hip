@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kCopyThreads) void copy_varlen_kernel(
   const int p = blockIdx.x / chunks_per_block;
   const int c = blockIdx.x - p * chunks_per_block;
   // In one-wave workgroups all the tables' words of the block in one trip, before anything depends on one of
-  // them: 4 MiB blocks 6.67 -> 6.77 TB/s (2 GiB there and back 1288 -> 1269 us).  Larger workgroups, of which the
+  // them: 4 MiB blocks 6.67 -> 6.79 TB/s (2 GiB there and back 1287 -> 1265 us).  Larger workgroups, of which the
   // ones past a ragged block's end leave at once, are better off with its length alone first (blocks of up
   // to 640 KiB, 16.5 us and 16.9 with all words).
   const int32_t count = n_count[p];

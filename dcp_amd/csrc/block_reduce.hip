@@ -602,7 +602,7 @@ __global__ __launch_bounds__(THREADS) void blockwise_sum_kernel(
   constexpr int WORDS = VN / Vec16<SRC>::N;  // 16-byte words of a source per word of the result
   const int s = blockIdx.x / chunks_per_sum;
   // All the tables' words of the sum in one trip, up to four of its sources among them (as in copy_varlen_kernel):
-  // 8192 ragged tokens of 8 heads, three sources, 8.3 -> 8.0 us
+  // 8192 ragged tokens of 8 heads, three sources, 8.00 -> 7.93 us
   const int32_t* offs = src_offsets + (int64_t)s * max_n_ops_per_block;
   const int64_t src_ptr = src_ptrs[s], dst_ptr = dst_ptrs[s];
   const int32_t n_elem = n_elements[s], n_ops = n_ops_per_block[s];

@@ -20,7 +20,8 @@ def share_of_a_part(tiles: Sequence[int], items_per_row: int, n_slots: int) -> O
     """How many key tiles a part takes, or None where nothing is split.  The shortest parts that are all
     on the device at once; if the rows alone are more than it holds, parts of the launch's mean work per
     slot (an item longer than that would end after all the others).  Partials and the kernel that adds
-    them cost about as much as eight tiles, so the longest row has to get shorter by more than that."""
+    them cost about as much as eight tiles, so the longest row has to get shorter by more than that.  (``tiles`` are
+    counted from the rows' keys, whatever the mask leaves of them to see.)"""
     longest = max(tiles, default=0)
     share = max(MIN_SHARE, -(-sum(tiles) * items_per_row // n_slots))
     if len(tiles) * items_per_row <= n_slots:

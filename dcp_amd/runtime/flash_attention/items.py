@@ -55,7 +55,11 @@ def one_workgroup_each(seqlens_q: Sequence[int], seqlens_kv: Sequence[int], n_he
     tokens, 8 heads) 103 / 96; 44 (18701 tokens) 76 / 65; 53 and 41 (two; 12926 tokens, size 64) 145 / 129; 53
     (5323 tokens, 40 heads of 64) 56.9 / 44.0; 56 (7604 tokens, 40 heads) 114 / 109; 98 (5269 tokens, 40 heads) 149 /
     152; 103 (16384 tokens, 16 heads) 197 / 199; 122 (28012 tokens, 32 heads) 348 / 363; 183 (32768 tokens, 8
-    heads) 340 / 356; 2297 (65536 tokens, 32 heads) 3762 / 3933."""
+    heads) 340 / 356; 2297 (65536 tokens, 32 heads) 3762 / 3933.  The line is on the low side: of ten launches of 65
+    to 102 tiles per slot one is better off with the queue (78: 153.9 / 156.5), one indifferent (93) and eight are
+    better off without it (65: 65.9 / 48.6; 74: 158.6 / 153.2; 82: 101.6 / 85.7; 85: 178.5 / 175.1; 98: 197.5 / 191.3;
+    102: 134.8 / 123.6).  Tiles are counted from the rows' keys: under a window or a shared prefix a row sees a part
+    of them, and such launches keep the queue at less work than the line says."""
     items = [-(-n // tile) for n in seqlens_q]
     return (sum(items) * n_heads > n_slots
             and sum(n * -(-k // 64) for n, k in zip(items, seqlens_kv)) * n_heads <= MAX_TILES_WITHOUT_QUEUE * n_slots)
