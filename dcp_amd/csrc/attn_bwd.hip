@@ -419,13 +419,11 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     // 341 -> 293; 4128 tokens 128 -> 111; 131072 tokens, window 4096, 21930 -> 21740; 65536 causal 11440 -> 11370
     // (runs of one build differ by 50).
     if (!unmasked) {
-      const int q = lane_here(), seqlen_kv = visit_lds[visit].seqlen_kv;
+      const int q = lane_here(), first_key = visit_lds[visit].k_row + w * 32, end_key = min(visit_lds[visit].seqlen_kv, first_key + 32);
       // (with one range the second range's planes hold the first's again: the union is the same)
-      const KeyRange range0 = key_range(rng_lds[st][0][q], rng_lds[st][1][q], seqlen_kv);
-      const KeyRange range1 = key_range(rng_lds[st][2][q], rng_lds[st][3][q], seqlen_kv);
-      const RangePair ranges = {range0.start, range0.len, range1.start, range1.len};
-      const uint32_t closed = ranges.closed_window(visit_lds[visit].k_row + w * 32);
-      closed_lds[w][q] = qt * BM + q < seqlen_q ? closed : 0xffffffffu;
+      const uint32_t open = open_window(rng_lds[st][0][q], rng_lds[st][1][q], first_key, end_key) |
+                            open_window(rng_lds[st][2][q], rng_lds[st][3][q], first_key, end_key);
+      closed_lds[w][q] = qt * BM + q < seqlen_q ? ~open : 0xffffffffu;
       // Other lanes of the wave read it below.  The LDS serves a wave's accesses in order, so nothing has to be
       // waited for, but the compiler must not take the reads before the store: these emit no instruction.
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

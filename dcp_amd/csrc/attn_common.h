@@ -521,6 +521,12 @@ struct RangePair {
     return ~(open(s0, len0) | open(s1, len1));
   }
 };
+// Bit p set = key base + p (p = 0..31) lies in [start, end) and before end_key (at most base + 32).  For a range that
+// is looked at once: the ends are cut to the window, whatever their values, and no length is taken.
+__device__ __forceinline__ uint32_t open_window(int start, int end, int base, int end_key) {
+  const int lo = min(max(start, base), base + 32), hi = max(min(end, end_key), lo);
+  return (uint32_t)((1ull << (hi - base)) - (1ull << (lo - base)));
+}
 // 0.0f where bit `bit` of `closed` is clear, -inf where it is set: the bit, sign-extended to 0 / -1,
 // shifted into the sign and exponent of a float.
 __device__ __forceinline__ float masked_start(uint32_t closed, int bit) {
