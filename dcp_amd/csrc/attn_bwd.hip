@@ -26,7 +26,7 @@
 // to end.  A step is one (q head, 64-query tile); the wave takes its two halves
 // of 32 queries one after the other (a sub-step):
 //
-//   S  = Q K^T          A = Q rows from LDS,   B = K held in registers
+//   S  = Q K^T          A = Q rows from LDS,   B = K held in registers (16x16x32 products)
 //   dP = dO V^T         A = dO rows from LDS,  B = V held in registers
 //   P  = exp2(S*c - lse), dS = P * (dP - delta)   accumulator layout: lane =
 //                                                 key, 4 consecutive queries
@@ -40,9 +40,15 @@
 // one that publishes its tiles) and LDS holds nothing but the Q and dO tiles, two
 // stages of each: everything a step reads is requested one step ahead.  With four
 // waves side by side along the keys, a Q/dO tile brought into LDS, a barrier and a
-// step's scalar control serve 64 matrix instructions per wave (with two waves
-// along the keys and two along the queries it was 32, and the two query halves
-// had to be added through LDS at the end).  The range mask enters S as the
+// step's scalar control serve twice the products per wave that two waves
+// along the keys and two along the queries had (whose two query halves
+// had to be added through LDS at the end).
+//
+// What bounds it on a full device is power: the clock falls to what the chip's limit allows, 1.49 GHz in this kernel
+// with 32x32x16 products (65536 causal tokens, 32 heads; 2.4-2.5 in a launch that leaves the device half empty), so
+// what counts is energy.  16x16x32 products move half the accumulators: 1.62 GHz, 8.05 -> 7.93 ms with 7 % more cycles
+// (an instruction more per 32 K operations), and the dQ kernel beside it 3.07 -> 3.00.  A launch of few, lone waves has
+// those cycles and no such clock: 4800 tokens, 8 kv heads, blocks of 1024, 68.6 -> 72 us.  The range mask enters S as the
 // accumulator's initial value (0 or -inf; a bit per key and query, worked out once a step).  dK/dV of a key never leave the wave
 // until the end, so the per-(row, kv block) private dKV blocks of the plan need
 // no atomics and are written whole (zeros where no query of the row attends).
@@ -124,12 +130,12 @@ struct DkvVisit {
 // WRITE_DS: the kernel also leaves dS (the storage type, zero where masked) in the workspace, for
 // the dQ kernel that contracts it with K instead of recomputing S and dP (attn_bwd_ds.hip).  A
 // piece is the dS of 64 keys x 32 queries of one head, 4 KiB, laid out as the lanes of this kernel
-// hold it: [32-key half][16-query half][key][4-query group within the 16: 2 x 2][4 queries].
+// hold it: [16 keys][key][4-query group][16-query half][4 queries].
 template <int DTYPE, int D, bool WRITE_DS>
 __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, int wg) {
   constexpr int BM = kBwdBM, BN = kDkvBN;
-  constexpr int KS = D / 16;  // k-steps over the head dim
-  constexpr int DT = D / 32;  // 32-dim blocks of dK^T / dV^T
+  constexpr int KS = D / 32;  // k-steps over the head dim
+  constexpr int DB = D / 16;  // 16-dim blocks of dK^T / dV^T
   typedef KvTile<D> Tile;     // the Q and dO tiles: 64 queries x D
 
   // two stages of everything a step reads: its Q and dO tiles and the per-query scalars
@@ -142,10 +148,10 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   // With D = 128 the accumulators (128 registers), K and V (64) and the products in flight do
   // not fit in 256 registers.  The compiler would spill to scratch memory, and a scratch
   // reload waits for every outstanding global load, i.e. for the tiles requested a step
-  // ahead.  So the last VL k-steps of V are parked in LDS instead (per lane, read back with
+  // ahead.  So the last k-step of V is parked in LDS instead (per lane, read back with
   // the other operands).
-  constexpr int VL = D == 128 ? 2 : 0;
-  __shared__ u32x4 v_park[VL > 0 ? kBwdThreads / 64 : 1][VL > 0 ? VL : 1][64];
+  constexpr int VL = D == 128 ? 1 : 0;
+  __shared__ u32x4 v_park[VL > 0 ? kBwdThreads / 64 : 1][2][64];
   // on a step that is not unmasked, per wave: which of its 32 keys each of the step's queries does not see
   __shared__ __attribute__((aligned(16))) uint32_t closed_lds[kBwdThreads / 64][BM];
 
@@ -153,8 +159,8 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   asm volatile("" : "+v"(tid));  // (per item: what is derived from it is not kept through the item before)
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's 32 keys of the tile
   const int lane = tid & 63;
-  const int c = lane & 31;
-  const int h = lane >> 5;
+  const int n = lane & 15;  // the lane's key in each of the wave's two 16-key columns
+  const int g = lane >> 4;  // and its four queries in each of a sub-step's two 16-query tiles
 
   // ---- which (kv block, 128-key tile, kv head), and the rows that attend to it ------------
   // Integer division runs on the vector unit, so its (uniform) results sit in vector registers
@@ -208,17 +214,17 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
                               (int64_t)tok0 * p.kv_token_stride + (int64_t)kv_head * D;
 
   // ---- K, V of this wave's 32 keys as B operands (lane = key, slots = dims) ------
-  u32x4 kreg[KS], vreg[KS - VL];
-  {
-    const int64_t off = kv_tile_off + (int64_t)c * p.kv_token_stride + h * 8;
+  u32x4 kreg[KS][2], vreg[KS - VL][2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int64_t off = kv_tile_off + (int64_t)(kk * 16 + n) * p.kv_token_stride + Tile::element16(g);
     const uint16_t* kp = reinterpret_cast<const uint16_t*>(p.k) + off;
     const uint16_t* vp = reinterpret_cast<const uint16_t*>(p.v) + off;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kreg[ks] = *reinterpret_cast<const u32x4*>(kp + ks * 16);
+    for (int ks = 0; ks < KS; ++ks) kreg[ks][kk] = *reinterpret_cast<const u32x4*>(kp + Tile::step16(ks));
 #pragma unroll
-    for (int ks = 0; ks < KS - VL; ++ks) vreg[ks] = *reinterpret_cast<const u32x4*>(vp + ks * 16);
-#pragma unroll
-    for (int j = 0; j < VL; ++j) v_park[w][j][lane] = *reinterpret_cast<const u32x4*>(vp + (KS - VL + j) * 16);
+    for (int ks = 0; ks < KS - VL; ++ks) vreg[ks][kk] = *reinterpret_cast<const u32x4*>(vp + Tile::step16(ks));
+    if constexpr (VL > 0) v_park[w][kk][lane] = *reinterpret_cast<const u32x4*>(vp + Tile::step16(KS - 1));
   }
 
   // ---- per visit: which 64-query tiles of its row see the keys (the same for every head) ------
@@ -250,18 +256,15 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   }
 
   // dK^T and dV^T of this wave's keys: (all dims) x (32 keys), complete when the loop ends
-  f32x16 dk_acc[DT], dv_acc[DT];
+  f32x4 dk_acc[DB][2], dv_acc[DB][2];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+  for (int d = 0; d < DB; ++d)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      dk_acc[dt][i] = 0.0f;
-      dv_acc[dt][i] = 0.0f;
-    }
+    for (int kk = 0; kk < 2; ++kk) dk_acc[d][kk] = dv_acc[d][kk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   // loop-invariant per-lane pieces of the addresses used in the loop
-  const int row_rd = Tile::row_base(c, h);
-  const int col_rd = Tile::col_base(lane, true);
+  const int row_rd = Tile::row_base16(n, g);
+  const int col_rd = Tile::col_base16(lane);
   const uint32_t tiles_at = lds_address(&tiles[0][0]);
   __syncthreads();
 
@@ -275,7 +278,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   // tile load idx of a step: the wave's group loads of the Q tile, then of the dO tile
   constexpr int NL = 2 * Tile::LPW;
   const uint64_t group_step = uniform64(Tile::group_global_step(q_row_stride));
-  static_assert(NL <= KS, "a sub-step carries half of the tile loads, one per two k-steps of its first phase");
+  static_assert(NL <= 2 * KS, "a sub-step carries half of the tile loads, one per k-step of its first phase");
   // Per-query values of a step, two dword loads per wave and no branches: wave 0 requests the
   // first range's starts and ends, wave 1 the second range's (the first's again, into planes
   // nobody reads, when there is one range), wave 2 the LSEs and wave 3 the deltas (each twice,
@@ -312,15 +315,15 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   // tile cu_seqlens_kv[b] / 64 + b (room for a last, partial tile of every row before it) and is laid
   // out [head][32-query chunk][64-key tile]: the pieces that a wave of the dQ kernel reads one after
   // another lie one after another (ordered by key tile first, they were 4 MiB apart at 32 heads and
-  // 1024-token blocks, every one in a memory page of its own).  ds_lane: the lane's 16 bytes within a
-  // [key][query half] plane of a piece.  (A wave whose 64-key half tile begins past the row's last
+  // 1024-token blocks, every one in a memory page of its own).  ds_lane: the lane's 16 bytes within the
+  // plane of the wave's first 16 keys.  (A wave whose 64-key half tile begins past the row's last
   // key has no piece -- it would be one of the next 32-query chunk's, or lie past the end of the
   // workspace -- and writes its zeros into a spare piece behind the last one instead, with a row of
   // no tiles: no branch around the stores.  The zeros of a wave without keys beside one with some
   // are the other half of that one's piece, which the dQ kernel reads whole.)
   uint64_t ds_visit = 0;
   uint32_t ds_row_tiles = 0;  // pieces from a 32-query chunk to the next
-  const int ds_lane = (w & 1) * 128 + 2 * c + h;
+  const int ds_lane = (w & 1) * 128 + 4 * n + g;
   auto begin_visit = [&](int v) {
     KernArgs<AttnBwdParams>& p = fresh_kernel_args<AttnBwdParams>();
     seqlen_q = visit_field(v, DkvVisit::kSeqlenQ);
@@ -437,45 +440,54 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     auto sub_step = [&](const int QI) {
       const int row_rd_q = row_rd + QI * Tile::ROW32, col_rd_q = col_rd + QI * Tile::ROW32;
       // ---- S = Q K^T, dP = dO V^T on 32 queries x 32 keys ---------------------------------
-      // (A = rows of the Q / dO tile, B = K / V in registers; lane = key, element i = query
-      // 32 QI + acc_row(i, h)).  The range mask enters S as the accumulator's initial value.
-      f32x16 s_acc, dp_acc;
+      // (A = rows of the Q / dO tile, B = K / V in registers; two by two 16x16 products: lane = key 16 kk + n,
+      // element r = query 32 QI + 16 qi + 4 g + r).  The range mask enters S as the accumulator's initial value.
+      f32x4 s_acc[2][2], dp_acc[2][2];  // [qi][kk]
       if (unmasked) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s_acc[i] = 0.0f;
+        for (int qi = 0; qi < 2; ++qi)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) s_acc[qi][kk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       } else {
-        const int my_bit = lane_here() & 31;
+        const int my_bit = lane_here() & 15;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const u32x4 closed = *reinterpret_cast<const u32x4*>(&closed_lds[w][QI * 32 + 8 * g + 4 * h]);
+        for (int qi = 0; qi < 2; ++qi) {
+          const u32x4 closed = *reinterpret_cast<const u32x4*>(&closed_lds[w][QI * 32 + 16 * qi + 4 * g]);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) s_acc[4 * g + r] = masked_start(closed[r], my_bit);
+          for (int r = 0; r < 4; ++r) {
+            s_acc[qi][0][r] = masked_start(closed[r], my_bit);
+            s_acc[qi][1][r] = masked_start(closed[r], 16 + my_bit);
+          }
         }
       }
       // dP starts from -delta of its query (dS = P (dP - delta)): the subtraction rides on the
       // accumulation instead of costing a vector instruction per element afterwards
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(&delta_lds[st][QI * 32 + 8 * g + 4 * h]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dp_acc[4 * g + r] = d4[r];
-      }
-      // Everything the sub-step's 32 MFMAs read from LDS forms one stream, read AHEAD entries
+      for (int qi = 0; qi < 2; ++qi)
+        dp_acc[qi][0] = dp_acc[qi][1] = *reinterpret_cast<const f32x4*>(&delta_lds[st][QI * 32 + 16 * qi + 4 * g]);
+      // Everything the sub-step's MFMAs read from LDS forms one stream, read AHEAD entries
       // ahead into four rotating registers, across both matrix phases (the first operand of the
-      // second phase is on its way while the vector phase runs):
-      //   phase 1, per k-step: Q rows (-> S), [the parked V k-step (B operand)], dO rows (-> dP)
-      //   phase 2, per (16-query step s2, 32-dim block d): dO^T (-> dV), Q^T (-> dK)
-      constexpr int N1 = 2 * KS + VL, N2 = 4 * DT, NS = N1 + N2, AHEAD = 2, RING = 4, PRE = 1;
-      constexpr int FIRST_PARKED = 2 * (KS - VL);  // stream index of the first k-step with a parked V
+      // second phase is on its way while the vector phase runs); an operand feeds two MFMAs, one per 16 keys:
+      //   phase 1, per k-step and 16 queries: Q rows (-> S), dO rows (-> dP), [the parked V k-step, two B operands]
+      //   phase 2, per 16-dim block d: dO^T (-> dV), Q^T (-> dK), over all 32 queries
+      constexpr int N1 = 4 * KS + 2 * VL, N2 = 2 * DB, NS = N1 + N2, AHEAD = 2, RING = 4, PRE = 1;
+      constexpr int FIRST_PARKED = 4 * (KS - VL);  // stream index of the k-step with the parked V
+      // (there: Q, Q, V of 16 keys, dO, dO, V of the other 16, which meets both dO)
+      enum { kQRows, kDoRows, kParkedV0, kParkedV1 };
+      auto kind_of = [](int o) {
+        constexpr int parked[6] = {kQRows, kQRows, kParkedV0, kDoRows, kDoRows, kParkedV1};
+        return o < FIRST_PARKED ? o & 1 : parked[(o - FIRST_PARKED) % 6];
+      };
+      auto step_of = [](int o) { return o < FIRST_PARKED ? o / 4 : KS - 1; };
+      auto queries_of = [](int o) { return o < FIRST_PARKED ? (o >> 1) & 1 : (o - FIRST_PARKED) % 6 == 1 || (o - FIRST_PARKED) % 6 == 4; };
       auto entry = [&](int o) -> u32x4 {
         if (o < N1) {
-          const int ks = o < FIRST_PARKED ? o / 2 : (KS - VL) + (o - FIRST_PARKED) / 3;
-          const int kind = o < FIRST_PARKED ? (o & 1) * 2 : (o - FIRST_PARKED) % 3;  // 0: Q, 1: parked V, 2: dO
-          if (kind == 1) return v_park[w][VL > 0 ? ks - (KS - VL) : 0][lane];
-          return Tile::read_row(kind == 0 ? q_lds : do_lds, row_rd_q, 0, ks);
+          const int kind = kind_of(o);
+          if (kind >= kParkedV0) return v_park[w][kind - kParkedV0][lane];
+          return Tile::read_row16(kind == kQRows ? q_lds : do_lds, row_rd_q, queries_of(o), step_of(o));
         }
-        const int i = o - N1, s2 = i / (2 * DT), d = (i % (2 * DT)) / 2;
-        return Tile::template read_col<true>((i & 1) ? q_lds : do_lds, col_rd_q, s2, d);
+        const int i = o - N1;
+        return Tile::read_col16((i & 1) ? q_lds : do_lds, col_rd_q, 0, i / 2);
       };
       // this sub-step's half of the next step's tile loads: the Q tile (QI = 0) or the dO tile
       static_assert(NL / 2 == Tile::LPW, "a sub-step loads one whole tile");
@@ -490,17 +502,26 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       if (QI == 0) request_scalars(head_next, qt_next, st ^ 1);
 #pragma unroll
       for (int o = 0; o < N1; ++o) {
-        const int ks = o < FIRST_PARKED ? o / 2 : (KS - VL) + (o - FIRST_PARKED) / 3;
-        const int kind = o < FIRST_PARKED ? (o & 1) * 2 : (o - FIRST_PARKED) % 3;
-        if (kind == 0) s_acc = mfma_32x32x16<DTYPE>(buf[o % RING], kreg[ks], s_acc);
-        else if (kind == 2 && ks < KS - VL) dp_acc = mfma_32x32x16<DTYPE>(buf[o % RING], vreg[ks < KS - VL ? ks : 0], dp_acc);
-        else if (kind == 2) dp_acc = mfma_32x32x16<DTYPE>(buf[o % RING], buf[(o - 1) % RING], dp_acc);
-        // the entry just used (and the one before it) are free: the next read goes there.  Only the
+        const int ks = step_of(o), kind = kind_of(o), qi = queries_of(o);
+        if (kind == kQRows) {
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) s_acc[qi][kk] = mfma_16x16x32<DTYPE>(buf[o % RING], kreg[ks][kk], s_acc[qi][kk]);
+        } else if (kind == kDoRows && ks < KS - VL) {
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk)
+            dp_acc[qi][kk] = mfma_16x16x32<DTYPE>(buf[o % RING], vreg[ks < KS - VL ? ks : 0][kk], dp_acc[qi][kk]);
+        } else if (kind == kDoRows) {
+          dp_acc[qi][0] = mfma_16x16x32<DTYPE>(buf[o % RING], buf[(o - 1 - qi) % RING], dp_acc[qi][0]);
+        } else if (kind == kParkedV1) {
+          dp_acc[0][1] = mfma_16x16x32<DTYPE>(buf[(o - 2) % RING], buf[o % RING], dp_acc[0][1]);
+          dp_acc[1][1] = mfma_16x16x32<DTYPE>(buf[(o - 1) % RING], buf[o % RING], dp_acc[1][1]);
+        }
+        // the entry just used (and the ones before it) are free: the next read goes there.  Only the
         // first operand of the second phase is requested before the vector phase (registers)
         if (o + AHEAD < N1 + PRE) buf[(o + AHEAD) % RING] = entry(o + AHEAD);
-        // this sub-step's half of the next step's tile loads, one per two k-steps
-        if (kind == 2 && ks % 2 == 0 && ks / 2 < NL / 2) {
-          Tile::load_group_at(load_at + (ks / 2) * (Tile::GROUP_STRIDE * 2), load_src, goff0);
+        // this sub-step's half of the next step's tile loads, one per k-step
+        if (o % 4 == 1 && o / 4 < NL / 2) {
+          Tile::load_group_at(load_at + Tile::group_of_load(o / 4) * (Tile::GROUP_STRIDE * 2), load_src, goff0);
           load_src = uniform64(load_src + group_step);
         }
         __builtin_amdgcn_sched_barrier(0);  // keeps the order: reads neither pile up in registers nor fall behind
@@ -508,21 +529,23 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       // ---- P = exp2(S c - lse), dS = P (dP - delta), packed in accumulator order: as B operands
       // they feed the next products without leaving the registers -------------------------------
       __builtin_amdgcn_s_setprio(kPrioVector);
-      u32x4 pb[2], dsb[2];
+      u32x4 pb[2], dsb[2];  // [kk]: the lane's key, queries 4 g.. and 16 + 4 g..
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int qrow = QI * 32 + 8 * g + 4 * h;
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(&lse_lds[st][qrow]);
-        float pv[4], dsv[4];
+      for (int qi = 0; qi < 2; ++qi) {
+        const f32x4 l4 = *reinterpret_cast<const f32x4*>(&lse_lds[st][QI * 32 + 16 * qi + 4 * g]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          pv[r] = fast_exp2(fmaf(s_acc[4 * g + r], p.scale_log2, -l4[r]));  // l4: lse * log2(e); masked: exp2(-inf) = 0
-          dsv[r] = pv[r] * dp_acc[4 * g + r];
+        for (int kk = 0; kk < 2; ++kk) {
+          float pv[4], dsv[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            pv[r] = fast_exp2(fmaf(s_acc[qi][kk][r], p.scale_log2, -l4[r]));  // l4: lse * log2(e); masked: exp2(-inf) = 0
+            dsv[r] = pv[r] * dp_acc[qi][kk][r];
+          }
+          pb[kk][qi * 2] = pack2<DTYPE>(pv[0], pv[1]);
+          pb[kk][qi * 2 + 1] = pack2<DTYPE>(pv[2], pv[3]);
+          dsb[kk][qi * 2] = pack2<DTYPE>(dsv[0], dsv[1]);
+          dsb[kk][qi * 2 + 1] = pack2<DTYPE>(dsv[2], dsv[3]);
         }
-        pb[g >> 1][(g & 1) * 2] = pack2<DTYPE>(pv[0], pv[1]);
-        pb[g >> 1][(g & 1) * 2 + 1] = pack2<DTYPE>(pv[2], pv[3]);
-        dsb[g >> 1][(g & 1) * 2] = pack2<DTYPE>(dsv[0], dsv[1]);
-        dsb[g >> 1][(g & 1) * 2 + 1] = pack2<DTYPE>(dsv[2], dsv[3]);
       }
       if constexpr (WRITE_DS) {
         // (non-temporal: the pieces are read once, by another kernel; they must not push the row's
@@ -544,13 +567,16 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       // transpose loads, in the accumulators' row order) ---------------------------------------
 #pragma unroll
       for (int o = N1; o < NS; ++o) {
-        const int i = o - N1, s2 = i / (2 * DT), d = (i % (2 * DT)) / 2;
-        if (i & 1) dk_acc[d] = mfma_32x32x16<DTYPE>(buf[o % RING], dsb[s2], dk_acc[d]);
-        else dv_acc[d] = mfma_32x32x16<DTYPE>(buf[o % RING], pb[s2], dv_acc[d]);
+        const int i = o - N1, d = i / 2;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          if (i & 1) dk_acc[d][kk] = mfma_16x16x32<DTYPE>(buf[o % RING], dsb[kk], dk_acc[d][kk]);
+          else dv_acc[d][kk] = mfma_16x16x32<DTYPE>(buf[o % RING], pb[kk], dv_acc[d][kk]);
+        }
         if (o + AHEAD < NS) buf[(o + AHEAD) % RING] = entry(o + AHEAD);
         if constexpr (WRITE_DS) {
           if (i == 3) __builtin_nontemporal_store(dsb[0], piece);
-          if (i == 2 * DT + 1) __builtin_nontemporal_store(dsb[1], piece + 64);  // (2 * 2 * DT iterations)
+          if (i == DB + 1) __builtin_nontemporal_store(dsb[1], piece + 64);  // (2 DB iterations)
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -576,52 +602,47 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   const int out_key = __builtin_amdgcn_readfirstlane(wg % args.kv_tiles_per_row) * BN + w * 32;
   // a group's result goes to a slot of dk/dv; or, where nothing else is added to it, to the caller's
   // unpadded tensor, of which only the block's own tokens may be written; or it is partial
-  int entry, where = 0, token = out_key + c;
+  int entry, where = 0, first = out_key, end = out_key + 32;  // the tokens of the entry that are written: [first, end)
   if (args.dkv_groups != nullptr) {
     const int32_t* grp = args.dkv_groups + (int64_t)out_item * kDkvGroupInts;
     entry = grp[1];
     where = grp[3];
-    if (token >= grp[2]) return;
+    end = min(end, grp[2]);
   } else {
     if (out_key >= visit_field(0, DkvVisit::kSeqlenKv)) return;  // a wave without keys
     const int blk = __builtin_amdgcn_readfirstlane(out_key / args.block_size);
     entry = args.dkv_block_table[(int64_t)visit_field(0, DkvVisit::kRow) * args.max_kv_blocks + blk];
-    token -= blk * args.block_size;
+    first -= blk * args.block_size;
+    end -= blk * args.block_size;
   }
   const float scale = args.scale;
-  if (where == 2) {  // a part's share, to be added to the other parts' by a sum kernel
-    const int64_t head_row = (int64_t)args.n_heads_kv * D;
-    float* dst = args.dkv_partials + ((int64_t)entry * args.block_size + token) * (2 * head_row) + (int64_t)out_head * D + 4 * h;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+  for (int kk = 0; kk < 2; ++kk) {
+    const int token = first + kk * 16 + n;
+    if (token >= end) continue;
+    if (where == 2) {  // a part's share, to be added to the other parts' by a sum kernel
+      const int64_t head_row = (int64_t)args.n_heads_kv * D;
+      float* dst = args.dkv_partials + ((int64_t)entry * args.block_size + token) * (2 * head_row) + (int64_t)out_head * D + 4 * g;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4 k4, v4;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          k4[r] = dk_acc[dt][4 * g + r] * scale;
-          v4[r] = dv_acc[dt][4 * g + r];
-        }
-        *reinterpret_cast<f32x4*>(dst + dt * 32 + 8 * g) = k4;
-        *reinterpret_cast<f32x4*>(dst + head_row + dt * 32 + 8 * g) = v4;
+      for (int d = 0; d < DB; ++d) {
+        *reinterpret_cast<f32x4*>(dst + d * 16) = dk_acc[d][kk] * scale;
+        *reinterpret_cast<f32x4*>(dst + head_row + d * 16) = dv_acc[d][kk];
       }
-    return;
-  }
-  const int64_t off = (int64_t)entry * (where ? args.dkv2_entry_stride : args.dkv_slot_stride) +
-                      (int64_t)(token) * (where ? args.dkv2_token_stride : args.dkv_token_stride) + (int64_t)out_head * D + 4 * h;
-  uint16_t* dv_dst = reinterpret_cast<uint16_t*>(where ? args.dv2 : args.dv) + off;
-  uint16_t* dk_dst = reinterpret_cast<uint16_t*>(where ? args.dk2 : args.dk) + off;
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int i = 4 * g;
-      u32x2 v4 = {pack2<DTYPE>(dv_acc[dt][i], dv_acc[dt][i + 1]), pack2<DTYPE>(dv_acc[dt][i + 2], dv_acc[dt][i + 3])};
-      *reinterpret_cast<u32x2*>(dv_dst + dt * 32 + 8 * g) = v4;
-      u32x2 k4 = {pack2<DTYPE>(dk_acc[dt][i] * scale, dk_acc[dt][i + 1] * scale),
-                  pack2<DTYPE>(dk_acc[dt][i + 2] * scale, dk_acc[dt][i + 3] * scale)};
-      *reinterpret_cast<u32x2*>(dk_dst + dt * 32 + 8 * g) = k4;
+      continue;
     }
+    const int64_t off = (int64_t)entry * (where ? args.dkv2_entry_stride : args.dkv_slot_stride) +
+                        (int64_t)(token) * (where ? args.dkv2_token_stride : args.dkv_token_stride) + (int64_t)out_head * D + 4 * g;
+    uint16_t* dv_dst = reinterpret_cast<uint16_t*>(where ? args.dv2 : args.dv) + off;
+    uint16_t* dk_dst = reinterpret_cast<uint16_t*>(where ? args.dk2 : args.dk) + off;
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+      const f32x4 v = dv_acc[d][kk], k = dk_acc[d][kk] * scale;
+      const u32x2 v4 = {pack2<DTYPE>(v[0], v[1]), pack2<DTYPE>(v[2], v[3])};
+      *reinterpret_cast<u32x2*>(dv_dst + d * 16) = v4;
+      const u32x2 k4 = {pack2<DTYPE>(k[0], k[1]), pack2<DTYPE>(k[2], k[3])};
+      *reinterpret_cast<u32x2*>(dk_dst + d * 16) = k4;
+    }
+  }
 }
 
 // Persistent where it works on groups of rows (131072 tokens, window 4096: 16.6 -> 15.6 ms; 65536 tokens,

@@ -13,7 +13,7 @@
 // every (64-query tile, 128-key tile) pair the dK/dV kernel visits.
 //
 // dS travels in pieces of 64 keys x 32 queries of one head (4 KiB), written by a wave of the dK/dV
-// kernel exactly as its lanes hold them (lane = key, four consecutive queries per register pair)
+// kernel exactly as its lanes hold them (lane = key, two times four consecutive queries)
 // in whole 1 KiB stores.  A wave here owns 32 queries (one piece per 64-key tile), brings its
 // pieces into a region of LDS of its own with global_load_lds and reads them as the B operand
 // through transposing loads, whose per-lane addresses undo the layout; no other wave touches the
@@ -56,7 +56,7 @@ constexpr int kDsFewItems = 4;        // per CU, see launch_bwd_through_ds
 template <int DTYPE, int D, int HH>
 __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, int item) {
   constexpr int BN = kDsBN;
-  constexpr int DT = D / 32;
+  constexpr int DB = D / 16;
   constexpr int KSTAGES = HH == 1 ? kDsStages : 2;  // K tiles requested two steps ahead: two tiles, or one
   typedef KvTile<D, kDsWaves> Tile;
   __shared__ __attribute__((aligned(16))) uint16_t k_lds[KSTAGES][Tile::SIZE];
@@ -66,8 +66,8 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  const int c = lane & 31;
-  const int h = lane >> 5;
+  const int n = lane & 15;
+  const int g4 = lane >> 4;
 
   int wg = item;
   const int qt = __builtin_amdgcn_readfirstlane(wg % p.dq_tiles_per_row);
@@ -82,8 +82,7 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   if (qt * kDsBM >= seqlen_q) return;
   const int kv_head = __builtin_amdgcn_readfirstlane(head / (p.n_heads_q / p.n_heads_kv));
   const int64_t q_row_stride = (int64_t)p.n_heads_q * D;
-  const int q_local = qt * kDsBM + w * 32 + c;
-  const bool q_valid = q_local < seqlen_q;
+  const int q_first = qt * kDsBM + w * 32;  // the wave's queries
 
   // ---- which key tiles: the 128-key tiles the dK/dV kernel visited for this wave's 64-query tile
   // (the same test on the same hulls: a piece that was never written is never read), and for the
@@ -123,22 +122,21 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   load_slot_table(slot_lds, kv_table, p.max_kv_blocks, tid, kDsThreads);
   __syncthreads();
 
-  f32x16 dq_acc[HH][DT];
+  f32x4 dq_acc[HH][DB][2];  // dims 16 d + 4 g4.. of query 16 qi + n
 #pragma unroll
   for (int hh = 0; hh < HH; ++hh)
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int d = 0; d < DB; ++d)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) dq_acc[hh][dt][i] = 0.0f;
+      for (int qi = 0; qi < 2; ++qi) dq_acc[hh][d][qi] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   const uint16_t* kg = reinterpret_cast<const uint16_t*>(p.k) + (int64_t)kv_head * D;
   const uint32_t kv_goff0 = Tile::lane_offset0(p.kv_token_stride, w, lane);
-  const int col_rd = Tile::col_base(lane, false);  // K^T, contraction index = key in plain order
-  // this lane's 8 bytes inside a piece for k-step 0 (see the file comment and attn_bwd.hip):
-  // 16-lane group L = lane >> 4: queries 16 (L & 1) + ..., keys 8 (L >> 1) + ...; lane j of the group
-  // supplies key row j >> 2 and the four queries 4 (j & 3)..
-  const int j = lane & 15, L = lane >> 4;
-  const int ds_rd = (L & 1) * 1024 + (2 * (8 * (L >> 1) + (j >> 2)) + (j & 1)) * 16 + ((j & 3) >> 1) * 8;  // bytes
+  const int col_rd = Tile::col_base16(lane);  // K^T; a lane's keys: 4 g4.. and 16 + 4 g4..
+  // This lane's 8 bytes inside a piece for keys 0..15 and queries 0..15 (see the file comment and attn_bwd.hip):
+  // lane j of the 16-lane group g4 supplies key 4 g4 + j / 4 and the queries 4 (j % 4)..: the 16 bytes of
+  // that key and query group, the lane's own number in the order of the piece.
+  const int ds_rd = lane * 16;
 
   const int tiles_per_block = p.block_size / BN;
   const int64_t tile_stride = (int64_t)BN * p.kv_token_stride;
@@ -175,31 +173,42 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
     if (cursor.index + 1 < n_tiles)
       cursor.advance(runs, tiles_per_block, slot_lds, kv_table, p.kv_slot_stride, tile_stride);
   };
-  auto compute = [&](f32x16 (&acc)[DT], int t64, const uint16_t* k_lds, const uint16_t* piece) {
+  auto compute = [&](f32x4 (&acc)[DB][2], int t64, const uint16_t* k_lds, const uint16_t* piece) {
     if (!wave_sees(t64)) return;
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
     const char* pb = reinterpret_cast<const char*>(piece) + ds_rd;
-    auto ds_operand = [&](int ks) -> u32x4 {
-      const char* p0 = pb + (ks >> 1) * 2048 + (ks & 1) * 512;
+    auto ds_operand = [&](int ks, int qi) -> u32x4 {
+      const char* p0 = pb + ks * 2048 + qi * 8;
       const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0));
-      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 128));
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 1024));
       const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
       return u32x4{l2[0], l2[1], h2[0], h2[1]};
     };
-    u32x4 kt_a[2][DT], dsb[2];
+    // operands in the order of their use, AHEAD of it: per 32 keys the two dS^T, then the K^T of every 16 dims, which
+    // feeds a product with either
+    constexpr int NK = BN / 32, N = NK * DB, AHEAD = 4, RING = 8;
+    u32x4 kt_a[RING], dsb[NK][2];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) kt_a[0][dt] = Tile::template read_col<false>(k_lds, col_rd, 0, dt);
-    dsb[0] = ds_operand(0);
+    for (int i = 0; i < AHEAD; ++i) {
+      if (i % DB == 0) {
+        dsb[i / DB][0] = ds_operand(i / DB, 0);
+        dsb[i / DB][1] = ds_operand(i / DB, 1);
+      }
+      kt_a[i] = Tile::read_col16(k_lds, col_rd, i / DB, i % DB);
+    }
 #pragma unroll
-    for (int ks = 0; ks < BN / 16; ++ks) {
-      if (ks + 1 < BN / 16) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) kt_a[(ks + 1) & 1][dt] = Tile::template read_col<false>(k_lds, col_rd, ks + 1, dt);
-        dsb[(ks + 1) & 1] = ds_operand(ks + 1);
+    for (int i = 0; i < N; ++i) {
+      const int nx = i + AHEAD;
+      if (nx < N) {
+        if (nx % DB == 0) {
+          dsb[nx / DB][0] = ds_operand(nx / DB, 0);
+          dsb[nx / DB][1] = ds_operand(nx / DB, 1);
+        }
+        kt_a[nx % RING] = Tile::read_col16(k_lds, col_rd, nx / DB, nx % DB);
       }
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) acc[dt] = mfma_32x32x16<DTYPE>(kt_a[ks & 1][dt], dsb[ks & 1], acc[dt]);
+      for (int qi = 0; qi < 2; ++qi) acc[i % DB][qi] = mfma_16x16x32<DTYPE>(kt_a[i % RING], dsb[i / DB][qi], acc[i % DB][qi]);
     }
   };
 
@@ -260,19 +269,21 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
     k_stage = k_stage == KSTAGES - 1 ? 0 : k_stage + 1;
   }
 
-  if (!q_valid) return;
 #pragma unroll
-  for (int hh = 0; hh < HH; ++hh) {
-    uint16_t* op = reinterpret_cast<uint16_t*>(p.dq) + (int64_t)p.dq_block_table[b] * p.dq_slot_stride +
-                   (int64_t)q_local * q_row_stride + (int64_t)(head + hh) * D + 4 * h;
+  for (int qi = 0; qi < 2; ++qi) {
+    const int q_local = q_first + qi * 16 + n;
+    if (q_local >= seqlen_q) continue;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int hh = 0; hh < HH; ++hh) {
+      uint16_t* op = reinterpret_cast<uint16_t*>(p.dq) + (int64_t)p.dq_block_table[b] * p.dq_slot_stride +
+                     (int64_t)q_local * q_row_stride + (int64_t)(head + hh) * D + 4 * g4;
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        u32x2 pk = {pack2<DTYPE>(dq_acc[hh][dt][4 * gq] * p.scale, dq_acc[hh][dt][4 * gq + 1] * p.scale),
-                    pack2<DTYPE>(dq_acc[hh][dt][4 * gq + 2] * p.scale, dq_acc[hh][dt][4 * gq + 3] * p.scale)};
-        *reinterpret_cast<u32x2*>(op + dt * 32 + 8 * gq) = pk;
+      for (int d = 0; d < DB; ++d) {
+        const f32x4 v = dq_acc[hh][d][qi] * p.scale;
+        const u32x2 pk = {pack2<DTYPE>(v[0], v[1]), pack2<DTYPE>(v[2], v[3])};
+        *reinterpret_cast<u32x2*>(op + d * 16) = pk;
       }
+    }
   }
 }
 

@@ -30,6 +30,24 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(u32x4 a, u32x4 b, f32x16 c) {
   }
 }
 
+// D(16x16, f32) += A(16x32) * B(32x16), 16-bit inputs.
+// Lane l = 16*g + n holds: A row n, k-slots 8g..8g+7; B column n, the same k-slots; D column n,
+// rows 4g..4g+3.
+// The same operations as the 32x32x16 form at half the accumulator traffic per operation, and on this device,
+// whose clock follows its power, the faster one: with random operands and nothing else in the kernel 2.08-2.15
+// PFLOP/s against 1.74-1.84; with an LDS read per 32 K operations 1.89 against 1.66; with the dK/dV kernel's mix of
+// FMAs, exponentials and LDS reads 1.69-1.70 against 1.53; with the forward's 1.49-1.51 against 1.42.
+template <int DTYPE>
+__device__ __forceinline__ f32x4 mfma_16x16x32(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (DTYPE == DCP_DTYPE_BF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
+}
+
 // Two fp32 -> one dword of two 16-bit values (round to nearest even).
 template <int DTYPE>
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
@@ -117,16 +135,17 @@ __device__ __forceinline__ constexpr int kslot_pos(int r) {
 // together must sit in different groups.  Groups are padded by 16 bytes, which
 // puts group g at bank-window offset 16g, and row r of the tile goes to
 //
-//   D = 128:  group 4*(r&3) + (r>>2)&3,   position r>>4 in the group
-//   D =  64:  group 4*(r&1) + (r>>2)&3,   position (r>>1)&1 + 2*(r>>4)
+//   D = 128:  group 4*(r&3) + swap((r>>2)&3),   position r>>4 in the group
+//   D =  64:  group 4*(r&1) + swap((r>>2)&3),   position (r>>1)&1 + 2*(r>>4)
 //
-// so that, within any aligned 16 rows, row r sits at window offset
-// 64*(r&3) + 16*((r>>2)&3) bytes:
+// (swap exchanges the two bits: 0, 2, 1, 3) so that, within any aligned 16 rows, row r sits at window offset
+// 64*(r&3) + 32*((r>>2)&1) + 16*((r>>3)&1) bytes:
 //  - row operand (8 consecutive elements of a row; 16 lanes read 16
 //    consecutive rows at one column): 16 different 16-byte slots;
-//  - column operand (transpose load: one column at 8 rows, the rows being the
-//    contraction index; 32 lanes touch 4 consecutive rows x 64 bytes): four
-//    64-byte windows.
+//  - column operand of a 32x32x16 product (transpose load: one column at 8 rows, the rows being the
+//    contraction index; 32 lanes touch 4 consecutive rows x 64 bytes): four 64-byte windows;
+//  - column operand of a 16x16x32 product (32 lanes touch 8 consecutive rows x 32 bytes): eight 32-byte
+//    windows, which is what the swap is for.
 // ---------------------------------------------------------------------------
 // LDS byte address of a __shared__ object
 template <typename T>
@@ -178,18 +197,24 @@ struct KvTile {
   static constexpr int LPW = NG / NW;             // group loads per wave (NW waves fill a tile)
   static constexpr int ROW32 = 256;               // element offset of row r + 32 (both head dims)
   static constexpr int ROW16 = 128;               // element offset of row r + 16
-  static constexpr int ROW8 = 2 * GROUP_STRIDE;   // row r + 8  (r % 16 < 8)
-  static constexpr int ROW4 = GROUP_STRIDE;       // row r + 4  (r % 16 in 0..3 or 8..11)
+  static constexpr int ROW8 = GROUP_STRIDE;       // row r + 8  (r % 16 < 8)
+  static constexpr int ROW4 = 2 * GROUP_STRIDE;   // row r + 4  (r % 16 in 0..3 or 8..11)
+
+  __device__ static __forceinline__ constexpr int swap(int x) { return ((x & 1) << 1) | (x >> 1); }  // of 0..3
+  // The wave's group loads in the order of their rows, which are then a constant step apart: which of the wave's groups
+  // the i-th one fills.
+  __device__ static __forceinline__ constexpr int group_of_load(int i) { return LPW == 4 ? swap(i) : i; }
+  static constexpr int LOAD_ROWS = LPW == 4 ? 4 : 8;  // rows from one of these loads to the next
 
   __device__ static __forceinline__ int at(int r, int e) {
-    const int grp = D == 128 ? 4 * (r & 3) + ((r >> 2) & 3) : 4 * (r & 1) + ((r >> 2) & 3);
+    const int grp = (D == 128 ? 4 * (r & 3) : 4 * (r & 1)) + swap((r >> 2) & 3);
     const int pos = D == 128 ? (r >> 4) : ((r >> 1) & 1) + 2 * (r >> 4);
     return grp * GROUP_STRIDE + pos * D + e;
   }
   // row held at position `pos` of group `grp`
   __device__ static __forceinline__ int row_of(int grp, int pos) {
-    return D == 128 ? 16 * pos + 4 * (grp & 3) + (grp >> 2)
-                    : 16 * (pos >> 1) + 4 * (grp & 3) + 2 * (pos & 1) + (grp >> 2);
+    return D == 128 ? 16 * pos + 4 * swap(grp & 3) + (grp >> 2)
+                    : 16 * (pos >> 1) + 4 * swap(grp & 3) + 2 * (pos & 1) + (grp >> 2);
   }
   // Byte offsets, from (row 0, the head's first element), of what this lane
   // fetches in each of its wave's group loads.  Loop-invariant.
@@ -224,8 +249,8 @@ struct KvTile {
   }
   // The same loads one at a time, so that a kernel can spread them between its matrix
   // instructions instead of issuing a burst (a burst fills the memory pipeline's queue
-  // and the wave sits at the last load until the queue drains).  The rows of group
-  // load i lie 4*i rows below those of group load 0, so one per-lane byte offset
+  // and the wave sits at the last load until the queue drains).  The rows of
+  // load i lie LOAD_ROWS*i rows below those of load 0, so one per-lane byte offset
   // (lane_offset0) serves all of them and the rest of the address is wave-uniform:
   // scalar base + vector offset addressing, no per-load address arithmetic.
   __device__ static __forceinline__ uint32_t lane_offset0(int64_t row_stride, int wave, int lane) {
@@ -236,8 +261,8 @@ struct KvTile {
   // `g` (wave-uniform) points at (row 0, the head's first element) of the tile.
   __device__ static __forceinline__ void load_group(uint32_t tile_at, const uint16_t* g, uint32_t off0,
                                                     int64_t row_stride, int wave, int i) {
-    const uint32_t lds_at = __builtin_amdgcn_readfirstlane(tile_at + (wave * LPW + i) * GROUP_STRIDE * 2);
-    const uint64_t a = reinterpret_cast<uint64_t>(g) + (uint64_t)(i * 8) * (uint64_t)row_stride;
+    const uint32_t lds_at = __builtin_amdgcn_readfirstlane(group_lds_at(tile_at, wave, i));
+    const uint64_t a = reinterpret_cast<uint64_t>(g) + (uint64_t)i * group_global_step(row_stride);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
     const uint64_t base = ((uint64_t)hi << 32) | lo;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -261,12 +286,11 @@ struct KvTile {
                  : "s"(lds_at), "v"(off0), "s"(base)
                  : "memory");
   }
-  // LDS byte address of the wave's group load i, and the global byte step between group loads (its
-  // rows lie four rows below those of load i - 1)
+  // LDS byte address of the wave's group load i, and the global byte step between group loads
   __device__ static __forceinline__ uint32_t group_lds_at(uint32_t tile_at, int wave, int i) {
-    return tile_at + (wave * LPW + i) * GROUP_STRIDE * 2;
+    return tile_at + (wave * LPW + group_of_load(i)) * GROUP_STRIDE * 2;
   }
-  __device__ static __forceinline__ uint64_t group_global_step(int64_t row_stride) { return (uint64_t)row_stride * 8; }
+  __device__ static __forceinline__ uint64_t group_global_step(int64_t row_stride) { return (uint64_t)row_stride * (2 * LOAD_ROWS); }
   // Row operand of lane (c, h): elements 16*ks + 8h.. of row 32*nt + c at
   //   tile + row_base(c, h) + nt*ROW32 + ks*16
   __device__ static __forceinline__ int row_base(int c, int h) { return at(c, 8 * h); }
@@ -292,6 +316,35 @@ struct KvTile {
   }
   __device__ static __forceinline__ u32x4 read_row(const uint16_t* tile, int base, int nt, int ks) {
     return *reinterpret_cast<const u32x4*>(tile + base + nt * ROW32 + ks * 16);
+  }
+  // The same for 16x16x32 products.  Row operand of lane (n, g): eight elements, from element16(g) + step16(ks), of row
+  // 16*nt + n.  Which of a row's elements are the contraction's slots of a lane is free as long as both operands agree,
+  // and is chosen by the banks: a 16-byte load serves the lanes whose bits 2, 3 and 4 have even parity together, and
+  // then the others, so the lanes of n / 4 = 0, 3 of one g meet those of n / 4 = 1, 2 of the next.  With both at the
+  // same 16 bytes of a 64-byte window the rows alone decide, and they were placed to differ; with g * 8, the plain
+  // order, every load took twice as long (an LDS-only loop: 9.3 against 5.9 clocks a load; the dK/dV kernel of 65536 causal
+  // tokens spent 16 % of its cycles on it).
+  __device__ static __forceinline__ constexpr int element16(int g) { return 32 * (g & 1) + 8 * (g >> 1); }
+  __device__ static __forceinline__ constexpr int step16(int ks) { return 16 * (ks & 1) + 64 * (ks >> 1); }
+  __device__ static __forceinline__ int row_base16(int n, int g) { return at(n, element16(g)); }
+  __device__ static __forceinline__ u32x4 read_row16(const uint16_t* tile, int base, int nt, int ks) {
+    return *reinterpret_cast<const u32x4*>(tile + base + nt * ROW16 + step16(ks));
+  }
+  // Column operand of lane (n, g): column 16*ct + n at rows 32*s2 + {4g..4g+3, 16+4g..16+4g+3}, the rows the lane holds in
+  // the accumulators of two 16-row tiles: those two, packed, are the other operand.
+  __device__ static __forceinline__ int col_base16(int lane) {
+    const int j = lane & 15, g = lane >> 4;
+    return at(4 * g + (j >> 2), 4 * (j & 3));
+  }
+  __device__ static __forceinline__ u32x4 read_col16(const uint16_t* tile, int base, int s2, int ct) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const uint16_t* p0 = tile + base + s2 * ROW32 + ct * 16;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + ROW16));
+    const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+    u32x4 out = {l2[0], l2[1], h2[0], h2[1]};
+    return out;
   }
 };
 
