@@ -83,6 +83,18 @@ __device__ __forceinline__ float halves_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// max / sum over the four 16-lane quarters of a wave, the same in all of them
+__device__ __forceinline__ float quarters_max(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // {quarters 0 0 2 2, quarters 1 1 3 3}
+  return halves_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+__device__ __forceinline__ float quarters_sum(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return halves_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+
 // Minimum / maximum over the wave, as a scalar.  Four DPP steps (row_shr 1, 2, 4, 8) leave each
 // 16-lane row's result in its last lane; the four row results are combined on the scalar unit.
 // (Butterfly shuffles would be six dependent trips through LDS each, and a workgroup's prologue
