@@ -213,20 +213,6 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   const int64_t kv_tile_off = (int64_t)(grouped ? grp[0] : p.kv_block_table[table_at]) * p.kv_slot_stride +
                               (int64_t)tok0 * p.kv_token_stride + (int64_t)kv_head * D;
 
-  // ---- K, V of this wave's 32 keys as B operands (lane = key, slots = dims) ------
-  u32x4 kreg[KS][2], vreg[KS - VL][2];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk) {
-    const int64_t off = kv_tile_off + (int64_t)(kk * 16 + n) * p.kv_token_stride + Tile::element16(g);
-    const uint16_t* kp = reinterpret_cast<const uint16_t*>(p.k) + off;
-    const uint16_t* vp = reinterpret_cast<const uint16_t*>(p.v) + off;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kreg[ks][kk] = *reinterpret_cast<const u32x4*>(kp + Tile::step16(ks));
-#pragma unroll
-    for (int ks = 0; ks < KS - VL; ++ks) vreg[ks][kk] = *reinterpret_cast<const u32x4*>(vp + Tile::step16(ks));
-    if constexpr (VL > 0) v_park[w][kk][lane] = *reinterpret_cast<const u32x4*>(vp + Tile::step16(KS - 1));
-  }
-
   // ---- per visit: which 64-query tiles of its row see the keys (the same for every head) ------
   // bit qt of `act`: some query of tile qt sees some of the workgroup's 128 keys; of the wave's
   // `unm`: every query of it sees all of the wave's 32.  Taken once from the per-tile hulls, so the
@@ -255,6 +241,24 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     }
   }
 
+  // ---- K, V of this wave's 32 keys as B operands (lane = key, slots = dims) ------
+  // (Requested after the hulls the masks are made of, and on their way while the masks are made and the first step's tiles
+  // requested: in front of them, each waited for by itself, a workgroup began its steps 2 us later.)
+  u32x4 kreg[KS][2], vreg[KS - VL][2], v_last[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int64_t off = kv_tile_off + (int64_t)(kk * 16 + n) * p.kv_token_stride + Tile::element16(g);
+    const uint16_t* kp = reinterpret_cast<const uint16_t*>(p.k) + off;
+    const uint16_t* vp = reinterpret_cast<const uint16_t*>(p.v) + off;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kreg[ks][kk] = *reinterpret_cast<const u32x4*>(kp + Tile::step16(ks));
+#pragma unroll
+    for (int ks = 0; ks < KS - VL; ++ks) vreg[ks][kk] = *reinterpret_cast<const u32x4*>(vp + Tile::step16(ks));
+    // (the kernel that leaves no dS has no registers for them over the masks)
+    if constexpr (VL > 0 && WRITE_DS) v_last[kk] = *reinterpret_cast<const u32x4*>(vp + Tile::step16(KS - 1));
+    else if constexpr (VL > 0) v_park[w][kk][lane] = *reinterpret_cast<const u32x4*>(vp + Tile::step16(KS - 1));
+  }
+
   // dK^T and dV^T of this wave's keys: (all dims) x (32 keys), complete when the loop ends
   f32x4 dk_acc[DB][2], dv_acc[DB][2];
 #pragma unroll
@@ -266,7 +270,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   const int row_rd = Tile::row_base16(n, g);
   const int col_rd = Tile::col_base16(lane);
   const uint32_t tiles_at = lds_address(&tiles[0][0]);
-  __syncthreads();
+  phase_barrier();  // (the masks; K and V may still be on their way)
 
   // Everything step (visit, head, qt) reads is requested a step ahead, straight into LDS stage st
   // and with nothing held in registers meanwhile: the Q and dO tiles, and one value per
@@ -367,6 +371,10 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
                        is_do ? i - Tile::LPW : i);
     }
   }
+  if constexpr (VL > 0 && WRITE_DS) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) v_park[w][kk][lane] = v_last[kk];
+  }
   if constexpr (WRITE_DS) wait_loads();  // (the wait at the top of a step counts on two stores behind the tile loads)
   while (visit < n_visits) {
     const int qt = __builtin_ctzll(rem);
@@ -466,11 +474,13 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       for (int qi = 0; qi < 2; ++qi)
         dp_acc[qi][0] = dp_acc[qi][1] = *reinterpret_cast<const f32x4*>(&delta_lds[st][QI * 32 + 16 * qi + 4 * g]);
       // Everything the sub-step's MFMAs read from LDS forms one stream, read AHEAD entries
-      // ahead into four rotating registers, across both matrix phases (the first operand of the
-      // second phase is on its way while the vector phase runs); an operand feeds two MFMAs, one per 16 keys:
+      // ahead into four rotating registers, across both matrix phases (the LSEs of the vector phase are on their way
+      // while the first runs, the first operands of the second while the vector phase does); an operand feeds two
+      // MFMAs, one per 16 keys:
       //   phase 1, per k-step and 16 queries: Q rows (-> S), dO rows (-> dP), [the parked V k-step, two B operands]
+      //   vector phase, per 16 queries: their LSEs
       //   phase 2, per 16-dim block d: dO^T (-> dV), Q^T (-> dK), over all 32 queries
-      constexpr int N1 = 4 * KS + 2 * VL, N2 = 2 * DB, NS = N1 + N2, AHEAD = 2, RING = 4, PRE = 1;
+      constexpr int N1 = 4 * KS + 2 * VL, NLSE = 2, P2 = N1 + NLSE, N2 = 2 * DB, NS = P2 + N2, AHEAD = 2, RING = 4;
       constexpr int FIRST_PARKED = 4 * (KS - VL);  // stream index of the k-step with the parked V
       // (there: Q, Q, V of 16 keys, dO, dO, V of the other 16, which meets both dO)
       enum { kQRows, kDoRows, kParkedV0, kParkedV1 };
@@ -486,7 +496,8 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
           if (kind >= kParkedV0) return v_park[w][kind - kParkedV0][lane];
           return Tile::read_row16(kind == kQRows ? q_lds : do_lds, row_rd_q, queries_of(o), step_of(o));
         }
-        const int i = o - N1;
+        if (o < P2) return *reinterpret_cast<const u32x4*>(&lse_lds[st][QI * 32 + 16 * (o - N1) + 4 * g]);
+        const int i = o - P2;
         return Tile::read_col16((i & 1) ? q_lds : do_lds, col_rd_q, 0, i / 2);
       };
       // this sub-step's half of the next step's tile loads: the Q tile (QI = 0) or the dO tile
@@ -516,9 +527,8 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
           dp_acc[0][1] = mfma_16x16x32<DTYPE>(buf[(o - 2) % RING], buf[o % RING], dp_acc[0][1]);
           dp_acc[1][1] = mfma_16x16x32<DTYPE>(buf[(o - 1) % RING], buf[o % RING], dp_acc[1][1]);
         }
-        // the entry just used (and the ones before it) are free: the next read goes there.  Only the
-        // first operand of the second phase is requested before the vector phase (registers)
-        if (o + AHEAD < N1 + PRE) buf[(o + AHEAD) % RING] = entry(o + AHEAD);
+        // the entry just used (and the ones before it) are free: the next read goes there
+        buf[(o + AHEAD) % RING] = entry(o + AHEAD);
         // this sub-step's half of the next step's tile loads, one per k-step
         if (o % 4 == 1 && o / 4 < NL / 2) {
           Tile::load_group_at(load_at + Tile::group_of_load(o / 4) * (Tile::GROUP_STRIDE * 2), load_src, goff0);
@@ -531,8 +541,11 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       __builtin_amdgcn_s_setprio(kPrioVector);
       u32x4 pb[2], dsb[2];  // [kk]: the lane's key, queries 4 g.. and 16 + 4 g..
 #pragma unroll
+      for (int o = P2; o < P2 + AHEAD; ++o) buf[o % RING] = entry(o);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
       for (int qi = 0; qi < 2; ++qi) {
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(&lse_lds[st][QI * 32 + 16 * qi + 4 * g]);
+        const f32x4 l4 = __builtin_bit_cast(f32x4, buf[(N1 + qi) % RING]);
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
           float pv[4], dsv[4];
@@ -560,14 +573,12 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       global_u32x4* piece = (global_u32x4*)(ds_step + (uint64_t)QI * ds_chunk_bytes) + ds_lane;
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(kPrioMatrix);
-#pragma unroll
-      for (int o = N1 + PRE; o < N1 + AHEAD; ++o) buf[o % RING] = entry(o);
       // ---- dV^T[dim, key] += dO^T[dim, q] P[q, key];  dK^T[dim, key] += Q^T[dim, q] dS[q, key]
       // over the sub-step's 32 queries (dO^T and Q^T come out of the row-major tiles by
       // transpose loads, in the accumulators' row order) ---------------------------------------
 #pragma unroll
-      for (int o = N1; o < NS; ++o) {
-        const int i = o - N1, d = i / 2;
+      for (int o = P2; o < NS; ++o) {
+        const int i = o - P2, d = i / 2;
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
           if (i & 1) dk_acc[d][kk] = mfma_16x16x32<DTYPE>(buf[o % RING], dsb[kk], dk_acc[d][kk]);
@@ -593,7 +604,8 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   }
 
   // ---- dK and dV of the wave's keys are complete: scale, round, store ---------------------
-  wait_loads();  // the last step's (unused) requests must land before the workgroup's LDS is released
+  wait_loads();  // the last step's (unused) requests must land before the workgroup's LDS is released, or used again
+  __syncthreads();
   // (what the loop did not need is worked out from the item's number again)
   KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
   asm volatile("" : "+s"(wg));
@@ -616,6 +628,10 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     end -= blk * args.block_size;
   }
   const float scale = args.scale;
+  const int64_t entry_off = (int64_t)entry * (where ? args.dkv2_entry_stride : args.dkv_slot_stride) + (int64_t)out_head * D;
+  const int64_t token_stride = where ? args.dkv2_token_stride : args.dkv_token_stride;
+  uint16_t* const dv_dst = reinterpret_cast<uint16_t*>(where ? args.dv2 : args.dv);
+  uint16_t* const dk_dst = reinterpret_cast<uint16_t*>(where ? args.dk2 : args.dk);
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     const int token = first + kk * 16 + n;
@@ -630,18 +646,50 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       }
       continue;
     }
-    const int64_t off = (int64_t)entry * (where ? args.dkv2_entry_stride : args.dkv_slot_stride) +
-                        (int64_t)(token) * (where ? args.dkv2_token_stride : args.dkv_token_stride) + (int64_t)out_head * D + 4 * g;
-    uint16_t* dv_dst = reinterpret_cast<uint16_t*>(where ? args.dv2 : args.dv) + off;
-    uint16_t* dk_dst = reinterpret_cast<uint16_t*>(where ? args.dk2 : args.dk) + off;
+    if (args.dkv_wide) continue;
+    const int64_t off = entry_off + (int64_t)token * token_stride + 4 * g;
 #pragma unroll
     for (int d = 0; d < DB; ++d) {
       const f32x4 v = dv_acc[d][kk], k = dk_acc[d][kk] * scale;
       const u32x2 v4 = {pack2<DTYPE>(v[0], v[1]), pack2<DTYPE>(v[2], v[3])};
-      *reinterpret_cast<u32x2*>(dv_dst + d * 16) = v4;
+      *reinterpret_cast<u32x2*>(dv_dst + off + d * 16) = v4;
       const u32x2 k4 = {pack2<DTYPE>(k[0], k[1]), pack2<DTYPE>(k[2], k[3])};
-      *reinterpret_cast<u32x2*>(dk_dst + d * 16) = k4;
+      *reinterpret_cast<u32x2*>(dk_dst + off + d * 16) = k4;
     }
+  }
+  if (where == 2 || !args.dkv_wide) return;
+  // A lane has four dims of a key, so its stores are eight bytes, 32 contiguous ones a key, and there are 64 of them a wave:
+  // 4.2 us at the end of every workgroup.  Through LDS (where the tiles were, a part of it to each wave) they
+  // become a quarter as many of whole rows, 1-2.
+  constexpr int ROW = D * 2 + 16;        // bytes of a key in LDS; the padding spreads a lane's eight over the banks
+  constexpr int PER_ROW = D * 2 / 16, ROWS = 64 / PER_ROW;  // lanes that store a key's row, keys in a store
+  static_assert(4 * 32 * ROW <= (int)sizeof(tiles), "a matrix of every wave fits where the tiles were");
+  const uint32_t at = tiles_at + w * (32 * ROW);
+  typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+  typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+#pragma unroll
+  for (int matrix = 0; matrix < 2; ++matrix) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const f32x4 x = matrix == 0 ? dv_acc[d][kk] : dk_acc[d][kk] * scale;
+        *(lds_u32x2*)(at + (kk * 16 + n) * ROW + d * 32 + g * 8) = u32x2{pack2<DTYPE>(x[0], x[1]), pack2<DTYPE>(x[2], x[3])};
+      }
+    // (other lanes of the wave read it: see closed_lds)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    uint16_t* dst = (matrix == 0 ? dv_dst : dk_dst) + entry_off + (lane % PER_ROW) * 8;
+#pragma unroll
+    for (int i = 0; i < 32 / ROWS; ++i) {
+      const int key = i * ROWS + lane / PER_ROW;
+      const u32x4 x = *(lds_u32x4*)(at + key * ROW + (lane % PER_ROW) * 16);
+      if (first + key < end) *reinterpret_cast<u32x4*>(dst + (int64_t)(first + key) * token_stride) = x;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 }
 
@@ -1189,6 +1237,9 @@ static int attn_bwd_launch(const void* dout, const void* q, const void* k, const
   p.dkv_partials = grouping ? grouping->partials : nullptr;
   p.dkv2_entry_stride = grouping ? grouping->entry_stride : 0;
   p.dkv2_token_stride = grouping ? grouping->token_stride : 0;
+  // 16-byte stores of dK and dV: everything a multiple of eight elements
+  p.dkv_wide = (((reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv) | reinterpret_cast<uintptr_t>(p.dk2) |
+                  reinterpret_cast<uintptr_t>(p.dv2)) & 15) | ((dkv_slot_stride | dkv_token_stride | p.dkv2_entry_stride | p.dkv2_token_stride) & 7)) == 0;
   p.kv_tiles_per_row = grouping ? block_size / kDkvBN : (int)(((int64_t)max_kv_blocks * block_size + kDkvBN - 1) / kDkvBN);
   p.n_dkv_items = (int64_t)(grouping ? grouping->n_groups : batch) * n_heads_kv * p.kv_tiles_per_row;
   p.n_dq_items = (int64_t)batch * n_heads_q * p.dq_tiles_per_row;

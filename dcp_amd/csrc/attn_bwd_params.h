@@ -66,6 +66,7 @@ struct AttnBwdParams {
   float* dkv_partials;        // where groups marked partial go
   int64_t dkv2_entry_stride;
   int64_t dkv2_token_stride;
+  int dkv_wide;          // dk, dv, dk2, dv2 and their strides allow 16-byte stores
   int dkv_xcd_group;     // dK/dV work items sharing one Q/dO stream (the key tiles of a row)
   int dq_xcd_group;      // dQ work items sharing one K/V stream
   int64_t n_dkv_items;   // (rows, or groups of rows) * n_heads_kv * kv_tiles_per_row
