@@ -63,7 +63,8 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   __shared__ __attribute__((aligned(16))) uint16_t ds_lds[kDsStages][kDsWaves][2048];  // [stage][wave]: one piece
   __shared__ int slot_lds[kSlotTableCap];
 
-  const int tid = threadIdx.x;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (per item: what is derived from it is not kept through the item before)
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int n = lane & 15;
@@ -75,10 +76,20 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   const int head = __builtin_amdgcn_readfirstlane(wg % (p.n_heads_q / HH)) * HH;  // the item's first head
   const int bi = __builtin_amdgcn_readfirstlane(wg / (p.n_heads_q / HH));
   const int b = __builtin_amdgcn_readfirstlane(p.row_order ? p.row_order[bi] : bi);
-  const int q_begin = p.cu_seqlens_q[b];
-  const int seqlen_q = p.cu_seqlens_q[b + 1] - q_begin;
-  const int kv_begin = p.cu_seqlens_kv[b];
-  const int seqlen_kv = p.cu_seqlens_kv[b + 1] - kv_begin;
+  // Everything the tables say of the row in one trip to memory: its bounds, where its dQ goes, its first kv slots (one a
+  // thread) and the hulls of the item's 64-query tiles (lanes 0..15: four words of each).
+  constexpr int T64 = kDsBM / 64;  // 64-query tiles of a workgroup
+  const int32_t* kv_table = p.kv_block_table + (int64_t)b * p.max_kv_blocks;
+  int q_begin = p.cu_seqlens_q[b], q_end = p.cu_seqlens_q[b + 1], kv_begin = p.cu_seqlens_kv[b], kv_end = p.cu_seqlens_kv[b + 1];
+  int dq_entry = p.dq_block_table[b], first_slots = 0, hulls = lane & 1 ? 0 : 0x7fffffff;  // (of a tile that is none: empty)
+  if (tid < min(p.max_kv_blocks, kSlotTableCap)) first_slots = kv_table[tid];
+  if (lane < 4 * T64 && T64 * qt + (lane >> 2) < p.q_tiles_per_row)
+    hulls = p.hull[((int64_t)b * p.q_tiles_per_row + T64 * qt + (lane >> 2)) * 8 + (lane & 3)];
+  asm volatile("" : "+v"(q_begin), "+v"(q_end), "+v"(kv_begin), "+v"(kv_end), "+v"(dq_entry), "+v"(first_slots), "+v"(hulls));
+  const int seqlen_q = __builtin_amdgcn_readfirstlane(q_end) - __builtin_amdgcn_readfirstlane(q_begin);
+  kv_begin = __builtin_amdgcn_readfirstlane(kv_begin);
+  dq_entry = __builtin_amdgcn_readfirstlane(dq_entry);
+  const int seqlen_kv = __builtin_amdgcn_readfirstlane(kv_end) - kv_begin;
   if (qt * kDsBM >= seqlen_q) return;
   const int kv_head = __builtin_amdgcn_readfirstlane(head / (p.n_heads_q / p.n_heads_kv));
   const int64_t q_row_stride = (int64_t)p.n_heads_q * D;
@@ -87,25 +98,17 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   // ---- which key tiles: the 128-key tiles the dK/dV kernel visited for this wave's 64-query tile
   // (the same test on the same hulls: a piece that was never written is never read), and for the
   // workgroup the hull of its two 64-query tiles -----------------------------------------------
-  constexpr int T64 = kDsBM / 64;  // 64-query tiles of a workgroup
-  const int qt64 = T64 * qt + (w >> 1);
-  const bool wave_has_tile = qt64 < p.q_tiles_per_row;
-  const int32_t* hull_row = p.hull + (int64_t)b * p.q_tiles_per_row * 8;
-  int hw[4] = {0x7fffffff, 0, 0x7fffffff, 0};
-  if (wave_has_tile) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) hw[i] = __builtin_amdgcn_readfirstlane(hull_row[qt64 * 8 + i]);
-  }
-  const TileRuns mine(hw[0], hw[1], hw[2], hw[3], 128);  // in 128-key tiles
+  const int own = w >> 1;  // of the item's 64-query tiles, the one this wave's queries lie in
+  const bool wave_has_tile = T64 * qt + own < p.q_tiles_per_row;
+  const TileRuns mine(__builtin_amdgcn_readlane(hulls, 4 * own), __builtin_amdgcn_readlane(hulls, 4 * own + 1),
+                      __builtin_amdgcn_readlane(hulls, 4 * own + 2), __builtin_amdgcn_readlane(hulls, 4 * own + 3), 128);  // in 128-key tiles
   int g[4] = {0x7fffffff, 0, 0x7fffffff, 0};
 #pragma unroll
   for (int t = 0; t < T64; ++t) {
-    if (T64 * qt + t >= p.q_tiles_per_row) continue;
-    const int32_t* hu = hull_row + (T64 * qt + t) * 8;
-    g[0] = min(g[0], __builtin_amdgcn_readfirstlane(hu[0]));
-    g[1] = max(g[1], __builtin_amdgcn_readfirstlane(hu[1]));
-    g[2] = min(g[2], __builtin_amdgcn_readfirstlane(hu[2]));
-    g[3] = max(g[3], __builtin_amdgcn_readfirstlane(hu[3]));
+    g[0] = min(g[0], __builtin_amdgcn_readlane(hulls, 4 * t));
+    g[1] = max(g[1], __builtin_amdgcn_readlane(hulls, 4 * t + 1));
+    g[2] = min(g[2], __builtin_amdgcn_readlane(hulls, 4 * t + 2));
+    g[3] = max(g[3], __builtin_amdgcn_readlane(hulls, 4 * t + 3));
   }
   TileRuns runs(g[0], g[1], g[2], g[3], 128);
   // as runs of 64-key tiles, none past the one that holds the row's last key
@@ -118,8 +121,8 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   if (runs.b1 < runs.a1) runs.b1 = runs.a1;
   const int n_tiles = runs.count();
 
-  const int32_t* kv_table = p.kv_block_table + (int64_t)b * p.max_kv_blocks;
-  load_slot_table(slot_lds, kv_table, p.max_kv_blocks, tid, kDsThreads);
+  if (tid < min(p.max_kv_blocks, kSlotTableCap)) slot_lds[tid] = first_slots;
+  load_slot_table(slot_lds, kv_table, p.max_kv_blocks, tid + kDsThreads, kDsThreads);
   __syncthreads();
 
   f32x4 dq_acc[HH][DB][2];  // dims 16 d + 4 g4.. of query 16 qi + n
@@ -275,7 +278,7 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
     if (q_local >= seqlen_q) continue;
 #pragma unroll
     for (int hh = 0; hh < HH; ++hh) {
-      uint16_t* op = reinterpret_cast<uint16_t*>(p.dq) + (int64_t)p.dq_block_table[b] * p.dq_slot_stride +
+      uint16_t* op = reinterpret_cast<uint16_t*>(p.dq) + (int64_t)dq_entry * p.dq_slot_stride +
                      (int64_t)q_local * q_row_stride + (int64_t)(head + hh) * D + 4 * g4;
 #pragma unroll
       for (int d = 0; d < DB; ++d) {
