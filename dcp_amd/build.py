@@ -10,6 +10,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -74,6 +75,24 @@ def build(verbose: bool = True) -> Path:
     return LIB_PATH
 
 
+PLAN_ANALYSIS_SRC = CSRC / "python" / "plan_analysis.cpp"
+PLAN_ANALYSIS_LIB = PKG_DIR / "_plan_analysis.so"
+
+
+def build_plan_analysis(verbose: bool = True) -> Path:
+    """Compiles the extension module ``dcp_amd._plan_analysis``: host code against Python's headers, so not a part of
+    the C-ABI library."""
+    # (not by hipcc, which would link a HIP runtime beside the one that torch brings)
+    cmd = [os.environ.get("CXX", "g++"), "-O3", "-std=c++17", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}",
+           str(PLAN_ANALYSIS_SRC), "-o", str(PLAN_ANALYSIS_LIB)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"plan analysis failed to build:\n{proc.stderr}")
+    if verbose:
+        print(f"built {PLAN_ANALYSIS_LIB}", file=sys.stderr)
+    return PLAN_ANALYSIS_LIB
+
+
 HOST_CHECK_SRC = PKG_DIR.parent / "tests" / "abi_host" / "abi_host_check.cpp"
 HOST_CHECK_BIN = HOST_CHECK_SRC.with_suffix("")
 
@@ -109,6 +128,7 @@ def build_bench_probes(verbose: bool = True) -> Path:
 
 if __name__ == "__main__":
     build()
+    build_plan_analysis()
     if LIB_PATH.name == "libdcp_hip.so":  # the host check links the library by its name
         build_abi_host_check()
         build_bench_probes()

@@ -35,6 +35,7 @@ from dcp_amd.core.instructions import (
     MemcpyInstr,
     SumInstr,
 )
+from dcp_amd.runtime.flash_attention import native
 
 
 @dataclass
@@ -66,10 +67,17 @@ _LOCAL_OF = {
 
 
 def analyse(plan: ExecutionPlan) -> DirectPlan:
-    result = DirectPlan()
     instrs = plan.instructions
     if any(isinstance(i, (CommLaunchInstr, CommWaitInstr, BarrierInstr)) for i in instrs):
-        return result
+        return DirectPlan()
+    found = native.direct(instrs)
+    return _analyse_any(plan) if found is None else DirectPlan(*found)
+
+
+def _analyse_any(plan: ExecutionPlan) -> DirectPlan:
+    """Of any plan; ``native.direct`` does the same for those that planners make."""
+    result = DirectPlan()
+    instrs = plan.instructions
 
     # A slot that holds a copy of a local block of the matching type: buffer type -> slot -> (memcpy
     # index, pair position, index and tokens of the local block)

@@ -37,6 +37,7 @@ from dcp_amd.core.instructions import (
     MemcpyInstr,
     SumInstr,
 )
+from dcp_amd.runtime.flash_attention import native
 from dcp_amd.runtime.flash_attention.direct import DirectPlan
 
 MAX_VISITS = 32  # DCP_ATTN_BWD_MAX_VISITS
@@ -202,6 +203,18 @@ def analyse(plan: ExecutionPlan, direct: DirectPlan, n_heads_kv: int, tiles_per_
                 n_visits, tiles_per_block * n_heads_kv, n_slots, q_heads_per_kv_head, 2 * tiles_per_block)
     if all(limit == 1 for limit in limits.values()) and all(p == (1, 1) for p in parts.values()):
         return result
+    if all(p == (1, 1) for p in parts.values()):  # (launches in parts have few pairs)
+        found = native.dkv(instrs, [limits.get(idx, 1) for idx in range(len(instrs))], direct.redirect_ops, Group)
+        if found is not None:
+            return DkvGroups(*found)
+    return _analyse_any(plan, direct, limits, parts, q_heads_per_kv_head)
+
+
+def _analyse_any(plan: ExecutionPlan, direct: DirectPlan, limits: Dict[int, int], parts: Dict[int, Tuple[int, int]],
+                 q_heads_per_kv_head: int) -> DkvGroups:
+    """Of any plan; ``native.dkv`` does the same for those that planners make, where no launch is in parts."""
+    result = DkvGroups()
+    instrs = plan.instructions
     visits = _Visits(instrs)
     row_of, pos_of, slot_of = visits.row, visits.pos, visits.slot
     # which visit wrote a BUFFER_dKV slot last, if a backward kernel did, and which sum op reads what it wrote

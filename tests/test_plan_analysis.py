@@ -1,0 +1,185 @@
+"""The native analyses of a plan (``runtime/flash_attention/native.py``) find what the Python ones find, in plans as
+planners make them and in plans changed at random, and leave to them what they do not take (CPU)."""
+
+import copy
+import random
+
+import numpy as np
+import pytest
+
+from dcp_amd.core.instructions import (
+    AttnBackwardInstr,
+    AttnInstr,
+    AttnReductionInstr,
+    BarrierInstr,
+    BufferBlock,
+    BufferType,
+    MemcpyInstr,
+    ReductionOp,
+    SumInstr,
+    SumOp,
+)
+from dcp_amd.runtime.flash_attention import direct, dkv_groups, executor, native
+from tests.plan_cases import make_case
+
+CASES = {
+    "causal_gqa": dict(seqlens=[1100, 300, 1, 129], block_size=128, n_heads=8, n_groups=2, head_dim=128, head_block=2),
+    "split": dict(seqlens=[900, 130], block_size=128, n_heads=4, n_groups=2, head_dim=64, head_block=1, n_kv_groups=2, kv_split="contiguous"),
+    "folded": dict(seqlens=[900, 130], block_size=128, n_heads=4, n_groups=2, head_dim=64, head_block=1, n_kv_groups=3, fold=True),
+    "lambda": dict(seqlens=[2500, 130], block_size=128, n_heads=4, n_groups=1, head_dim=128, head_block=2, mask="lambda",
+                   mask_kwargs=dict(n_starting=16, l_pretrain=300)),
+    "many_rows": dict(seqlens=[41 * 128 - 5], block_size=128, n_heads=2, n_groups=2, head_dim=128, head_block=2),
+}
+
+
+def _plans(name):
+    case = make_case(**CASES[name])
+    return case["fw"], case["bw"]
+
+
+def _same_direct(plan):
+    found = native.direct(plan.instructions)
+    assert found is not None
+    assert direct.DirectPlan(*found) == direct._analyse_any(plan)
+
+
+def _same_groups(plan, limit, analysed):
+    limits = {i: limit for i, instr in enumerate(plan.instructions) if isinstance(instr, AttnBackwardInstr)}
+    found = native.dkv(plan.instructions, [limits.get(i, 1) for i in range(len(plan.instructions))], analysed.redirect_ops, dkv_groups.Group)
+    assert found is not None
+    expected = dkv_groups._analyse_any(plan, analysed, limits, {i: (1, 1) for i in limits}, 1)
+    assert dkv_groups.DkvGroups(*found) == expected
+    assert list(found[0]) == list(expected.groups)
+
+
+def test_the_module_is_built():
+    assert native._plan_analysis is not None
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_plans_of_the_planner(name):
+    for plan in _plans(name):
+        _same_direct(plan)
+        for limit in (2, 3, 8, 32):
+            for analysed in (direct.DirectPlan(), direct._analyse_any(plan)):
+                _same_groups(plan, limit, analysed)
+
+
+def _changed(plan, rng):
+    """The plan with a few blocks, ops and pairs exchanged, dropped, repeated or of another size or type."""
+    plan = copy.copy(plan)
+    plan.instructions = instrs = [copy.copy(i) for i in plan.instructions]
+
+    def other(block):
+        how = rng.randrange(4)
+        if how == 0:
+            return BufferBlock(block.buffer_type, max(0, block.index + rng.choice((-1, 1, 40))), block.n_tokens)
+        if how == 1:
+            return BufferBlock(block.buffer_type, block.index, block.n_tokens + rng.choice((-1, 1)))
+        if how == 2:
+            return BufferBlock(rng.choice([v for k, v in vars(BufferType).items() if k[:2] in ("LO", "BU")]), block.index, block.n_tokens)
+        return BufferBlock(str(b"".join([block.buffer_type.encode()]), "ascii"), block.index, block.n_tokens)  # a string of its own
+
+    def in_list(items, change):
+        items = list(items)
+        if not items:
+            return items
+        at, how = rng.randrange(len(items)), rng.randrange(6)
+        if how == 0:
+            items.insert(rng.randrange(len(items)), items[at])
+        elif how == 1 and len(items) > 1:
+            del items[at]
+        elif how == 2:
+            rng.shuffle(items)
+        else:
+            items[at] = change(items[at])
+        return items
+
+    for _ in range(rng.randint(1, 6)):
+        instr = rng.choice(instrs)
+        if isinstance(instr, MemcpyInstr):
+            instr.src_dst_pairs = in_list(instr.src_dst_pairs, lambda p: (other(p[0]), p[1]) if rng.random() < 0.5 else (p[0], other(p[1])))
+        elif isinstance(instr, (AttnInstr, AttnBackwardInstr)):
+            names = ["q_block_table", "kv_block_table", "out_block_table"]
+            names += ["dq_block_table", "dkv_block_table"] if isinstance(instr, AttnBackwardInstr) else []
+            name = rng.choice(names)
+            table = [list(row) for row in getattr(instr, name)]
+            row = table[rng.randrange(len(table))]
+            at = rng.randrange(len(row))
+            row[at] = other(row[at])
+            setattr(instr, name, table)
+        elif isinstance(instr, SumInstr):
+            instr.ops = in_list(instr.ops, lambda op: SumOp(in_list(op.src_buffers, other), op.dst_buffer) if rng.random() < 0.5
+                                else SumOp(op.src_buffers, other(op.dst_buffer)))
+        elif isinstance(instr, AttnReductionInstr):
+            instr.ops = in_list(instr.ops, lambda op: ReductionOp(in_list(op.src_buffers, lambda p: p), op.dst_buffer))
+    if rng.random() < 0.2:
+        instrs.insert(rng.randrange(len(instrs) + 1), copy.copy(rng.choice(instrs)))
+    return plan
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_changed_plans(name):
+    rng = random.Random(name)
+    taken = 0
+    for plan in _plans(name):
+        for _ in range(60):
+            changed = _changed(plan, rng)
+            try:
+                expected = direct._analyse_any(changed)
+            except (IndexError, TypeError, AttributeError):
+                assert native.direct(changed.instructions) is None  # the Python code raises it
+                continue
+            found = native.direct(changed.instructions)
+            if found is not None:
+                taken += 1
+                assert direct.DirectPlan(*found) == expected
+            for limit in (2, 5, 32):
+                try:
+                    _ = dkv_groups._analyse_any(changed, expected, {i: limit for i, x in enumerate(changed.instructions) if isinstance(x, AttnBackwardInstr)},
+                                                {i: (1, 1) for i, x in enumerate(changed.instructions) if isinstance(x, AttnBackwardInstr)}, 1)
+                except (IndexError, KeyError):
+                    continue
+                _same_groups(changed, limit, expected)
+    assert taken > 60
+
+
+def test_what_is_left_to_the_python_code():
+    class Block(BufferBlock):
+        pass
+
+    class Other:
+        ops, output_is_unpadded = [], 0
+
+    block = BufferBlock(BufferType.BUFFER_Q, 3, 128)
+    local = BufferBlock(BufferType.LOCAL_Q, 3, 128)
+    for bad in (Block(BufferType.BUFFER_Q, 3, 128), BufferBlock("AnotherBuffer", 3, 128), BufferBlock(BufferType.BUFFER_Q, -1, 128),
+                BufferBlock(BufferType.BUFFER_Q, 1 << 40, 128), BufferBlock(BufferType.BUFFER_Q, 1 << 70, 128), BufferBlock(BufferType.BUFFER_Q, True, 128)):
+        assert native.direct([MemcpyInstr([(local, block)])]) is not None
+        assert native.direct([MemcpyInstr([(local, bad)])]) is None
+    assert native.direct([MemcpyInstr([(local, block, block)])]) is None
+    assert native.direct([MemcpyInstr(iter([(local, block)]))]) is None
+    assert native.direct([SumInstr([], 0)]) is not None and native.direct([Other()]) is None
+    assert native.direct([BarrierInstr()]) is None
+    with pytest.raises(AttributeError):
+        instr = MemcpyInstr([(local, block)])
+        del instr.src_dst_pairs
+        native.direct([instr])
+
+
+def test_padded_tables():
+    rng = random.Random(0)
+    cu = [rng.randrange(1 << 30) for _ in range(50)]
+    for width in (1, 3, 17):
+        rows = [[rng.randrange(50) for _ in range(rng.randint(0, width))] for _ in range(40)]
+        blocks = [[BufferBlock(BufferType.BUFFER_KV, i, 1) for i in row] for row in rows]
+        for got, expected in ((native.padded(rows, width, cu), executor._padded([[cu[i] for i in row] for row in rows], width)),
+                              (native.padded(blocks, width), executor._padded(rows, width))):
+            assert got.dtype == np.int32 and np.array_equal(got, expected)
+    single = [rng.randrange(50) for _ in range(9)]
+    assert np.array_equal(native.padded(single, 1, cu), [[cu[i]] for i in single])
+    assert np.array_equal(native.padded(single, 3, cu), [[cu[i], -1, -1] for i in single])
+    block = BufferBlock(BufferType.BUFFER_KV, 1 << 31, 1)
+    for rows, width, starts in (([[0, 1]], 1, cu), ([[50]], 1, cu), ([[-1]], 1, cu), ([0, [1]], 1, cu), ([[0]], 1, [1 << 31]), ([], 1, cu),
+                                ([[]], 0, cu), ([[block]], 1, None), ([[0]], 1, None)):
+        assert native.padded(rows, width, starts) is None
