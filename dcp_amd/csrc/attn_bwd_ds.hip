@@ -28,8 +28,10 @@
 // head has an even number of q heads a work item takes two of them, alternating between them tile
 // by tile: a K tile in LDS serves both heads' pieces (half the K loads again), and the waves meet at
 // a barrier only where the K tile changes, every other step.  On the 65536-token causal benchmark
-// (16.8 GB of dS) the kernel takes 3.0 ms, 5.9 TB/s out of HBM; with one head per item 3.2 ms;
-// with four-wave workgroups, two stages and a full wait per tile 3.4 ms.  A kernel that only
+// (16.8 GB of dS) the kernel takes 2.95-3.0 ms, 6.1 TB/s out of HBM; with one head per item 3.2 ms;
+// with four-wave workgroups, two stages and a full wait per tile 3.4 ms.  Four-wave workgroups with four (head size 128)
+// or six (64) stages, where a launch leaves CUs idle, are no faster either: backward of 40 items 45.6 -> 45.8 us, of 144
+// 122.4 -> 122.4, of 176 of head size 64 72.0 -> 78.4, of 448 262 -> 289.  A kernel that only
 // streams 4 KiB pieces per wave into LDS the same way reads 7.0 TB/s (6.6 with a workgroup barrier
 // per step, 6.0-6.2 with a K tile's loads beside it); the rest is the start of every work item (a
 // chain of dependent table reads and an empty pipeline: with no tiles at all the kernel takes
@@ -77,7 +79,8 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
   const int bi = __builtin_amdgcn_readfirstlane(wg / (p.n_heads_q / HH));
   const int b = __builtin_amdgcn_readfirstlane(p.row_order ? p.row_order[bi] : bi);
   // Everything the tables say of the row in one trip to memory: its bounds, where its dQ goes, its first kv slots (one a
-  // thread) and the hulls of the item's 64-query tiles (lanes 0..15: four words of each).
+  // thread) and the hulls of the item's 64-query tiles (lanes 0..15: four words of each).  Backward of 4800 tokens, 8 kv
+  // heads, 96.9 -> 96.2 us; 1024 tokens 59.7 -> 58.3; 16384 tokens of 16 heads in blocks of 256 709 -> 706.
   constexpr int T64 = kDsBM / 64;  // 64-query tiles of a workgroup
   const int32_t* kv_table = p.kv_block_table + (int64_t)b * p.max_kv_blocks;
   int q_begin = p.cu_seqlens_q[b], q_end = p.cu_seqlens_q[b + 1], kv_begin = p.cu_seqlens_kv[b], kv_end = p.cu_seqlens_kv[b + 1];
