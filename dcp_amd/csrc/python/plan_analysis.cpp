@@ -8,11 +8,17 @@
 // These functions take the plans that planners make: lists and tuples of BufferBlock, ReductionOp and SumOp
 // themselves, plain integers and strings, slot numbers that index an array.  For anything else they return None and
 // change nothing, and the Python code, which takes every plan, does it.
+//
+// They read a plan without owning it: its lists' storage, its blocks, its strings.  So nothing of Python's may run before
+// the last look at it -- no call of a class or of an object's methods, and no new object that the garbage collector
+// counts, since a collection runs finalisers and either may let another thread in, which may change the plan.  An analysis
+// therefore has two parts: it reads the whole plan, and takes references to what the results hold; then it makes them.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <algorithm>
 #include <cstdint>
+#include <map>
 #include <memory>
 #include <new>
 #include <utility>
@@ -31,6 +37,10 @@ typedef std::unique_ptr<PyObject, Drop> Ref;
 Ref own(PyObject* o) {
   if (o == nullptr) throw PythonError();
   return Ref(o);
+}
+Ref share(PyObject* borrowed) {
+  Py_INCREF(borrowed);
+  return Ref(borrowed);
 }
 void check(int status) {
   if (status != 0) throw PythonError();
@@ -162,9 +172,8 @@ struct Instrs {
   }
   bool flag(Py_ssize_t i, const char* name) {
     const Ref value = own(PyObject_GetAttrString(list[i], name));
-    const int truth = PyObject_IsTrue(value.get());
-    if (truth < 0) throw PythonError();
-    return truth != 0;
+    if (PyBool_Check(value.get())) return value.get() == Py_True;
+    return integer(value.get()) != 0;  // (any other object's truth is its own code's to say)
   }
 };
 Seq op_sources(PyObject* op, PyTypeObject* type) {
@@ -369,7 +378,7 @@ PyObject* direct(PyObject* instr_list, PyObject* kind_list) {
   std::vector<std::pair<int, int>> skip_ops;
   struct Redirect {
     int instr, pos;
-    PyObject* dst;
+    Ref dst;
   };
   std::vector<Redirect> redirects;
   for (Py_ssize_t idx = 0; idx < instrs.size(); ++idx) {
@@ -412,14 +421,14 @@ PyObject* direct(PyObject* instr_list, PyObject* kind_list) {
         PyObject* dst = dst_of(*p, kSum);
         const Block to = reader.block(dst);
         if (!is_local(to.type) || to.n_tokens != reader.block(field(ops[pos], s_dst_buffer)).n_tokens) continue;
-        redirects.push_back({(int)idx, (int)pos, dst});
+        redirects.push_back({(int)idx, (int)pos, share(dst)});
         skip_ops.emplace_back(p->instr, p->pos);
       }
     }
   }
   for (const int c : blocked) copied[copies[c].instr][copies[c].pos] = 0;
 
-  // ---- as Python objects ----
+  // ---- as Python objects (the plan is not looked at from here on) ----
   const Ref skip_pairs = own(PyDict_New()), operand_dict = own(PyDict_New()), skip_dict = own(PyDict_New()), redirect_dict = own(PyDict_New());
   auto entry = [](PyObject* dict, int64_t key, PyObject* (*make)()) {  // dict.setdefault(key, make()), borrowed
     const Ref k = own(PyLong_FromLongLong(key));
@@ -463,7 +472,7 @@ PyObject* direct(PyObject* instr_list, PyObject* kind_list) {
   for (const auto& [instr, pos] : skip_ops) add(entry(skip_dict.get(), instr, new_set), pos);
   for (const Redirect& r : redirects) {
     const Ref pos = own(PyLong_FromLong(r.pos));
-    check(PyDict_SetItem(entry(redirect_dict.get(), r.instr, new_dict), pos.get(), r.dst));
+    check(PyDict_SetItem(entry(redirect_dict.get(), r.instr, new_dict), pos.get(), r.dst.get()));
   }
   return PyTuple_Pack(4, skip_pairs.get(), operand_dict.get(), skip_dict.get(), redirect_dict.get());
 }
@@ -484,7 +493,19 @@ std::vector<int> chunk_sizes(int n_visits, int limit) {
 PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, PyObject* redirect_ops, PyObject* group_type) {
   Instrs instrs(instr_list, kind_list);
   const Seq limits(limit_list);  // rows a group may visit, per instruction
-  if (limits.n != instrs.size() || !PyDict_CheckExact(redirect_ops)) throw NotTaken();
+  if (limits.n != instrs.size()) throw NotTaken();
+  std::map<std::pair<int64_t, int64_t>, PyObject*> redirects;  // sum instruction and position of the op -> where it goes
+  {
+    auto for_each = [](PyObject* dict, auto&& body) {  // (a lookup would compare its keys, with their own code)
+      if (!PyDict_CheckExact(dict)) throw NotTaken();
+      Py_ssize_t at = 0;
+      PyObject *key, *value;
+      while (PyDict_Next(dict, &at, &key, &value)) body(integer(key), value);
+    };
+    for_each(redirect_ops, [&](int64_t instr, PyObject* of_instr) {
+      for_each(of_instr, [&](int64_t pos, PyObject* dst) { redirects[{instr, pos}] = dst; });
+    });
+  }
   Reader reader;
   constexpr int kUnread = -1, kElsewhere = -2;
   struct Visit {
@@ -559,7 +580,13 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
     }
   }
 
-  const Ref groups_of = own(PyDict_New()), skip_dict = own(PyDict_New()), source_dict = own(PyDict_New());
+  struct Group {
+    std::vector<int> visits;
+    PyObject* dst;  // borrowed from the plan while it is read
+    int rank, component;
+    Ref owned;  // dst
+  };
+  std::vector<std::pair<Py_ssize_t, std::vector<Group>>> groups_of;  // of the backward instructions
   std::vector<std::vector<char>> gone_of(sums.size());  // per sum op, its sources that the kernel has added already
   std::vector<char> filtered(sums.size(), 0), skipped(sums.size(), 0);
   for (Py_ssize_t idx = 0; idx < instrs.size(); ++idx) {
@@ -628,13 +655,9 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
       number = most.first;
       window = number > 2 && 2 * most.second > (int)(together.size() + alone.size());
     }
-    struct Group {
-      std::vector<int> visits;
-      PyObject* dst;  // borrowed from the plan
-      int rank, component;
-    };
     std::vector<Group> groups;
-    for (const int v : alone) groups.push_back({{v}, visits[v].slot, 0, 0});
+    auto add_group = [&](std::vector<int> taken, PyObject* dst) { groups.push_back({std::move(taken), dst, 0, 0, nullptr}); };
+    for (const int v : alone) add_group({v}, visits[v].slot);
     for (Together& t : together) {
       std::stable_sort(t.taken.begin(), t.taken.end(), [&](int a, int b) {
         const int ra = visits[a].row, rb = visits[b].row;
@@ -645,20 +668,12 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
       const Seq sources = op_sources(sum.op, sum_op_type);
       const int rows = (int)t.taken.size();
       PyObject* dst = nullptr;  // where the sum goes, if that is an unpadded tensor
-      {
-        const Ref j = own(PyLong_FromLong(sum.instr)), pos = own(PyLong_FromLong(sum.pos));
-        PyObject* of_instr = PyDict_GetItemWithError(redirect_ops, j.get());
-        if (of_instr != nullptr) {
-          if (!PyDict_CheckExact(of_instr)) throw NotTaken();
-          dst = PyDict_GetItemWithError(of_instr, pos.get());
-        }
-        if (PyErr_Occurred()) throw PythonError();
-      }
+      if (const auto known = redirects.find({sum.instr, sum.pos}); known != redirects.end()) dst = known->second;
       if (dst == nullptr && instrs.flag(sum.instr, "output_is_unpadded")) dst = field(sum.op, s_dst_buffer);
       if (rows <= limit && rows == sources.n && dst != nullptr) {
         const Block to = reader.block(dst);
         if (to.type == kLocaldKV && to.n_tokens == visits[t.taken[0]].n_tokens && named.get(to.index) == 1) {
-          groups.push_back({t.taken, dst, 0, 0});
+          add_group(t.taken, dst);
           skipped[t.who] = 1;
           continue;
         }
@@ -669,7 +684,7 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
       SlotMap<char> added(0);
       int at = 0;
       for (const int size : rows > limit ? chunk_sizes(rows, limit) : std::vector<int>{rows}) {
-        groups.push_back({std::vector<int>(t.taken.begin() + at, t.taken.begin() + at + size), visits[t.taken[at]].slot, 0, 0});
+        add_group(std::vector<int>(t.taken.begin() + at, t.taken.begin() + at + size), visits[t.taken[at]].slot);
         for (int i = 1; i < size; ++i) added.set(visits[t.taken[at + i]].index, 1);
         at += size;
       }
@@ -721,6 +736,20 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
       if (a.visits.size() != b.visits.size()) return a.visits.size() > b.visits.size();
       return a.rank != b.rank ? a.rank < b.rank : a.component < b.component;
     });
+    for (Group& g : groups) g.owned = share(g.dst);
+    groups_of.emplace_back(idx, std::move(groups));
+  }
+  std::vector<std::vector<Ref>> left_of(sums.size());  // what a sum op still adds
+  for (size_t who = 0; who < sums.size(); ++who) {
+    if (!filtered[who]) continue;
+    const Seq sources = op_sources(sums[who].op, sum_op_type);
+    for (Py_ssize_t i = 0; i < sources.n; ++i)
+      if (!gone_of[who][i]) left_of[who].push_back(share(sources[i]));
+  }
+
+  // ---- as Python objects (the plan is not looked at from here on) ----
+  const Ref group_dict = own(PyDict_New()), skip_dict = own(PyDict_New()), source_dict = own(PyDict_New());
+  for (const auto& [idx, groups] : groups_of) {
     const Ref list = own(PyList_New(groups.size()));
     for (size_t i = 0; i < groups.size(); ++i) {
       Ref pairs = own(PyList_New(groups[i].visits.size()));
@@ -729,10 +758,10 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
         Ref row = own(PyLong_FromLong(v.row)), pos = own(PyLong_FromLong(v.pos));
         PyList_SET_ITEM(pairs.get(), k, own(PyTuple_Pack(2, row.get(), pos.get())).release());
       }
-      PyList_SET_ITEM(list.get(), i, own(PyObject_CallFunctionObjArgs(group_type, pairs.get(), groups[i].dst, nullptr)).release());
+      PyList_SET_ITEM(list.get(), i, own(PyObject_CallFunctionObjArgs(group_type, pairs.get(), groups[i].owned.get(), nullptr)).release());
     }
     const Ref key = own(PyLong_FromSsize_t(idx));
-    check(PyDict_SetItem(groups_of.get(), key.get(), list.get()));
+    check(PyDict_SetItem(group_dict.get(), key.get(), list.get()));
   }
   auto entry = [](PyObject* dict, int key, bool set) {
     const Ref k = own(PyLong_FromLong(key));
@@ -747,13 +776,11 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
     const Ref pos = own(PyLong_FromLong(sums[who].pos));
     if (skipped[who]) check(PySet_Add(entry(skip_dict.get(), sums[who].instr, true), pos.get()));
     if (!filtered[who]) continue;
-    const Seq sources = op_sources(sums[who].op, sum_op_type);
-    const Ref left = own(PyList_New(0));
-    for (Py_ssize_t i = 0; i < sources.n; ++i)
-      if (!gone_of[who][i]) check(PyList_Append(left.get(), sources[i]));
+    const Ref left = own(PyList_New(left_of[who].size()));
+    for (size_t i = 0; i < left_of[who].size(); ++i) PyList_SET_ITEM(left.get(), i, left_of[who][i].release());
     check(PyDict_SetItem(entry(source_dict.get(), sums[who].instr, false), pos.get(), left.get()));
   }
-  return PyTuple_Pack(3, groups_of.get(), skip_dict.get(), source_dict.get());
+  return PyTuple_Pack(3, group_dict.get(), skip_dict.get(), source_dict.get());
 }
 
 // ---- a block table as int32 [rows, width], filled up with -1 (executor.py: _padded) -------------------

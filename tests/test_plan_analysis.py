@@ -183,3 +183,49 @@ def test_padded_tables():
     for rows, width, starts in (([[0, 1]], 1, cu), ([[50]], 1, cu), ([[-1]], 1, cu), ([0, [1]], 1, cu), ([[0]], 1, [1 << 31]), ([], 1, cu),
                                 ([[]], 0, cu), ([[block]], 1, None), ([[0]], 1, None)):
         assert native.padded(rows, width, starts) is None
+
+
+@pytest.mark.parametrize("name", list(CASES))
+@pytest.mark.parametrize("limit", [2, 32])
+def test_the_plan_is_read_before_anything_of_pythons_runs(name, limit):
+    """The groups are instances of a class of Python's, whose code may change the plan, or let a thread in that
+    does: the plan has been read by then."""
+    plan = copy.deepcopy(_plans(name)[1])
+    instrs = plan.instructions
+    limits = [limit if isinstance(i, AttnBackwardInstr) else 1 for i in instrs]
+    analysed = direct._analyse_any(plan)
+    expected = native.dkv(copy.deepcopy(instrs), limits, copy.deepcopy(analysed.redirect_ops), dkv_groups.Group)
+
+    class Emptying(dkv_groups.Group):
+        __eq__ = dkv_groups.Group.__eq__
+
+        def __init__(self, *args):
+            super().__init__(*args)
+            for i in instrs:
+                if isinstance(i, AttnBackwardInstr):
+                    for row in i.kv_block_table + i.dkv_block_table:
+                        row[:] = [BufferBlock(BufferType.BUFFER_dKV, 0, 1)]
+                elif isinstance(i, SumInstr):
+                    for op in i.ops:
+                        op.src_buffers, op.dst_buffer = [], None
+            for ops in analysed.redirect_ops.values():
+                ops.clear()
+
+    fields = lambda groups: {i: [(g.visits, g.dst) for g in of] for i, of in groups.items()}
+    found = native.dkv(instrs, limits, analysed.redirect_ops, Emptying)
+    assert fields(found[0]) == fields(expected[0]) and found[1:] == expected[1:]
+    assert all(not op.src_buffers for i in instrs if isinstance(i, SumInstr) for op in i.ops)  # (it was changed)
+
+
+def test_a_flag_with_a_truth_of_its_own_is_left_to_the_python_code():
+    class Flag:
+        def __bool__(self):
+            raise AssertionError("asked while the plan is read")
+
+    for flag, taken in ((0, True), (1, True), (True, True), (-3, True), (np.int64(1), False), (None, False), (Flag(), False)):
+        assert (native.direct([SumInstr([], flag)]) is not None) == taken
+    block, local = BufferBlock(BufferType.BUFFER_dKV, 3, 128), BufferBlock(BufferType.LOCAL_dKV, 3, 128)
+    back = AttnBackwardInstr.__new__(AttnBackwardInstr)
+    back.kv_block_table, back.dkv_block_table = [[block]], [[block]]
+    for flag, taken in ((1, True), (Flag(), False)):
+        assert (native.dkv([back, SumInstr([SumOp([block], local)], flag)], [2, 1], {}, dkv_groups.Group) is not None) == taken
