@@ -3,6 +3,7 @@ planners make them and in plans changed at random, and leave to them what they d
 
 import copy
 import random
+import time
 
 import numpy as np
 import pytest
@@ -229,3 +230,28 @@ def test_a_flag_with_a_truth_of_its_own_is_left_to_the_python_code():
     back.kv_block_table, back.dkv_block_table = [[block]], [[block]]
     for flag, taken in ((1, True), (Flag(), False)):
         assert (native.dkv([back, SumInstr([SumOp([block], local)], flag)], [2, 1], {}, dkv_groups.Group) is not None) == taken
+
+
+def test_high_slot_numbers_cost_no_more_than_in_python():
+    """What the native analysis keeps per slot number is kept once, not once a sum op."""
+    plan = make_case(seqlens=[16384], block_size=128, n_heads=4, n_groups=4, head_dim=64, head_block=1)["bw"]
+    high = lambda b: BufferBlock(b.buffer_type, b.index + 4100000, b.n_tokens) if b.buffer_type == BufferType.BUFFER_dKV else b
+    plan.instructions = [copy.copy(i) for i in plan.instructions]
+    for i in plan.instructions:
+        if isinstance(i, AttnBackwardInstr):
+            i.dkv_block_table = [[high(b) for b in row] for row in i.dkv_block_table]
+        elif isinstance(i, SumInstr):
+            i.ops = [SumOp([high(b) for b in op.src_buffers], high(op.dst_buffer)) for op in i.ops]
+    analysed = direct._analyse_any(plan)
+    _same_groups(plan, 8, analysed)
+    limits = {i: 8 for i, x in enumerate(plan.instructions) if isinstance(x, AttnBackwardInstr)}
+
+    def seconds(analysis):
+        begin = time.process_time()
+        analysis()
+        return time.process_time() - begin
+
+    by_instr = [limits.get(i, 1) for i in range(len(plan.instructions))]
+    natively = min(seconds(lambda: native.dkv(plan.instructions, by_instr, analysed.redirect_ops, dkv_groups.Group)) for _ in range(3))
+    in_python = min(seconds(lambda: dkv_groups._analyse_any(plan, analysed, limits, {i: (1, 1) for i in limits}, 1)) for _ in range(3))
+    assert natively < in_python, (natively, in_python)
