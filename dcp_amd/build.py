@@ -11,8 +11,10 @@ import os
 import subprocess
 import sys
 import sysconfig
+import warnings
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
+from typing import Optional
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
@@ -76,18 +78,27 @@ def build(verbose: bool = True) -> Path:
 
 
 PLAN_ANALYSIS_SRC = CSRC / "python" / "plan_analysis.cpp"
-PLAN_ANALYSIS_LIB = PKG_DIR / "_plan_analysis.so"
+# (with the tag of this Python's ABI: any other would load a file without one, and the module is not of the stable ABI)
+PLAN_ANALYSIS_LIB = PKG_DIR / f"_plan_analysis{sysconfig.get_config_var('EXT_SUFFIX')}"
 
 
-def build_plan_analysis(verbose: bool = True) -> Path:
+def build_plan_analysis(verbose: bool = True) -> Optional[Path]:
     """Compiles the extension module ``dcp_amd._plan_analysis``: host code against Python's headers, so not a part of
-    the C-ABI library."""
+    the C-ABI library.  The package does without it (preparing a plan then takes longer), so where there is no compiler
+    or no header it is left out, with a warning, and None is returned."""
+    for older in (PLAN_ANALYSIS_LIB, PLAN_ANALYSIS_LIB.with_name("_plan_analysis.so")):
+        older.unlink(missing_ok=True)
     # (not by hipcc, which would link a HIP runtime beside the one that torch brings)
     cmd = [os.environ.get("CXX", "g++"), "-O3", "-std=c++17", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}",
            str(PLAN_ANALYSIS_SRC), "-o", str(PLAN_ANALYSIS_LIB)]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"plan analysis failed to build:\n{proc.stderr}")
+    try:
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        error = proc.stderr if proc.returncode != 0 else None
+    except OSError as e:
+        error = str(e)
+    if error is not None:
+        warnings.warn(f"built without the native plan analysis: {error}", RuntimeWarning, stacklevel=2)
+        return None
     if verbose:
         print(f"built {PLAN_ANALYSIS_LIB}", file=sys.stderr)
     return PLAN_ANALYSIS_LIB
@@ -128,7 +139,7 @@ def build_bench_probes(verbose: bool = True) -> Path:
 
 if __name__ == "__main__":
     build()
-    build_plan_analysis()
     if LIB_PATH.name == "libdcp_hip.so":  # the host check links the library by its name
         build_abi_host_check()
         build_bench_probes()
+    build_plan_analysis()
