@@ -233,8 +233,9 @@ def test_a_flag_with_a_truth_of_its_own_is_left_to_the_python_code():
 
 
 def test_high_slot_numbers_cost_no_more_than_in_python():
-    """What the native analysis keeps per slot number is kept once, not once a sum op."""
-    plan = make_case(seqlens=[16384], block_size=128, n_heads=4, n_groups=4, head_dim=64, head_block=1)["bw"]
+    """What the native analysis keeps per slot number is kept once, not once a sum op (3200 of the ops here are added in
+    part: 0.57 s with a map each, 0.08 with one, in Python 0.11)."""
+    plan = make_case(seqlens=[384] * 800, block_size=128, n_heads=4, n_groups=4, head_dim=64, head_block=1)["bw"]
     high = lambda b: BufferBlock(b.buffer_type, b.index + 4100000, b.n_tokens) if b.buffer_type == BufferType.BUFFER_dKV else b
     plan.instructions = [copy.copy(i) for i in plan.instructions]
     for i in plan.instructions:
@@ -243,8 +244,8 @@ def test_high_slot_numbers_cost_no_more_than_in_python():
         elif isinstance(i, SumInstr):
             i.ops = [SumOp([high(b) for b in op.src_buffers], high(op.dst_buffer)) for op in i.ops]
     analysed = direct._analyse_any(plan)
-    _same_groups(plan, 8, analysed)
-    limits = {i: 8 for i, x in enumerate(plan.instructions) if isinstance(x, AttnBackwardInstr)}
+    _same_groups(plan, 2, analysed)
+    limits = {i: 2 for i, x in enumerate(plan.instructions) if isinstance(x, AttnBackwardInstr)}
 
     def seconds(analysis):
         begin = time.process_time()
@@ -254,4 +255,4 @@ def test_high_slot_numbers_cost_no_more_than_in_python():
     by_instr = [limits.get(i, 1) for i in range(len(plan.instructions))]
     natively = min(seconds(lambda: native.dkv(plan.instructions, by_instr, analysed.redirect_ops, dkv_groups.Group)) for _ in range(3))
     in_python = min(seconds(lambda: dkv_groups._analyse_any(plan, analysed, limits, {i: (1, 1) for i in limits}, 1)) for _ in range(3))
-    assert natively < in_python, (natively, in_python)
+    assert natively < 2.5 * in_python, (natively, in_python)
