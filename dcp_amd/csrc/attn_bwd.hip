@@ -132,7 +132,7 @@ struct DkvVisit {
 // piece is the dS of 64 keys x 32 queries of one head, 4 KiB, laid out as the lanes of this kernel
 // hold it: [16 keys][key][4-query group][16-query half][4 queries].
 template <int DTYPE, int D, bool WRITE_DS>
-__device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, int wg) {
+__device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, int wg, const int wave) {
   constexpr int BM = kBwdBM, BN = kDkvBN;
   constexpr int KS = D / 32;  // k-steps over the head dim
   constexpr int DB = D / 16;  // 16-dim blocks of dK^T / dV^T
@@ -155,9 +155,11 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   // on a step that is not unmasked, per wave: which of its 32 keys each of the step's queries does not see
   __shared__ __attribute__((aligned(16))) uint32_t closed_lds[kBwdThreads / 64][BM];
 
-  int tid = threadIdx.x;
+  // (the kernel that leaves no dS is at the register limit in its steps, so nothing of a lane is kept over them in it: its
+  // number is worked out here and at the end again; kept, with V's last step as it is, one register was spilled)
+  int tid = WRITE_DS ? threadIdx.x : wave * 64 + lane_here();
   asm volatile("" : "+v"(tid));  // (per item: what is derived from it is not kept through the item before)
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // this wave's 32 keys of the tile
+  const int w = WRITE_DS ? __builtin_amdgcn_readfirstlane(tid >> 6) : wave;  // this wave's 32 keys of the tile
   const int lane = tid & 63;
   const int n = lane & 15;  // the lane's key in each of the wave's two 16-key columns
   const int g = lane >> 4;  // and its four queries in each of a sub-step's two 16-query tiles
@@ -606,6 +608,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   // ---- dK and dV of the wave's keys are complete: scale, round, store ---------------------
   wait_loads();  // the last step's (unused) requests must land before the workgroup's LDS is released, or used again
   __syncthreads();
+  const int out_lane = WRITE_DS ? lane : lane_here(), out_n = out_lane & 15, out_g = out_lane >> 4;
   // (what the loop did not need is worked out from the item's number again)
   KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
   asm volatile("" : "+s"(wg));
@@ -634,11 +637,11 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
   uint16_t* const dk_dst = reinterpret_cast<uint16_t*>(where ? args.dk2 : args.dk);
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
-    const int token = first + kk * 16 + n;
+    const int token = first + kk * 16 + out_n;
     if (token >= end) continue;
     if (where == 2) {  // a part's share, to be added to the other parts' by a sum kernel
       const int64_t head_row = (int64_t)args.n_heads_kv * D;
-      float* dst = args.dkv_partials + ((int64_t)entry * args.block_size + token) * (2 * head_row) + (int64_t)out_head * D + 4 * g;
+      float* dst = args.dkv_partials + ((int64_t)entry * args.block_size + token) * (2 * head_row) + (int64_t)out_head * D + 4 * out_g;
 #pragma unroll
       for (int d = 0; d < DB; ++d) {
         *reinterpret_cast<f32x4*>(dst + d * 16) = dk_acc[d][kk] * scale;
@@ -647,7 +650,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
       continue;
     }
     if (args.dkv_wide) continue;
-    const int64_t off = entry_off + (int64_t)token * token_stride + 4 * g;
+    const int64_t off = entry_off + (int64_t)token * token_stride + 4 * out_g;
 #pragma unroll
     for (int d = 0; d < DB; ++d) {
       const f32x4 v = dv_acc[d][kk], k = dk_acc[d][kk] * scale;
@@ -674,17 +677,17 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
 #pragma unroll
       for (int d = 0; d < DB; ++d) {
         const f32x4 x = matrix == 0 ? dv_acc[d][kk] : dk_acc[d][kk] * scale;
-        *(lds_u32x2*)(at + (kk * 16 + n) * ROW + d * 32 + g * 8) = u32x2{pack2<DTYPE>(x[0], x[1]), pack2<DTYPE>(x[2], x[3])};
+        *(lds_u32x2*)(at + (kk * 16 + out_n) * ROW + d * 32 + out_g * 8) = u32x2{pack2<DTYPE>(x[0], x[1]), pack2<DTYPE>(x[2], x[3])};
       }
     // (other lanes of the wave read it: see closed_lds)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    uint16_t* dst = (matrix == 0 ? dv_dst : dk_dst) + entry_off + (lane % PER_ROW) * 8;
+    uint16_t* dst = (matrix == 0 ? dv_dst : dk_dst) + entry_off + (out_lane % PER_ROW) * 8;
 #pragma unroll
     for (int i = 0; i < 32 / ROWS; ++i) {
-      const int key = i * ROWS + lane / PER_ROW;
-      const u32x4 x = *(lds_u32x4*)(at + key * ROW + (lane % PER_ROW) * 16);
+      const int key = i * ROWS + out_lane / PER_ROW;
+      const u32x4 x = *(lds_u32x4*)(at + key * ROW + (out_lane % PER_ROW) * 16);
       if (first + key < end) *reinterpret_cast<u32x4*>(dst + (int64_t)(first + key) * token_stride) = x;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -700,6 +703,7 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
 template <int DTYPE, int D, bool WRITE_DS>
 __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const AttnBwdParams p) {
   __shared__ int ticket_lds;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int item = 0;
   {
     KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
@@ -709,7 +713,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_dkv_kernel(const Attn
     KernArgs<AttnBwdParams>& args = fresh_kernel_args<AttnBwdParams>();
     if (item < 0) item = next_item({args.dkv_tickets, kTicketStride, args.n_dkv_items, args.dkv_xcd_group}, &ticket_lds);
     if (item < 0) break;
-    attn_bwd_dkv_item<DTYPE, D, WRITE_DS>(args, item);
+    attn_bwd_dkv_item<DTYPE, D, WRITE_DS>(args, item, wave);
     item = -1;
   }
 }

@@ -1,10 +1,17 @@
-"""The native plan analysis is an optional part of the build, for this Python alone (CPU)."""
+"""The build: the native plan analysis is an optional part of it, for this Python alone; what the compiler made of the
+kernels (CPU)."""
 
 import importlib.machinery
+import struct
+import subprocess
+from pathlib import Path
 
 import pytest
+import yaml
 
 from dcp_amd import build
+
+READELF = Path(build.HIPCC).resolve().parents[1] / "lib" / "llvm" / "bin" / "llvm-readelf"
 
 
 @pytest.fixture
@@ -32,3 +39,33 @@ def test_a_build_without(elsewhere, monkeypatch, what):
     with pytest.warns(RuntimeWarning, match="without the native plan analysis"):
         assert build.build_plan_analysis(verbose=False) is None
     assert list(elsewhere.iterdir()) == []
+
+
+def _kernels(library: Path, where: Path):
+    """What the code objects in a library say of their kernels."""
+    data, magic, found = library.read_bytes(), b"__CLANG_OFFLOAD_BUNDLE__", {}
+    at = data.find(magic)
+    while at >= 0:
+        n, entry = struct.unpack_from("<Q", data, at + len(magic))[0], at + len(magic) + 8
+        for _ in range(n):
+            offset, size, name_size = struct.unpack_from("<3Q", data, entry)
+            name = data[entry + 24 : entry + 24 + name_size]
+            entry += 24 + name_size
+            if name.startswith(b"hip") and size:
+                (where / "code_object").write_bytes(data[at + offset : at + offset + size])
+                notes = subprocess.run([READELF, "--notes", str(where / "code_object")], capture_output=True, text=True, check=True).stdout
+                metadata = yaml.safe_load(notes[notes.index("---") : notes.index("\n...")])
+                found.update({k[".name"]: k for k in metadata["amdhsa.kernels"]})
+        at = data.find(magic, at + 1)
+    return found
+
+
+def test_no_kernel_spills_vector_registers(tmp_path):
+    """A reload from scratch memory waits for every global load in flight, the tiles requested a step ahead among them."""
+    if not build.LIB_PATH.exists():
+        build.build(verbose=False)
+    kernels = _kernels(build.LIB_PATH, tmp_path)
+    for name in ("attn_fwd_kernel", "attn_bwd_dkv_kernel", "attn_bwd_dq_kernel", "attn_bwd_dq_ds_kernel", "attn_bwd_fused_kernel"):
+        assert sum(name in k for k in kernels) >= 2
+    assert {name: k[".private_segment_fixed_size"] for name, k in kernels.items()
+            if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]} == {}
