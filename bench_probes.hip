@@ -66,11 +66,12 @@ __global__ __launch_bounds__(kProbeThreads, 1) void mfma_probe_kernel(const u32x
 
 // What the matrix cores sustain when every wave also issues, evenly spread between its MFMAs and
 // with no dependency on anything loaded, the other instructions an attention kernel needs per
-// NM MFMAs: NV plain vector instructions (FMAs), NE exponentials, NB128 16-byte and NB64 8-byte LDS
-// reads per lane.  Two workgroups per CU (64 KiB of LDS each), i.e. two waves per SIMD, like the
-// attention kernels.  No tile loads, no barriers, no waits on data: an upper bound for a kernel
-// with that instruction mix, whatever its schedule.
-template <int NM, int NV, int NE, int NB128, int NB64>
+// NM MFMAs (32x32x16, or 16x16x32 with SMALL): NV plain vector instructions (FMAs), NE exponentials, NB128 16-byte and
+// NB64 8-byte LDS reads per lane.  Two workgroups per CU (64 KiB of LDS each), i.e. two waves per SIMD, like the
+// attention kernels.  No tile loads, no barriers, no waits on data but for an LDS read RING
+// reads before: what the device sustains of that instruction mix, to a few per cent for how it is spread (65536 causal
+// tokens: the dK/dV kernel runs at 0.70 of it, the forward at 0.79).
+template <bool SMALL, int NM, int NV, int NE, int NB128, int NB64>
 __global__ __launch_bounds__(kProbeThreads, 2) void mfma_mix_probe_kernel(const u32x4* operands, float* out, int iters,
                                                                          float s, float t) {
   __shared__ __attribute__((aligned(16))) u32x4 lds[4096];  // 64 KiB: two workgroups per CU
@@ -78,51 +79,72 @@ __global__ __launch_bounds__(kProbeThreads, 2) void mfma_mix_probe_kernel(const 
   __syncthreads();
   const size_t base = ((size_t)blockIdx.x * kProbeThreads + threadIdx.x) * 16;
   const u32x4 a = operands[base], b = operands[base + 8];
-  f32x16 acc[4];
+  typedef typename std::conditional<SMALL, f32x4, f32x16>::type Acc;
+  constexpr int NA = SMALL ? 16 : 4, N_ELEM = sizeof(Acc) / 4;  // accumulators in turn
+  Acc acc[NA];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < NA; ++j)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[j][i] = 0.0f;
+    for (int i = 0; i < N_ELEM; ++i) acc[j][i] = 0.0f;
   float x[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) x[i] = threadIdx.x * 0.001f + i * 0.01f;
-  const uint32_t at = lds_address(&lds[0]) + (threadIdx.x & 63) * 16;
+  typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+  typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+  uint32_t at = lds_address(&lds[0]) + (threadIdx.x & 63) * 16;
+  constexpr int RING = 8;  // reads in flight, of each kind
+  u32x4 wide[RING];
+  u32x2 narrow[RING];
+#pragma unroll
+  for (int i = 0; i < RING; ++i) {
+    wide[i] = u32x4{0, 0, 0, 0};
+    narrow[i] = u32x2{0, 0};
+  }
   for (int it = 0; it < iters; ++it) {
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-      acc[m & 3] = mfma_32x32x16<DCP_DTYPE_BF16>(a, b, acc[m & 3]);
+      if constexpr (SMALL) acc[m % NA] = mfma_16x16x32<DCP_DTYPE_BF16>(a, b, acc[m % NA]);
+      else acc[m % NA] = mfma_32x32x16<DCP_DTYPE_BF16>(a, b, acc[m % NA]);
       // the m-th share of each kind: floor((m + 1) N / NM) - floor(m N / NM) instructions
+      // (the empty asm holds them here: the compiler moved them all behind the last MFMA)
 #pragma unroll
-      for (int k = m * NV / NM; k < (m + 1) * NV / NM; ++k) x[k & 15] = __builtin_fmaf(x[k & 15], s, t);
+      for (int k = m * NV / NM; k < (m + 1) * NV / NM; ++k) {
+        x[k & 15] = __builtin_fmaf(x[k & 15], s, t);
+        asm volatile("" : "+v"(x[k & 15]));
+      }
 #pragma unroll
-      for (int k = m * NE / NM; k < (m + 1) * NE / NM; ++k) x[k & 15] = fast_exp2(x[k & 15]);
+      for (int k = m * NE / NM; k < (m + 1) * NE / NM; ++k) {
+        x[k & 15] = fast_exp2(x[k & 15]);
+        asm volatile("" : "+v"(x[k & 15]));
+      }
+      // (a read's register is given up where the read RING after it goes into it: the asm is that use, and makes the
+      // address one that the next read cannot share)
 #pragma unroll
       for (int k = m * NB128 / NM; k < (m + 1) * NB128 / NM; ++k) {
-        u32x4 v;
-        asm volatile("ds_read_b128 %0, %1 offset:1024" : "=v"(v) : "v"(at));
-        asm volatile("" ::"v"(v));
+        asm volatile("" : "+v"(at) : "v"(wide[k % RING]));
+        wide[k % RING] = *(lds_u32x4*)(at + 1024);
       }
 #pragma unroll
       for (int k = m * NB64 / NM; k < (m + 1) * NB64 / NM; ++k) {
-        u32x2 v;
-        asm volatile("ds_read_b64 %0, %1 offset:2048" : "=v"(v) : "v"(at));
-        asm volatile("" ::"v"(v));
+        asm volatile("" : "+v"(at) : "v"(narrow[k % RING]));
+        narrow[k % RING] = *(lds_u32x2*)(at + 2048);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    asm volatile("s_waitcnt lgkmcnt(0)");
     if ((it & 63) == 63) {  // keep the sums finite
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < NA; ++j)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[j][i] *= 1e-6f;
+        for (int i = 0; i < N_ELEM; ++i) acc[j][i] *= 1e-6f;
     }
   }
+#pragma unroll
+  for (int i = 0; i < RING; ++i) asm volatile("" ::"v"(wide[i]), "v"(narrow[i]));
   float r = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < NA; ++j)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) r += acc[j][i];
+    for (int i = 0; i < N_ELEM; ++i) r += acc[j][i];
 #pragma unroll
   for (int i = 0; i < 16; ++i) r += x[i];
   out[2 + (size_t)blockIdx.x * kProbeThreads + threadIdx.x] = r;
@@ -222,27 +244,28 @@ extern "C" int bench_mfma_probe(const void* operands, float* out, int n_workgrou
 
 
 // The MFMA probe with an attention kernel's other instructions beside the MFMAs (see
-// mfma_mix_probe_kernel): `mix` 0 = forward (per 32 MFMAs: 112 FMAs, 32 exponentials, 16 + 32 LDS
-// reads), 1 = dK/dV kernel (per 32: 58, 16, 20 + 32), 2 = dQ kernel (per 48: 80, 32, 32 + 32).
+// mfma_mix_probe_kernel): `mix` 0 = forward (per 32 32x32x16 MFMAs: 112 FMAs, 32 exponentials, 16 + 32 LDS
+// reads), 1 = dK/dV kernel (per 64 16x16x32 ones, a sub-step without a mask: 72, 16, 22 + 32), 2 = dQ kernel that
+// recomputes S and dP (per 48 32x32x16 ones: 80, 32, 32 + 32).
 // `n_workgroups` workgroups of 256 threads, two per CU; `operands` and `out` as for
 // bench_mfma_probe (at least 4096 x 16 bytes of operands).  *flop = the MFMAs' operations.
 extern "C" int bench_mfma_mix_probe(const void* operands, float* out, int n_workgroups, int iters, int mix, double* flop,
                                     void* stream) {
   DCP_REQUIRE(operands && out && flop, "mfma_mix_probe: null argument");
   DCP_REQUIRE(n_workgroups >= 16 && iters > 0, "mfma_mix_probe: at least 16 workgroups and one iteration");
-  const int per_iter = mix == 2 ? 48 : 32;
-  *flop = (double)n_workgroups * (kProbeThreads / 64) * (double)iters * per_iter * (2.0 * 32 * 32 * 16);
+  const double flop_per_iter = mix == 2 ? 48 * (2.0 * 32 * 32 * 16) : mix == 1 ? 64 * (2.0 * 16 * 16 * 32) : 32 * (2.0 * 32 * 32 * 16);
+  *flop = (double)n_workgroups * (kProbeThreads / 64) * (double)iters * flop_per_iter;
   dim3 grid(n_workgroups), block(kProbeThreads);
   const u32x4* ops = (const u32x4*)operands;
   switch (mix) {
     case 0:
-      hipLaunchKernelGGL((mfma_mix_probe_kernel<32, 112, 32, 16, 32>), grid, block, 0, (hipStream_t)stream, ops, out, iters, 1.0001f, 0.5f);
+      hipLaunchKernelGGL((mfma_mix_probe_kernel<false, 32, 112, 32, 16, 32>), grid, block, 0, (hipStream_t)stream, ops, out, iters, 1.0001f, 0.5f);
       break;
     case 1:
-      hipLaunchKernelGGL((mfma_mix_probe_kernel<32, 58, 16, 20, 32>), grid, block, 0, (hipStream_t)stream, ops, out, iters, 1.0001f, 0.5f);
+      hipLaunchKernelGGL((mfma_mix_probe_kernel<true, 64, 72, 16, 22, 32>), grid, block, 0, (hipStream_t)stream, ops, out, iters, 1.0001f, 0.5f);
       break;
     case 2:
-      hipLaunchKernelGGL((mfma_mix_probe_kernel<48, 80, 32, 32, 32>), grid, block, 0, (hipStream_t)stream, ops, out, iters, 1.0001f, 0.5f);
+      hipLaunchKernelGGL((mfma_mix_probe_kernel<false, 48, 80, 32, 32, 32>), grid, block, 0, (hipStream_t)stream, ops, out, iters, 1.0001f, 0.5f);
       break;
     default:
       return fail(DCP_ERR_UNSUPPORTED, "mfma_mix_probe: mix %d unsupported (0, 1 or 2)", mix);
