@@ -64,14 +64,7 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 // below 2^-126 flush to zero, which is what a softmax weight that small is).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// The value the other half of the wave holds (lane ^ 32), by one register swap on the vector
-// unit (no trip through LDS).
-__device__ __forceinline__ float xor32(float x) {
-  const unsigned u = __float_as_uint(x);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // {lanes 0-31 twice, lanes 32-63 twice}
-  return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
-}
-// max / sum over the two halves, the same in both
+// max / sum over the two halves of a wave, the same in both (one register swap on the vector unit, no trip through LDS)
 __device__ __forceinline__ float halves_max(float x) {
   const unsigned u = __float_as_uint(x);
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
@@ -81,18 +74,6 @@ __device__ __forceinline__ float halves_sum(float x) {
   const unsigned u = __float_as_uint(x);
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// max / sum over the four 16-lane quarters of a wave, the same in all of them
-__device__ __forceinline__ float quarters_max(float x) {
-  const unsigned u = __float_as_uint(x);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // {quarters 0 0 2 2, quarters 1 1 3 3}
-  return halves_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
-}
-__device__ __forceinline__ float quarters_sum(float x) {
-  const unsigned u = __float_as_uint(x);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return halves_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
 // Minimum / maximum over the wave, as a scalar.  Four DPP steps (row_shr 1, 2, 4, 8) leave each
@@ -117,22 +98,6 @@ __device__ __forceinline__ int wave_reduce_minmax(int x) {
 }
 __device__ __forceinline__ int wave_min(int x) { return wave_reduce_minmax<true>(x); }
 __device__ __forceinline__ int wave_max(int x) { return wave_reduce_minmax<false>(x); }
-
-// Row index (within a 32-row MFMA tile) of accumulator element i for a lane
-// in half h.
-__device__ __forceinline__ constexpr int acc_row(int i, int h) {
-  return 8 * (i / 4) + 4 * h + (i % 4);
-}
-
-// Position, inside a group of 16 contraction indices stored contiguously in
-// LDS, of the 4-index subgroup r (indices 4r..4r+3), chosen so that a lane in
-// half h reads its 8 k-slots {4h..4h+3, 8+4h..8+4h+3} with one 16-byte load at
-// position 8h.  These are exactly the rows a lane holds in accumulator
-// elements 0..7 of a 32x32 tile, so an accumulator feeds the next MFMA as its
-// B operand without any cross-lane movement.
-__device__ __forceinline__ constexpr int kslot_pos(int r) {
-  return r == 0 ? 0 : r == 1 ? 8 : r == 2 ? 4 : 12;
-}
 
 // ---------------------------------------------------------------------------
 // LDS tile of 64 rows x D 16-bit elements, filled by NW waves straight from global memory
@@ -228,38 +193,7 @@ struct KvTile {
     return D == 128 ? 16 * pos + 4 * swap(grp & 3) + (grp >> 2)
                     : 16 * (pos >> 1) + 4 * swap(grp & 3) + 2 * (pos & 1) + (grp >> 2);
   }
-  // Byte offsets, from (row 0, the head's first element), of what this lane
-  // fetches in each of its wave's group loads.  Loop-invariant.
-  __device__ static __forceinline__ void lane_offsets(uint32_t (&off)[LPW], int64_t row_stride, int wave, int lane) {
-    constexpr int CH = D / 8;
-#pragma unroll
-    for (int i = 0; i < LPW; ++i)
-      off[i] = (uint32_t)((row_of(wave * LPW + i, lane / CH) * row_stride + (lane % CH) * 8) * 2);
-  }
-  // `g` (wave-uniform) points at (row 0, the head's first element) of the tile.
-  //
-  // The load is written as assembly on purpose.  Through the builtin the compiler sees
-  // an instruction that touches both global memory and LDS, and as long as one is in
-  // flight it turns every LDS wait of the wave into a wait for ALL outstanding LDS
-  // reads (lgkmcnt(0)), which serialises operand prefetch with the MFMAs for the whole
-  // time a tile is streaming in, i.e. always.  Here the compiler tracks nothing, so the
-  // kernels must (and do) order these loads themselves: s_waitcnt vmcnt(0) and a
-  // workgroup barrier between a load and the first read of its stage, a barrier between
-  // the last read of a stage and the load that refills it.
-  // `tile_at` is the tile's LDS byte address (lds_address() of the array).
-  __device__ static __forceinline__ void load_async(uint32_t tile_at, const uint16_t* g, const uint32_t (&off)[LPW],
-                                                    int wave) {
-    const char* gb = reinterpret_cast<const char*>(g);
-#pragma unroll
-    for (int i = 0; i < LPW; ++i) {
-      const uint32_t lds_at = __builtin_amdgcn_readfirstlane(tile_at + (wave * LPW + i) * GROUP_STRIDE * 2);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                   :
-                   : "s"(lds_at), "v"(gb + off[i])
-                   : "memory");
-    }
-  }
-  // The same loads one at a time, so that a kernel can spread them between its matrix
+  // A wave fills its groups of a tile one load at a time, so that a kernel can spread them between its matrix
   // instructions instead of issuing a burst (a burst fills the memory pipeline's queue
   // and the wave sits at the last load until the queue drains).  The rows of
   // load i lie LOAD_ROWS*i rows below those of load 0, so one per-lane byte offset
@@ -270,7 +204,17 @@ struct KvTile {
     static_assert((LPW & (LPW - 1)) == 0 && LPW <= 4, "group loads of a wave must not carry into grp >> 2");
     return (uint32_t)((row_of(wave * LPW, lane / CH) * row_stride + (lane % CH) * 8) * 2);
   }
-  // `g` (wave-uniform) points at (row 0, the head's first element) of the tile.
+  // `tile_at` is the tile's LDS byte address (lds_address() of the array), `g` (wave-uniform) points at (row 0, the
+  // head's first element) of the tile.
+  //
+  // The loads are written as assembly on purpose.  Through the builtin the compiler sees
+  // an instruction that touches both global memory and LDS, and as long as one is in
+  // flight it turns every LDS wait of the wave into a wait for ALL outstanding LDS
+  // reads (lgkmcnt(0)), which serialises operand prefetch with the MFMAs for the whole
+  // time a tile is streaming in, i.e. always.  Here the compiler tracks nothing, so the
+  // kernels must (and do) order these loads themselves: s_waitcnt vmcnt(0) and a
+  // workgroup barrier between a load and the first read of its stage, a barrier between
+  // the last read of a stage and the load that refills it.
   __device__ static __forceinline__ void load_group(uint32_t tile_at, const uint16_t* g, uint32_t off0,
                                                     int64_t row_stride, int wave, int i) {
     const uint32_t lds_at = __builtin_amdgcn_readfirstlane(group_lds_at(tile_at, wave, i));
@@ -572,9 +516,6 @@ __device__ __forceinline__ KeyRange key_range(int start, int end, int seqlen_kv)
 
 struct RangePair {
   int s0, len0, s1, len1;  // of each range, see KeyRange
-  __device__ __forceinline__ bool contains(int k) const {
-    return ((unsigned)(k - s0) < (unsigned)len0) | ((unsigned)(k - s1) < (unsigned)len1);
-  }
   // Bit p set = key base + p (p = 0..31) lies in neither range.  A dozen vector instructions
   // for a 32-key window, after which an accumulator's initial value costs two (masked_start)
   // where a range test per element costs seven.
