@@ -18,7 +18,6 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <map>
 #include <memory>
 #include <new>
 #include <utility>
@@ -494,7 +493,7 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
   Instrs instrs(instr_list, kind_list);
   const Seq limits(limit_list);  // rows a group may visit, per instruction
   if (limits.n != instrs.size()) throw NotTaken();
-  std::map<std::pair<int64_t, int64_t>, PyObject*> redirects;  // sum instruction and position of the op -> where it goes
+  std::vector<SlotMap<PyObject*>> redirects(instrs.size(), SlotMap<PyObject*>(nullptr));  // sum -> position of an op -> where it goes
   {
     auto for_each = [](PyObject* dict, auto&& body) {  // (a lookup would compare its keys, with their own code)
       if (!PyDict_CheckExact(dict)) throw NotTaken();
@@ -503,7 +502,10 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
       while (PyDict_Next(dict, &at, &key, &value)) body(integer(key), value);
     };
     for_each(redirect_ops, [&](int64_t instr, PyObject* of_instr) {
-      for_each(of_instr, [&](int64_t pos, PyObject* dst) { redirects[{instr, pos}] = dst; });
+      for_each(of_instr, [&](int64_t pos, PyObject* dst) {
+        if (instr < 0 || instr >= instrs.size() || pos < 0 || pos >= kMaxIndex) throw NotTaken();
+        redirects[instr].set(pos, dst);
+      });
     });
   }
   Reader reader;
@@ -672,8 +674,7 @@ PyObject* dkv(PyObject* instr_list, PyObject* kind_list, PyObject* limit_list, P
       const SumOf& sum = sums[t.who];
       const Seq sources = op_sources(sum.op, sum_op_type);
       const int rows = (int)t.taken.size();
-      PyObject* dst = nullptr;  // where the sum goes, if that is an unpadded tensor
-      if (const auto known = redirects.find({sum.instr, sum.pos}); known != redirects.end()) dst = known->second;
+      PyObject* dst = redirects[sum.instr].get(sum.pos);  // where the sum goes, if that is an unpadded tensor
       if (dst == nullptr && instrs.flag(sum.instr, "output_is_unpadded")) dst = field(sum.op, s_dst_buffer);
       if (rows <= limit && rows == sources.n && dst != nullptr) {
         const Block to = reader.block(dst);
