@@ -47,7 +47,8 @@
 // What bounds it on a full device is power: the clock falls to what the chip's limit allows, 1.49 GHz in this kernel
 // with 32x32x16 products (65536 causal tokens, 32 heads; 2.4-2.5 in a launch that leaves the device half empty), so
 // what counts is energy.  16x16x32 products move half the accumulators: 1.62 GHz, 8.05 -> 7.93 ms with 7 % more cycles
-// (an instruction more per 32 K operations), and the dQ kernel beside it 3.07 -> 3.00.  A launch of few, lone waves has
+// (an instruction more per 32 K operations; 7.7 ms with 4 % more since a workgroup's ends are shorter), and the dQ
+// kernel beside it 3.07 -> 3.00.  A launch of few, lone waves has
 // those cycles and no such clock: 4800 tokens, 8 kv heads, blocks of 1024, 68.6 -> 72 us.  The range mask enters S as the
 // accumulator's initial value (0 or -inf; a bit per key and query, worked out once a step).  dK/dV of a key never leave the wave
 // until the end, so the per-(row, kv block) private dKV blocks of the plan need
@@ -426,8 +427,8 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     const uint64_t ds_chunk_bytes = (uint64_t)ds_row_tiles << 12;
 
     // The range test of a masked step, a lane a query: 32 keys in a dozen vector instructions, left as a bit
-    // mask that the lanes, which hold a key each, read back for their sixteen queries at a time.  Every lane
-    // testing its key against every query's ranges was ten instructions an element, 320 a step, behind 32
+    // mask that the lanes read back for the eight queries they hold of a sub-step, at each of their two keys.  Every lane
+    // testing a key against every query's ranges was ten instructions an element, 320 a step, behind 32
     // reads of LDS.  Backward, us: 5269 tokens in shared prefixes, 40 heads, 685 -> 522; 12678 tokens, 8 heads,
     // 341 -> 293; 4128 tokens 128 -> 111; 131072 tokens, window 4096, 21930 -> 21740; 65536 causal 11440 -> 11370
     // (runs of one build differ by 50).
@@ -661,9 +662,9 @@ __device__ __forceinline__ void attn_bwd_dkv_item(KernArgs<AttnBwdParams>& p, in
     }
   }
   if (where == 2 || !args.dkv_wide) return;
-  // A lane has four dims of a key, so its stores are eight bytes, 32 contiguous ones a key, and there are 64 of them a wave:
-  // 4.2 us at the end of every workgroup.  Through LDS (where the tiles were, a part of it to each wave) they
-  // become a quarter as many of whole rows, 1-2.
+  // A lane has four dims of a key, so its stores are eight bytes, 32 contiguous ones a key, and there are 32 of them a wave (16 at
+  // head size 64): 4.2 us at the end of every workgroup.  Through LDS (where the tiles were, a part of it to each wave) they
+  // become half as many, of whole rows, 1-2.
   constexpr int ROW = D * 2 + 16;        // bytes of a key in LDS; the padding spreads a lane's eight over the banks
   constexpr int PER_ROW = D * 2 / 16, ROWS = 64 / PER_ROW;  // lanes that store a key's row, keys in a store
   static_assert(4 * 32 * ROW <= (int)sizeof(tiles), "a matrix of every wave fits where the tiles were");

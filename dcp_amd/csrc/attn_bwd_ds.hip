@@ -33,9 +33,11 @@
 // or six (64) stages, where a launch leaves CUs idle, are no faster either: backward of 40 items 45.6 -> 45.8 us, of 144
 // 122.4 -> 122.4, of 176 of head size 64 72.0 -> 78.4, of 448 262 -> 289.  A kernel that only
 // streams 4 KiB pieces per wave into LDS the same way reads 7.0 TB/s (6.6 with a workgroup barrier
-// per step, 6.0-6.2 with a K tile's loads beside it); the rest is the start of every work item (a
-// chain of dependent table reads and an empty pipeline: with no tiles at all the kernel takes
-// 0.21 ms, and every item waits once for its first tile).
+// per step, 6.0-6.2 with a K tile's loads beside it); the rest is the start of every work item (a trip to
+// memory for its tables and an empty pipeline: every item waits once for its first tile; when its tables were a chain of
+// trips, the kernel took 0.21 ms with no tiles at all).  The pieces are read from LDS 8 bytes a lane at a stride
+// of 16, which is half of the banks: with 65536 tokens a conflict cycle for every other MFMA, beside a stream that is
+// slower than either.
 #include <math.h>
 
 #include <algorithm>
@@ -100,7 +102,7 @@ __device__ __forceinline__ void attn_bwd_dq_ds_item(KernArgs<AttnBwdParams>& p, 
 
   // ---- which key tiles: the 128-key tiles the dK/dV kernel visited for this wave's 64-query tile
   // (the same test on the same hulls: a piece that was never written is never read), and for the
-  // workgroup the hull of its two 64-query tiles -----------------------------------------------
+  // workgroup the hull of its four 64-query tiles -----------------------------------------------
   const int own = w >> 1;  // of the item's 64-query tiles, the one this wave's queries lie in
   const bool wave_has_tile = T64 * qt + own < p.q_tiles_per_row;
   const TileRuns mine(__builtin_amdgcn_readlane(hulls, 4 * own), __builtin_amdgcn_readlane(hulls, 4 * own + 1),

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void attn_bwd_fused_kernel(const At
   const uint32_t qdo_at = lds_address(&qdo[0][0]);
   // A step's tile is one 64-row tile: Q of its 32 queries in rows 0..31, dO in rows 32..63, so a
   // group load takes its lanes 0..31 from Q and 32..63 from dO.  Per lane: which array, which of
-  // the 32 queries (group load i of the wave adds 4 i rows) and which 16 bytes of the row.
+  // the 32 queries (load i of the wave adds LOAD_ROWS * i rows) and which 16 bytes of the row.
   const char* lane_src;
   {
     constexpr int CH = D / 8;

@@ -473,8 +473,8 @@ __device__ __forceinline__ void attn_fwd_item(KernArgs<AttnFwdParams>& p, int it
   // pipe and the vector ALU of the SIMD are busy at the same time.  Operands are read
   // three ahead.  The softmax of a pair of elements goes through three stages an MFMA apart -- the argument of pair
   // c2 + 1, the exponential of pair c2, sum and packing of pair c2 - 1 -- so that no instruction waits for the one before
-  // it: 1024 tokens, 8 heads 23.4 -> 22.2 us, 1000 tokens 13.4 -> 13.1, 65536 causal tokens 3845 -> 3805, 32768 of
-  // head size 64 638 -> 635.
+  // it: 1024 tokens, 8 heads 23.4 -> 22.2 us, 1000 tokens 13.4 -> 13.1; large launches gain less than they vary by (65536
+  // causal tokens 0.8 % with the tables' reads above).
   auto multiply_qk_with_softmax = [&](const uint16_t* k_lds, f32x16 (&s_out)[2][QB], const f32x16 (&sc)[2][QB]) {
     constexpr int N = 2 * KS;     // operands, QB MFMAs each
     constexpr int AHEAD = 3;
